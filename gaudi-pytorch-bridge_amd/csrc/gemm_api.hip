@@ -1,5 +1,8 @@
 // fp8_gemm_v2 C entry point: argument checks, kernel choice, and the any-shape
 // fallback kernel.  The MFMA tile kernels live in gemm_tile.h.
+#include <algorithm>
+#include <cmath>
+
 #include "gemm_dispatch.h"
 
 namespace mi355q {
@@ -71,6 +74,45 @@ inline bool tiled_ok(const void* A, int trans_a, int64_t lda, const void* B, int
   return M > 0 && N > 0 && K > 0;
 }
 
+// The cut that is expected to take least.  The figures (microseconds, bytes per microsecond) are fits to 60 problems of 1 to
+// 128 rows, K from 2048 to 14336 and N from 1024 to 38400, most of which they meet within two microseconds:
+//  * a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where more of them run;
+//  * in the strip kernel A's tile travels along (a quarter of its bytes count with a K-major B, half with the shorter
+//    pieces of an MN-major one);
+//  * fixed costs, and with more than one part the meeting: each part's sums out, and all of them into the last one.
+SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+  SplitPlan best;
+  if (M > 128 || M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
+  const double cus = (double)compute_units();
+  double best_us = 0.0;
+  auto consider = [&](bool stream, int64_t nb, int64_t tile_rows, int64_t unit) {
+    const int64_t strips = (N + nb - 1) / nb, groups = strips * batch, units = (K + unit - 1) / unit;
+    const int64_t rows = M < 32 ? M : tile_rows;  // rows of sums that travel
+    const double width = (double)nb + (stream ? 0.0 : (double)tile_rows * (b_kmajor ? 0.25 : 0.5));
+    for (int64_t parts = 1; parts <= 32 && parts <= units; ++parts) {
+      if (parts > 1 && (!may_split || groups > kMaxTickets || (double)(groups * parts) > 2.0 * cus)) break;
+      const double wgs = (double)(groups * parts), rounds = std::ceil(wgs / cus);
+      const double rate = std::min(37e3, 6.5e6 / std::min(wgs, cus));
+      double us = rounds * (double)((units + parts - 1) / parts * unit) * width / rate + 4.5;
+      if (parts > 1)
+        us += stream ? 0.5 + 0.2 * (double)parts + (double)rows * (0.15 + 0.005 * (double)parts)
+                     : 2.0 + 0.25 * (double)parts + ((double)parts + 1.5) * (double)(rows * nb * 4) / 50e3;
+      if (best.nb != 0 && us >= best_us) continue;
+      best_us = us;
+      best.stream = stream;
+      best.nb = (int)nb;
+      best.strips = (int)strips;
+      best.parts = (int)parts;
+      best.tile_rows = tile_rows;
+      best.batch = batch;
+    }
+  };
+  // (the stream kernel addresses an operand with 31-bit offsets)
+  if (a_kmajor && !b_kmajor && M <= 16 && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) consider(true, 256, 16, 256);
+  consider(false, 128, !a_kmajor ? 128 : (M <= 32 ? 32 : (M <= 64 ? 64 : 128)), kBK);
+  return best;
+}
+
 }  // namespace mi355q
 
 using namespace mi355q;
@@ -87,8 +129,15 @@ const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64
       case mi355q::TileChoice::k128x128: return "tile128x128x128_mfma32x32x64";
     }
   }
+  if (mi355q::split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, 1, true).stream) return "stream_Mx256_registers_mfma16x16";
   if (M <= 128) return "strip_Mx128x128_ring_mfma32x32x64";
   return "tile128x128x128_mfma32x32x64";
+}
+
+size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                       int64_t batch) {
+  if (lda % 16 || ldb % 16 || !k_chunks_ok(trans_a, trans_b, K)) return 0;
+  return batch > 65535 ? 0 : split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, true).workspace_bytes();
 }
 
 int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
@@ -98,6 +147,18 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const vo
                     int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
                     int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
                     int64_t stride_bias, void* stream) {
+  return mi355q_fp8_gemm_ws(A, fmt_a, trans_a, lda, B, fmt_b, trans_b, ldb, C, out_dtype, ldc, M, N, K, sa_dev, sa_host,
+                            sa_mode, sb_dev, sb_host, sb_mode, bias, bias_mode, ldbias, D, ldd, batch, stride_a, stride_b,
+                            stride_c, stride_d, stride_bias, nullptr, 0, stream);
+}
+
+int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
+                       int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
+                       int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
+                       const float* sb_dev, float sb_host, int sb_mode, const void* bias,
+                       int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
+                       int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
+                       int64_t stride_bias, void* workspace, size_t workspace_bytes, void* stream) {
   auto fmt_ok = [](int f) { return f == MI355Q_E4M3FN || f == MI355Q_E5M2; };
   auto mode_ok = [](int m, const float* p) {
     if (m < MI355Q_GS_NONE || m > MI355Q_GS_PER_COL) return false;
@@ -154,10 +215,19 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const vo
     gb.fast_epi = epilogue_fast_ok(gb, nb);
     if (tiled_ok(gb.A, trans_a, lda, gb.B, trans_b, ldb, M, N, K, stride_a, stride_b)) {
       const bool ak = !trans_a, bk = trans_b != 0;
-      if (ak && bk) launch_gemm_kk(gb, fmt_a, fmt_b, nb, st);
-      else if (ak) launch_gemm_km(gb, fmt_a, fmt_b, nb, st);
-      else if (bk) launch_gemm_mk(gb, fmt_a, fmt_b, nb, st);
-      else launch_gemm_mm(gb, fmt_a, fmt_b, nb, st);
+      // (few rows: K is walked in parts if the caller brought the room where they meet)
+      const SplitPlan plan = split_plan(ak, lda, bk, ldb, M, N, K, nb, workspace != nullptr && nb == batch);
+      SplitArgs split{plan.parts, nullptr, nullptr};
+      if (plan.parts > 1) {
+        if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;
+        split.tickets = static_cast<uint32_t*>(workspace);
+        split.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
+      }
+      if (plan.stream) launch_gemm_stream(gb, fmt_a, fmt_b, plan, split, nb, st);
+      else if (ak && bk) launch_gemm_kk(gb, split, fmt_a, fmt_b, nb, st);
+      else if (ak) launch_gemm_km(gb, split, fmt_a, fmt_b, nb, st);
+      else if (bk) launch_gemm_mk(gb, split, fmt_a, fmt_b, nb, st);
+      else launch_gemm_mm(gb, split, fmt_a, fmt_b, nb, st);
     } else {
       const int64_t a_sm = trans_a ? 1 : lda, a_sk = trans_a ? lda : 1;
       const int64_t b_sk = trans_b ? 1 : ldb, b_sn = trans_b ? ldb : 1;

@@ -80,7 +80,7 @@ void launch_256x256(const GemmArgs& g, int64_t batch, hipStream_t st) {
 }
 
 template <bool AK, bool BK_, int FA, int FB>
-void launch_by_size(const GemmArgs& g, int64_t batch, hipStream_t st) {
+void launch_by_size(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
   if (g.M > 128 && g.N > 128) {
     switch (choose_tiles(g.M, g.N, batch)) {
       case TileChoice::k256x256: {
@@ -101,7 +101,7 @@ void launch_by_size(const GemmArgs& g, int64_t batch, hipStream_t st) {
       case TileChoice::k128x128: launch_tile<128, 128, 4, false, AK, BK_, FA, FB, 2>(g, batch, st); break;
     }
   } else if (g.M <= 128) {
-    launch_skinny_by_m<AK, BK_, FA, FB>(g, batch, st);
+    launch_skinny_by_m<AK, BK_, FA, FB>(g, split, batch, st);
   } else {
     launch_tile<128, 128, 4, false, AK, BK_, FA, FB, 2>(g, batch, st);
   }
@@ -109,11 +109,20 @@ void launch_by_size(const GemmArgs& g, int64_t batch, hipStream_t st) {
 
 // One translation unit per operand layout instantiates this (gemm_inst_*.hip).
 template <bool AK, bool BK_>
-void launch_by_format(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st) {
-  if (fmt_a == MI355Q_E4M3FN && fmt_b == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E4M3FN, MI355Q_E4M3FN>(g, batch, st);
-  else if (fmt_a == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E4M3FN, MI355Q_E5M2>(g, batch, st);
-  else if (fmt_b == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E5M2, MI355Q_E4M3FN>(g, batch, st);
-  else launch_by_size<AK, BK_, MI355Q_E5M2, MI355Q_E5M2>(g, batch, st);
+void launch_by_format(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st) {
+  if (fmt_a == MI355Q_E4M3FN && fmt_b == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E4M3FN, MI355Q_E4M3FN>(g, split, batch, st);
+  else if (fmt_a == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E4M3FN, MI355Q_E5M2>(g, split, batch, st);
+  else if (fmt_b == MI355Q_E4M3FN) launch_by_size<AK, BK_, MI355Q_E5M2, MI355Q_E4M3FN>(g, split, batch, st);
+  else launch_by_size<AK, BK_, MI355Q_E5M2, MI355Q_E5M2>(g, split, batch, st);
 }
+
+// A K-major / B K-major etc.; defined in gemm_inst_*.hip
+void launch_gemm_kk(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+void launch_gemm_km(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+void launch_gemm_mk(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+void launch_gemm_mm(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+
+// K-major A, MN-major B, few rows; defined in gemm_stream.hip
+void launch_gemm_stream(const GemmArgs& g, int fmt_a, int fmt_b, const SplitPlan& p, const SplitArgs& split, int64_t batch, hipStream_t st);
 
 }  // namespace mi355q

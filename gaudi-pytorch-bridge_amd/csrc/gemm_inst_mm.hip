@@ -2,7 +2,7 @@
 #include "gemm_dispatch.h"
 
 namespace mi355q {
-void launch_gemm_mm(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st) {
-  launch_by_format<false, false>(g, fmt_a, fmt_b, batch, st);
+void launch_gemm_mm(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st) {
+  launch_by_format<false, false>(g, split, fmt_a, fmt_b, batch, st);
 }
 }  // namespace mi355q

@@ -9,10 +9,13 @@
 // multiplies the whole A tile by its own 32 columns; fragments are read right
 // before use (the matrix pipes are mostly idle anyway).
 //
+// Where the strips alone leave compute units idle (N = 4096: 32 strips for 256 units), K is cut into parts walked
+// by a workgroup each, whose sums meet through the caller's workspace (gemm_split.h); SplitPlan says how.
+//
 // The global->LDS loads, LDS geometry, fragment reads and epilogues are those
 // of the large-tile kernel (gemm_tile.h).
 #pragma once
-#include "gemm_tile.h"
+#include "gemm_split.h"
 
 namespace mi355q {
 
@@ -28,7 +31,7 @@ constexpr int skinny_stages() {
 }
 
 template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
-__global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g) {
+__global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g, SplitArgs split) {
   constexpr int MT = BM / 32;
   constexpr int S = skinny_stages<BM>();
   constexpr int kStageBytes = (BM + kSkBN) * kBK;
@@ -42,7 +45,14 @@ __global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g)
   __shared__ __attribute__((aligned(1024))) uint8_t lds[S * kStageBytes];
 
   const int64_t batch = blockIdx.y;
-  const int n0 = blockIdx.x * kSkBN;
+  const int strips = g.tiles_n, strip = blockIdx.x % strips, part = blockIdx.x / strips;
+  const int n0 = strip * kSkBN;
+  // this workgroup's part of K, whole stages
+  const int kt_all = (g.K + kBK - 1) / kBK;
+  const int kt0 = (int)((int64_t)part * kt_all / split.parts), kt1 = (int)((int64_t)(part + 1) * kt_all / split.parts);
+  g.K = (g.K < kt1 * kBK ? g.K : kt1 * kBK) - kt0 * kBK;
+  g.A += (int64_t)kt0 * kBK * (A_KMAJOR ? 1 : g.lda);
+  g.B += (int64_t)kt0 * kBK * (B_KMAJOR ? 1 : g.ldb);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = wave * 32;
 
@@ -67,7 +77,7 @@ __global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g)
   // k row are contiguous in memory and walking in step is the better order.)
   // (Not with an MN-major A and a ragged K: the stage that holds the K tail then has loads that
   // fall outside A's descriptor altogether, and the counted waits below need it to be the last.)
-  const int first = (B_KMAJOR && (A_KMAJOR || g.K % kBK == 0)) ? (int)(((int64_t)blockIdx.x * KT) / gridDim.x) : 0;
+  const int first = (B_KMAJOR && (A_KMAJOR || g.K % kBK == 0)) ? (int)(((int64_t)strip * KT) / strips) : 0;
   int at = 0;  // the stage the loaders' descriptors point at
   // Issues the loads of the i-th stage in walking order; beyond the KT-th they
   // fall outside the descriptors and arrive as zeros, so that every step issues
@@ -136,9 +146,25 @@ __global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g)
     wr_off += kStageBytes;
     if (wr_off == S * kStageBytes) wr_off = 0;
   }
+  const int slot = (int)batch * strips + strip;
+  const uint32_t seen = split.parts > 1 ? split_look(split, slot) : 0;
   // the ring is idle (zero-fill loads of the stages past K included) before the epilogue overlays it
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
+  if (split.parts > 1) {
+    uint32_t* word = reinterpret_cast<uint32_t*>(lds);  // (nothing else in the ring is live)
+    if (threadIdx.x == 0) *word = seen;
+    __syncthreads();
+    const bool others_in = *word == (uint32_t)split.parts - 1;
+    __syncthreads();
+    // with one row tile the lanes of rows past M have nothing to add
+    const bool mine = MT > 1 || (int)(threadIdx.x & 31) < g.M;
+    if (!split_exchange<16 * MT, kSkThreads>(
+            split, slot, strips * gridDim.y, part, mine, others_in, word, [&](int j) { return acc[j / 16][0][j % 16]; },
+            [&](int j, float v) { acc[j / 16][0][j % 16] = v; }))
+      return;
+    __syncthreads();  // the word has been read
+  }
   float* stage_area = reinterpret_cast<float*>(lds) + wave * epilogue_stage_floats<MT, 1>();
   if (g.fast_epi) {
     epilogue_bf16_fast_any<MT, 1>(g, batch, acc, 0, n0 + wn, stage_area);
@@ -148,23 +174,23 @@ __global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g)
 }
 
 template <int BM, bool AK, bool BK_, int FA, int FB>
-void launch_skinny(const GemmArgs& g, int64_t batch, hipStream_t st) {
+void launch_skinny(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
   GemmArgs a = g;
   a.tiles_m = 1;
   a.tiles_n = (g.N + kSkBN - 1) / kSkBN;
-  dim3 grid((unsigned)a.tiles_n, (unsigned)batch);
-  fp8_gemm_skinny_kernel<BM, AK, BK_, FA, FB><<<grid, kSkThreads, 0, st>>>(a);
+  dim3 grid((unsigned)(a.tiles_n * split.parts), (unsigned)batch);
+  fp8_gemm_skinny_kernel<BM, AK, BK_, FA, FB><<<grid, kSkThreads, 0, st>>>(a, split);
 }
 
 // M <= 128.  An MN-major A tile has rows of BM bytes in LDS, for which only
 // 128 has a conflict-free swizzle, so trans_a problems always take BM = 128.
 template <bool AK, bool BK_, int FA, int FB>
-void launch_skinny_by_m(const GemmArgs& g, int64_t batch, hipStream_t st) {
+void launch_skinny_by_m(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
   if constexpr (AK) {
-    if (g.M <= 32) return launch_skinny<32, AK, BK_, FA, FB>(g, batch, st);
-    if (g.M <= 64) return launch_skinny<64, AK, BK_, FA, FB>(g, batch, st);
+    if (g.M <= 32) return launch_skinny<32, AK, BK_, FA, FB>(g, split, batch, st);
+    if (g.M <= 64) return launch_skinny<64, AK, BK_, FA, FB>(g, split, batch, st);
   }
-  launch_skinny<128, AK, BK_, FA, FB>(g, batch, st);
+  launch_skinny<128, AK, BK_, FA, FB>(g, split, batch, st);
 }
 
 }  // namespace mi355q

@@ -1196,10 +1196,4 @@ void launch_tile(const GemmArgs& g, int64_t batch, hipStream_t st) {
   fp8_gemm_tile_kernel<BM, BN, WN, AK, BK_, FA, FB, FAST_ONLY><<<grid, kWavesM * WN * 64, 0, st>>>(a);
 }
 
-// A K-major / B K-major etc.; defined in gemm_inst_*.hip
-void launch_gemm_kk(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
-void launch_gemm_km(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
-void launch_gemm_mk(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
-void launch_gemm_mm(const GemmArgs& g, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
-
 }  // namespace mi355q

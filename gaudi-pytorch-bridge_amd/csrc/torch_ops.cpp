@@ -325,6 +325,70 @@ Tensor cast_from_fp8_scalar_list(const Tensor& input, c10::ArrayRef<double> scal
   return cast_from_fp8_impl(input, IValue(scale.vec()), out_dtype, to_opt_shape(scale_shape));
 }
 
+// --------------------------------------------------------- kept workspaces
+//
+// Kernels that split a reduction over workgroups (the K split of the GEMMs for few rows and of the 4-bit GEMMs, the
+// key splits of the attention kernel for few queries) keep arrival counters in their workspace, which have to be zero
+// when a call starts and are left zero by every call: one zero-filled buffer per (device, stream, op) is kept here and
+// grown on demand, so that a call launches one kernel and nothing else.  Calls on one stream run in order, which is
+// all the sharing the buffer allows; the ops lay their counters out differently and do not share.  At most
+// kKeptWorkspaces buffers are kept: past that the one that was used least recently is given back (to the caching
+// allocator, which hands it out again only to work queued behind what still uses it).  While a stream is being captured into a graph no kept
+// buffer is handed out (its memory would belong to the graph's pool, and replays of two graphs could overlap): the
+// call takes a buffer of the graph's own and clears its counters with a fill kernel that is part of the graph
+// (captured_ticket_workspace).
+enum TicketWorkspaceOp { kWsW4a8 = 0, kWsSdpa = 1, kWsW4a16 = 2, kWsGemm = 3 };
+constexpr size_t kKeptWorkspaces = 64;
+struct TicketWorkspaceCache {
+  struct Entry {
+    Tensor buffer;
+    uint64_t used = 0;
+  };
+  std::mutex mu;
+  uint64_t clock = 0;
+  std::map<std::tuple<int, void*, int>, Entry> map;
+};
+TicketWorkspaceCache& ticket_workspace_cache() {
+  // never destroyed: a static Tensor would be freed after the HIP runtime has shut down
+  static auto* cache = new TicketWorkspaceCache();
+  return *cache;
+}
+bool stream_is_capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// Undefined for bytes == 0 (the problem does not split).
+Tensor ticket_workspace(const Tensor& like, size_t bytes, TicketWorkspaceOp op) {
+  if (bytes == 0 || stream_is_capturing()) return Tensor();
+  TicketWorkspaceCache& c = ticket_workspace_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  const auto key = std::make_tuple((int)like.device().index(), current_stream(like), (int)op);
+  TicketWorkspaceCache::Entry& e = c.map[key];
+  e.used = ++c.clock;
+  if (!e.buffer.defined() || (size_t)e.buffer.numel() < bytes) e.buffer = at::zeros({(int64_t)bytes}, like.options().dtype(at::kByte));
+  Tensor t = e.buffer;
+  if (c.map.size() > kKeptWorkspaces) {
+    auto oldest = c.map.begin();
+    for (auto it = c.map.begin(); it != c.map.end(); ++it)
+      if (it->second.used < oldest->second.used) oldest = it;
+    c.map.erase(oldest);
+  }
+  return t;
+}
+// While the stream is being captured: a buffer out of the graph's pool, its counters (the first `counters` bytes)
+// zeroed by a small fill kernel, which every replay runs again; the rest (partial sums that are written before they
+// are read) as it comes.
+Tensor captured_ticket_workspace(const Tensor& like, size_t bytes, int64_t counters) {
+  Tensor t = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+  t.narrow(0, 0, std::min<int64_t>((int64_t)bytes, counters)).zero_();
+  return t;
+}
+// After a call that used the buffer has failed: its counters may be left non-zero (no workgroup then draws a
+// group's last ticket and the output stays unwritten), so the buffer is dropped and the next call starts from a
+// zero-filled one.
+void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
+  TicketWorkspaceCache& c = ticket_workspace_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  c.map.erase(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
+}
+
 // --------------------------------------------------------------- fp8_gemm_v2
 
 // torch.matmul shape rule with optional transposes of the last two dims
@@ -441,6 +505,10 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   for (auto d : batch_shape) batch *= d;
 
   auto prep = [&](const Tensor& t, int64_t rows, int64_t cols, int64_t* stride) {
+    if (t.dim() == 2 && t.is_contiguous()) {  // (what a layer passes: no view to make, no dispatch)
+      *stride = 0;
+      return t;
+    }
     int64_t tb_numel = t.numel() / std::max<int64_t>(rows * cols, 1);
     if (rows * cols == 0) tb_numel = 1;
     Tensor c;
@@ -547,14 +615,19 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
     stride_d = M * N;
   }
 
-  check_status(
-      mi355q_fp8_gemm(ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
+  const size_t ws_bytes = mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
+  const bool kept = ws_bytes == 0 || !stream_is_capturing();
+  Tensor ws = kept ? ticket_workspace(A, ws_bytes, kWsGemm) : captured_ticket_workspace(A, ws_bytes, 65536);
+  const int st =
+      mi355q_fp8_gemm_ws(ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
                       bc_t.data_ptr(), to_mi355q_dtype(B.scalar_type()), tb ? 1 : 0, ldb,
                       out.data_ptr(), to_mi355q_dtype(out_dtype), N, m_call, N, k_call, sa.dev, sa.host, sa.mode,
                       sb.dev, sb.host, sb.mode, bias_mode != MI355Q_BIAS_NONE ? bias_t.data_ptr() : nullptr,
                       bias_mode, ldbias, accumulate ? d_t.data_ptr() : nullptr, N, batch_call, stride_a,
-                      stride_b, M * N, stride_d, stride_bias, current_stream(A)),
-      "mi355q_fp8_gemm");
+                      stride_b, M * N, stride_d, stride_bias, ws.defined() ? ws.data_ptr() : nullptr,
+                      ws.defined() ? (size_t)ws.numel() : 0, current_stream(A));
+  if (st != MI355Q_OK && ws.defined() && kept) drop_ticket_workspace(A, kWsGemm);
+  check_status(st, "mi355q_fp8_gemm");
   return out;
 }
 
@@ -750,54 +823,7 @@ Tensor convert_from_uint4(const Tensor& input, const Tensor& scale,
 // matrix in between.  out = out_dtype((A @ ((q - z) * s)) * A_scale_inv + bias).  The reference has no
 // fused op; shapes the kernel does not take raise (there is no second route to the same bits).
 //
-// The kernel's split over K keeps arrival counters in its workspace, which have to be zero when a
-// call starts and are left zero by every call (the key splits of the attention kernel for few
-// queries do the same): one zero-filled buffer per (device, stream, op) is kept here and grown on
-// demand, so that a call launches one kernel and nothing else.  Calls on one stream run in order,
-// which is all the sharing the buffer allows; the two ops lay their counters out differently and
-// do not share.  While a stream is being captured into a graph no kept buffer is handed out (its
-// memory would belong to the graph's pool, and replays of two graphs could overlap): the call takes
-// a buffer of the graph's own and clears its counters with a fill kernel that is part of the graph
-// (captured_ticket_workspace).
-enum TicketWorkspaceOp { kWsW4a8 = 0, kWsSdpa = 1, kWsW4a16 = 2 };
-struct TicketWorkspaceCache {
-  std::mutex mu;
-  std::map<std::tuple<int, void*, int>, Tensor> map;
-};
-TicketWorkspaceCache& ticket_workspace_cache() {
-  // never destroyed: a static Tensor would be freed after the HIP runtime has shut down
-  static auto* cache = new TicketWorkspaceCache();
-  return *cache;
-}
-void ticket_workspace_cache_erase(int device, void* stream, int op) {
-  TicketWorkspaceCache& c = ticket_workspace_cache();
-  std::lock_guard<std::mutex> lock(c.mu);
-  c.map.erase(std::make_tuple(device, stream, op));
-}
-Tensor ticket_workspace(const Tensor& like, size_t bytes, TicketWorkspaceOp op) {
-  if (bytes == 0 || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return Tensor();
-  TicketWorkspaceCache& c = ticket_workspace_cache();
-  std::lock_guard<std::mutex> lock(c.mu);
-  Tensor& t = c.map[std::make_tuple((int)like.device().index(), current_stream(like), (int)op)];
-  if (!t.defined() || (size_t)t.numel() < bytes) t = at::zeros({(int64_t)bytes}, like.options().dtype(at::kByte));
-  return t;
-}
-// While the stream is being captured: a buffer out of the graph's pool, its first KiB (the arrival counters of
-// every op that uses one) zeroed by a small fill kernel, which every replay runs again; the rest (partial sums
-// that are written before they are read) as it comes.
-Tensor captured_ticket_workspace(const Tensor& like, size_t bytes) {
-  Tensor t = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
-  t.narrow(0, 0, std::min<int64_t>((int64_t)bytes, 1024)).zero_();
-  return t;
-}
-bool stream_is_capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
-// After a call that used the buffer has failed: its counters may be left non-zero (no workgroup then draws a
-// group's last ticket and the output stays unwritten), so the buffer is dropped and the next call starts from a
-// zero-filled one.
-void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
-  ticket_workspace_cache_erase((int)like.device().index(), current_stream(like), (int)op);
-}
-
+// (The workspace of its split over K: see ticket_workspace.)
 Tensor w4a8_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, const c10::optional<Tensor>& zero_point,
                  bool is_signed, at::ScalarType out_dtype, const c10::optional<Tensor>& A_scale_inv,
                  const c10::optional<Tensor>& bias) {
@@ -855,7 +881,7 @@ Tensor w4a8_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, con
   // the buffer kept per stream, or under graph capture one of the graph's own with its counters cleared
   const size_t ws_bytes = mi355q_w4a8_gemm_workspace_bytes(M, N, K, group, to_mi355q_dtype(s.scalar_type()));
   const bool kept = !stream_is_capturing();
-  Tensor ws = kept ? ticket_workspace(a, ws_bytes, kWsW4a8) : (ws_bytes ? captured_ticket_workspace(a, ws_bytes) : Tensor());
+  Tensor ws = kept ? ticket_workspace(a, ws_bytes, kWsW4a8) : (ws_bytes ? captured_ticket_workspace(a, ws_bytes, 1024) : Tensor());
   const int st = mi355q_w4a8_gemm(a.data_ptr(), to_mi355q_dtype(a.scalar_type()), K, w.data_ptr<int32_t>(), N / 8, s.data_ptr(),
                                   to_mi355q_dtype(s.scalar_type()), has_zp ? z.data_ptr<int32_t>() : nullptr, is_signed ? 1 : 0,
                                   group, out.data_ptr(), to_mi355q_dtype(out_dtype), N, M, N, K, sa_dev, 1.0f, sa_mode,
@@ -911,7 +937,7 @@ Tensor w4a16_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, co
   // the buffer kept per stream starts zero-filled, which the split over K needs; under graph capture a buffer of the
   // graph's own with its counters cleared
   const bool kept = !stream_is_capturing();
-  Tensor ws = kept ? ticket_workspace(a, bytes, kWsW4a16) : captured_ticket_workspace(a, bytes);
+  Tensor ws = kept ? ticket_workspace(a, bytes, kWsW4a16) : captured_ticket_workspace(a, bytes, 1024);
   const int st = mi355q_w4a16_gemm(a.data_ptr(), MI355Q_BF16, K, w.data_ptr<int32_t>(), N / 8, s.data_ptr(),
                                    to_mi355q_dtype(s.scalar_type()), has_zp ? z.data_ptr<int32_t>() : nullptr, is_signed ? 1 : 0, group,
                                    out.data_ptr(), to_mi355q_dtype(out_dtype), N, M, N, K, has_bias ? b.data_ptr() : nullptr,

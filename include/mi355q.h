@@ -238,6 +238,31 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda,
                     void* stream);
 
 /*
+ * The same with a workspace.  Products of at most 128 rows of A are bound by
+ * streaming B; where N alone does not give every compute unit a share of it,
+ * K is walked in parts by several workgroups whose fp32 sums meet through
+ * `workspace` (device memory, 16-byte aligned, at least
+ * mi355q_fp8_gemm_workspace_bytes() bytes; 0: the problem does not split).
+ * It begins with 64 KiB of arrival counters (the same place for every shape):
+ * zero-filled once before its first use, left zero by every call; calls that
+ * may overlap in time need workspaces of their own.  NULL: the same result
+ * (sums in another order) without the split.
+ */
+size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb,
+                                       int64_t M, int64_t N, int64_t K, int64_t batch);
+int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
+                    const void* B, int fmt_b, int trans_b, int64_t ldb,
+                    void* C, int out_dtype, int64_t ldc,
+                    int64_t M, int64_t N, int64_t K,
+                    const float* sa_dev, float sa_host, int sa_mode,
+                    const float* sb_dev, float sb_host, int sb_mode,
+                    const void* bias, int bias_mode, int64_t ldbias,
+                    const void* D, int64_t ldd,
+                    int64_t batch, int64_t stride_a, int64_t stride_b,
+                    int64_t stride_c, int64_t stride_d, int64_t stride_bias,
+                    void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Fused int4-dequant GEMM, fp8 activations times 4-bit weights (W4A8):
  *   C = out_dtype( (A @ W) * sa + bias ),   W[k, n] = (q[k, n] - z[k / group, n]) * s[k / group, n],
  * with the weights as convert_from_int4 / convert_from_uint4 take them and mi355q_dequant_4bit

@@ -1,0 +1,81 @@
+"""Products of at most 128 rows of A: the kernel that streams B into registers (gemm_stream.h), the strip kernel, and the
+split of K over workgroups with which both run.  Operands are small integers and scales powers of two, so that every
+fp32 sum is exact in any order and the result must match bit for bit."""
+import ctypes
+
+import pytest
+import torch
+
+import isa_check
+from helpers import E4, E5
+
+# rows at the edges of the kernels' tiles; N off the strips' 128 and 256 columns; K from one unit of 16 up, off the
+# stages' 128, and long enough for many parts
+CASES = [(1, 16, 8), (1, 4096, 1024), (15, 4112, 1000), (16, 14336, 520), (16, 8192, 4104), (17, 2064, 384), (32, 4096, 264),
+         (33, 2048, 1016), (64, 14336, 256), (65, 1040, 2048), (128, 8192, 640), (3, 272, 33288)]
+
+
+def operands(M, K, N, trans_b, fa, fb, dev):
+    g = torch.Generator().manual_seed(M * 7 + K * 3 + N)
+    a = torch.randint(-3, 4, (M, K), generator=g).float()
+    b = torch.randint(-3, 4, (K, N), generator=g).float()
+    return a, b, a.to(fa).to(dev), (b.t().contiguous() if trans_b else b).to(fb).to(dev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,K,N", CASES)
+def test_split_products_are_exact(M, K, N, trans_b, dev):
+    fa, fb = ((E4, E4), (E4, E5), (E5, E4), (E5, E5))[(M + K + N) % 4]
+    a, b, a8, b8 = operands(M, K, N, trans_b, fa, fb, dev)
+    ops = torch.ops.hpu
+    sa, sb = (torch.arange(M) % 3 - 1.0).exp2(), (torch.arange(N) % 2 - 1.0).exp2()
+    bias = (torch.arange(N) % 5 - 2).float()
+    ref = ((a @ b) * sa[:, None]) * sb[None] + bias
+    for out_dtype in (torch.float32, torch.bfloat16):
+        for _ in range(2):  # the counters of the first call are back at zero
+            c = ops.fp8_gemm_v2(a8, False, b8, trans_b, None, out_dtype, sa[:, None].to(dev), sb.to(dev), bias.to(out_dtype).to(dev), False, [1, N])
+            assert torch.equal(c.cpu(), ref.to(out_dtype)), (M, K, N, out_dtype)
+    # accumulate input, full bias, scalar scales
+    d = torch.randint(-4, 5, (M, N)).bfloat16()
+    c = ops.fp8_gemm_v2(a8, False, b8, trans_b, d.to(dev), torch.bfloat16, torch.tensor(0.5).to(dev), torch.tensor(2.0).to(dev), d.to(dev), True)
+    assert torch.equal(c.cpu(), (a @ b + d.float() * 2).bfloat16())
+
+
+@pytest.mark.gpu
+def test_one_workspace_serves_several_shapes(pkg, dev):
+    """The C entry with a caller's workspace: shapes one after the other, counters left zero, too small a workspace
+    refused, and no workspace accepted."""
+    lib = pkg.capi()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    shapes = [(1, 4096, 1024), (16, 8192, 4096), (64, 4096, 512), (2, 2048, 2048)]
+    need = max(lib.mi355q_fp8_gemm_workspace_bytes(0, k, 0, n, m, n, k, 1) for m, k, n in shapes)
+    assert need > 64 * 1024
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    for m, k, n in shapes:
+        a, b, a8, b8 = operands(m, k, n, False, E4, E4, dev)
+        ref = a @ b
+        c = torch.empty(m, n, device=dev)
+        for ptr, size, want in ((ws.data_ptr(), need, 0), (None, 0, 0), (ws.data_ptr(), 1024, None)):
+            status = lib.mi355q_fp8_gemm_ws(a8.data_ptr(), pkg.E4M3FN, 0, k, b8.data_ptr(), pkg.E4M3FN, 0, n, c.data_ptr(), pkg.F32, n, m, n, k,
+                                            None, 1.0, pkg.GS_NONE, None, 1.0, pkg.GS_NONE, None, pkg.BIAS_NONE, 0, None, 0, 1, 0, 0, 0, 0, 0,
+                                            ptr, size, st)
+            if want is None:
+                assert status != 0
+                continue
+            assert status == 0
+            assert torch.equal(c.cpu(), ref)
+        assert int(ws[: 64 * 1024].count_nonzero()) == 0
+
+
+@pytest.mark.timeout(600)
+def test_parts_of_k_meet_by_device_scope_accesses_in_order():
+    """Sums stored (sc1), acknowledged, barrier, ticket, barrier, counter reset, sums read (sc1); nothing cache-wide."""
+    import re
+    for src, least in (("gemm_stream.hip", 4), ("gemm_inst_kk.hip", 12)):
+        text = isa_check.compile_to_isa(src)
+        orders = isa_check.exchange_order(text)
+        assert len(orders) >= least and isa_check.scratch_bytes(text) == {}, src
+        for name, seq in orders.items():
+            assert "F" not in seq and seq.count("A") == 1, name
+            assert re.search(r"S+W+BAW?BS?W?L+", seq), (name, seq)
