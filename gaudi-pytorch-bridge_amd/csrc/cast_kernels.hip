@@ -554,12 +554,41 @@ __global__ __launch_bounds__(kThreads) void split_rows_vec_kernel(const uint16_t
 // the row is read from HBM once.  Results are bit-identical to the three
 // separate steps (rowwise_amax, an fp32 division, cast_to_fp8 with per-row
 // scales); scale_inv = 1 / scale is what the GEMM takes as A_scale_inv.
-template <bool BF16_IN, int FMT, int VPT>
-__global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
+//
+// A workgroup has as many waves as the row needs (row_shape below): a wave whose lanes are all past the row's end
+// would issue the same instructions as the others.  SAT: target may lie above the largest finite code, so the scaled
+// values need the saturating conversion.
+template <int FMT, bool SAT>
+__device__ __forceinline__ uint32_t row_cvt_fp8x4(float a, float b, float c, float d) {
+  if constexpr (SAT) return cvt_fp8x4<FMT>(a, b, c, d);
+  else return cvt_fp8x4_in_range<FMT>(a, b, c, d);
+}
+
+constexpr int kMaxRowThreads = 1024;
+
+// The row's amax (a non-negative fp32 bit pattern) from every lane's; then the row's scale, stored by thread 0.
+__device__ __forceinline__ float row_scale_of_block(uint32_t am, float target, int64_t row, float* scale_out, float* scale_inv_out) {
+  __shared__ uint32_t wave_part[kMaxRowThreads / 64];
+  am = wave_max_u32(am);
+  if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = am;
+  __syncthreads();
+  uint32_t r = wave_part[0];
+  const int waves = (int)(blockDim.x >> 6);
+  for (int w = 1; w < waves; ++w) r = r > wave_part[w] ? r : wave_part[w];
+  const float scale = row_scale(target, __uint_as_float(r));
+  if (threadIdx.x == 0) {
+    if (scale_out) scale_out[row] = scale;
+    if (scale_inv_out) scale_inv_out[row] = 1.0f / scale;
+  }
+  return scale;
+}
+
+template <bool BF16_IN, int FMT, int VPT, bool SAT>
+__global__ __launch_bounds__(kMaxRowThreads) void quantize_rows_kernel(
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, int64_t vec_per_row, float target,
     float* __restrict__ scale_out, float* __restrict__ scale_inv_out) {
-  __shared__ uint32_t wave_part[kThreads / 64];
   const int64_t row = blockIdx.x;
+  const int threads = (int)blockDim.x;
   // Descriptors over the row: a lane past its end loads zeros and its store is
   // dropped, so the body has no divergent branch and all loads are in flight
   // before the first is used.
@@ -572,7 +601,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
   uint32_t am = 0;
 #pragma unroll
   for (int u = 0; u < VPT; ++u)
-    in[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rin, ((int)threadIdx.x + u * kThreads) * 16, 0, 2));
+    in[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rin, ((int)threadIdx.x + u * threads) * 16, 0, 2));
 #pragma unroll
   for (int u = 0; u < VPT; ++u) {
 #pragma unroll
@@ -590,22 +619,11 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
     const uint32_t lo = am & 0xffffu, hi = am >> 16;
     am = (lo > hi ? lo : hi) << 16;
   }
-  am = wave_max_u32(am);
-  if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = am;
-  __syncthreads();
-  uint32_t r = wave_part[0];
-#pragma unroll
-  for (int w = 1; w < kThreads / 64; ++w) r = r > wave_part[w] ? r : wave_part[w];
-  const float amax = __uint_as_float(r);
-  const float scale = row_scale(target, amax);
-  if (threadIdx.x == 0) {
-    if (scale_out) scale_out[row] = scale;
-    if (scale_inv_out) scale_inv_out[row] = 1.0f / scale;
-  }
+  const float scale = row_scale_of_block(am, target, row, scale_out, scale_inv_out);
   const float s = BF16_IN ? round_to_bf16(scale) : scale;
 #pragma unroll
   for (int u = 0; u < VPT; ++u) {
-    const int off = ((int)threadIdx.x + u * kThreads) * OUT_BYTES;
+    const int off = ((int)threadIdx.x + u * threads) * OUT_BYTES;
     if constexpr (BF16_IN) {
       float p[8];
 #pragma unroll
@@ -613,11 +631,11 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
         p[2 * i] = round_to_bf16(__uint_as_float(in[u][i] << 16) * s);
         p[2 * i + 1] = round_to_bf16(__uint_as_float(in[u][i] & 0xffff0000u) * s);
       }
-      const u32x2 o = {cvt_fp8x4<FMT>(p[0], p[1], p[2], p[3]), cvt_fp8x4<FMT>(p[4], p[5], p[6], p[7])};
+      const u32x2 o = {row_cvt_fp8x4<FMT, SAT>(p[0], p[1], p[2], p[3]), row_cvt_fp8x4<FMT, SAT>(p[4], p[5], p[6], p[7])};
       __builtin_amdgcn_raw_buffer_store_b64(o, rout, off, 0, 2);
     } else {
-      const uint32_t o = cvt_fp8x4<FMT>(__uint_as_float(in[u][0]) * s, __uint_as_float(in[u][1]) * s,
-                                        __uint_as_float(in[u][2]) * s, __uint_as_float(in[u][3]) * s);
+      const uint32_t o = row_cvt_fp8x4<FMT, SAT>(__uint_as_float(in[u][0]) * s, __uint_as_float(in[u][1]) * s,
+                                                 __uint_as_float(in[u][2]) * s, __uint_as_float(in[u][3]) * s);
       __builtin_amdgcn_raw_buffer_store_b32(o, rout, off, 0, 2);
     }
   }
@@ -629,13 +647,19 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(
 // projection of a decoder MLP block; gate and up may be column ranges of one
 // wider matrix (row pitches ld_gate, ld_up in elements).  h_out, when given,
 // receives the bf16 products.
-template <int FMT, int VPT>
-__global__ __launch_bounds__(kThreads) void silu_mul_quantize_rows_kernel(
+//
+// Bound by vector issue where the chip is full and by one compute unit's where there is one row, hence the spelling of
+// silu_for_bf16 and the maximum over the unrounded products (rounding is monotonic, so the largest rounded product is
+// the rounded largest product; the maximum passes a NaN on).  1 x 14336: 4.8 us (7.5 with an IEEE exponential and
+// division per element), 1024 x 14336: 14.9 (22.7), 4096 x 14336: 51 us, 5.8 TB/s (60 with bf16(silu) looked up in a
+// table in LDS that every workgroup built).
+template <int FMT, int VPT, bool SAT>
+__global__ __launch_bounds__(kMaxRowThreads) void silu_mul_quantize_rows_kernel(
     const uint16_t* __restrict__ gate, int64_t ld_gate, const uint16_t* __restrict__ up, int64_t ld_up,
     uint8_t* __restrict__ y, uint16_t* __restrict__ h_out, int64_t vec_per_row, float target,
     float* __restrict__ scale_out, float* __restrict__ scale_inv_out) {
-  __shared__ uint32_t wave_part[kThreads / 64];
   const int64_t row = blockIdx.x;
+  const int threads = (int)blockDim.x;
   // Descriptors over the row (zeros past its end, stores dropped there): no
   // divergent branch, and every load is in flight before the first is used.
   const int row_bytes = (int)vec_per_row * 16;
@@ -645,10 +669,10 @@ __global__ __launch_bounds__(kThreads) void silu_mul_quantize_rows_kernel(
       h_out ? h_out + row * vec_per_row * 8 : nullptr, 0, h_out ? row_bytes : 0, 0x00020000);
   const __amdgpu_buffer_rsrc_t rout = __builtin_amdgcn_make_buffer_rsrc(y + row * vec_per_row * 8, 0, (int)vec_per_row * 8, 0x00020000);
   u32x4 gv[VPT], h[VPT];
-  uint32_t am = 0;
+  float am = 0.0f;
 #pragma unroll
   for (int u = 0; u < VPT; ++u) {
-    const int off = ((int)threadIdx.x + u * kThreads) * 16;
+    const int off = ((int)threadIdx.x + u * threads) * 16;
     gv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rg, off, 0, 2));
     h[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, off, 0, 2));
   }
@@ -656,31 +680,16 @@ __global__ __launch_bounds__(kThreads) void silu_mul_quantize_rows_kernel(
   for (int u = 0; u < VPT; ++u) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float s0 = round_to_bf16(silu_f32(__uint_as_float(gv[u][i] << 16)));
-      const float s1 = round_to_bf16(silu_f32(__uint_as_float(gv[u][i] & 0xffff0000u)));
-      h[u][i] = pack_bf16x2(s0 * __uint_as_float(h[u][i] << 16), s1 * __uint_as_float(h[u][i] & 0xffff0000u));
-      const u16x2 a = __builtin_bit_cast(u16x2, h[u][i] & 0x7fff7fffu);
-      am = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, __builtin_bit_cast(u16x2, am)));
+      const uint32_t s = pack_bf16x2(silu_for_bf16(__uint_as_float(gv[u][i] << 16)), silu_for_bf16(__uint_as_float(gv[u][i] & 0xffff0000u)));
+      const float h0 = __uint_as_float(s << 16) * __uint_as_float(h[u][i] << 16);
+      const float h1 = __uint_as_float(s & 0xffff0000u) * __uint_as_float(h[u][i] & 0xffff0000u);
+      am = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(h0), __builtin_fabsf(h1)), am);
+      h[u][i] = pack_bf16x2(h0, h1);
     }
     // without h_out the descriptor is empty and the store goes nowhere
-    __builtin_amdgcn_raw_buffer_store_b128(h[u], rh, ((int)threadIdx.x + u * kThreads) * 16, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(h[u], rh, ((int)threadIdx.x + u * threads) * 16, 0, 0);
   }
-  {
-    const uint32_t lo = am & 0xffffu, hi = am >> 16;
-    am = (lo > hi ? lo : hi) << 16;
-  }
-  am = wave_max_u32(am);
-  if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = am;
-  __syncthreads();
-  uint32_t r = wave_part[0];
-#pragma unroll
-  for (int w = 1; w < kThreads / 64; ++w) r = r > wave_part[w] ? r : wave_part[w];
-  const float amax = __uint_as_float(r);
-  const float scale = row_scale(target, amax);
-  if (threadIdx.x == 0) {
-    if (scale_out) scale_out[row] = scale;
-    if (scale_inv_out) scale_inv_out[row] = 1.0f / scale;
-  }
+  const float scale = row_scale_of_block(__float_as_uint(round_to_bf16(am)) & 0x7fffffffu, target, row, scale_out, scale_inv_out);
   const float s = round_to_bf16(scale);
 #pragma unroll
   for (int u = 0; u < VPT; ++u) {
@@ -690,148 +699,8 @@ __global__ __launch_bounds__(kThreads) void silu_mul_quantize_rows_kernel(
       p[2 * i] = round_to_bf16(__uint_as_float(h[u][i] << 16) * s);
       p[2 * i + 1] = round_to_bf16(__uint_as_float(h[u][i] & 0xffff0000u) * s);
     }
-    const u32x2 o = {cvt_fp8x4<FMT>(p[0], p[1], p[2], p[3]), cvt_fp8x4<FMT>(p[4], p[5], p[6], p[7])};
-    __builtin_amdgcn_raw_buffer_store_b64(o, rout, ((int)threadIdx.x + u * kThreads) * 8, 0, 2);
-  }
-}
-
-// The same, for many rows: bf16(silu(gate)) comes from a table in LDS.
-//
-// bf16(silu(x)) is a function of one bf16 value, 65536 cases in all, and most of
-// them need no arithmetic: for |x| < 2^-8 it equals bf16(x / 2); for x >= 128 it
-// is x; for finite x <= -128 it is -0 (silu_f32 returns -0 below -88.5).  The
-// 2 x 1920 values in between are computed once per workgroup with silu_f32, the
-// very function the kernel above calls per element, and kept in LDS; a workgroup
-// then walks several rows.  An element costs about 20 vector instructions instead
-// of about 50 (the exp and the IEEE division were 28 of them), which takes the
-// kernel from the vector ALU's bound to HBM's.  Index arithmetic and the range
-// fix-ups run on pairs of 16-bit lanes.  Results are bit-identical to the
-// kernel above (checked on all 65536 gate values).
-typedef short i16x2 __attribute__((ext_vector_type(2)));
-constexpr int kSiluLo = 0x3b80;                     // bf16 bits of 2^-8
-constexpr int kSiluHi = 0x4300;                     // bf16 bits of 128
-constexpr int kSiluEntries = kSiluHi - kSiluLo;     // per sign
-
-__device__ __forceinline__ void silu_table_build(uint16_t* tbl) {
-  for (int i = threadIdx.x; i < 2 * kSiluEntries; i += kThreads) {
-    const int sign = i >= kSiluEntries;
-    const uint32_t bits = (uint32_t)(kSiluLo + (i - sign * kSiluEntries)) | ((uint32_t)sign << 15);
-    tbl[i] = (uint16_t)(__float_as_uint(round_to_bf16(silu_f32(__uint_as_float(bits << 16)))) >> 16);
-  }
-}
-
-// Packed 16-bit integer instructions, spelled out: written as C on 16-bit vector types the
-// compiler turns the sign-mask idiom (x >> 15) back into compares and selects per half,
-// three times the instructions.
-#define MI355Q_PK_OP(name, mnemonic)                                                    \
-  __device__ __forceinline__ uint32_t name(uint32_t a, uint32_t b) {                    \
-    uint32_t r;                                                                         \
-    asm(mnemonic " %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));                             \
-    return r;                                                                           \
-  }
-MI355Q_PK_OP(pk_sub_u16, "v_pk_sub_u16")          // a - b per half, wrapping
-MI355Q_PK_OP(pk_min_u16, "v_pk_min_u16")
-MI355Q_PK_OP(pk_ashrrev_i16, "v_pk_ashrrev_i16")  // b >> a per half, arithmetic
-MI355Q_PK_OP(pk_lshrrev_b16, "v_pk_lshrrev_b16")  // b >> a per half, logical
-MI355Q_PK_OP(pk_lshlrev_b16, "v_pk_lshlrev_b16")  // b << a per half
-#undef MI355Q_PK_OP
-__device__ __forceinline__ uint32_t pk_mad_u16(uint32_t a, uint32_t b, uint32_t c) {
-  uint32_t r;
-  asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-__device__ __forceinline__ uint32_t select_bits(uint32_t mask, uint32_t if_set, uint32_t if_clear) {
-  return (if_set & mask) | (if_clear & ~mask);  // v_bfi_b32
-}
-
-// bf16(silu(x)) of the two bf16 values in w, as two bf16 values.
-__device__ __forceinline__ uint32_t silu_bf16x2_lookup(uint32_t w, const uint16_t* tbl) {
-  constexpr uint32_t k15 = 0x000f000fu, k1 = 0x00010001u;
-  constexpr uint32_t kLo = (uint32_t)kSiluLo * 0x00010001u, kHiM1 = (uint32_t)(kSiluHi - 1) * 0x00010001u;
-  constexpr uint32_t kN = (uint32_t)kSiluEntries * 0x00010001u, kNM1 = (uint32_t)(kSiluEntries - 1) * 0x00010001u;
-  const uint32_t a = w & 0x7fff7fffu;
-  const uint32_t d = pk_sub_u16(a, kLo);                              // negative as int16: |x| < 2^-8
-  const uint32_t m_small = pk_ashrrev_i16(k15, d);
-  const uint32_t m_big = pk_ashrrev_i16(k15, pk_sub_u16(kHiM1, a));   // |x| >= 128, inf, NaN
-  const uint32_t idx = pk_mad_u16(pk_lshrrev_b16(k15, w), kN, pk_min_u16(d, kNM1));
-  const uint32_t off = pk_lshlrev_b16(k1, idx);                       // byte offsets into the table
-  const uint8_t* tb = reinterpret_cast<const uint8_t*>(tbl);
-  const uint32_t t = (uint32_t)*reinterpret_cast<const uint16_t*>(tb + (off & 0xffffu)) |
-                     ((uint32_t)*reinterpret_cast<const uint16_t*>(tb + (off >> 16)) << 16);
-  // |x| < 2^-8: bf16(x / 2)
-  const uint32_t small = pack_bf16x2(__uint_as_float(w << 16) * 0.5f, __uint_as_float(w & 0xffff0000u) * 0.5f);
-  // |x| >= 128: x when positive; -0 when negative and finite, NaN for -inf (= -inf / inf) and NaN
-  const uint32_t m_naninf = pk_ashrrev_i16(k15, pk_sub_u16(0x7f7f7f7fu, a));
-  const uint32_t neg = 0x80008000u | (m_naninf & 0x7fc07fc0u);
-  const uint32_t big = select_bits(pk_ashrrev_i16(k15, w), neg, w);
-  return select_bits(m_small, small, select_bits(m_big, big, t));
-}
-
-template <int FMT, int VPT>
-__global__ __launch_bounds__(kThreads) void silu_mul_quantize_rows_table_kernel(
-    const uint16_t* __restrict__ gate, int64_t ld_gate, const uint16_t* __restrict__ up, int64_t ld_up,
-    uint8_t* __restrict__ y, uint16_t* __restrict__ h_out, int64_t rows, int64_t vec_per_row, float target,
-    float* __restrict__ scale_out, float* __restrict__ scale_inv_out) {
-  __shared__ uint16_t tbl[2 * kSiluEntries];
-  __shared__ uint32_t wave_part[2][kThreads / 64];
-  silu_table_build(tbl);
-  __syncthreads();
-  const int row_bytes = (int)vec_per_row * 16;
-  int parity = 0;
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x, parity ^= 1) {
-    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(gate) + row * ld_gate, 0, row_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(up) + row * ld_up, 0, row_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
-        h_out ? h_out + row * vec_per_row * 8 : nullptr, 0, h_out ? row_bytes : 0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rout = __builtin_amdgcn_make_buffer_rsrc(y + row * vec_per_row * 8, 0, (int)vec_per_row * 8, 0x00020000);
-    u32x4 gv[VPT], h[VPT];
-    uint32_t am = 0;
-#pragma unroll
-    for (int u = 0; u < VPT; ++u) {
-      const int off = ((int)threadIdx.x + u * kThreads) * 16;
-      gv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rg, off, 0, 2));
-      h[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ru, off, 0, 2));
-    }
-#pragma unroll
-    for (int u = 0; u < VPT; ++u) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t s = silu_bf16x2_lookup(gv[u][i], tbl);
-        h[u][i] = pack_bf16x2(__uint_as_float(s << 16) * __uint_as_float(h[u][i] << 16),
-                              __uint_as_float(s & 0xffff0000u) * __uint_as_float(h[u][i] & 0xffff0000u));
-        const u16x2 a = __builtin_bit_cast(u16x2, h[u][i] & 0x7fff7fffu);
-        am = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, __builtin_bit_cast(u16x2, am)));
-      }
-      __builtin_amdgcn_raw_buffer_store_b128(h[u], rh, ((int)threadIdx.x + u * kThreads) * 16, 0, 0);
-    }
-    {
-      const uint32_t lo = am & 0xffffu, hi = am >> 16;
-      am = (lo > hi ? lo : hi) << 16;
-    }
-    am = wave_max_u32(am);
-    // two exchange areas, used in turn: a wave may start the next row while another still reads this one's
-    if ((threadIdx.x & 63) == 0) wave_part[parity][threadIdx.x >> 6] = am;
-    __syncthreads();
-    uint32_t r = wave_part[parity][0];
-#pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) r = r > wave_part[parity][w] ? r : wave_part[parity][w];
-    const float scale = row_scale(target, __uint_as_float(r));
-    if (threadIdx.x == 0) {
-      if (scale_out) scale_out[row] = scale;
-      if (scale_inv_out) scale_inv_out[row] = 1.0f / scale;
-    }
-    const float s = round_to_bf16(scale);
-#pragma unroll
-    for (int u = 0; u < VPT; ++u) {
-      float p[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        p[2 * i] = round_to_bf16(__uint_as_float(h[u][i] << 16) * s);
-        p[2 * i + 1] = round_to_bf16(__uint_as_float(h[u][i] & 0xffff0000u) * s);
-      }
-      const u32x2 o = {cvt_fp8x4<FMT>(p[0], p[1], p[2], p[3]), cvt_fp8x4<FMT>(p[4], p[5], p[6], p[7])};
-      __builtin_amdgcn_raw_buffer_store_b64(o, rout, ((int)threadIdx.x + u * kThreads) * 8, 0, 2);
-    }
+    const u32x2 o = {row_cvt_fp8x4<FMT, SAT>(p[0], p[1], p[2], p[3]), row_cvt_fp8x4<FMT, SAT>(p[4], p[5], p[6], p[7])};
+    __builtin_amdgcn_raw_buffer_store_b64(o, rout, ((int)threadIdx.x + u * threads) * 8, 0, 2);
   }
 }
 
@@ -1130,53 +999,54 @@ inline bool scale_args_ok(const float* scale, int mode, int64_t outer, int64_t m
   return true;
 }
 
-template <bool BF16_IN, int FMT>
-int quantize_rows_launch(const uint8_t* x, uint8_t* y, int64_t rows, int64_t vpr, float target,
-                                float* scale_out, float* scale_inv_out, hipStream_t st) {
-  const unsigned grid = (unsigned)rows;
-  if (vpr <= kThreads) quantize_rows_kernel<BF16_IN, FMT, 1><<<grid, kThreads, 0, st>>>(x, y, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 2 * kThreads) quantize_rows_kernel<BF16_IN, FMT, 2><<<grid, kThreads, 0, st>>>(x, y, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 4 * kThreads) quantize_rows_kernel<BF16_IN, FMT, 4><<<grid, kThreads, 0, st>>>(x, y, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 8 * kThreads) quantize_rows_kernel<BF16_IN, FMT, 8><<<grid, kThreads, 0, st>>>(x, y, vpr, target, scale_out, scale_inv_out);
-  else return MI355Q_ERR_UNSUPPORTED;
-  return launch_status();
+// How a row of vpr vectors is spread over a workgroup: vectors per thread, and threads, whole waves of them.
+// Few rows leave compute units idle, and a row's time is that of its slowest thread: one vector per thread, two where
+// 1024 threads do not suffice.  With many rows four vectors per thread keep more loads in flight and several
+// workgroups on a compute unit (three, five or seven: 3 to 10 % slower at 1024 x 14336 and 2048 x 5632; at 512 rows
+// the two forms cross).
+constexpr int64_t kFewRows = 512;
+constexpr int kBulkVectors = 4;
+struct RowShape {
+  int vpt;
+  unsigned threads;
+};
+inline RowShape row_shape(int64_t rows, int64_t vpr) {
+  const int vpt = rows < kFewRows ? (vpr <= kMaxRowThreads ? 1 : 2) : kBulkVectors;
+  return {vpt, (unsigned)(((vpr + vpt - 1) / vpt + 63) / 64 * 64)};
+}
+constexpr int64_t kMaxRowVectors = 2 * kMaxRowThreads;
+
+// Calls f(vectors per thread, saturate, threads); false: the row does not fit a workgroup.
+template <int FMT, typename F>
+bool with_row_shape(int64_t rows, int64_t vpr, float target, F&& f) {
+  if (vpr > kMaxRowVectors) return false;
+  const RowShape s = row_shape(rows, vpr);
+  if (!(target <= kFp8Max[FMT - MI355Q_E4M3FN])) f(std::integral_constant<int, 2>{}, std::true_type{}, (unsigned)kMaxRowThreads);
+  else if (s.vpt == 1) f(std::integral_constant<int, 1>{}, std::false_type{}, s.threads);
+  else if (s.vpt == 2) f(std::integral_constant<int, 2>{}, std::false_type{}, s.threads);
+  else f(std::integral_constant<int, kBulkVectors>{}, std::false_type{}, s.threads);
+  return true;
 }
 
-// The table kernel pays for its table (15 silu evaluations per thread) once per workgroup:
-// it runs from this many rows on, with a fixed number of workgroups.
-constexpr int64_t kSiluTableMinRows = 2048;
-inline int silu_table_workgroups() {
-  static const int n = [] {
-    int dev = 0, cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
-      cu = 256;
-    return cu * 4;  // measured at 4096 x 14336: 2 per compute unit 70 us, 4: 62.5, 8: 63.7
-  }();
-  return n;
+template <bool BF16_IN, int FMT>
+int quantize_rows_launch(const uint8_t* x, uint8_t* y, int64_t rows, int64_t vpr, float target,
+                         float* scale_out, float* scale_inv_out, hipStream_t st) {
+  const bool ok = with_row_shape<FMT>(rows, vpr, target, [&](auto v, auto sat, unsigned threads) {
+    quantize_rows_kernel<BF16_IN, FMT, decltype(v)::value, decltype(sat)::value>
+        <<<(unsigned)rows, threads, 0, st>>>(x, y, vpr, target, scale_out, scale_inv_out);
+  });
+  return ok ? launch_status() : MI355Q_ERR_UNSUPPORTED;
 }
 
 template <int FMT>
 int silu_mul_quantize_rows_launch(const uint16_t* gate, int64_t ld_gate, const uint16_t* up, int64_t ld_up,
                                   uint8_t* y, uint16_t* h_out, int64_t rows, int64_t vpr, float target,
                                   float* scale_out, float* scale_inv_out, hipStream_t st) {
-  // Many rows: workgroups that build the silu table once and walk several rows each.
-  if (rows >= kSiluTableMinRows && vpr <= 8 * kThreads) {
-    const int64_t want = (int64_t)silu_table_workgroups();
-    const unsigned tg = (unsigned)(rows < want ? rows : want);
-    if (vpr <= kThreads) silu_mul_quantize_rows_table_kernel<FMT, 1><<<tg, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, rows, vpr, target, scale_out, scale_inv_out);
-    else if (vpr <= 2 * kThreads) silu_mul_quantize_rows_table_kernel<FMT, 2><<<tg, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, rows, vpr, target, scale_out, scale_inv_out);
-    else if (vpr <= 4 * kThreads) silu_mul_quantize_rows_table_kernel<FMT, 4><<<tg, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, rows, vpr, target, scale_out, scale_inv_out);
-    else silu_mul_quantize_rows_table_kernel<FMT, 8><<<tg, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, rows, vpr, target, scale_out, scale_inv_out);
-    return launch_status();
-  }
-  const unsigned grid = (unsigned)rows;
-  if (vpr <= kThreads) silu_mul_quantize_rows_kernel<FMT, 1><<<grid, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 2 * kThreads) silu_mul_quantize_rows_kernel<FMT, 2><<<grid, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 4 * kThreads) silu_mul_quantize_rows_kernel<FMT, 4><<<grid, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, vpr, target, scale_out, scale_inv_out);
-  else if (vpr <= 8 * kThreads) silu_mul_quantize_rows_kernel<FMT, 8><<<grid, kThreads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, vpr, target, scale_out, scale_inv_out);
-  else return MI355Q_ERR_UNSUPPORTED;
-  return launch_status();
+  const bool ok = with_row_shape<FMT>(rows, vpr, target, [&](auto v, auto sat, unsigned threads) {
+    silu_mul_quantize_rows_kernel<FMT, decltype(v)::value, decltype(sat)::value>
+        <<<(unsigned)rows, threads, 0, st>>>(gate, ld_gate, up, ld_up, y, h_out, vpr, target, scale_out, scale_inv_out);
+  });
+  return ok ? launch_status() : MI355Q_ERR_UNSUPPORTED;
 }
 
 }  // namespace mi355q

@@ -44,37 +44,17 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, r);
 }
 
-// exp(t) for -87 <= t <= 88 as a fixed sequence of IEEE operations (Cody-Waite
-// reduction by ln 2 in two parts, the degree-5 polynomial of Cephes' expf, an
-// exact scaling by a power of two): the CPU oracle runs the same sequence and
-// gets the same bits, which a library or hardware exp would not guarantee.
-// Contraction is off so that no multiply and add merge that the oracle keeps apart.
-__device__ __forceinline__ float exp_spelled_out(float t) {
-#pragma clang fp contract(off)
-  const float n = __builtin_rintf(t * 1.44269504088896341f);
-  float r = __builtin_fmaf(n, -0.693145751953125f, t);
-  r = __builtin_fmaf(n, -1.42860682030941723212e-6f, r);
-  float q = 1.9875691500e-4f;
-  q = __builtin_fmaf(q, r, 1.3981999507e-3f);
-  q = __builtin_fmaf(q, r, 8.3334519073e-3f);
-  q = __builtin_fmaf(q, r, 4.1665795894e-2f);
-  q = __builtin_fmaf(q, r, 1.6666665459e-1f);
-  q = __builtin_fmaf(q, r, 5.0000001201e-1f);
-  float y = __builtin_fmaf(q, r * r, r);
-  y = y + 1.0f;
-  return __builtin_ldexpf(y, (int)n);
-}
-
-// x / (1 + exp(-x)) in fp32, branch-free; results smaller than 3.3e-37 in
-// magnitude (x <= -88.5) are -0, NaN stays NaN.
-__device__ __forceinline__ float silu_f32(float x) {
-#pragma clang fp contract(off)
-  const float t = -x;
-  // fmin / fmax return the other operand for a NaN, so the exp below never sees one
-  float e = exp_spelled_out(__builtin_fminf(__builtin_fmaxf(t, -87.0f), 88.0f));
-  e = t > 88.0f ? __builtin_inff() : e;
-  e = t < -87.0f ? 0.0f : e;
-  return x / (1.0f + e);
+// x / (1 + exp(-x)) for a bf16 x, accurate enough that rounding the result to bf16 gives the bits of the CPU
+// oracle's fixed sequence of IEEE operations for every one of the 65536 values x can take (a test compares them all).
+// With t = |x| exp(-|x|) / (1 + exp(-|x|)) it is max(x, -0) - t: nothing overflows and nothing cancels.  The
+// exponential carries a factor of 2, which keeps it a normal number down to x = -88, the last value with a result;
+// below that v_exp_f32 gives 0 and the result is -0.  -inf gives inf * 0 = NaN, and a NaN passes through the maximum.
+// Nine instructions, two of them transcendental; the IEEE sequence took fifty.
+__device__ __forceinline__ float silu_for_bf16(float x) {
+  const float xm = __builtin_fminf(x, 128.0f);
+  const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(__builtin_fabsf(xm), -1.44269504088896341f, 1.0f));
+  const float p = __builtin_fabsf(xm) * (e * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0.5f, 1.0f)));
+  return __builtin_fmaf(-p, 0.5f, __builtin_elementwise_maximum(x, -0.0f));
 }
 
 // Clamp to the finite fp8 range.  minimum/maximum propagate NaN, so a NaN
@@ -93,6 +73,22 @@ __device__ __forceinline__ uint32_t cvt_fp8x4(float a, float b, float c, float d
   b = sat_fp8<FMT>(b);
   c = sat_fp8<FMT>(c);
   d = sat_fp8<FMT>(d);
+  int r;
+  if constexpr (FMT == MI355Q_E5M2) {
+    r = __builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false);
+    r = __builtin_amdgcn_cvt_pk_bf8_f32(c, d, r, true);
+  } else {
+    r = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+    r = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, r, true);
+  }
+  return (uint32_t)r;
+}
+
+// The same for values known to lie below the halfway point past the largest finite code (464; 61440), which round to
+// that code by themselves: what a row scaled by target / amax with target <= the largest finite value holds, whatever
+// the roundings on the way (at most 449.8; 57570).  NaN stays NaN.
+template <int FMT>
+__device__ __forceinline__ uint32_t cvt_fp8x4_in_range(float a, float b, float c, float d) {
   int r;
   if constexpr (FMT == MI355Q_E5M2) {
     r = __builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false);
