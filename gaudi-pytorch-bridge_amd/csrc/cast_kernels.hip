@@ -23,6 +23,15 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t v) { *p = v; }
 // 32 MiB).
 constexpr int kAmaxThreads = 1024;
 constexpr int kAmaxBlocks = 256;
+// The cast with amax: up to kAmaxBlocks workgroups of 512 threads with eight vectors in flight per lane, of 256 threads
+// while those suffice (short tensors: more compute units take part).  With the amax starting at zero, bf16, us:
+//   elements              2^12   2^20   2^22   2^23   2^24   2^26   2^28
+//   this                   4.2    4.5    6.1    7.4   11.4   34.1    131
+//   256 x 1024 threads     4.6    5.7    7.3    9.1   11.5   34.9    136
+//   up to 2048 x 256       4.3    4.7   11.3   24.6     94     97    154    (atomics on one word: 13 to 45 ns each)
+constexpr int kCastAmaxMaxThreads = 512;
+constexpr int kCastAmaxU = 8;
+constexpr int64_t kCastAmaxSmall = int64_t(1) << 21;  // elements
 
 // Block-level max of abs-value bit patterns, then one atomicMax per block.
 // Bit patterns of non-negative floats order like the floats, and a NaN
@@ -61,16 +70,16 @@ __device__ __forceinline__ void block_amax_commit(uint32_t m, uint32_t* amax) {
 // load the compiler cannot tell that the previous iteration's load into the
 // same registers was consumed, and makes every load wait for all earlier ones.)
 template <bool BF16_IN, int FMT, int SK, bool AMAX, int U>
-__global__ __launch_bounds__(AMAX ? kAmaxThreads : kThreads) void cast_to_fp8_vec8(
+__global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to_fp8_vec8(
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
     float scale_host, int scale_is_dev, int64_t vec_per_row, int64_t blocks_per_row,
     int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax) {
-  constexpr int THREADS = AMAX ? kAmaxThreads : kThreads;
+  const int THREADS = AMAX ? (int)blockDim.x : kThreads;
   constexpr int IN_BYTES = BF16_IN ? 16 : 32;
   constexpr int kNt = 2;  // non-temporal
   uint32_t am = 0;
   // a logical block is THREADS * U consecutive vectors of one row; without amax
-  // the grid holds one workgroup per logical block and this loop runs once
+  // (or with few enough of them) the grid holds one workgroup per logical block and this loop runs once
   for (int64_t lb = blockIdx.x; lb < total_blocks; lb += gridDim.x) {
     const int64_t row = lb / blocks_per_row;
     const int64_t vec0 = (lb - row * blocks_per_row) * (int64_t)(THREADS * U);  // first vector, within the row
@@ -148,6 +157,17 @@ __global__ __launch_bounds__(AMAX ? kAmaxThreads : kThreads) void cast_to_fp8_ve
       out.x = cvt_fp8x4<FMT>(v[0], v[1], v[2], v[3]);
       out.y = cvt_fp8x4<FMT>(v[4], v[5], v[6], v[7]);
       __builtin_amdgcn_raw_buffer_store_b64(out, rout, ((int)threadIdx.x + u * THREADS) * 8, 0, kNt);
+      if constexpr (AMAX) {
+        // Where every workgroup has one logical block they all end at once, find the word still at zero and queue up
+        // at it.  One wave of each hands in what it has seen halfway, so that most find a larger value at the end and
+        // skip (2^22 elements: 6.1 instead of 7.0 us).  Longer tensors spread by themselves and only lose by it.
+        if (u == U / 2 - 1 && total_blocks == gridDim.x && threadIdx.x < 64) {
+          uint32_t m = am;
+          if constexpr (BF16_IN) m = ((m & 0xffffu) > (m >> 16) ? m & 0xffffu : m >> 16) << 16;
+          m = wave_max_u32(m);
+          if (threadIdx.x == 0) atomicMax(amax, m);
+        }
+      }
     }
   }
 
@@ -882,12 +902,14 @@ inline bool plan_vectors(int mode, int64_t outer, int64_t mid, int64_t inner, in
 
 constexpr int kCastU = 4;  // 16-byte loads in flight per thread
 
+inline unsigned cast_amax_threads(int64_t elements) { return elements <= kCastAmaxSmall ? kThreads : kCastAmaxMaxThreads; }
+
 template <bool BF16_IN, int FMT, bool AMAX>
 void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale,
                         float sh, int is_dev, int64_t vpr, int64_t bpr, int64_t total, int64_t mid,
                         uint32_t* amax) {
-  constexpr int U = kCastU;
-  constexpr int T = AMAX ? kAmaxThreads : kThreads;
+  constexpr int U = AMAX ? kCastAmaxU : kCastU;
+  const unsigned T = AMAX ? cast_amax_threads(vpr * (total / bpr) * 8) : kThreads;
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
   switch (sk) {
     case SK_SCALAR:
@@ -908,7 +930,6 @@ void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, co
 template <bool BF16_IN, int FMT>
 int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh, int mode,
                      int64_t outer, int64_t mid, int64_t inner, uint32_t* amax, hipStream_t st) {
-  constexpr int U = kCastU;
   const int64_t n = outer * mid * inner;
   VecPlan p;
   const bool vec = aligned(x, 16) && aligned(y, 8) &&
@@ -919,7 +940,7 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
     // In flat modes the row length need not be a multiple of 8: the tail goes
     // to the generic kernel.  In 2-D modes plan_vectors has required it.
     if (vpr > 0) {
-      const int64_t per_block = (int64_t)(amax ? kAmaxThreads : kThreads) * U;
+      const int64_t per_block = amax ? (int64_t)cast_amax_threads(vpr * p.rows * 8) * kCastAmaxU : (int64_t)kThreads * kCastU;
       const int64_t bpr = (vpr + per_block - 1) / per_block;
       const int64_t total = bpr * p.rows;
       if (total > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
@@ -1229,9 +1250,9 @@ int mi355q_silu_mul_quantize_rows(const void* gate, int64_t ld_gate, const void*
   return silu_mul_quantize_rows_launch<MI355Q_E5M2>(g, ld_gate, u, ld_up, yb, hb, rows, cols / 8, target, scale_out, scale_inv_out, st);
 }
 
-int mi355q_cast_to_fp8(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
+static int cast_to_fp8_rne(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
                        float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
-                       float* amax_out, void* stream) {
+                       float* amax_out, bool zero_amax, void* stream) {
   if (fp8_fmt != MI355Q_E4M3FN && fp8_fmt != MI355Q_E5M2) return MI355Q_ERR_INVALID_ARGUMENT;
   if (!scale_args_ok(scale_dev, scale_mode, outer, mid, inner)) return MI355Q_ERR_INVALID_ARGUMENT;
   const int64_t n = outer * mid * inner;
@@ -1258,7 +1279,7 @@ int mi355q_cast_to_fp8(const void* x, int x_dtype, void* y, int fp8_fmt, const f
   if (x_dtype != MI355Q_F32 && x_dtype != MI355Q_BF16) return MI355Q_ERR_INVALID_ARGUMENT;
 
   uint32_t* am = reinterpret_cast<uint32_t*>(amax_out);
-  if (am) fill_u32_kernel<<<1, 1, 0, st>>>(am, 0u);
+  if (am && zero_amax) fill_u32_kernel<<<1, 1, 0, st>>>(am, 0u);
   if (n == 0) return launch_status();
   if (x_dtype == MI355Q_BF16) {
     if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<true, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
@@ -1266,6 +1287,19 @@ int mi355q_cast_to_fp8(const void* x, int x_dtype, void* y, int fp8_fmt, const f
   }
   if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<false, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
   return cast_to_dispatch<false, MI355Q_E5M2>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
+}
+
+int mi355q_cast_to_fp8(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
+                       float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
+                       float* amax_out, void* stream) {
+  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, amax_out, true, stream);
+}
+
+int mi355q_cast_to_fp8_running_amax(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
+                                    float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
+                                    float* running_amax, void* stream) {
+  if (running_amax == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
+  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, running_amax, false, stream);
 }
 
 int mi355q_cast_from_fp8(const void* x, int fp8_fmt, void* y, int out_dtype, const float* scale_dev,

@@ -202,8 +202,12 @@ bool sr_flush_to_zero_mode() {
 }
 
 // One call for both rounding modes.
-int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* amax, bool stochastic) {
+// amax_zeroed: *amax holds zero (round to nearest only).
+int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* amax, bool stochastic, bool amax_zeroed = false) {
   const int xd = to_mi355q_dtype(x.scalar_type()), od = to_mi355q_dtype(out.scalar_type());
+  if (amax_zeroed)
+    return mi355q_cast_to_fp8_running_amax(x.data_ptr(), xd, out.data_ptr(), od, cs.dev, cs.host, cs.mode, cs.outer, cs.mid,
+                                           cs.inner, amax, current_stream(x));
   if (!stochastic)
     return mi355q_cast_to_fp8(x.data_ptr(), xd, out.data_ptr(), od, cs.dev, cs.host, cs.mode, cs.outer, cs.mid,
                               cs.inner, amax, current_stream(x));
@@ -212,6 +216,101 @@ int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* ama
   const bool sftz = sr_flush_to_zero_mode() && x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kFloat8_e5m2;
   return mi355q_cast_to_fp8_sr(x.data_ptr(), xd, out.data_ptr(), od, cs.dev, cs.host, cs.mode, cs.outer, cs.mid,
                                cs.inner, amax, r.first, r.second, sftz ? 1 : 0, current_stream(x));
+}
+
+// --------------------------------------------------------- kept workspaces
+//
+// Kernels that split a reduction over workgroups (the K split of the GEMMs for few rows and of the 4-bit GEMMs, the
+// key splits of the attention kernel for few queries) keep arrival counters in their workspace, which have to be zero
+// when a call starts and are left zero by every call: one zero-filled buffer per (device, stream, op) is kept here and
+// grown on demand, so that a call launches one kernel and nothing else.  Calls on one stream run in order, which is
+// all the sharing the buffer allows; the ops lay their counters out differently and do not share.  At most
+// kKeptWorkspaces buffers are kept: past that the one that was used least recently is given back (to the caching
+// allocator, which hands it out again only to work queued behind what still uses it).  While a stream is being captured into a graph no kept
+// buffer is handed out (its memory would belong to the graph's pool, and replays of two graphs could overlap): the
+// call takes a buffer of the graph's own and clears its counters with a fill kernel that is part of the graph
+// (captured_ticket_workspace).
+enum TicketWorkspaceOp { kWsW4a8 = 0, kWsSdpa = 1, kWsW4a16 = 2, kWsGemm = 3 };
+constexpr size_t kKeptWorkspaces = 64;
+struct TicketWorkspaceCache {
+  struct Entry {
+    Tensor buffer;
+    uint64_t used = 0;
+  };
+  std::mutex mu;
+  uint64_t clock = 0;
+  std::map<std::tuple<int, void*, int>, Entry> map;
+};
+template <typename Map>
+void drop_least_recent(Map& map) {
+  auto oldest = map.begin();
+  for (auto it = map.begin(); it != map.end(); ++it)
+    if (it->second.used < oldest->second.used) oldest = it;
+  map.erase(oldest);
+}
+TicketWorkspaceCache& ticket_workspace_cache() {
+  // never destroyed: a static Tensor would be freed after the HIP runtime has shut down
+  static auto* cache = new TicketWorkspaceCache();
+  return *cache;
+}
+bool stream_is_capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// Undefined for bytes == 0 (the problem does not split).
+Tensor ticket_workspace(const Tensor& like, size_t bytes, TicketWorkspaceOp op) {
+  if (bytes == 0 || stream_is_capturing()) return Tensor();
+  TicketWorkspaceCache& c = ticket_workspace_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  const auto key = std::make_tuple((int)like.device().index(), current_stream(like), (int)op);
+  TicketWorkspaceCache::Entry& e = c.map[key];
+  e.used = ++c.clock;
+  if (!e.buffer.defined() || (size_t)e.buffer.numel() < bytes) e.buffer = at::zeros({(int64_t)bytes}, like.options().dtype(at::kByte));
+  Tensor t = e.buffer;
+  if (c.map.size() > kKeptWorkspaces) drop_least_recent(c.map);
+  return t;
+}
+// While the stream is being captured: a buffer out of the graph's pool, its counters (the first `counters` bytes)
+// zeroed by a small fill kernel, which every replay runs again; the rest (partial sums that are written before they
+// are read) as it comes.
+Tensor captured_ticket_workspace(const Tensor& like, size_t bytes, int64_t counters) {
+  Tensor t = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+  t.narrow(0, 0, std::min<int64_t>((int64_t)bytes, counters)).zero_();
+  return t;
+}
+// After a call that used the buffer has failed: its counters may be left non-zero (no workgroup then draws a
+// group's last ticket and the output stays unwritten), so the buffer is dropped and the next call starts from a
+// zero-filled one.
+void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
+  TicketWorkspaceCache& c = ticket_workspace_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  c.map.erase(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
+}
+
+// Zeroed words for results that kernels accumulate into (amax), so that a call needs no launch that clears one: a
+// block of them is cleared at once, per (device, stream), and every word is handed out once, as a tensor that shares
+// the block's memory; words are a cache line apart.  Not while the stream is being captured (a replay would find the
+// word as the last one left it).
+struct ZeroWords {
+  static constexpr int64_t kWords = 256, kStride = 16;
+  struct Entry {
+    Tensor block;
+    int64_t next = kWords;
+    uint64_t used = 0;
+  };
+  std::mutex mu;
+  uint64_t clock = 0;
+  std::map<std::pair<int, void*>, Entry> map;
+};
+Tensor zero_word(const Tensor& like) {
+  static auto* z = new ZeroWords();  // never destroyed, as above
+  std::lock_guard<std::mutex> lock(z->mu);
+  ZeroWords::Entry& e = z->map[std::make_pair((int)like.device().index(), current_stream(like))];
+  e.used = ++z->clock;
+  if (e.next == ZeroWords::kWords) {
+    e.block = at::zeros({ZeroWords::kWords * ZeroWords::kStride}, like.options().dtype(at::kFloat));
+    e.next = 0;
+  }
+  Tensor word = e.block.as_strided({}, {}, ZeroWords::kStride * e.next++);
+  if (z->map.size() > kKeptWorkspaces) drop_least_recent(z->map);
+  return word;
 }
 
 // ------------------------------------------------------------ cast_to_fp8_v2
@@ -268,15 +367,17 @@ void cast_to_fp8_v2_boxed(const c10::OperatorHandle& op, c10::DispatchKeySet, to
     DeviceGuard guard(input.device());
     Tensor x = input.contiguous();
     out = at::empty(x.sizes(), x.options().dtype(dst));
-    amax = at::empty(is_amax ? std::vector<int64_t>{} : std::vector<int64_t>{0},
-                     x.options().dtype(at::kFloat));
+    const bool zeroed = is_amax && !sr && !stream_is_capturing();
+    if (zeroed) amax = zero_word(x);
+    else if (is_amax) amax = at::empty({}, x.options().dtype(at::kFloat));
+    else amax = at::empty({0}, x.options().dtype(at::kFloat));
     CastScale cs;
     if (is_fp8(x.scalar_type())) {
       cs.outer = x.numel();  // fp8 -> same fp8: copy, scale plays no part
     } else {
       cs = resolve_cast_scale(scale, scale_shape, x);
     }
-    check_status(launch_cast_to(x, out, cs, is_amax ? amax.data_ptr<float>() : nullptr, sr), "mi355q_cast_to_fp8");
+    check_status(launch_cast_to(x, out, cs, is_amax ? amax.data_ptr<float>() : nullptr, sr, zeroed), "mi355q_cast_to_fp8");
   }
   torch::jit::drop(*stack, 6);
   stack->emplace_back(std::move(out));
@@ -323,70 +424,6 @@ Tensor cast_from_fp8_scalar(const Tensor& input, double scale, at::ScalarType ou
 Tensor cast_from_fp8_scalar_list(const Tensor& input, c10::ArrayRef<double> scale,
                                  at::ScalarType out_dtype, at::OptionalIntArrayRef scale_shape) {
   return cast_from_fp8_impl(input, IValue(scale.vec()), out_dtype, to_opt_shape(scale_shape));
-}
-
-// --------------------------------------------------------- kept workspaces
-//
-// Kernels that split a reduction over workgroups (the K split of the GEMMs for few rows and of the 4-bit GEMMs, the
-// key splits of the attention kernel for few queries) keep arrival counters in their workspace, which have to be zero
-// when a call starts and are left zero by every call: one zero-filled buffer per (device, stream, op) is kept here and
-// grown on demand, so that a call launches one kernel and nothing else.  Calls on one stream run in order, which is
-// all the sharing the buffer allows; the ops lay their counters out differently and do not share.  At most
-// kKeptWorkspaces buffers are kept: past that the one that was used least recently is given back (to the caching
-// allocator, which hands it out again only to work queued behind what still uses it).  While a stream is being captured into a graph no kept
-// buffer is handed out (its memory would belong to the graph's pool, and replays of two graphs could overlap): the
-// call takes a buffer of the graph's own and clears its counters with a fill kernel that is part of the graph
-// (captured_ticket_workspace).
-enum TicketWorkspaceOp { kWsW4a8 = 0, kWsSdpa = 1, kWsW4a16 = 2, kWsGemm = 3 };
-constexpr size_t kKeptWorkspaces = 64;
-struct TicketWorkspaceCache {
-  struct Entry {
-    Tensor buffer;
-    uint64_t used = 0;
-  };
-  std::mutex mu;
-  uint64_t clock = 0;
-  std::map<std::tuple<int, void*, int>, Entry> map;
-};
-TicketWorkspaceCache& ticket_workspace_cache() {
-  // never destroyed: a static Tensor would be freed after the HIP runtime has shut down
-  static auto* cache = new TicketWorkspaceCache();
-  return *cache;
-}
-bool stream_is_capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
-// Undefined for bytes == 0 (the problem does not split).
-Tensor ticket_workspace(const Tensor& like, size_t bytes, TicketWorkspaceOp op) {
-  if (bytes == 0 || stream_is_capturing()) return Tensor();
-  TicketWorkspaceCache& c = ticket_workspace_cache();
-  std::lock_guard<std::mutex> lock(c.mu);
-  const auto key = std::make_tuple((int)like.device().index(), current_stream(like), (int)op);
-  TicketWorkspaceCache::Entry& e = c.map[key];
-  e.used = ++c.clock;
-  if (!e.buffer.defined() || (size_t)e.buffer.numel() < bytes) e.buffer = at::zeros({(int64_t)bytes}, like.options().dtype(at::kByte));
-  Tensor t = e.buffer;
-  if (c.map.size() > kKeptWorkspaces) {
-    auto oldest = c.map.begin();
-    for (auto it = c.map.begin(); it != c.map.end(); ++it)
-      if (it->second.used < oldest->second.used) oldest = it;
-    c.map.erase(oldest);
-  }
-  return t;
-}
-// While the stream is being captured: a buffer out of the graph's pool, its counters (the first `counters` bytes)
-// zeroed by a small fill kernel, which every replay runs again; the rest (partial sums that are written before they
-// are read) as it comes.
-Tensor captured_ticket_workspace(const Tensor& like, size_t bytes, int64_t counters) {
-  Tensor t = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
-  t.narrow(0, 0, std::min<int64_t>((int64_t)bytes, counters)).zero_();
-  return t;
-}
-// After a call that used the buffer has failed: its counters may be left non-zero (no workgroup then draws a
-// group's last ticket and the output stays unwritten), so the buffer is dropped and the next call starts from a
-// zero-filled one.
-void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
-  TicketWorkspaceCache& c = ticket_workspace_cache();
-  std::lock_guard<std::mutex> lock(c.mu);
-  c.map.erase(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
 }
 
 // --------------------------------------------------------------- fp8_gemm_v2

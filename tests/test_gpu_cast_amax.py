@@ -1,0 +1,56 @@
+"""cast_to_fp8 with amax at the edges of its launch shapes (one workgroup, up to 2^21 elements, one logical block per
+workgroup, several), many calls in a row (amax words are handed out from cleared blocks), streams, and the C entry that
+raises a running maximum."""
+import ctypes
+
+import pytest
+import torch
+
+from helpers import E4
+
+pytestmark = pytest.mark.gpu
+SIZES = [1, 8, 4096, 16384, 16392, 2 ** 21, 2 ** 21 + 8, 2 ** 23, 2 ** 23 + 40, 2 ** 24 + 3]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_amax_and_codes(oracle, dev, n, dtype):
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n, generator=g).to(dtype)
+    x[torch.randint(0, n, (1,), generator=g)] = -7.25  # the maximum somewhere
+    scale = torch.tensor(40.0)
+    y, amax = torch.ops.hpu.cast_to_fp8_v2(x.to(dev), scale.to(dev), False, True, E4)
+    y_ref, _ = oracle.c_cast_to_fp8(x, scale, E4, True)
+    assert amax.shape == () and amax.item() == 7.25
+    assert torch.equal(y.cpu().view(torch.uint8), y_ref.view(torch.uint8))
+
+
+def test_every_call_has_its_own_word(dev):
+    """More calls than a block of words holds, on two streams, all results kept."""
+    xs = [torch.full((5,), float(i + 1), device=dev).bfloat16() for i in range(8)]
+    side = torch.cuda.Stream()
+    got = []
+    for i in range(600):
+        if i % 3 == 2:
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                got.append((i, torch.ops.hpu.cast_to_fp8_v2(xs[i % 8], None, False, True, E4)[1]))
+        else:
+            got.append((i, torch.ops.hpu.cast_to_fp8_v2(xs[i % 8], None, False, True, E4)[1]))
+    torch.cuda.synchronize()
+    assert all(a.item() == i % 8 + 1 for i, a in got)
+    got[0][1].fill_(99.0)  # writing to one result leaves the others alone
+    assert all(a.item() == i % 8 + 1 for i, a in got[1:])
+
+
+def test_running_maximum(pkg, dev):
+    lib = pkg.capi()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    am = torch.tensor([2.0], device=dev)
+    y = torch.empty(64, dtype=E4, device=dev)
+    for top, want in ((1.0, 2.0), (3.5, 3.5), (0.25, 3.5)):
+        x = torch.full((64,), -top, device=dev)
+        assert lib.mi355q_cast_to_fp8_running_amax(x.data_ptr(), pkg.F32, y.data_ptr(), pkg.E4M3FN, None, 1.0, pkg.SCALE_NONE, 64, 1, 1,
+                                                   am.data_ptr(), st) == 0
+        assert am.item() == want
+    assert lib.mi355q_cast_to_fp8_running_amax(x.data_ptr(), pkg.F32, y.data_ptr(), pkg.E4M3FN, None, 1.0, pkg.SCALE_NONE, 64, 1, 1, None, st) != 0
