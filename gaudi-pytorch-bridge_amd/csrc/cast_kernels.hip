@@ -567,6 +567,39 @@ __global__ __launch_bounds__(kThreads) void split_rows_vec_kernel(const uint16_t
   }
 }
 
+// Bytes c .. c + 15 of a row of `bytes` bytes that starts anywhere; zeros past its end.  One unaligned 16-byte load: the
+// chunk that reaches past the row's end is read so that it ends with the row and shifted into place, so nothing
+// outside the row is touched (rows shorter than a chunk: byte by byte).
+struct __attribute__((packed, aligned(1))) UnalignedChunk {
+  u32x4 v;
+};
+__device__ __forceinline__ u32x4 ragged_chunk(const uint8_t* row, int c, int bytes) {
+  const int n = bytes - c;
+  if (bytes < 16) {
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+    for (int i = 0; i < n; ++i) w[i >> 2] |= (uint32_t)row[c + i] << (8 * (i & 3));
+    return u32x4{w[0], w[1], w[2], w[3]};
+  }
+  const int back = n < 16 ? 16 - n : 0;
+  const u32x4 v = reinterpret_cast<const UnalignedChunk*>(row + c - back)->v;
+  if (back == 0) return v;
+  const int words = back >> 2, bits = 8 * (back & 3);
+  const uint32_t w[8] = {v[0], v[1], v[2], v[3], 0u, 0u, 0u, 0u};
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (k == words) {
+        lo = w[i + k];
+        hi = w[i + k + 1];
+      }
+    o[i] = (uint32_t)((((uint64_t)hi << 32) | lo) >> bits);
+  }
+  return o;
+}
+
 // ------------------------------------------------- dynamic per-row quantisation
 //
 // One pass of "per-row amax -> scale = target / amax -> cast with that scale":
@@ -657,6 +690,59 @@ __global__ __launch_bounds__(kMaxRowThreads) void quantize_rows_kernel(
       const uint32_t o = row_cvt_fp8x4<FMT, SAT>(__uint_as_float(in[u][0]) * s, __uint_as_float(in[u][1]) * s,
                                                  __uint_as_float(in[u][2]) * s, __uint_as_float(in[u][3]) * s);
       __builtin_amdgcn_raw_buffer_store_b32(o, rout, off, 0, 2);
+    }
+  }
+}
+
+// The same for rows that are no whole number of vectors or start at any address: unaligned 16-byte loads and 8-byte
+// stores, a row's last few codes byte by byte.  (As separate operations, row maxima, division and a cast an element per
+// thread, such a call kept the host busy for 28 us.)
+template <bool BF16_IN, int FMT>
+__global__ __launch_bounds__(kMaxRowThreads) void quantize_ragged_rows_kernel(
+    const uint8_t* __restrict__ x, uint8_t* __restrict__ y, int cols, float target,
+    float* __restrict__ scale_out, float* __restrict__ scale_inv_out) {
+  constexpr int ES = BF16_IN ? 2 : 4, EPV = 16 / ES, VPT = 2;
+  const int64_t row = blockIdx.x;
+  const int threads = (int)blockDim.x;
+  const uint8_t* xr = x + row * cols * ES;
+  uint8_t* yr = y + row * cols;
+  u32x4 in[VPT];
+  uint32_t am = 0;
+#pragma unroll
+  for (int u = 0; u < VPT; ++u) {
+    const int e = ((int)threadIdx.x + u * threads) * EPV;
+    in[u] = e < cols ? ragged_chunk(xr, e * ES, cols * ES) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w = in[u][i];
+      const uint32_t a = BF16_IN ? (w << 16) & 0x7fffffffu : w & 0x7fffffffu, b = BF16_IN ? w & 0x7fff0000u : 0u;
+      am = am > a ? am : a;
+      am = am > b ? am : b;
+    }
+  }
+  const float scale = row_scale_of_block(am, target, row, scale_out, scale_inv_out);
+  const float s = BF16_IN ? round_to_bf16(scale) : scale;
+#pragma unroll
+  for (int u = 0; u < VPT; ++u) {
+    const int e = ((int)threadIdx.x + u * threads) * EPV, n = cols - e;
+    if (n <= 0) continue;
+    float p[EPV];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (BF16_IN) {
+        p[2 * i] = round_to_bf16(__uint_as_float(in[u][i] << 16) * s);
+        p[2 * i + 1] = round_to_bf16(__uint_as_float(in[u][i] & 0xffff0000u) * s);
+      } else {
+        p[i] = __uint_as_float(in[u][i]) * s;
+      }
+    }
+    uint32_t o[EPV / 4];
+#pragma unroll
+    for (int i = 0; i < EPV / 4; ++i) o[i] = cvt_fp8x4<FMT>(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
+    if (n >= EPV) {
+      __builtin_memcpy(yr + e, o, EPV);
+    } else {
+      for (int i = 0; i < n; ++i) yr[e + i] = (uint8_t)(o[i >> 2] >> (8 * (i & 3)));
     }
   }
 }
@@ -859,6 +945,56 @@ __global__ __launch_bounds__(kThreads) void copy_vec16_kernel(const uint8_t* __r
 #pragma unroll
   for (int u = 0; u < kCopyU; ++u)
     __builtin_amdgcn_raw_buffer_store_b128(t[u], rout, ((int)threadIdx.x + u * kThreads) * 16, 0, 2);
+}
+
+// ------------------------------------------------------------- padded copies
+//
+// Byte matrices whose rows start at any address, copied into rows of whole 16-byte chunks with zeros behind the data
+// (what the GEMM's MFMA kernels take): both operands of a product in one launch.  A thread writes kPadU chunks of the
+// destination and reads each with one unaligned 16-byte load; the last chunk of a row is read so that it ends with
+// the row and shifted into place, so nothing outside the matrix is touched.
+struct PadJob {
+  const uint8_t* src;
+  uint8_t* dst;
+  int64_t src_ld, src_stride, dst_stride;  // bytes
+  int32_t rows, cols, dst_rows, dst_chunks;
+  int32_t batch;
+  int64_t chunks;                          // of all matrices
+};
+struct PadJobs {
+  PadJob job[2];
+};
+constexpr int kPadU = 4;
+
+// The chunk `k` chunks behind the start of row `row0` (of all matrices' rows).
+__device__ __forceinline__ u32x4 pad_chunk(const PadJob& j, int64_t row0, uint32_t k) {
+  const uint32_t down = k / (uint32_t)j.dst_chunks;
+  const int c = (int)(k - down * (uint32_t)j.dst_chunks) * 16;
+  const int64_t row_all = row0 + down;
+  int64_t b = 0, r = row_all;
+  if (j.batch > 1) {
+    b = row_all / j.dst_rows;
+    r = row_all - b * j.dst_rows;
+  }
+  if (r >= j.rows || c >= j.cols) return u32x4{0u, 0u, 0u, 0u};
+  return ragged_chunk(j.src + b * j.src_stride + r * j.src_ld, c, j.cols);
+}
+
+__global__ __launch_bounds__(kThreads) void pad_rows_kernel(PadJobs jobs, int64_t blocks0) {
+  const bool second = blockIdx.x >= blocks0;
+  const PadJob& j = jobs.job[second ? 1 : 0];
+  const int64_t start = ((int64_t)blockIdx.x - (second ? blocks0 : 0)) * (kThreads * kPadU), first = start + threadIdx.x;
+  const int64_t row0 = start / j.dst_chunks;
+  const uint32_t k0 = (uint32_t)(start - row0 * j.dst_chunks) + threadIdx.x;
+  u32x4 v[kPadU];
+#pragma unroll
+  for (int u = 0; u < kPadU; ++u)
+    v[u] = first + u * kThreads < j.chunks ? pad_chunk(j, row0, k0 + u * kThreads) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int u = 0; u < kPadU; ++u) {
+    const int64_t chunk = first + u * kThreads;
+    if (chunk < j.chunks) *reinterpret_cast<u32x4*>(j.dst + chunk * 16) = v[u];
+  }
 }
 
 // --------------------------------------------------------------- host helpers
@@ -1214,12 +1350,22 @@ int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
   if (x == nullptr || y == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
   if (rows > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
   const int epv = x_dtype == MI355Q_BF16 ? 8 : 4;
-  // whole 16-byte vectors only; the row has to fit the registers of one workgroup
-  if (cols % epv != 0 || !aligned(x, 16) || !aligned(y, epv)) return MI355Q_ERR_UNSUPPORTED;
-  const int64_t vpr = cols / epv;
+  const int64_t vpr = (cols + epv - 1) / epv;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint8_t* xb = static_cast<const uint8_t*>(x);
   uint8_t* yb = static_cast<uint8_t*>(y);
+  if (cols % epv != 0 || !aligned(x, 16) || !aligned(y, epv)) {
+    if (vpr > kMaxRowVectors || !aligned(x, epv == 8 ? 2 : 4)) return MI355Q_ERR_UNSUPPORTED;
+    const unsigned grid = (unsigned)rows, threads = (unsigned)(((vpr + 1) / 2 + 63) / 64 * 64);
+    if (x_dtype == MI355Q_BF16) {
+      if (fp8_fmt == MI355Q_E4M3FN) quantize_ragged_rows_kernel<true, MI355Q_E4M3FN><<<grid, threads, 0, st>>>(xb, yb, (int)cols, target, scale_out, scale_inv_out);
+      else quantize_ragged_rows_kernel<true, MI355Q_E5M2><<<grid, threads, 0, st>>>(xb, yb, (int)cols, target, scale_out, scale_inv_out);
+    } else {
+      if (fp8_fmt == MI355Q_E4M3FN) quantize_ragged_rows_kernel<false, MI355Q_E4M3FN><<<grid, threads, 0, st>>>(xb, yb, (int)cols, target, scale_out, scale_inv_out);
+      else quantize_ragged_rows_kernel<false, MI355Q_E5M2><<<grid, threads, 0, st>>>(xb, yb, (int)cols, target, scale_out, scale_inv_out);
+    }
+    return launch_status();
+  }
   if (x_dtype == MI355Q_BF16) {
     if (fp8_fmt == MI355Q_E4M3FN) return quantize_rows_launch<true, MI355Q_E4M3FN>(xb, yb, rows, vpr, target, scale_out, scale_inv_out, st);
     return quantize_rows_launch<true, MI355Q_E5M2>(xb, yb, rows, vpr, target, scale_out, scale_inv_out, st);
@@ -1320,6 +1466,37 @@ int mi355q_cast_from_fp8(const void* x, int fp8_fmt, void* y, int out_dtype, con
   }
   if (out_dtype == MI355Q_BF16) return cast_from_dispatch<MI355Q_E5M2, true>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, st);
   return cast_from_dispatch<MI355Q_E5M2, false>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, st);
+}
+
+int mi355q_pad_rows(const mi355q_pad_desc* desc, int count, void* stream) {
+  if (desc == nullptr || count < 1 || count > 2) return MI355Q_ERR_INVALID_ARGUMENT;
+  PadJobs jobs{};
+  int64_t blocks[2] = {0, 0};
+  for (int i = 0; i < count; ++i) {
+    const mi355q_pad_desc& d = desc[i];
+    if (d.batch < 0 || d.rows < 0 || d.cols < 0 || d.dst_rows < d.rows || d.dst_ld < d.cols || d.dst_ld % 16 || d.src_ld < d.cols)
+      return MI355Q_ERR_INVALID_ARGUMENT;
+    if (d.batch == 0 || d.dst_rows == 0 || d.dst_ld == 0) continue;
+    if (d.dst == nullptr || !aligned(d.dst, 16) || (d.rows > 0 && d.cols > 0 && d.src == nullptr)) return MI355Q_ERR_INVALID_ARGUMENT;
+    if (d.rows > 0x7fffffffLL || d.dst_rows > 0x7fffffffLL || d.dst_ld > 0x7fffffffLL || d.batch > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
+    PadJob& j = jobs.job[i];
+    j.src = static_cast<const uint8_t*>(d.src);
+    j.dst = static_cast<uint8_t*>(d.dst);
+    j.src_ld = d.src_ld;
+    j.src_stride = d.src_stride;
+    j.dst_stride = d.dst_rows * d.dst_ld;
+    j.rows = (int32_t)d.rows;
+    j.cols = (int32_t)d.cols;
+    j.dst_rows = (int32_t)d.dst_rows;
+    j.dst_chunks = (int32_t)(d.dst_ld / 16);
+    j.batch = (int32_t)d.batch;
+    j.chunks = d.batch * d.dst_rows * (d.dst_ld / 16);
+    blocks[i] = (j.chunks + kThreads * kPadU - 1) / (kThreads * kPadU);
+  }
+  if (blocks[0] + blocks[1] == 0) return MI355Q_OK;
+  if (blocks[0] + blocks[1] > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
+  pad_rows_kernel<<<(unsigned)(blocks[0] + blocks[1]), kThreads, 0, static_cast<hipStream_t>(stream)>>>(jobs, blocks[0]);
+  return launch_status();
 }
 
 }  // extern "C"

@@ -105,8 +105,9 @@ int mi355q_rowwise_amax(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * quantises activations on the fly.  The reference has no such op
  * (fp8_ops.cpp:170-178: its amax is one scalar and the scale is computed by
  * the caller).  Rows of up to 2048 16-byte vectors (16384 bf16 / 8192 fp32
- * elements), x 16-byte aligned, cols a multiple of 8 (bf16) or 4 (fp32);
- * otherwise MI355Q_ERR_UNSUPPORTED and the caller takes the three-step route.
+ * elements), x aligned to its elements; fastest where x is 16-byte aligned and
+ * cols a multiple of 8 (bf16) or 4 (fp32).  Longer rows:
+ * MI355Q_ERR_UNSUPPORTED, and the caller takes the three-step route.
  */
 int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
                          void* y, int fp8_fmt, float target,
@@ -465,6 +466,23 @@ int mi355q_fp8_sdpa_fwd(const void* q, const void* k, const void* v, int fp8_fmt
                         float softmax_scale, int is_causal, const float* const* scale_dev,
                         const float* scale_host, float* amax_s, float* amax_o, void* workspace,
                         size_t workspace_bytes, void* stream);
+
+/*
+ * Byte matrices whose rows may start anywhere, copied into rows of whole
+ * 16-byte chunks with zeros behind the data: what a caller of mi355q_fp8_gemm
+ * does with operands that miss its alignment rules (zeros along K add nothing).
+ * One launch for one or two operands (count).
+ *   src  `batch` matrices src_stride bytes apart of [rows, cols] bytes, row
+ *        pitch src_ld >= cols, any alignment
+ *   dst  `batch` matrices of [dst_rows, dst_ld] bytes, one after the other;
+ *        dst_rows >= rows, dst_ld >= cols a multiple of 16, 16-byte aligned
+ */
+typedef struct mi355q_pad_desc {
+  const void* src;
+  void* dst;
+  int64_t batch, rows, cols, src_ld, src_stride, dst_rows, dst_ld;
+} mi355q_pad_desc;
+int mi355q_pad_rows(const mi355q_pad_desc* desc, int count, void* stream);
 
 /* Name of the kernel variant mi355q_fp8_gemm would pick for a problem
  * (for logs and profiles; static string). */
