@@ -1,7 +1,6 @@
 // fp8_gemm_v2 C entry point: argument checks, kernel choice, and the any-shape
 // fallback kernel.  The MFMA tile kernels live in gemm_tile.h.
 #include <algorithm>
-#include <cmath>
 
 #include "gemm_dispatch.h"
 
@@ -80,9 +79,39 @@ inline bool tiled_ok(const void* A, int trans_a, int64_t lda, const void* B, int
 //  * in the strip kernel A's tile travels along (a quarter of its bytes count with a K-major B, half with the shorter
 //    pieces of an MN-major one);
 //  * fixed costs, and with more than one part the meeting: each part's sums out, and all of them into the last one.
+//
+// More than 128 rows (tile_split_plan): the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where that beats
+// the unsplit launch by 10 % and 2 us (short products whose weights sit in the Infinity Cache are that much faster than
+// tile_us says); the fits are those of tile_us with 4.5 us for the first meeting of 128 x 128 sums and
+// 3.5 for each further one (6.5 each at 256 x 128).
+SplitPlan tile_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  SplitPlan best;
+  const int64_t cus = compute_units(), pairs = (K + 2 * kBK - 1) / (2 * kBK);
+  const TileChoice whole = N > 128 ? choose_tiles(M, N, K, batch) : TileChoice::k128x128;
+  if (whole == TileChoice::k256x256 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= cus) return best;
+  double best_us = 0.9 * tile_us(whole, M, N, K, batch) - 2.0;
+  for (const int64_t bm : {128, 256}) {
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + 127) / 128);
+    for (int64_t parts = 2; parts <= pairs && parts * tiles * batch <= cus; ++parts) {
+      const double stages = 2.0 * (double)((pairs + parts - 1) / parts), levels = std::ceil(std::log2((double)parts));
+      const double us = bm == 128 ? stages * 0.8 + 6.0 + 3.5 * levels : stages * 1.06 + 5.0 + 6.5 * levels;
+      if (us >= best_us) continue;
+      best_us = us;
+      best.tile = bm == 128 ? SplitTile::k128x128 : SplitTile::k256x128;
+      best.nb = 128;
+      best.strips = (int)tiles;
+      best.parts = (int)parts;
+      best.tile_rows = bm;
+      best.batch = batch;
+    }
+  }
+  return best;
+}
+
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
   SplitPlan best;
-  if (M > 128 || M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
+  if (M > 128) return may_split ? tile_split_plan(M, N, K, batch) : best;
   const double cus = (double)compute_units();
   double best_us = 0.0;
   auto consider = [&](bool stream, int64_t nb, int64_t tile_rows, int64_t unit) {
@@ -123,7 +152,7 @@ const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64
                                     int64_t N, int64_t K) {
   if (lda % 16 || ldb % 16 || !mi355q::k_chunks_ok(trans_a, trans_b, K)) return "simple";
   if (M > 128 && N > 128) {
-    switch (mi355q::choose_tiles(M, N, 1)) {
+    switch (mi355q::choose_tiles(M, N, K, 1)) {
       case mi355q::TileChoice::k256x256: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
       case mi355q::TileChoice::k256x128: return "tile256x128x128_mfma32x32x64";
       case mi355q::TileChoice::k128x128: return "tile128x128x128_mfma32x32x64";
@@ -215,13 +244,14 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const
     gb.fast_epi = epilogue_fast_ok(gb, nb);
     if (tiled_ok(gb.A, trans_a, lda, gb.B, trans_b, ldb, M, N, K, stride_a, stride_b)) {
       const bool ak = !trans_a, bk = trans_b != 0;
-      // (few rows: K is walked in parts if the caller brought the room where they meet)
+      // (K is walked in parts if the caller brought the room where they meet)
       const SplitPlan plan = split_plan(ak, lda, bk, ldb, M, N, K, nb, workspace != nullptr && nb == batch);
       SplitArgs split{plan.parts, nullptr, nullptr};
       if (plan.parts > 1) {
         if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;
         split.tickets = static_cast<uint32_t*>(workspace);
         split.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
+        split.tile = plan.tile;
       }
       if (plan.stream) launch_gemm_stream(gb, fmt_a, fmt_b, plan, split, nb, st);
       else if (ak && bk) launch_gemm_kk(gb, split, fmt_a, fmt_b, nb, st);

@@ -1,5 +1,5 @@
 // The meeting of workgroups that each hold one part of K of the same columns of C (split K), used by the kernels for
-// few rows of A.
+// few rows of A; gemm_tile_split.h has the form for the larger tiles.
 //
 // A workgroup stores its fp32 sums with device-scope atomic accesses, which go past the caches of its XCD to the level
 // of memory that all XCDs share (no cache is written back or invalidated as a whole, which a fence would do), waits
@@ -20,19 +20,23 @@ constexpr int kTicketStride = 16;                         // 32-bit words: one c
 constexpr size_t kTicketBytes = 64 * 1024;                // the counters' area, in front of the sums, the same for every shape
 constexpr int kMaxTickets = (int)(kTicketBytes / (kTicketStride * 4));
 
+enum class SplitTile { kStrip, k128x128, k256x128 };  // kStrip: the kernels for at most 128 rows
+
 struct SplitArgs {
-  int parts;           // workgroups that share a strip of C, one part of K each
+  int parts;           // workgroups that share a strip or tile of C, one part of K each
   uint32_t* tickets;   // counters, zero between launches
   float* partials;
+  SplitTile tile = SplitTile::kStrip;
 };
 
-// How a product of at most 128 rows of A is cut.
+// How a product is cut.
 struct SplitPlan {
   bool stream = false;       // the kernel of gemm_stream.h (else the strip kernel of gemm_skinny.h)
-  int nb = 0;                // columns per strip; 0: neither kernel (M > 128)
-  int strips = 0, parts = 1;
+  int nb = 0;                // columns per strip or tile; 0: not cut, and more than 128 rows
+  int strips = 0, parts = 1;   // strips, or tiles
   int64_t tile_rows = 0;     // rows of sums a workgroup leaves in the workspace
   int64_t batch = 1;
+  SplitTile tile = SplitTile::kStrip;
   size_t workspace_bytes() const {
     return parts < 2 ? 0 : kTicketBytes + (size_t)parts * strips * batch * tile_rows * nb * sizeof(float);
   }

@@ -249,8 +249,8 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda,
                     void* stream);
 
 /*
- * The same with a workspace.  Products of at most 128 rows of A are bound by
- * streaming B; where N alone does not give every compute unit a share of it,
+ * The same with a workspace.  Where the strips or tiles of C do not give every
+ * compute unit work (few rows of A, or up to a few thousand with a narrow N),
  * K is walked in parts by several workgroups whose fp32 sums meet through
  * `workspace` (device memory, 16-byte aligned, at least
  * mi355q_fp8_gemm_workspace_bytes() bytes; 0: the problem does not split).
