@@ -284,15 +284,16 @@ void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
   c.map.erase(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
 }
 
-// Zeroed words for results that kernels accumulate into (amax), so that a call needs no launch that clears one: a
-// block of them is cleared at once, per (device, stream), and every word is handed out once, as a tensor that shares
-// the block's memory; words are a cache line apart.  Not while the stream is being captured (a replay would find the
-// word as the last one left it).
+// Zeroed words for results that kernels accumulate into (amax), so that a call needs no launch that clears one:
+// kWords of them are cleared by one launch, per (device, stream), and each is handed out once.  Every word is an
+// allocation of its own and becomes a tensor only when it is handed out, so that what a caller gets is what at::empty
+// would give: its own storage (it can be saved, resized, recorded on a stream), its own version counter, and an
+// inference tensor or not by the mode of the call that gets it.  Not while the stream is being captured (a replay
+// would find the word as the last one left it).
 struct ZeroWords {
-  static constexpr int64_t kWords = 256, kStride = 16;
+  static constexpr int64_t kWords = 64;  // what one launch of _foreach_zero_ takes
   struct Entry {
-    Tensor block;
-    int64_t next = kWords;
+    std::vector<c10::Storage> words;
     uint64_t used = 0;
   };
   std::mutex mu;
@@ -301,15 +302,24 @@ struct ZeroWords {
 };
 Tensor zero_word(const Tensor& like) {
   static auto* z = new ZeroWords();  // never destroyed, as above
-  std::lock_guard<std::mutex> lock(z->mu);
-  ZeroWords::Entry& e = z->map[std::make_pair((int)like.device().index(), current_stream(like))];
-  e.used = ++z->clock;
-  if (e.next == ZeroWords::kWords) {
-    e.block = at::zeros({ZeroWords::kWords * ZeroWords::kStride}, like.options().dtype(at::kFloat));
-    e.next = 0;
+  c10::Storage storage;
+  {
+    std::lock_guard<std::mutex> lock(z->mu);
+    ZeroWords::Entry& e = z->map[std::make_pair((int)like.device().index(), current_stream(like))];
+    e.used = ++z->clock;
+    if (e.words.empty()) {
+      std::vector<Tensor> fresh;
+      for (int64_t i = 0; i < ZeroWords::kWords; ++i) fresh.push_back(at::empty({}, like.options().dtype(at::kFloat)));
+      at::_foreach_zero_(fresh);
+      for (const Tensor& t : fresh) e.words.push_back(t.storage());
+    }
+    storage = std::move(e.words.back());
+    e.words.pop_back();
+    if (z->map.size() > kKeptWorkspaces) drop_least_recent(z->map);
   }
-  Tensor word = e.block.as_strided({}, {}, ZeroWords::kStride * e.next++);
-  if (z->map.size() > kKeptWorkspaces) drop_least_recent(z->map);
+  Tensor word = at::detail::make_tensor<c10::TensorImpl>(std::move(storage), c10::DispatchKeySet(c10::DispatchKey::CUDA),
+                                                         caffe2::TypeMeta::Make<float>());
+  word.unsafeGetTensorImpl()->set_sizes_contiguous({});
   return word;
 }
 

@@ -1,5 +1,5 @@
 """cast_to_fp8 with amax at the edges of its launch shapes (one workgroup, up to 2^21 elements, one logical block per
-workgroup, several), many calls in a row (amax words are handed out from cleared blocks), streams, and the C entry that
+workgroup, several), many calls in a row (zeroed words are cleared many at a time), streams, and the C entry that
 raises a running maximum."""
 import ctypes
 
@@ -26,7 +26,7 @@ def test_amax_and_codes(oracle, dev, n, dtype):
 
 
 def test_every_call_has_its_own_word(dev):
-    """More calls than a block of words holds, on two streams, all results kept."""
+    """More calls than one launch clears words for, on two streams, all results kept."""
     xs = [torch.full((5,), float(i + 1), device=dev).bfloat16() for i in range(8)]
     side = torch.cuda.Stream()
     got = []
@@ -41,6 +41,23 @@ def test_every_call_has_its_own_word(dev):
     assert all(a.item() == i % 8 + 1 for i, a in got)
     got[0][1].fill_(99.0)  # writing to one result leaves the others alone
     assert all(a.item() == i % 8 + 1 for i, a in got[1:])
+
+
+def test_amax_is_an_ordinary_tensor(dev):
+    """Whatever mode the words were cleared in: own storage and version, resizable, an inference tensor only by the call's own mode."""
+    x = torch.tensor([-3.0, 1.0], device=dev).bfloat16()
+    call = lambda: torch.ops.hpu.cast_to_fp8_v2(x, None, False, True, E4)[1]  # noqa: E731
+    for _ in range(70):
+        with torch.inference_mode():
+            inside = call()
+        first, second = call(), call()
+        assert inside.is_inference() and not first.is_inference()
+        assert first.untyped_storage().nbytes() == 4 and first.storage_offset() == 0 and first._base is None
+        version = second._version
+        first.mul_(2)  # refused for an inference tensor
+        assert second._version == version
+        first.resize_(100).fill_(-1.0)
+        assert second.item() == 3.0 and inside.item() == 3.0
 
 
 def test_running_maximum(pkg, dev):
