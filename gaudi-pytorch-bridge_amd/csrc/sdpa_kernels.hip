@@ -701,60 +701,131 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
 // what is split: over `nsplit` workgroups, and inside a workgroup over its four waves, block by
 // block.  Each wave streams its own blocks through LDS stages of its own (no barrier in the loop)
 // and keeps its own running maximum, sum and O; the four are merged through LDS at the end, and
-// the splits' results (unnormalised O, m, l per row) through a workspace by a second small kernel.
+// the splits' results (unnormalised O, m, l per row) through a workspace (sdpa_decode_finish).
 
 constexpr int kDecodeTileFloats(int DVT) { return 32 * DVT * 32 + 64; }  // O^T [dv][row], m[row], l[row]
 
-// merges `n` partial results for row `row`, columns dv0, dv0 + dvstep, ...; returns the row's 1 / l
-// (0 for a row with nothing to attend to) and leaves the merged, normalised values in `val`
-template <int DVT>
-__device__ __forceinline__ float sdpa_merge(const float* parts, int n, int stride_floats, int row, int dv0, int dvstep, float qs,
-                                            float (&val)[DVT * 32 / 8]) {
-  float M = -__builtin_inff();
-  for (int w = 0; w < n; ++w) M = __builtin_fmaxf(M, parts[(int64_t)w * stride_floats + 32 * DVT * 32 + row]);
-  float L = 0.0f;
+// The end of a workgroup of the decoding kernel: merge the four waves' results (LDS, [dv][32 rows], then m and l), exchange
+// them with the other splits, store the rows.  R: the tile's rows that hold queries, rounded up to 8, 16 or 32; the threads
+// are laid over those alone (row tid % R, columns tid / R, + 256 / R, ...), so the rest is neither merged nor sent.
+// What bounds it is latency: a store, a ticket and a read, each a trip to the memory level that the XCDs share, while
+// nothing else runs.  So the last workgroup has the results of four splits on their way at a time, their maxima with them
+// (one split after the other was a trip each, and one more for each maximum).  Against that and all 32 rows merged and
+// sent: 8 x 8192 keys, 8 key / value heads of 4 queries (4 splits), 31.9 -> 28.2 us, 4.2 -> 4.8 TB/s, the same bits.
+template <int DVT, int R>
+__device__ __forceinline__ void sdpa_decode_finish(const SdpaArgs& a, uint8_t* lds, int64_t grp, int split, int64_t o_off, float qs) {
+  constexpr int kTile = kDecodeTileFloats(DVT), kML = 32 * DVT * 32;  // m[row] from kML on, l[row] 32 further
+  constexpr int STEP = kSdpaThreads / R, NV = DVT * 32 / STEP;
+  const int tid = threadIdx.x, row = tid & (R - 1), dv0 = tid / R;
+  const float* parts = reinterpret_cast<const float*>(lds);
+  float M = -__builtin_inff(), L = 0.0f, val[NV];
+  for (int w = 0; w < 4; ++w) M = __builtin_fmaxf(M, parts[w * kTile + kML + row]);
 #pragma unroll
-  for (int i = 0; i < DVT * 32 / 8; ++i) val[i] = 0.0f;
-  for (int w = 0; w < n; ++w) {
-    const float* pw = parts + (int64_t)w * stride_floats;
-    const float mw = pw[32 * DVT * 32 + row];
+  for (int i = 0; i < NV; ++i) val[i] = 0.0f;
+  for (int w = 0; w < 4; ++w) {
+    const float* pw = parts + w * kTile;
+    const float mw = pw[kML + row];
     const float wgt = mw == -__builtin_inff() ? 0.0f : fast_exp2(mw - M);
-    L += pw[32 * DVT * 32 + 32 + row] * wgt;
+    L += pw[kML + 32 + row] * wgt;
 #pragma unroll
-    for (int i = 0; i < DVT * 32 / 8; ++i) val[i] += pw[(dv0 + i * dvstep) * 32 + row] * wgt;
+    for (int i = 0; i < NV; ++i) val[i] += pw[(dv0 + i * STEP) * 32 + row] * wgt;
   }
-  const float l = L / qs;
-  const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
+  if (a.nsplit > 1) {
+    // Unnormalised: the merged maximum, the merged sum and O of this split go to the workspace; the workgroup
+    // that draws the group's last ticket merges the splits in their order, whoever came last, and stores the
+    // rows.  The partial results are written and read with device-scope atomic accesses, which go past this
+    // XCD's cache to where the other XCDs see them: no cache has to be written back or invalidated as a whole,
+    // which a fence would do.  The last one returns the counter to zero for the next launch.
+    float* group_parts = a.ws + (int64_t)grp * a.nsplit * kTile;
+    float* out = group_parts + (int64_t)split * kTile;
+    if (row < a.rows) {
 #pragma unroll
-  for (int i = 0; i < DVT * 32 / 8; ++i) val[i] *= inv_l;
-  return inv_l;
-}
-
-// final scaling, rounding and store of one row's merged values (columns dv0 + i dvstep), amax updates
-template <int DVT>
-__device__ __forceinline__ void sdpa_store_row(const SdpaArgs& a, uint8_t* orow, bool row_ok, float inv_l, int dv0, int dvstep,
-                                               const float (&val)[DVT * 32 / 8]) {
-  const float dv = sdpa_scale(a, 2, 1.0f), qs = sdpa_scale(a, 3, 1.0f), ds = sdpa_scale(a, 5, 1.0f / qs);
+      for (int i = 0; i < NV; ++i) __hip_atomic_store(out + (dv0 + i * STEP) * R + row, val[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (dv0 == 0) {
+        __hip_atomic_store(out + kML + row, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(out + kML + 32 + row, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the stores have been acknowledged before the ticket is drawn
+    __syncthreads();
+    uint32_t* drawn = reinterpret_cast<uint32_t*>(lds);  // the tiles in LDS have been read
+    if (tid == 0) {
+      const uint32_t t = __hip_atomic_fetch_add(a.tickets + grp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (t == (uint32_t)a.nsplit - 1) __hip_atomic_store(a.tickets + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *drawn = t;
+    }
+    __syncthreads();
+    if (*drawn != (uint32_t)a.nsplit - 1) return;
+    // (a row past a.rows reads the last row that was sent: in bounds, and not stored)
+    const float* mine = group_parts + (row < a.rows ? row : a.rows - 1);
+    constexpr int kAhead = 4;
+    float m[kAhead], l[kAhead], v[kAhead][NV];
+    auto fetch = [&](int w0) {
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        const float* pw = mine + (int64_t)(w0 + q < a.nsplit ? w0 + q : a.nsplit - 1) * kTile;
+        m[q] = __hip_atomic_load(pw + kML, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        l[q] = __hip_atomic_load(pw + kML + 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[q][i] = __hip_atomic_load(pw + (dv0 + i * STEP) * R, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    };
+    fetch(0);
+    M = -__builtin_inff();
+    for (int w0 = kAhead; w0 < a.nsplit; w0 += 8) {  // the maxima that are not among those
+      float mm[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        mm[q] = __hip_atomic_load(mine + (int64_t)(w0 + q < a.nsplit ? w0 + q : a.nsplit - 1) * kTile + kML, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) M = __builtin_fmaxf(M, mm[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) M = __builtin_fmaxf(M, m[q]);
+    L = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) val[i] = 0.0f;
+    for (int w0 = 0; w0 < a.nsplit; w0 += kAhead) {
+      if (w0 > 0) fetch(w0);
+#pragma unroll
+      for (int q = 0; q < kAhead; ++q) {
+        if (w0 + q < a.nsplit) {
+          const float wgt = m[q] == -__builtin_inff() ? 0.0f : fast_exp2(m[q] - M);
+          L += l[q] * wgt;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) val[i] += v[q][i] * wgt;
+        }
+      }
+    }
+  }
+  // normalise (0 for a row with nothing to attend to), scale, round and store; the amax updates
+  const float lsum = L / qs;
+  const float inv_l = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+  const bool row_ok = row < a.rows;
+  const int rin = a.pack ? row / a.L : 0, rq = a.pack ? row - rin * a.L : row;
+  uint8_t* orow = a.out + (o_off + (int64_t)rin * a.o_bs[2] + (int64_t)rq * a.ldo) * (a.out_fp8 ? 1 : 2);
+  const float dv = sdpa_scale(a, 2, 1.0f), ds = sdpa_scale(a, 5, 1.0f / qs);
   const float qo = a.out_fp8 ? sdpa_scale(a, 4, 1.0f) : 1.0f;
   float amax_o = 0.0f;
 #pragma unroll
-  for (int i = 0; i < DVT * 32 / 8; ++i) {
-    const int d = dv0 + i * dvstep;
-    const float v = val[i] * (ds * dv);
+  for (int i = 0; i < NV; ++i) {
+    const int d = dv0 + i * STEP;
+    const float x = val[i] * inv_l * (ds * dv);
     if (row_ok && d < a.Dv) {
-      amax_o = __builtin_fmaxf(amax_o, __builtin_fabsf(v));
-      if (a.out_fp8) orow[d] = (uint8_t)(cvt_fp8x4<MI355Q_E4M3FN>(v * qo, 0.f, 0.f, 0.f) & 0xffu);
-      else reinterpret_cast<uint16_t*>(orow)[d] = (uint16_t)(pack_bf16x2(v, 0.f) & 0xffffu);
+      amax_o = __builtin_fmaxf(amax_o, __builtin_fabsf(x));
+      if (a.out_fp8) orow[d] = (uint8_t)(cvt_fp8x4<MI355Q_E4M3FN>(x * qo, 0.f, 0.f, 0.f) & 0xffu);
+      else reinterpret_cast<uint16_t*>(orow)[d] = (uint16_t)(pack_bf16x2(x, 0.f) & 0xffffu);
     }
   }
-  const int lane = threadIdx.x & 63;
+  const int lane = tid & 63;
   if (a.amax_s != nullptr) {
-    const uint32_t m = wave_max_u32(__float_as_uint(row_ok ? inv_l : 0.0f));
-    if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_s), m);
+    const uint32_t mx = wave_max_u32(__float_as_uint(row_ok && dv0 == 0 ? inv_l : 0.0f));
+    if (lane == 0 && mx != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_s), mx);
   }
   if (a.amax_o != nullptr) {
-    const uint32_t m = wave_max_u32(__float_as_uint(amax_o));
-    if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), m);
+    const uint32_t mx = wave_max_u32(__float_as_uint(amax_o));
+    if (lane == 0 && mx != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), mx);
   }
 }
 
@@ -904,76 +975,9 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
     tile[32 * DVT * 32 + 32 + lq] = l_tot;
   }
   __syncthreads();
-  const int row = tid & 31, dvg = tid >> 5;  // a thread merges columns dvg, dvg + 8, ... of one row
-  const float* parts = reinterpret_cast<const float*>(lds);
-  if (a.nsplit == 1) {
-    float val[DVT * 32 / 8];
-    const float inv_l = sdpa_merge<DVT>(parts, 4, kDecodeTileFloats(DVT), row, dvg, 8, qs, val);
-    const int rin = a.pack ? row / a.L : 0, rq = a.pack ? row - rin * a.L : row;
-    uint8_t* orow = a.out + (o_off + (int64_t)rin * a.o_bs[2] + (int64_t)rq * a.ldo) * (a.out_fp8 ? 1 : 2);
-    sdpa_store_row<DVT>(a, orow, row < a.rows, dvg == 0 ? inv_l : 0.0f, dvg, 8, val);
-  } else {
-    // Unnormalised: the merged maximum, the merged sum and O of this split go to the workspace; the workgroup
-    // that draws the group's last ticket merges the splits in their order, whoever came last, and stores the
-    // rows.  The partial results are written and read with device-scope atomic accesses, which go past this
-    // XCD's cache to where the other XCDs see them: no cache has to be written back or invalidated as a whole,
-    // which a fence would do.  The last one returns the counter to zero for the next launch.
-    float M = -__builtin_inff();
-    for (int w = 0; w < 4; ++w) M = __builtin_fmaxf(M, parts[w * kDecodeTileFloats(DVT) + 32 * DVT * 32 + row]);
-    float L = 0.0f, val[DVT * 32 / 8];
-#pragma unroll
-    for (int i = 0; i < DVT * 32 / 8; ++i) val[i] = 0.0f;
-    for (int w = 0; w < 4; ++w) {
-      const float* pw = parts + w * kDecodeTileFloats(DVT);
-      const float mw = pw[32 * DVT * 32 + row];
-      const float wgt = mw == -__builtin_inff() ? 0.0f : fast_exp2(mw - M);
-      L += pw[32 * DVT * 32 + 32 + row] * wgt;
-#pragma unroll
-      for (int i = 0; i < DVT * 32 / 8; ++i) val[i] += pw[(dvg + 8 * i) * 32 + row] * wgt;
-    }
-    float* group_parts = a.ws + (int64_t)grp * a.nsplit * kDecodeTileFloats(DVT);
-    float* out = group_parts + (int64_t)split * kDecodeTileFloats(DVT);
-#pragma unroll
-    for (int i = 0; i < DVT * 32 / 8; ++i)
-      __hip_atomic_store(out + (dvg + 8 * i) * 32 + row, val[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (dvg == 0) {
-      __hip_atomic_store(out + 32 * DVT * 32 + row, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(out + 32 * DVT * 32 + 32 + row, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __builtin_amdgcn_s_waitcnt(0);  // the stores have been acknowledged before the ticket is drawn
-    __syncthreads();
-    uint32_t* drawn = reinterpret_cast<uint32_t*>(lds);  // the tiles in LDS have been read
-    if (tid == 0) {
-      const uint32_t t = __hip_atomic_fetch_add(a.tickets + grp, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (t == (uint32_t)a.nsplit - 1) __hip_atomic_store(a.tickets + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      *drawn = t;
-    }
-    __syncthreads();
-    if (*drawn != (uint32_t)a.nsplit - 1) return;
-    M = -__builtin_inff();
-    for (int w = 0; w < a.nsplit; ++w)
-      M = __builtin_fmaxf(M, __hip_atomic_load(group_parts + (int64_t)w * kDecodeTileFloats(DVT) + 32 * DVT * 32 + row, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT));
-    L = 0.0f;
-#pragma unroll
-    for (int i = 0; i < DVT * 32 / 8; ++i) val[i] = 0.0f;
-    for (int w = 0; w < a.nsplit; ++w) {
-      const float* pw = group_parts + (int64_t)w * kDecodeTileFloats(DVT);
-      const float mw = __hip_atomic_load(pw + 32 * DVT * 32 + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float wgt = mw == -__builtin_inff() ? 0.0f : fast_exp2(mw - M);
-      L += __hip_atomic_load(pw + 32 * DVT * 32 + 32 + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * wgt;
-#pragma unroll
-      for (int i = 0; i < DVT * 32 / 8; ++i)
-        val[i] += __hip_atomic_load(pw + (dvg + 8 * i) * 32 + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * wgt;
-    }
-    const float l = L / qs;
-    const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
-#pragma unroll
-    for (int i = 0; i < DVT * 32 / 8; ++i) val[i] *= inv_l;
-    const int rin = a.pack ? row / a.L : 0, rq = a.pack ? row - rin * a.L : row;
-    uint8_t* orow = a.out + (o_off + (int64_t)rin * a.o_bs[2] + (int64_t)rq * a.ldo) * (a.out_fp8 ? 1 : 2);
-    sdpa_store_row<DVT>(a, orow, row < a.rows, dvg == 0 ? inv_l : 0.0f, dvg, 8, val);
-  }
+  if (a.rows <= 8) sdpa_decode_finish<DVT, 8>(a, lds, grp, split, o_off, qs);
+  else if (a.rows <= 16) sdpa_decode_finish<DVT, 16>(a, lds, grp, split, o_off, qs);
+  else sdpa_decode_finish<DVT, 32>(a, lds, grp, split, o_off, qs);
 }
 
 template <int DKC, int DVT>

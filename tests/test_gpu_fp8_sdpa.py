@@ -322,6 +322,24 @@ def test_few_queries_against_many_keys(oracle, pkg, dev, case):
     check_fp8(out8, ref8, str(case))
 
 
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("S, D", [(512, 128), (1088, 128), (2600, 64), (4224, 80), (8192, 128)])
+def test_few_queries_row_layouts_and_splits(oracle, pkg, dev, rows, S, D):
+    """The end of the decoding kernel at the edges of its row layouts (8, 16, 32 rows) and of the splits that are read at a
+    time (4), and again with the same bits."""
+    gen = torch.Generator().manual_seed(100 * rows + S)
+    q, k, v = make_qkv(gen, (1, 2, rows, 1, D), (1, 2, 1, S, D), (1, 2, 1, S, D))
+    sc = (0.5, 2.0, 0.25, 128.0, None, 1 / 128.0)
+    out, _, _, _, amax_s, amax_o = run_op(dev, q, k, v, scales=sc, amax_s=True, amax_o=True)
+    ref, ref_as, ref_ao = oracle.torch_fp8_sdpa(q, k, v, d_scale_q=0.5, d_scale_k=2.0, d_scale_v=0.25, q_scale_s=128.0,
+                                                d_scale_s=1 / 128.0, key_streams=key_walk(pkg, q, k, v))
+    check_bf16(out, ref, f"{rows} rows, {S} keys")
+    assert abs(float(amax_s.cpu()) - float(ref_as)) <= 1e-4 * float(ref_as)
+    assert abs(float(amax_o.cpu()) - float(ref_ao)) <= 2e-3 * float(ref_ao)
+    for _ in range(3):
+        assert torch.equal(run_op(dev, q, k, v, scales=sc)[0], out)
+
+
 def test_few_queries_without_a_workspace(oracle, pkg, dev):
     """The C entry point without the workspace it asks for: one workgroup per group walks all the keys."""
     gen = torch.Generator().manual_seed(21)
