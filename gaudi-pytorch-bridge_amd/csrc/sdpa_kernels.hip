@@ -846,7 +846,7 @@ __device__ __forceinline__ void sdpa_group_offsets(const SdpaArgs& a, int64_t g,
   }
 }
 
-template <int DKC, int DVT, int FMT>
+template <int DKC, int DVT, int FMT, int R>
 __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const SdpaArgs a) {
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = 128;
@@ -975,16 +975,21 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
     tile[32 * DVT * 32 + 32 + lq] = l_tot;
   }
   __syncthreads();
-  if (a.rows <= 8) sdpa_decode_finish<DVT, 8>(a, lds, grp, split, o_off, qs);
-  else if (a.rows <= 16) sdpa_decode_finish<DVT, 16>(a, lds, grp, split, o_off, qs);
-  else sdpa_decode_finish<DVT, 32>(a, lds, grp, split, o_off, qs);
+  sdpa_decode_finish<DVT, R>(a, lds, grp, split, o_off, qs);
+}
+
+template <int DKC, int DVT, int FMT>
+static void sdpa_decode_launch_rows(const SdpaArgs& a, dim3 grid, hipStream_t st) {
+  if (a.rows <= 8) hipLaunchKernelGGL((fp8_sdpa_decode_kernel<DKC, DVT, FMT, 8>), grid, dim3(kSdpaThreads), 0, st, a);
+  else if (a.rows <= 16) hipLaunchKernelGGL((fp8_sdpa_decode_kernel<DKC, DVT, FMT, 16>), grid, dim3(kSdpaThreads), 0, st, a);
+  else hipLaunchKernelGGL((fp8_sdpa_decode_kernel<DKC, DVT, FMT, 32>), grid, dim3(kSdpaThreads), 0, st, a);
 }
 
 template <int DKC, int DVT>
 static int sdpa_decode_launch(const SdpaArgs& a, int fmt, int64_t groups, hipStream_t st) {
   const dim3 grid((unsigned)(groups * a.nsplit));
-  if (fmt == MI355Q_E5M2) hipLaunchKernelGGL((fp8_sdpa_decode_kernel<DKC, DVT, MI355Q_E5M2>), grid, dim3(kSdpaThreads), 0, st, a);
-  else hipLaunchKernelGGL((fp8_sdpa_decode_kernel<DKC, DVT, MI355Q_E4M3FN>), grid, dim3(kSdpaThreads), 0, st, a);
+  if (fmt == MI355Q_E5M2) sdpa_decode_launch_rows<DKC, DVT, MI355Q_E5M2>(a, grid, st);
+  else sdpa_decode_launch_rows<DKC, DVT, MI355Q_E4M3FN>(a, grid, st);
   return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;
 }
 
