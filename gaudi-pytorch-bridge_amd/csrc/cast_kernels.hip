@@ -5,6 +5,7 @@
 // loads in flight.  Rounding and saturation use the CDNA4 conversion
 // instructions (v_cvt_pk_{fp8,bf8}_f32, v_cvt_pk_f32_{fp8,bf8},
 // v_cvt_pk_bf16_f32); see device_common.h.
+#include <cmath>
 #include <type_traits>
 
 #include "device_common.h"
@@ -609,8 +610,8 @@ __device__ __forceinline__ u32x4 ragged_chunk(const uint8_t* row, int c, int byt
 // scales); scale_inv = 1 / scale is what the GEMM takes as A_scale_inv.
 //
 // A workgroup has as many waves as the row needs (row_shape below): a wave whose lanes are all past the row's end
-// would issue the same instructions as the others.  SAT: target may lie above the largest finite code, so the scaled
-// values need the saturating conversion.
+// would issue the same instructions as the others.  SAT: target's magnitude lies above the largest finite code (or is a
+// NaN), so the scaled values need the saturating conversion.
 template <int FMT, bool SAT>
 __device__ __forceinline__ uint32_t row_cvt_fp8x4(float a, float b, float c, float d) {
   if constexpr (SAT) return cvt_fp8x4<FMT>(a, b, c, d);
@@ -1178,7 +1179,7 @@ template <int FMT, typename F>
 bool with_row_shape(int64_t rows, int64_t vpr, float target, F&& f) {
   if (vpr > kMaxRowVectors) return false;
   const RowShape s = row_shape(rows, vpr);
-  if (!(target <= kFp8Max[FMT - MI355Q_E4M3FN])) f(std::integral_constant<int, 2>{}, std::true_type{}, (unsigned)kMaxRowThreads);
+  if (!(std::fabs(target) <= kFp8Max[FMT - MI355Q_E4M3FN])) f(std::integral_constant<int, 2>{}, std::true_type{}, (unsigned)kMaxRowThreads);
   else if (s.vpt == 1) f(std::integral_constant<int, 1>{}, std::false_type{}, s.threads);
   else if (s.vpt == 2) f(std::integral_constant<int, 2>{}, std::false_type{}, s.threads);
   else f(std::integral_constant<int, kBulkVectors>{}, std::false_type{}, s.threads);

@@ -85,8 +85,8 @@ __device__ __forceinline__ uint32_t cvt_fp8x4(float a, float b, float c, float d
 }
 
 // The same for values known to lie below the halfway point past the largest finite code (464; 61440), which round to
-// that code by themselves: what a row scaled by target / amax with target <= the largest finite value holds, whatever
-// the roundings on the way (at most 449.8; 57570).  NaN stays NaN.
+// that code by themselves: what a row scaled by target / amax with |target| <= the largest finite value holds, whatever
+// the roundings on the way (at most 450; 57600).  NaN stays NaN.
 template <int FMT>
 __device__ __forceinline__ uint32_t cvt_fp8x4_in_range(float a, float b, float c, float d) {
   int r;

@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from helpers import E4, E5
+from helpers import E4, E5, assert_fp8_equal
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,32 @@ def test_target_past_the_largest_code_saturates(pkg, dev):
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     assert lib.mi355q_quantize_rows(x.data_ptr(), pkg.BF16, 1, 8, y.data_ptr(), pkg.E4M3FN, 1024.0, None, inv.data_ptr(), st) == 0
     assert y.cpu().float()[0].tolist() == [256.0, -448.0, 448.0, 448.0, -448.0, 128.0, 0.0, 384.0]
+
+
+@pytest.mark.parametrize("target", [-448.0, -1024.0, -60000.0, -1e5, 1e5, float("-inf")])
+@pytest.mark.parametrize("fmt", [E4, E5])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_target_of_any_sign_saturates(oracle, pkg, dev, target, fmt, dtype):
+    """Codes past the largest finite one are that code, whatever the sign of the target, on aligned rows, on ragged ones and
+    behind silu(gate) * up."""
+    lib = pkg.capi()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator().manual_seed(9)
+    gate, up = torch.randn(5, 136, generator=g).to(dtype), torch.randn(5, 136, generator=g).to(dtype)
+
+    def reference(x):
+        amax = x.float().abs().amax(1)
+        scale = torch.clamp_max(torch.full_like(amax, target) / amax, oracle.ROW_SCALE_CAP)
+        return oracle.c_cast_to_fp8(x, scale, fmt, scale_shape=[x.shape[0], 1])[0]
+
+    code = {E4: pkg.E4M3FN, E5: pkg.E5M2}[fmt]
+    for cols in (136, 133):
+        x = gate[:, :cols].contiguous()
+        y, xd = torch.empty(5, cols, dtype=fmt, device=dev), x.to(dev)
+        assert lib.mi355q_quantize_rows(xd.data_ptr(), pkg.BF16 if dtype == torch.bfloat16 else pkg.F32, 5, cols, y.data_ptr(), code, target, None,
+                                        None, st) == 0
+        assert_fp8_equal(y, reference(x), fmt, f"{cols} columns")
+    if dtype == torch.bfloat16:
+        y, gd, ud = torch.empty(5, 136, dtype=fmt, device=dev), gate.to(dev), up.to(dev)
+        assert lib.mi355q_silu_mul_quantize_rows(gd.data_ptr(), 136, ud.data_ptr(), 136, 5, 136, y.data_ptr(), code, target, None, None, None, st) == 0
+        assert_fp8_equal(y, reference(oracle.c_silu_mul_bf16(gate, up)), fmt, "silu")
