@@ -1179,10 +1179,15 @@ template <int FMT, typename F>
 bool with_row_shape(int64_t rows, int64_t vpr, float target, F&& f) {
   if (vpr > kMaxRowVectors) return false;
   const RowShape s = row_shape(rows, vpr);
-  if (!(std::fabs(target) <= kFp8Max[FMT - MI355Q_E4M3FN])) f(std::integral_constant<int, 2>{}, std::true_type{}, (unsigned)kMaxRowThreads);
-  else if (s.vpt == 1) f(std::integral_constant<int, 1>{}, std::false_type{}, s.threads);
-  else if (s.vpt == 2) f(std::integral_constant<int, 2>{}, std::false_type{}, s.threads);
-  else f(std::integral_constant<int, kBulkVectors>{}, std::false_type{}, s.threads);
+  auto with_vectors = [&](auto saturate) {
+    if (s.vpt == 1) f(std::integral_constant<int, 1>{}, saturate, s.threads);
+    else if (s.vpt == 2) f(std::integral_constant<int, 2>{}, saturate, s.threads);
+    else f(std::integral_constant<int, kBulkVectors>{}, saturate, s.threads);
+  };
+  // (both conversions with the same shapes: a saturating form with 1024 threads for every row took 23 instead of 7 us at
+  // 4096 x 1024 and 45 instead of 8 at 8192 x 512)
+  if (!(std::fabs(target) <= kFp8Max[FMT - MI355Q_E4M3FN])) with_vectors(std::true_type{});
+  else with_vectors(std::false_type{});
   return true;
 }
 

@@ -62,3 +62,42 @@ def test_a_target_of_any_sign_saturates(oracle, pkg, dev, target, fmt, dtype):
         y, gd, ud = torch.empty(5, 136, dtype=fmt, device=dev), gate.to(dev), up.to(dev)
         assert lib.mi355q_silu_mul_quantize_rows(gd.data_ptr(), 136, ud.data_ptr(), 136, 5, 136, y.data_ptr(), code, target, None, None, None, st) == 0
         assert_fp8_equal(y, reference(oracle.c_silu_mul_bf16(gate, up)), fmt, "silu")
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 8192), (2, 8200), (511, 520), (512, 520), (513, 16384)])
+def test_saturating_form_at_every_row_shape(oracle, pkg, dev, rows, cols):
+    """The codes of a target past the largest finite one at the row shapes of the first test."""
+    lib = pkg.capi()
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=g).bfloat16()
+    xd, y = x.to(dev), torch.empty(rows, cols, dtype=E4, device=dev)
+
+    def call(target):
+        st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert lib.mi355q_quantize_rows(xd.data_ptr(), pkg.BF16, rows, cols, y.data_ptr(), pkg.E4M3FN, target, None, None, st) == 0
+
+    call(1024.0)
+    amax = x.float().abs().amax(1)
+    ref = oracle.c_cast_to_fp8(x, torch.full_like(amax, 1024.0) / amax, E4, scale_shape=[rows, 1])[0]
+    assert_fp8_equal(y, ref, E4)
+
+
+def test_saturating_form_is_as_fast(pkg, dev):
+    lib = pkg.capi()
+    rows, cols = 8192, 512
+    x, y = torch.randn(rows, cols, device=dev).bfloat16(), torch.empty(rows, cols, dtype=E4, device=dev)
+
+    def best(target):
+        st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        times = []
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(40):
+                lib.mi355q_quantize_rows(x.data_ptr(), pkg.BF16, rows, cols, y.data_ptr(), pkg.E4M3FN, target, None, None, st)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    assert best(1024.0) < 2.0 * best(448.0)  # 7.8 with 1024 threads for every row, 1.1 with the rows' own shape
