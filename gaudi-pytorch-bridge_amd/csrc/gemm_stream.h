@@ -55,10 +55,15 @@ __device__ __forceinline__ void st_transpose4(uint32_t w0, uint32_t w1, uint32_t
 }
 
 // Row and column factors and the bias vector of the workgroup's rows and columns, fetched before the stream starts
-// (read at its end they would be cold misses, one after the other, with nothing left to hide them under).
+// (read at its end they would be cold misses, one after the other, with nothing left to hide them under).  A's scale and
+// B's stay apart, one as the row's factor and one as the column's: their product can leave fp32's range where neither
+// sums nor results do.  Where both are per row, or both per column, the second one is B's.
 struct StreamFactors {
-  float row[kStRows], col[kStBN], bias[kStBN];
+  float row[kStRows], col[kStBN], bias[kStBN], second[kStBN];
 };
+__device__ __forceinline__ bool st_two_of_a_kind(const GemmArgs& g) {
+  return g.sa_mode == g.sb_mode && (g.sa_mode == MI355Q_GS_PER_ROW || g.sa_mode == MI355Q_GS_PER_COL);
+}
 // Requested without a branch (a factor the problem does not have is an empty buffer, which reads as zero and touches
 // no memory): a branch here would make the compiler wait for the values in front of the stream's first loads.
 struct StreamFactorLoads {
@@ -85,11 +90,17 @@ struct StreamFactorLoads {
     const auto scalar = [&](int mode, float host, uint32_t loaded) {
       return mode == MI355Q_GS_HOST ? host : (mode == MI355Q_GS_DEV || mode == MI355Q_GS_PER_ROW ? __uint_as_float(loaded) : 1.0f);
     };
+    const float a_here = scalar(g.sa_mode, g.sa_host, a_row), b_here = scalar(g.sb_mode, g.sb_host, b_row);
+    const bool a_in_col = g.sa_mode == MI355Q_GS_PER_COL, b_in_col = g.sb_mode == MI355Q_GS_PER_COL;
+    const bool a_in_row = g.sa_mode == MI355Q_GS_PER_ROW, b_in_row = g.sb_mode == MI355Q_GS_PER_ROW;
+    // the row's factor is A's scale and the column's B's, scalars too, but where A's is per column or only B's per row
+    const bool turned = (a_in_col && !b_in_col) || (b_in_row && !a_in_row);
     if (threadIdx.x < kStBN) {
-      f.col[threadIdx.x] = (g.sa_mode == MI355Q_GS_PER_COL ? __uint_as_float(a_col) : 1.0f) * (g.sb_mode == MI355Q_GS_PER_COL ? __uint_as_float(b_col) : 1.0f);
+      f.col[threadIdx.x] = a_in_col ? __uint_as_float(a_col) : (turned ? a_here : (b_in_col ? __uint_as_float(b_col) : b_here));
       f.bias[threadIdx.x] = g.out_bf16 ? bf16_bits_to_f32(bias16) : __uint_as_float(bias32);
+      if (st_two_of_a_kind(g)) f.second[threadIdx.x] = b_in_col ? __uint_as_float(b_col) : b_here;
     }
-    if (threadIdx.x < kStRows) f.row[threadIdx.x] = scalar(g.sa_mode, g.sa_host, a_row) * scalar(g.sb_mode, g.sb_host, b_row);
+    if (threadIdx.x < kStRows) f.row[threadIdx.x] = turned ? b_here : a_here;
   }
 };
 
@@ -101,8 +112,14 @@ __device__ __forceinline__ void st_store8(const GemmArgs& g, int64_t batch, int 
   const int es = g.out_bf16 ? 2 : 4;
   const float rf = f.row[m];
   float v[8];
+  if (st_two_of_a_kind(g)) {
+    const bool rows = g.sa_mode == MI355Q_GS_PER_ROW;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(acc[e] * rf, f.col[col + e], f.bias[col + e]);
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(acc[e] * (rows ? rf : f.col[col + e]), f.second[rows ? m : col + e], f.bias[col + e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(acc[e] * rf, f.col[col + e], f.bias[col + e]);
+  }
   if (g.D != nullptr || g.bias_mode == MI355Q_BIAS_FULL) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {

@@ -43,6 +43,38 @@ def test_split_products_are_exact(M, K, N, trans_b, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 8, 17])
+@pytest.mark.parametrize("exponent", [70, -72])
+@pytest.mark.parametrize("kind_a", ["scalar", "row", "col"])
+@pytest.mark.parametrize("kind_b", ["scalar", "row", "col"])
+def test_scales_are_applied_one_after_the_other(M, exponent, kind_a, kind_b, dev):
+    """fp32 results whose scales multiply to something outside fp32's range, while sums and results lie inside it: 2^140
+    is infinite and 2^-144 has five bits left of a scale with seven."""
+    K = N = 4096
+    unit = 2.0 ** -14 if exponent > 0 else 2.0 ** 9
+    a, b = torch.full((M, K), unit), torch.full((K, N), unit)
+    a[M - 1, 1:] = 0.0
+    b[:, 5] = 0.0
+    sums = torch.full((M, N), K * unit * unit, dtype=torch.float64)
+    sums[M - 1] = unit * unit
+    sums[:, 5] = 0.0
+
+    def scale(kind, mantissa):
+        s = torch.tensor(mantissa * 2.0 ** exponent)
+        if kind == "row":
+            return (s * (1.0 - 0.25 * (torch.arange(M) % 2)))[:, None]
+        return s if kind == "scalar" else (s * (1.0 - 0.25 * (torch.arange(N) % 2)))[None]
+
+    sa, sb = scale(kind_a, 1.0 + 2.0 ** -6), scale(kind_b, 1.0)
+    c = torch.ops.hpu.fp8_gemm_v2(a.to(E5).to(dev), False, b.to(E5).to(dev), False, None, torch.float32, sa.to(dev), sb.to(dev), None, False,
+                                  list(sb.shape) if kind_b != "scalar" else None)
+    ref = (sums * sa.double() * sb.double()).float()
+    assert bool(ref.isfinite().all()) and int((ref == 0).sum()) == M
+    # (results below 2^-126 are rounded to a whole number of 2^-149)
+    assert torch.allclose(c.cpu(), ref, rtol=2.0 ** -22, atol=2.0 ** -149)
+
+
+@pytest.mark.gpu
 def test_one_workspace_serves_several_shapes(pkg, dev):
     """The C entry with a caller's workspace: shapes one after the other, counters left zero, too small a workspace
     refused, and no workspace accepted."""
