@@ -578,16 +578,20 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   Tensor out = at::empty(out_shape, A.options().dtype(out_dtype));
   if (out.numel() == 0) return out;
 
-  // The MFMA kernels move 16-byte chunks: they need 16-byte aligned operands and pitches and, where
-  // K is an operand's contiguous dimension, K % 16 == 0; anything else runs on a kernel that takes 80 ns per k
-  // (1 x 3001 x 8000: 0.7 ms).  From K = 96 on, or for a large product, such operands therefore go into zero-filled
-  // buffers with every extent rounded up to 16, both in one launch (zeros along K add nothing to any sum; padding along
-  // m or n is never read into a stored output).  1 x 3001 x 8000: 726 -> 25 us with the quantisation, 7 x 600 x 501: 64 -> 18.
+  // The MFMA kernels move 16-byte chunks: they need 16-byte aligned operands and pitches and, where K is an operand's
+  // contiguous dimension, K % 16 == 0; anything else runs on a kernel that takes about 80 ns per k (1 x 3001 x 8000:
+  // 0.7 ms).  Where that is more than a second launch costs, such operands go into zero-filled buffers with every extent
+  // rounded up to 16, both in one launch (zeros along K add nothing to any sum; padding along m or n is never read into
+  // a stored output).  Without -> with the copies, us a call:
+  //   1 x 33       K = 97: 9.2 -> 13.1, 161: 13.5 -> 11       300 x 501  K = 81: 10.8 -> 12.7, 129: 15.5 -> 12.7
+  //   300 x 501, B [N, K] (a wave's threads read it a row of B apart)    K = 49: 13 -> 13, 81: 21.8 -> 12.6
+  //   1 x 3001 x 8000: 726 -> 25 with the quantisation, 7 x 600 x 501: 64 -> 18, 2000 x 81 x 2001: 29 (four launches) -> 17
   int64_t lda = ac, ldb = bc, k_call = K;
   auto misaligned = [](const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) != 0; };
   const bool k_ragged = K % 16 != 0 && !(ta && !tb);
+  const double outputs = (double)M * (double)N;
   if ((ac % 16 || bc % 16 || k_ragged || misaligned(ac_t) || misaligned(bc_t)) &&
-      (K >= 96 || (double)M * (double)N * (double)K >= (double)(1 << 22))) {
+      (K >= 128 || outputs * (double)K >= (double)(1 << 26) || (tb && K >= 64 && outputs >= (double)(1 << 17)))) {
     const int64_t kp = (ta && !tb) ? K : (K + 15) / 16 * 16;  // K is contiguous in neither operand: any K
     mi355q_pad_desc jobs[2];
     int count = 0;

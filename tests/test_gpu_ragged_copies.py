@@ -35,7 +35,7 @@ def test_pad_rows(pkg, dev, batch, rows, cols, offset):
 
 
 # around the size from which operands are copied, one and both operands ragged, every layout, batches
-@pytest.mark.parametrize("M,K,N", [(1, 95, 33), (1, 97, 33), (3, 1111, 999), (17, 4096, 257), (130, 333, 144), (64, 100, 5)])
+@pytest.mark.parametrize("M,K,N", [(1, 95, 33), (1, 97, 33), (1, 127, 33), (1, 129, 33), (300, 63, 501), (3, 1111, 999), (17, 4096, 257), (130, 333, 144), (64, 100, 5)])
 @pytest.mark.parametrize("trans_a,trans_b", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("batch", [0, 3])
 def test_ragged_products_are_exact(dev, M, K, N, trans_a, trans_b, batch):
@@ -47,6 +47,22 @@ def test_ragged_products_are_exact(dev, M, K, N, trans_a, trans_b, batch):
     b8 = (b.transpose(-1, -2).contiguous() if trans_b else b).to(E5).to(dev)
     c = torch.ops.hpu.fp8_gemm_v2(a8, trans_a, b8, trans_b, None, torch.float32, None, None, None, False)
     assert torch.equal(c.cpu(), a @ b)
+
+
+# both sides of each line of the rule: the operands are copied where that is faster than the kernel for any shape
+@pytest.mark.parametrize("M,K,N,trans_b,copied", [(1, 97, 33, False, 0), (1, 127, 33, True, 0), (1, 129, 33, False, 2), (1, 129, 33, True, 2),
+                                                  (300, 81, 501, False, 0), (300, 81, 501, True, 2), (5000, 49, 31, True, 0), (30, 81, 33, True, 0),
+                                                  (300, 126, 501, False, 0), (2000, 20, 2001, False, 2), (64, 128, 5, False, 1)])
+def test_which_ragged_products_are_copied(dev, M, K, N, trans_b, copied):
+    a8, b8 = torch.zeros(M, K, device=dev).to(E4), torch.zeros((N, K) if trans_b else (K, N), device=dev).to(E4)
+
+    def call():
+        return torch.ops.hpu.fp8_gemm_v2(a8, False, b8, trans_b, None, torch.float32, None, None, None, False)
+
+    call()
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    c = call()
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 1 + copied and c.shape == (M, N)
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (2, 9), (5, 1021), (600, 515), (1, 16383), (2, 8191)])
