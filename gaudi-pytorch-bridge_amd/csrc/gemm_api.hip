@@ -73,14 +73,7 @@ inline bool tiled_ok(const void* A, int trans_a, int64_t lda, const void* B, int
   return M > 0 && N > 0 && K > 0;
 }
 
-// The cut that is expected to take least.  The figures (microseconds, bytes per microsecond) are fits to 60 problems of 1 to
-// 128 rows, K from 2048 to 14336 and N from 1024 to 38400, most of which they meet within two microseconds:
-//  * a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where more of them run;
-//  * in the strip kernel A's tile travels along (a quarter of its bytes count with a K-major B, half with the shorter
-//    pieces of an MN-major one);
-//  * fixed costs, and with more than one part the meeting: each part's sums out, and all of them into the last one.
-//
-// More than 128 rows (tile_split_plan): the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where that beats
+// More than 128 rows: the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where that beats
 // the unsplit launch by 10 % and 2 us (short products whose weights sit in the Infinity Cache are that much faster than
 // tile_us says); the fits are those of tile_us with 4.5 us for the first meeting of 128 x 128 sums and
 // 3.5 for each further one (6.5 each at 256 x 128).
@@ -108,6 +101,20 @@ SplitPlan tile_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   return best;
 }
 
+// The cut that is expected to take least.  More than 128 rows: tile_split_plan.  For fewer the figures (microseconds, bytes
+// per microsecond) are fits to 60 problems of 1 to 128 rows, K from 2048 to 14336 and N from 1024 to 38400, most of which
+// they meet within two microseconds:
+//  * a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where more of them run;
+//  * in the strip kernel A's tile travels along (a quarter of its bytes count with a K-major B, half with the shorter
+//    pieces of an MN-major one);
+//  * fixed costs, and with more than one part the meeting: each part's sums out, and all of them into the last one.
+// Short products stay whole where the meeting costs them more than the parts save.  Whole and in parts, us a launch,
+// weights hot in the caches / cold:
+//  * the strip kernel below K = 1792: 1 x 1280 x 512, B [N, K], 8.9 / 8.9 and 9.5 / 9.4; 8 x 1536 x 512 8.2 / 9.3 and 8.8 / 9.0
+//    (2048: 8 x 2048 x 512 9.5 / 10.7 and 9.1 / 9.5);
+//  * the stream kernel below K = 2048, against the strip kernel whole: 1 x 1024 x 2048 6.8 / 8.5 and 10.3 / 10.1;
+//  * no part of the stream kernel shorter than 512, two turns of its eight waves, since in a part of 256 a wave's first
+//    loads have none behind them: 8 x 2048 x 4096 in eight of those 12.1 / 12.0, in four parts on the strip kernel 10.0 / 10.2.
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
   SplitPlan best;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
@@ -115,11 +122,14 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   const double cus = (double)compute_units();
   double best_us = 0.0;
   auto consider = [&](bool stream, int64_t nb, int64_t tile_rows, int64_t unit) {
+    const int64_t shortest = stream ? 512 : unit;  // part
+    const bool in_parts = may_split && K >= (stream ? 2048 : 1792);
     const int64_t strips = (N + nb - 1) / nb, groups = strips * batch, units = (K + unit - 1) / unit;
     const int64_t rows = M < 32 ? M : tile_rows;  // rows of sums that travel
     const double width = (double)nb + (stream ? 0.0 : (double)tile_rows * (b_kmajor ? 0.25 : 0.5));
     for (int64_t parts = 1; parts <= 32 && parts <= units; ++parts) {
-      if (parts > 1 && (!may_split || groups > kMaxTickets || (double)(groups * parts) > 2.0 * cus)) break;
+      if (parts > 1 && (!in_parts || groups > kMaxTickets || (double)(groups * parts) > 2.0 * cus)) break;
+      if (parts > 1 && (units + parts - 1) / parts * unit < shortest) break;
       const double wgs = (double)(groups * parts), rounds = std::ceil(wgs / cus);
       const double rate = std::min(37e3, 6.5e6 / std::min(wgs, cus));
       double us = rounds * (double)((units + parts - 1) / parts * unit) * width / rate + 4.5;

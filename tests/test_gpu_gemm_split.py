@@ -100,6 +100,21 @@ def test_one_workspace_serves_several_shapes(pkg, dev):
         assert int(ws[: 64 * 1024].count_nonzero()) == 0
 
 
+def test_short_products_stay_whole(pkg):
+    """K below which a product was slower in parts than whole, and longer ones that stay in parts; without a workspace none is."""
+    need = pkg.capi().mi355q_fp8_gemm_workspace_bytes
+    bytes_of = lambda m, k, n, nk: need(0, k, nk, k if nk else n, m, n, k, 1)  # noqa: E731
+    for m in (1, 4, 8, 16, 17, 64, 128):
+        for n in (128, 512, 2048, 4096, 11264):
+            for nk in (0, 1):
+                assert all(bytes_of(m, k, n, nk) == 0 for k in (16, 512, 1024, 1280, 1536, 1776)), (m, n, nk)
+                assert bytes_of(m, 8192, n, nk) > 0, (m, n, nk)
+    counters = 64 * 1024
+    for n in (512, 1024, 4096):  # sums of 16 rows and 256 columns: parts of the stream kernel, 512 k each at least
+        parts = (bytes_of(1, 4096, n, 0) - counters) // (n * 16 * 4)
+        assert 2 <= parts <= 8, (n, parts)
+
+
 @pytest.mark.timeout(600)
 def test_parts_of_k_meet_by_device_scope_accesses_in_order():
     """Sums stored (sc1), acknowledged, barrier, ticket, barrier, counter reset, sums read (sc1); nothing cache-wide."""
