@@ -45,14 +45,20 @@ __global__ __launch_bounds__(kSkThreads) void fp8_gemm_skinny_kernel(GemmArgs g,
   __shared__ __attribute__((aligned(1024))) uint8_t lds[S * kStageBytes];
 
   const int64_t batch = blockIdx.y;
-  const int strips = g.tiles_n, strip = blockIdx.x % strips, part = blockIdx.x / strips;
+  const int strips = g.tiles_n;
+  int strip = blockIdx.x, part = 0;
+  if (split.parts > 1) {
+    // This workgroup's part of K, whole stages.  (Behind a branch and in 32 bits: nothing is on its way from memory yet, and
+    // the 64-bit divisions that stood here for every launch took 0.4 us.)
+    part = blockIdx.x / (unsigned)strips;
+    strip = blockIdx.x - part * strips;
+    const unsigned kt_all = (g.K + kBK - 1) / kBK;
+    const int kt0 = (int)(part * kt_all / (unsigned)split.parts), kt1 = (int)((part + 1) * kt_all / (unsigned)split.parts);
+    g.K = (g.K < kt1 * kBK ? g.K : kt1 * kBK) - kt0 * kBK;
+    g.A += (int64_t)kt0 * kBK * (A_KMAJOR ? 1 : g.lda);
+    g.B += (int64_t)kt0 * kBK * (B_KMAJOR ? 1 : g.ldb);
+  }
   const int n0 = strip * kSkBN;
-  // this workgroup's part of K, whole stages
-  const int kt_all = (g.K + kBK - 1) / kBK;
-  const int kt0 = (int)((int64_t)part * kt_all / split.parts), kt1 = (int)((int64_t)(part + 1) * kt_all / split.parts);
-  g.K = (g.K < kt1 * kBK ? g.K : kt1 * kBK) - kt0 * kBK;
-  g.A += (int64_t)kt0 * kBK * (A_KMAJOR ? 1 : g.lda);
-  g.B += (int64_t)kt0 * kBK * (B_KMAJOR ? 1 : g.ldb);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wn = wave * 32;
 
