@@ -73,26 +73,34 @@ inline bool tiled_ok(const void* A, int trans_a, int64_t lda, const void* B, int
   return M > 0 && N > 0 && K > 0;
 }
 
-// More than 128 rows: the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where that beats
-// the unsplit launch by 10 % and 2 us (short products whose weights sit in the Infinity Cache are that much faster than
-// tile_us says); the fits are those of tile_us with 4.5 us for the first meeting of 128 x 128 sums and
-// 3.5 for each further one (6.5 each at 256 x 128).
+// More than 128 rows: the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where they are expected to beat
+// the uncut launch.  The estimates (us; `fill` is the share of the compute units that have a workgroup) are least-squares fits
+// to 590 products of 130 to 4000 rows, K from 1536 to 14336 and N from 64 to 8192, whole and in 2 to 16 parts, each timed with
+// the weights hot in the caches and cold and counted half and half, since a cut hides the cold weights' latency but costs the
+// same meeting when they are hot: 500 x 3072 x 2048 takes 13.2 / 23.8 whole, 14.8 / 18.4 in two parts, 20.9 / 21.1 in four.
+// Most are within 10 %.  The meeting costs more the fuller the chip is.  Beyond 16 parts nothing was faster.
 SplitPlan tile_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
   SplitPlan best;
   const int64_t cus = compute_units(), pairs = (K + 2 * kBK - 1) / (2 * kBK);
   const TileChoice whole = N > 128 ? choose_tiles(M, N, K, batch) : TileChoice::k128x128;
   if (whole == TileChoice::k256x256 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= cus) return best;
-  double best_us = 0.9 * tile_us(whole, M, N, K, batch) - 2.0;
+  auto tiles_of = [&](int64_t bm) { return ((M + bm - 1) / bm) * ((N + 127) / 128) * batch; };
+  const double all_stages = (double)((K + kBK - 1) / kBK);
+  double best_us = 0.85 * tile_us(whole, M, N, K, batch);
+  if (whole == TileChoice::k128x128) best_us = all_stages * (0.52 + 0.29 * (double)tiles_of(128) / (double)cus) + 2.7;
+  if (whole == TileChoice::k256x128) best_us = all_stages * 0.83 + 2.7 + (all_stages * 0.07 + 3.9) * (double)tiles_of(256) / (double)cus;
   for (const int64_t bm : {128, 256}) {
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + 127) / 128);
-    for (int64_t parts = 2; parts <= pairs && parts * tiles * batch <= cus; ++parts) {
-      const double stages = 2.0 * (double)((pairs + parts - 1) / parts), levels = std::ceil(std::log2((double)parts));
-      const double us = bm == 128 ? stages * 0.8 + 6.0 + 3.5 * levels : stages * 1.06 + 5.0 + 6.5 * levels;
+    const int64_t tiles = tiles_of(bm);
+    for (int64_t parts = 2; parts <= 16 && parts <= pairs && parts * tiles <= cus; ++parts) {
+      const double stages = 2.0 * (double)((pairs + parts - 1) / parts), levels = std::log2((double)parts);
+      const double fill = (double)(parts * tiles) / (double)cus;
+      const double us = bm == 128 ? stages * (0.51 + 0.13 * fill) + levels * (3.0 - 0.84 * fill) + 7.3 * fill + 2.9
+                                  : stages * (0.72 + 0.07 * fill) + levels * (5.8 - 0.82 * fill) + 9.1 * fill + 4.3;
       if (us >= best_us) continue;
       best_us = us;
       best.tile = bm == 128 ? SplitTile::k128x128 : SplitTile::k256x128;
       best.nb = 128;
-      best.strips = (int)tiles;
+      best.strips = (int)(tiles / batch);
       best.parts = (int)parts;
       best.tile_rows = bm;
       best.batch = batch;

@@ -1,7 +1,8 @@
 // The 128 x 128 and 256 x 128 tiles of gemm_tile.h with K in parts over workgroups, for products of more than 128 rows
 // whose tiles leave compute units idle (256 x 14336 x 4096 is 64 tiles of 128 x 128 for 256 units: 104 us unsplit, 40 us
 // in four parts).  What bounds them: a compute unit takes in about 40 KB of panels a microsecond, and on top the
-// meeting: 4 to 5 us for the first pair of 128 x 128 sums, 3.5 for each further level, 6.5 each at 256 x 128.  With two
+// meeting, 2 to 3 us a level for 128 x 128 sums and 5 to 6 for 256 x 128, with 7 to 9 on top on a full chip (the fits that
+// choose are in gemm_api.hip).  With two
 // workgroups per compute unit the same product takes 47 us (the panels come in no faster), so the grid stops at one.
 // 256 x 256 tiles in parts were no faster on any of 18 products (sums of 256 KB: 15 us to meet), but for 2000 x 14336 x
 // 4096 in two parts (105 against 120 us).  Measured before -> after, weights [K, N], bf16 out:

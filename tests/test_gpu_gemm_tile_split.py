@@ -61,3 +61,15 @@ def test_plans_of_the_cases(pkg):
         for n in (128, 1024, 4096, 8192):
             for k in (1024, 4096, 14336):
                 assert need(0, k, 0, n, m, n, k, 1) <= 64 * 1024 + 256 * 256 * 128 * 4
+
+
+def test_few_and_long_parts(pkg):
+    """Short products on a chip that their parts fill are cut in two at most (in four they took up to 57 % longer than whole), and
+    nothing into more than 16 parts."""
+    need = pkg.capi().mi355q_fp8_gemm_workspace_bytes
+    sums = lambda m, k, n: need(0, k, 0, n, m, n, k, 1)  # noqa: E731
+    for m, k, n in [(130, 3072, 4096), (256, 3072, 4096), (384, 3072, 2048), (500, 3072, 2048), (768, 3072, 1024), (1000, 3072, 1024)]:
+        tiles = (m + 127) // 128 * (n // 128)
+        assert sums(m, k, n) <= 64 * 1024 + 2 * tiles * 128 * 128 * 4, (m, k, n)
+    for k in (14336, 16384, 32768):
+        assert 64 * 1024 < sums(130, k, 128) <= 64 * 1024 + 16 * 2 * 128 * 128 * 4, k
