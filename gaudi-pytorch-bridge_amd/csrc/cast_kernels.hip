@@ -1039,28 +1039,49 @@ inline bool plan_vectors(int mode, int64_t outer, int64_t mid, int64_t inner, in
 
 constexpr int kCastU = 4;  // 16-byte loads in flight per thread
 
-inline unsigned cast_amax_threads(int64_t elements) { return elements <= kCastAmaxSmall ? kThreads : kCastAmaxMaxThreads; }
+// How a cast with amax runs: threads of a workgroup, and vectors in flight per thread.  Where rows have scales of their own, or
+// columns have, a workgroup walks row by row and a thread has no more vectors to ask for than the row holds: eight at a
+// time would be empty steps and, with the amax kernels' few workgroups, little in flight.  bf16, us, with 8 and with this:
+//   4096 x 4096 per column 52 -> 17 (46 as 1024 threads x 4), per row 41 -> 17 (38)     512 x 16384 per column 10.8 -> 7.8 (9.6)
+//   16384 x 64 per column 110 -> 35 (157)     4096 x 512 per column 29 -> 9 (42)     256 x 4096 per column 6.6 -> 4.1 (7.5)
+struct CastAmaxShape {
+  unsigned threads;
+  int vectors;
+};
+inline CastAmaxShape cast_amax_shape(int sk, int64_t rows, int64_t vpr) {
+  const bool small = rows * vpr * 8 <= kCastAmaxSmall;
+  const unsigned threads = small ? kThreads : kCastAmaxMaxThreads;
+  if (sk == SK_SCALAR || sk == SK_FULL) return {threads, kCastAmaxU};
+  return {threads, small || vpr <= kCastAmaxMaxThreads ? 1 : (vpr <= 2 * kCastAmaxMaxThreads ? 2 : (vpr <= 4 * kCastAmaxMaxThreads ? 4 : kCastAmaxU))};
+}
+
+template <bool BF16_IN, int FMT, bool AMAX, int U>
+void launch_cast_to_rows(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, int64_t vpr, int64_t bpr,
+                         int64_t total, int64_t mid, unsigned threads, uint32_t* amax) {
+  const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
+  if (sk == SK_ROW) cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax);
+  else cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax);
+}
 
 template <bool BF16_IN, int FMT, bool AMAX>
-void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale,
-                        float sh, int is_dev, int64_t vpr, int64_t bpr, int64_t total, int64_t mid,
-                        uint32_t* amax) {
+void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, float sh, int is_dev, int64_t vpr,
+                        int64_t bpr, int64_t total, int64_t mid, CastAmaxShape shape, uint32_t* amax) {
   constexpr int U = AMAX ? kCastAmaxU : kCastU;
-  const unsigned T = AMAX ? cast_amax_threads(vpr * (total / bpr) * 8) : kThreads;
+  const unsigned T = AMAX ? shape.threads : kThreads;
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
-  switch (sk) {
-    case SK_SCALAR:
-      cast_to_fp8_vec8<BF16_IN, FMT, SK_SCALAR, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
-      break;
-    case SK_ROW:
-      cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
-      break;
-    case SK_COL:
-      cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
-      break;
-    default:
-      cast_to_fp8_vec8<BF16_IN, FMT, SK_FULL, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
-      break;
+  if (sk == SK_SCALAR) {
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_SCALAR, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
+  } else if (sk == SK_FULL) {
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_FULL, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
+  } else if constexpr (!AMAX) {
+    launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax);
+  } else {
+    switch (shape.vectors) {
+      case 1: launch_cast_to_rows<BF16_IN, FMT, AMAX, 1>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
+      case 2: launch_cast_to_rows<BF16_IN, FMT, AMAX, 2>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
+      case 4: launch_cast_to_rows<BF16_IN, FMT, AMAX, 4>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
+      default: launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
+    }
   }
 }
 
@@ -1077,13 +1098,14 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
     // In flat modes the row length need not be a multiple of 8: the tail goes
     // to the generic kernel.  In 2-D modes plan_vectors has required it.
     if (vpr > 0) {
-      const int64_t per_block = amax ? (int64_t)cast_amax_threads(vpr * p.rows * 8) * kCastAmaxU : (int64_t)kThreads * kCastU;
+      const CastAmaxShape shape = cast_amax_shape(p.sk, p.rows, vpr);
+      const int64_t per_block = amax ? (int64_t)shape.threads * shape.vectors : (int64_t)kThreads * kCastU;
       const int64_t bpr = (vpr + per_block - 1) / per_block;
       const int64_t total = bpr * p.rows;
       if (total > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
       const int is_dev = mode == MI355Q_SCALE_DEV;
-      if (amax) launch_cast_to_vec<BF16_IN, FMT, true>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, amax);
-      else launch_cast_to_vec<BF16_IN, FMT, false>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, amax);
+      if (amax) launch_cast_to_vec<BF16_IN, FMT, true>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax);
+      else launch_cast_to_vec<BF16_IN, FMT, false>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax);
       done = p.rows == 1 ? vpr * 8 : n;
     }
   }
