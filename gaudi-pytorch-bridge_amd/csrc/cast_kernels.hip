@@ -18,6 +18,11 @@ constexpr int kThreads = 256;
 
 __global__ void fill_u32_kernel(uint32_t* p, uint32_t v) { *p = v; }
 
+// The word that the stream's next call raises to its amax, cleared on the way instead of by a launch of its own.
+__device__ __forceinline__ void clear_next(uint32_t* next) {
+  if (next != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *next = 0u;
+}
+
 // Kernels that reduce an amax run as at most kAmaxBlocks fat workgroups that
 // stride over the data: the number of same-address atomics, not the streaming,
 // is what bounds them otherwise (2048 blocks: ~30 us; 256 blocks: ~7 us for
@@ -74,11 +79,12 @@ template <bool BF16_IN, int FMT, int SK, bool AMAX, int U>
 __global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to_fp8_vec8(
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
     float scale_host, int scale_is_dev, int64_t vec_per_row, int64_t blocks_per_row,
-    int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax) {
+    int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
   const int THREADS = AMAX ? (int)blockDim.x : kThreads;
   constexpr int IN_BYTES = BF16_IN ? 16 : 32;
   constexpr int kNt = 2;  // non-temporal
   uint32_t am = 0;
+  if constexpr (AMAX) clear_next(next);
   // a logical block is THREADS * U consecutive vectors of one row; without amax
   // (or with few enough of them) the grid holds one workgroup per logical block and this loop runs once
   for (int64_t lb = blockIdx.x; lb < total_blocks; lb += gridDim.x) {
@@ -186,9 +192,10 @@ template <bool BF16_IN, int FMT>
 __global__ __launch_bounds__(kThreads) void cast_to_fp8_generic(
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
     float scale_host, int mode, int64_t start, int64_t n, int64_t mid, int64_t inner,
-    uint32_t* __restrict__ amax) {
+    uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
   const int64_t i = start + (int64_t)blockIdx.x * kThreads + threadIdx.x;
   uint32_t am = 0;
+  clear_next(next);
   if (i < n) {
     float s = 1.0f;
     if (mode == MI355Q_SCALE_HOST) s = scale_host;
@@ -1057,37 +1064,37 @@ inline CastAmaxShape cast_amax_shape(int sk, int64_t rows, int64_t vpr) {
 
 template <bool BF16_IN, int FMT, bool AMAX, int U>
 void launch_cast_to_rows(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, int64_t vpr, int64_t bpr,
-                         int64_t total, int64_t mid, unsigned threads, uint32_t* amax) {
+                         int64_t total, int64_t mid, unsigned threads, uint32_t* amax, uint32_t* next) {
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
-  if (sk == SK_ROW) cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax);
-  else cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax);
+  if (sk == SK_ROW) cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
+  else cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
 }
 
 template <bool BF16_IN, int FMT, bool AMAX>
 void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, float sh, int is_dev, int64_t vpr,
-                        int64_t bpr, int64_t total, int64_t mid, CastAmaxShape shape, uint32_t* amax) {
+                        int64_t bpr, int64_t total, int64_t mid, CastAmaxShape shape, uint32_t* amax, uint32_t* next) {
   constexpr int U = AMAX ? kCastAmaxU : kCastU;
   const unsigned T = AMAX ? shape.threads : kThreads;
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
   if (sk == SK_SCALAR) {
-    cast_to_fp8_vec8<BF16_IN, FMT, SK_SCALAR, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_SCALAR, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax, next);
   } else if (sk == SK_FULL) {
-    cast_to_fp8_vec8<BF16_IN, FMT, SK_FULL, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax);
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_FULL, AMAX, U><<<grid, T, 0, st>>>(x, y, scale, sh, is_dev, vpr, bpr, total, mid, amax, next);
   } else if constexpr (!AMAX) {
-    launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax);
+    launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax, next);
   } else {
     switch (shape.vectors) {
-      case 1: launch_cast_to_rows<BF16_IN, FMT, AMAX, 1>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
-      case 2: launch_cast_to_rows<BF16_IN, FMT, AMAX, 2>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
-      case 4: launch_cast_to_rows<BF16_IN, FMT, AMAX, 4>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
-      default: launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax); break;
+      case 1: launch_cast_to_rows<BF16_IN, FMT, AMAX, 1>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax, next); break;
+      case 2: launch_cast_to_rows<BF16_IN, FMT, AMAX, 2>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax, next); break;
+      case 4: launch_cast_to_rows<BF16_IN, FMT, AMAX, 4>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax, next); break;
+      default: launch_cast_to_rows<BF16_IN, FMT, AMAX, U>(sk, st, x, y, scale, vpr, bpr, total, mid, T, amax, next); break;
     }
   }
 }
 
 template <bool BF16_IN, int FMT>
 int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh, int mode,
-                     int64_t outer, int64_t mid, int64_t inner, uint32_t* amax, hipStream_t st) {
+                     int64_t outer, int64_t mid, int64_t inner, uint32_t* amax, uint32_t* next, hipStream_t st) {
   const int64_t n = outer * mid * inner;
   VecPlan p;
   const bool vec = aligned(x, 16) && aligned(y, 8) &&
@@ -1104,8 +1111,8 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
       const int64_t total = bpr * p.rows;
       if (total > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
       const int is_dev = mode == MI355Q_SCALE_DEV;
-      if (amax) launch_cast_to_vec<BF16_IN, FMT, true>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax);
-      else launch_cast_to_vec<BF16_IN, FMT, false>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax);
+      if (amax) launch_cast_to_vec<BF16_IN, FMT, true>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax, next);
+      else launch_cast_to_vec<BF16_IN, FMT, false>(p.sk, st, x, y, scale, sh, is_dev, vpr, bpr, total, p.mid, shape, amax, next);
       done = p.rows == 1 ? vpr * 8 : n;
     }
   }
@@ -1113,7 +1120,7 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
     const int64_t rest = n - done;
     const int64_t grid = (rest + kThreads - 1) / kThreads;
     if (grid > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
-    cast_to_fp8_generic<BF16_IN, FMT><<<(unsigned)grid, kThreads, 0, st>>>(x, y, scale, sh, mode, done, n, mid, inner, amax);
+    cast_to_fp8_generic<BF16_IN, FMT><<<(unsigned)grid, kThreads, 0, st>>>(x, y, scale, sh, mode, done, n, mid, inner, amax, done > 0 ? nullptr : next);
   }
   return launch_status();
 }
@@ -1426,7 +1433,7 @@ int mi355q_silu_mul_quantize_rows(const void* gate, int64_t ld_gate, const void*
 
 static int cast_to_fp8_rne(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
                        float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
-                       float* amax_out, bool zero_amax, void* stream) {
+                       float* amax_out, bool zero_amax, float* next_amax, void* stream) {
   if (fp8_fmt != MI355Q_E4M3FN && fp8_fmt != MI355Q_E5M2) return MI355Q_ERR_INVALID_ARGUMENT;
   if (!scale_args_ok(scale_dev, scale_mode, outer, mid, inner)) return MI355Q_ERR_INVALID_ARGUMENT;
   const int64_t n = outer * mid * inner;
@@ -1452,28 +1459,38 @@ static int cast_to_fp8_rne(const void* x, int x_dtype, void* y, int fp8_fmt, con
   }
   if (x_dtype != MI355Q_F32 && x_dtype != MI355Q_BF16) return MI355Q_ERR_INVALID_ARGUMENT;
 
-  uint32_t* am = reinterpret_cast<uint32_t*>(amax_out);
+  uint32_t *am = reinterpret_cast<uint32_t*>(amax_out), *next = reinterpret_cast<uint32_t*>(next_amax);
   if (am && zero_amax) fill_u32_kernel<<<1, 1, 0, st>>>(am, 0u);
-  if (n == 0) return launch_status();
-  if (x_dtype == MI355Q_BF16) {
-    if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<true, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
-    return cast_to_dispatch<true, MI355Q_E5M2>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
+  if (n == 0) {
+    if (next) fill_u32_kernel<<<1, 1, 0, st>>>(next, 0u);
+    return launch_status();
   }
-  if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<false, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
-  return cast_to_dispatch<false, MI355Q_E5M2>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, st);
+  if (x_dtype == MI355Q_BF16) {
+    if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<true, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, next, st);
+    return cast_to_dispatch<true, MI355Q_E5M2>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, next, st);
+  }
+  if (fp8_fmt == MI355Q_E4M3FN) return cast_to_dispatch<false, MI355Q_E4M3FN>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, next, st);
+  return cast_to_dispatch<false, MI355Q_E5M2>(xb, yb, scale_dev, scale_host, scale_mode, outer, mid, inner, am, next, st);
 }
 
 int mi355q_cast_to_fp8(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
                        float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
                        float* amax_out, void* stream) {
-  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, amax_out, true, stream);
+  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, amax_out, true, nullptr, stream);
 }
 
 int mi355q_cast_to_fp8_running_amax(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
                                     float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
                                     float* running_amax, void* stream) {
   if (running_amax == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
-  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, running_amax, false, stream);
+  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, running_amax, false, nullptr, stream);
+}
+
+int mi355q_cast_to_fp8_amax_chain(const void* x, int x_dtype, void* y, int fp8_fmt, const float* scale_dev,
+                                  float scale_host, int scale_mode, int64_t outer, int64_t mid, int64_t inner,
+                                  float* amax, int amax_is_zero, float* next_amax, void* stream) {
+  if (amax == nullptr || amax == next_amax) return MI355Q_ERR_INVALID_ARGUMENT;
+  return cast_to_fp8_rne(x, x_dtype, y, fp8_fmt, scale_dev, scale_host, scale_mode, outer, mid, inner, amax, amax_is_zero == 0, next_amax, stream);
 }
 
 int mi355q_cast_from_fp8(const void* x, int fp8_fmt, void* y, int out_dtype, const float* scale_dev,

@@ -202,12 +202,8 @@ bool sr_flush_to_zero_mode() {
 }
 
 // One call for both rounding modes.
-// amax_zeroed: *amax holds zero (round to nearest only).
-int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* amax, bool stochastic, bool amax_zeroed = false) {
+int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* amax, bool stochastic) {
   const int xd = to_mi355q_dtype(x.scalar_type()), od = to_mi355q_dtype(out.scalar_type());
-  if (amax_zeroed)
-    return mi355q_cast_to_fp8_running_amax(x.data_ptr(), xd, out.data_ptr(), od, cs.dev, cs.host, cs.mode, cs.outer, cs.mid,
-                                           cs.inner, amax, current_stream(x));
   if (!stochastic)
     return mi355q_cast_to_fp8(x.data_ptr(), xd, out.data_ptr(), od, cs.dev, cs.host, cs.mode, cs.outer, cs.mid,
                               cs.inner, amax, current_stream(x));
@@ -284,43 +280,52 @@ void drop_ticket_workspace(const Tensor& like, TicketWorkspaceOp op) {
   c.map.erase(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
 }
 
-// Zeroed words for results that kernels accumulate into (amax), so that a call needs no launch that clears one:
-// kWords of them are cleared by one launch, per (device, stream), and each is handed out once.  Every word is an
-// allocation of its own and becomes a tensor only when it is handed out, so that what a caller gets is what at::empty
-// would give: its own storage (it can be saved, resized, recorded on a stream), its own version counter, and an
-// inference tensor or not by the mode of the call that gets it.  Not while the stream is being captured (a replay
-// would find the word as the last one left it).
-struct ZeroWords {
-  static constexpr int64_t kWords = 64;  // what one launch of _foreach_zero_ takes
+// The zeroed word that a stream's next cast raises to its amax: every call clears one for the next in its own kernel, so
+// that no call needs a launch that clears, and no call pays for others (64 words cleared by one launch took every 64th call
+// 60 to 90 us on the host, with a process-wide lock held).  One word per (device, stream); a second thread that calls
+// meanwhile finds none and has its own cleared by a launch.  A word is an allocation of its own and becomes a tensor only
+// when it is handed out, so that what a caller gets is what at::empty would give: its own storage (it can be saved,
+// resized, recorded on a stream), its own version counter, and an inference tensor or not by the mode of the call that
+// gets it.  Not while the stream is being captured (a replay would find the word as the last one left it).
+struct NextWords {
   struct Entry {
-    std::vector<c10::Storage> words;
+    c10::Storage word;
     uint64_t used = 0;
   };
   std::mutex mu;
   uint64_t clock = 0;
   std::map<std::pair<int, void*>, Entry> map;
 };
-Tensor zero_word(const Tensor& like) {
-  static auto* z = new ZeroWords();  // never destroyed, as above
+NextWords& next_words() {
+  static auto* words = new NextWords();  // never destroyed, as above
+  return *words;
+}
+// Undefined where the stream has none.
+Tensor take_zero_word(const Tensor& like) {
   c10::Storage storage;
   {
-    std::lock_guard<std::mutex> lock(z->mu);
-    ZeroWords::Entry& e = z->map[std::make_pair((int)like.device().index(), current_stream(like))];
-    e.used = ++z->clock;
-    if (e.words.empty()) {
-      std::vector<Tensor> fresh;
-      for (int64_t i = 0; i < ZeroWords::kWords; ++i) fresh.push_back(at::empty({}, like.options().dtype(at::kFloat)));
-      at::_foreach_zero_(fresh);
-      for (const Tensor& t : fresh) e.words.push_back(t.storage());
-    }
-    storage = std::move(e.words.back());
-    e.words.pop_back();
-    if (z->map.size() > kKeptWorkspaces) drop_least_recent(z->map);
+    NextWords& w = next_words();
+    std::lock_guard<std::mutex> lock(w.mu);
+    const auto it = w.map.find(std::make_pair((int)like.device().index(), current_stream(like)));
+    if (it == w.map.end() || !it->second.word) return Tensor();
+    storage = std::move(it->second.word);
+    it->second.word = c10::Storage();
   }
   Tensor word = at::detail::make_tensor<c10::TensorImpl>(std::move(storage), c10::DispatchKeySet(c10::DispatchKey::CUDA),
                                                          caffe2::TypeMeta::Make<float>());
   word.unsafeGetTensorImpl()->set_sizes_contiguous({});
   return word;
+}
+// After the launch that clears it.  (Where another thread has put one meanwhile this one goes, after the lock.)
+void put_zero_word(const Tensor& like, c10::Storage word) {
+  c10::Storage dropped;
+  NextWords& w = next_words();
+  std::lock_guard<std::mutex> lock(w.mu);
+  NextWords::Entry& e = w.map[std::make_pair((int)like.device().index(), current_stream(like))];
+  e.used = ++w.clock;
+  std::swap(e.word, word);
+  dropped = std::move(word);
+  if (w.map.size() > kKeptWorkspaces) drop_least_recent(w.map);
 }
 
 // ------------------------------------------------------------ cast_to_fp8_v2
@@ -377,17 +382,27 @@ void cast_to_fp8_v2_boxed(const c10::OperatorHandle& op, c10::DispatchKeySet, to
     DeviceGuard guard(input.device());
     Tensor x = input.contiguous();
     out = at::empty(x.sizes(), x.options().dtype(dst));
-    const bool zeroed = is_amax && !sr && !stream_is_capturing();
-    if (zeroed) amax = zero_word(x);
-    else if (is_amax) amax = at::empty({}, x.options().dtype(at::kFloat));
-    else amax = at::empty({0}, x.options().dtype(at::kFloat));
+    const auto words = x.options().dtype(at::kFloat);
+    const bool chained = is_amax && !sr && !is_fp8(x.scalar_type()) && !stream_is_capturing();
+    if (chained) amax = take_zero_word(x);
+    const bool zeroed = amax.defined();
+    if (!zeroed) amax = is_amax ? at::empty({}, words) : at::empty({0}, words);
     CastScale cs;
     if (is_fp8(x.scalar_type())) {
       cs.outer = x.numel();  // fp8 -> same fp8: copy, scale plays no part
     } else {
       cs = resolve_cast_scale(scale, scale_shape, x);
     }
-    check_status(launch_cast_to(x, out, cs, is_amax ? amax.data_ptr<float>() : nullptr, sr, zeroed), "mi355q_cast_to_fp8");
+    if (chained) {
+      Tensor next = at::empty({}, words);
+      check_status(mi355q_cast_to_fp8_amax_chain(x.data_ptr(), to_mi355q_dtype(x.scalar_type()), out.data_ptr(), to_mi355q_dtype(dst), cs.dev,
+                                                 cs.host, cs.mode, cs.outer, cs.mid, cs.inner, amax.data_ptr<float>(), zeroed ? 1 : 0,
+                                                 next.data_ptr<float>(), current_stream(x)),
+                   "mi355q_cast_to_fp8");
+      put_zero_word(x, next.storage());
+    } else {
+      check_status(launch_cast_to(x, out, cs, is_amax ? amax.data_ptr<float>() : nullptr, sr), "mi355q_cast_to_fp8");
+    }
   }
   torch::jit::drop(*stack, 6);
   stack->emplace_back(std::move(out));

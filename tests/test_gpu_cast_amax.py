@@ -1,7 +1,8 @@
 """cast_to_fp8 with amax at the edges of its launch shapes (one workgroup, up to 2^21 elements, one logical block per
-workgroup, several), many calls in a row (zeroed words are cleared many at a time), streams, and the C entry that
-raises a running maximum."""
+workgroup, several), many calls in a row (each clears the next one's word), streams, threads, and the C entries that
+raise a running maximum and chain calls."""
 import ctypes
+import threading
 
 import pytest
 import torch
@@ -62,7 +63,7 @@ def test_column_scales_cost_little_more_than_one_scale(dev):
 
 
 def test_every_call_has_its_own_word(dev):
-    """More calls than one launch clears words for, on two streams, all results kept."""
+    """Many calls on two streams, all results kept."""
     xs = [torch.full((5,), float(i + 1), device=dev).bfloat16() for i in range(8)]
     side = torch.cuda.Stream()
     got = []
@@ -80,7 +81,7 @@ def test_every_call_has_its_own_word(dev):
 
 
 def test_amax_is_an_ordinary_tensor(dev):
-    """Whatever mode the words were cleared in: own storage and version, resizable, an inference tensor only by the call's own mode."""
+    """Whatever mode the call was made in that cleared the word: own storage and version, resizable, an inference tensor only by the call's own mode."""
     x = torch.tensor([-3.0, 1.0], device=dev).bfloat16()
     call = lambda: torch.ops.hpu.cast_to_fp8_v2(x, None, False, True, E4)[1]  # noqa: E731
     for _ in range(70):
@@ -94,6 +95,63 @@ def test_amax_is_an_ordinary_tensor(dev):
         assert second._version == version
         first.resize_(100).fill_(-1.0)
         assert second.item() == 3.0 and inside.item() == 3.0
+
+
+def test_no_call_pays_for_others(dev):
+    """Every call allocates its codes, and its own or the next call's word: no call makes a stock for later ones."""
+    x = torch.ones(4096, device=dev).bfloat16()
+    kept = []
+    for _ in range(200):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        kept.append(torch.ops.hpu.cast_to_fp8_v2(x, None, False, True, E4))
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] - before <= 3
+    assert all(a.item() == 1.0 for _, a in kept)
+
+
+def test_threads_on_one_stream_and_on_their_own(dev):
+    """Threads that share a stream find no word now and then and clear their own; none sees another's."""
+    tops = [float(2 ** i) for i in range(8)]
+    xs = [torch.full((1000 + i,), t, device=dev).bfloat16() for i, t in enumerate(tops)]
+    torch.cuda.synchronize()
+    shared = torch.cuda.Stream()
+    got, errors = [[] for _ in tops], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(shared if i < 5 else torch.cuda.Stream()):
+                for _ in range(100):
+                    got[i].append(torch.ops.hpu.cast_to_fp8_v2(xs[i], None, False, True, E4)[1])
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for i, t in enumerate(tops):
+        assert torch.stack(got[i]).cpu().eq(t).all()
+
+
+@pytest.mark.parametrize("n", [0, 5, 4096, 4099, 2 ** 22 + 3])
+def test_chained_calls(pkg, dev, n):
+    """The C entry: each call's maximum in the word that the call before it cleared, tails and empty tensors among them."""
+    lib = pkg.capi()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    words = torch.full((4,), 77.0, device=dev)
+    y = torch.empty(n, dtype=E4, device=dev)
+    word = lambda i: words.data_ptr() + 4 * i  # noqa: E731
+    for i, top in enumerate((5.0, 3.0, 4.0)):
+        x = torch.full((n,), -top, device=dev).bfloat16()
+        assert lib.mi355q_cast_to_fp8_amax_chain(x.data_ptr(), pkg.BF16, y.data_ptr(), pkg.E4M3FN, None, 1.0, pkg.SCALE_NONE, n, 1, 1, word(i),
+                                                 int(i > 0), word(i + 1) if i < 2 else None, st) == 0
+    assert words.tolist() == ([5.0, 3.0, 4.0] if n else [0.0, 0.0, 0.0]) + [77.0]
+    for amax, following in ((None, word(0)), (word(0), word(0))):
+        assert lib.mi355q_cast_to_fp8_amax_chain(x.data_ptr(), pkg.BF16, y.data_ptr(), pkg.E4M3FN, None, 1.0, pkg.SCALE_NONE, n, 1, 1, amax, 1, following,
+                                                 st) != 0
 
 
 def test_running_maximum(pkg, dev):
