@@ -507,7 +507,7 @@ def bench_gemm_c3(ops, oracle, pkg, dev, steps, warmup, cpu):
             "ms_nk": ms_nk, "tflops_nk": flop / (ms_nk * 1e-3) / 1e12, "variant_nk": variant_nk}
 
 
-def bench_gemm_decode(ops, oracle, dev, steps, warmup):
+def bench_gemm_decode(ops, oracle, pkg, dev, steps, warmup):
     """benchmark configuration 4: per-token x per-channel scales, K = 8192, N = 28672."""
     out = []
     gen = torch.Generator().manual_seed(SEED)
@@ -550,7 +550,8 @@ def bench_gemm_decode(ops, oracle, dev, steps, warmup):
         out.append(hbm_entry(f"fp8_gemm_v2_decode_M{M}",
                              f"C4 fp8_gemm_v2 M={M} K=8192 N=28672 per-token x per-channel scales -> bf16",
                              nbytes, ms, steps, "fp8_gemm_stream_kernel" if M <= 16 else "fp8_gemm_skinny_kernel" if M <= 128 else "fp8_gemm_tile_kernel<256,128>",
-                             extra={"tflops": round(flop / (ms * 1e-3) / 1e12, 2), "library_gemm_ms_same_shape": lib_ms}))
+                             extra={"kernel_variant": pkg.capi().mi355q_fp8_gemm_ws_variant(0, K, 0, N, M, N, K, 1).decode(),
+                                    "tflops": round(flop / (ms * 1e-3) / 1e12, 2), "library_gemm_ms_same_shape": lib_ms}))
     return out
 
 
@@ -791,7 +792,7 @@ def main():
     if "mlp" in which:
         ops_out.append(bench_mlp(ops, dev, max(args.steps // 2, 5), args.warmup))
     if "decode" in which:
-        ops_out += bench_gemm_decode(ops, oracle, dev, args.steps, args.warmup)
+        ops_out += bench_gemm_decode(ops, oracle, pkg, dev, args.steps, args.warmup)
     if "int4" in which:
         ops_out += bench_int4(pkg, oracle, dev, k_stream, w_stream, cpu)
     if "cast" in which or "castlarge" in which:

@@ -160,6 +160,24 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   return best;
 }
 
+// What launch_by_size and launch_gemm_stream run; may_split: the caller brings the workspace.
+const char* variant_name(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+  if (lda % 16 || ldb % 16 || lda > (1LL << 22) || ldb > (1LL << 22) || !k_chunks_ok(trans_a, trans_b, K)) return "simple";
+  const SplitPlan p = split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, may_split);
+  if (M <= 128) {
+    if (p.stream) return p.parts > 1 ? "split_stream_Mx256_registers_mfma16x16" : "stream_Mx256_registers_mfma16x16";
+    return p.parts > 1 ? "split_strip_Mx128x128_ring_mfma32x32x64" : "strip_Mx128x128_ring_mfma32x32x64";
+  }
+  if (p.tile == SplitTile::k128x128) return "split_tile128x128x128_mfma32x32x64";
+  if (p.tile == SplitTile::k256x128) return "split_tile256x128x128_mfma32x32x64";
+  switch (N > 128 ? choose_tiles(M, N, K, batch) : TileChoice::k128x128) {
+    case TileChoice::k256x256: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
+    case TileChoice::k256x128: return "tile256x128x128_mfma32x32x64";
+    case TileChoice::k128x128: break;
+  }
+  return "tile128x128x128_mfma32x32x64";
+}
+
 }  // namespace mi355q
 
 using namespace mi355q;
@@ -168,17 +186,12 @@ extern "C" {
 
 const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
                                     int64_t N, int64_t K) {
-  if (lda % 16 || ldb % 16 || !mi355q::k_chunks_ok(trans_a, trans_b, K)) return "simple";
-  if (M > 128 && N > 128) {
-    switch (mi355q::choose_tiles(M, N, K, 1)) {
-      case mi355q::TileChoice::k256x256: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
-      case mi355q::TileChoice::k256x128: return "tile256x128x128_mfma32x32x64";
-      case mi355q::TileChoice::k128x128: return "tile128x128x128_mfma32x32x64";
-    }
-  }
-  if (mi355q::split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, 1, true).stream) return "stream_Mx256_registers_mfma16x16";
-  if (M <= 128) return "strip_Mx128x128_ring_mfma32x32x64";
-  return "tile128x128x128_mfma32x32x64";
+  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, 1, false);
+}
+
+const char* mi355q_fp8_gemm_ws_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
+                                       int64_t N, int64_t K, int64_t batch) {
+  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
 }
 
 size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,

@@ -496,10 +496,14 @@ typedef struct mi355q_pad_desc {
 } mi355q_pad_desc;
 int mi355q_pad_rows(const mi355q_pad_desc* desc, int count, void* stream);
 
-/* Name of the kernel variant mi355q_fp8_gemm would pick for a problem
- * (for logs and profiles; static string). */
+/* Name of the kernel variant that mi355q_fp8_gemm picks for a problem of one
+ * batch with 16-byte aligned operands, and of the one that mi355q_fp8_gemm_ws
+ * picks with a workspace ("split_...": K in parts over workgroups).  For logs
+ * and profiles; static strings. */
 const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb,
                                     int64_t M, int64_t N, int64_t K);
+const char* mi355q_fp8_gemm_ws_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb,
+                                       int64_t M, int64_t N, int64_t K, int64_t batch);
 
 #ifdef __cplusplus
 }

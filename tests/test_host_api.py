@@ -80,6 +80,31 @@ def test_variant_names(pkg):
     assert lib.mi355q_fp8_gemm_variant(0, 1040, 0, 1008, 515, 1001, 1030) == b"simple"       # K contiguous and ragged
 
 
+def test_variant_names_are_those_of_the_entry(pkg):
+    """mi355q_fp8_gemm has no workspace, so it never splits, and its choice among the kernels for few rows is the one made
+    without parts; mi355q_fp8_gemm_ws splits exactly where it asks for a workspace."""
+    lib = pkg.capi()
+    names = lambda m, k, n, nk=0: (lib.mi355q_fp8_gemm_variant(0, k, nk, k if nk else n, m, n, k),  # noqa: E731
+                                   lib.mi355q_fp8_gemm_ws_variant(0, k, nk, k if nk else n, m, n, k, 1))
+    for m, k, n in [(1, 4096, 1024), (1, 14336, 4096), (1, 4096, 4096)]:
+        plain, ws = names(m, k, n)
+        assert plain.startswith(b"strip_") and ws.startswith(b"split_stream_"), (m, k, n, plain, ws)
+    assert names(64, 14336, 4096)[1].startswith(b"split_strip_")
+    assert names(256, 14336, 1024)[1].startswith(b"split_tile128x128")
+    assert names(8192, 4096, 14336) == (b"tile256x256x128_mfma16x16x128",) * 2
+    for m in (1, 8, 16, 17, 64, 128, 129, 256, 300, 1000, 4096):
+        for k in (512, 2048, 4096, 14336):
+            for n in (16, 128, 1024, 4096, 28672):
+                for nk in (0, 1):
+                    plain, ws = names(m, k, n, nk)
+                    assert not plain.startswith(b"split_")
+                    need = lib.mi355q_fp8_gemm_workspace_bytes(0, k, nk, k if nk else n, m, n, k, 1)
+                    assert ws.startswith(b"split_") == (need > 0), (m, k, n, nk, ws)
+                    assert need > 0 or ws == plain or m <= 128, (m, k, n, nk, plain, ws)
+    # more columns than the tiles' 31-bit offsets reach
+    assert lib.mi355q_fp8_gemm_variant(0, 64, 0, (1 << 22) + 16, 8, 1 << 22, 64) == b"simple"
+
+
 @pytest.mark.parametrize("key", sorted(REFERENCE_SCHEMAS))
 def test_schemas_are_the_references(pkg, key):
     name, overload = key
