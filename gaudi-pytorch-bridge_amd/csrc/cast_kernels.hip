@@ -187,34 +187,44 @@ __global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to
   }
 }
 
-// One element per thread, any alignment, any broadcast: tails and odd shapes.
-template <bool BF16_IN, int FMT>
+// Element by element, any alignment, any broadcast: tails and odd shapes.
+// A form of its own without amax (with the amax chain's clearing in it, that too, such calls took 6.9 and 11.1 instead of
+// 6.4 and 10.2 us, 3001 x 1001 and 16384 x 333 fp32 per column).  With amax a thread takes kGenericAmaxU elements, which
+// makes that many fewer workgroups meet at one word: one, four, eight, sixteen elements 22.6, 13.9, 14.4, 12.6 us at
+// 3001 x 1001 bf16, 72, 52, 41, 37 at 4095 x 4095, 11.7, 8.3, 7.1, 9.8 at 100 x 3001.
+constexpr int kGenericAmaxU = 8;
+template <bool BF16_IN, int FMT, bool AMAX>
 __global__ __launch_bounds__(kThreads) void cast_to_fp8_generic(
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
     float scale_host, int mode, int64_t start, int64_t n, int64_t mid, int64_t inner,
     uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
-  const int64_t i = start + (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  constexpr int U = AMAX ? kGenericAmaxU : 1;
   uint32_t am = 0;
-  clear_next(next);
-  if (i < n) {
-    float s = 1.0f;
-    if (mode == MI355Q_SCALE_HOST) s = scale_host;
-    else if (mode == MI355Q_SCALE_DEV) s = scale[0];
-    else if (mode == MI355Q_SCALE_MID) s = scale[(i / inner) % mid];
-    else if (mode == MI355Q_SCALE_FULL) s = scale[i];
-    float v, p;
-    if constexpr (BF16_IN) {
-      const uint32_t h = reinterpret_cast<const uint16_t*>(x)[i];
-      v = bf16_bits_to_f32(h);
-      p = round_to_bf16(v * round_to_bf16(s));
-    } else {
-      v = reinterpret_cast<const float*>(x)[i];
-      p = v * s;
+  if constexpr (AMAX) clear_next(next);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = start + ((int64_t)blockIdx.x * U + u) * kThreads + threadIdx.x;
+    if (i < n) {
+      float s = 1.0f;
+      if (mode == MI355Q_SCALE_HOST) s = scale_host;
+      else if (mode == MI355Q_SCALE_DEV) s = scale[0];
+      else if (mode == MI355Q_SCALE_MID) s = scale[(i / inner) % mid];
+      else if (mode == MI355Q_SCALE_FULL) s = scale[i];
+      float v, p;
+      if constexpr (BF16_IN) {
+        const uint32_t h = reinterpret_cast<const uint16_t*>(x)[i];
+        v = bf16_bits_to_f32(h);
+        p = round_to_bf16(v * round_to_bf16(s));
+      } else {
+        v = reinterpret_cast<const float*>(x)[i];
+        p = v * s;
+      }
+      const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
+      am = am > a ? am : a;
+      y[i] = (uint8_t)(cvt_fp8x4<FMT>(p, p, p, p) & 0xffu);
     }
-    am = __float_as_uint(v) & 0x7fffffffu;
-    y[i] = (uint8_t)(cvt_fp8x4<FMT>(p, p, p, p) & 0xffu);
   }
-  if (amax != nullptr) block_amax_commit(am, amax);
+  if constexpr (AMAX) block_amax_commit(am, amax);
 }
 
 // Stochastic rounding with flush to zero (round mode CAST_ROUND_SFTZ of GetCastParams,
@@ -1118,9 +1128,10 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
   }
   if (done < n) {
     const int64_t rest = n - done;
-    const int64_t grid = (rest + kThreads - 1) / kThreads;
+    const int64_t per_block = (int64_t)kThreads * (amax ? kGenericAmaxU : 1), grid = (rest + per_block - 1) / per_block;
     if (grid > 0x7fffffffLL) return MI355Q_ERR_UNSUPPORTED;
-    cast_to_fp8_generic<BF16_IN, FMT><<<(unsigned)grid, kThreads, 0, st>>>(x, y, scale, sh, mode, done, n, mid, inner, amax, done > 0 ? nullptr : next);
+    if (amax) cast_to_fp8_generic<BF16_IN, FMT, true><<<(unsigned)grid, kThreads, 0, st>>>(x, y, scale, sh, mode, done, n, mid, inner, amax, done > 0 ? nullptr : next);
+    else cast_to_fp8_generic<BF16_IN, FMT, false><<<(unsigned)grid, kThreads, 0, st>>>(x, y, scale, sh, mode, done, n, mid, inner, nullptr, nullptr);
   }
   return launch_status();
 }

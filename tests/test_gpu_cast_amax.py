@@ -43,6 +43,21 @@ def test_amax_and_codes_with_row_and_column_scales(oracle, dev, rows, cols, dtyp
     assert torch.equal(y.cpu().view(torch.uint8), y_ref.view(torch.uint8))
 
 
+# no whole vectors in a row: an element per thread without amax, eight with it (2048 a workgroup)
+@pytest.mark.parametrize("rows,cols", [(1, 3), (3, 683), (2048, 1), (293, 7), (3001, 1001)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("is_amax", [False, True])
+def test_ragged_rows_with_column_scales(oracle, dev, rows, cols, dtype, is_amax):
+    g = torch.Generator().manual_seed(cols)
+    x = torch.randn(rows, cols, generator=g).to(dtype)
+    x.view(-1)[-1] = 9.5  # in the last element
+    scale = torch.rand(cols, generator=g) + 20
+    y, amax = torch.ops.hpu.cast_to_fp8_v2(x.to(dev), scale.to(dev), False, is_amax, E4, [1, cols])
+    y_ref, _ = oracle.c_cast_to_fp8(x, scale, E4, True, scale_shape=[1, cols])
+    assert torch.equal(y.cpu().view(torch.uint8), y_ref.view(torch.uint8))
+    assert amax.item() == 9.5 if is_amax else amax.shape == (0,)
+
+
 def test_column_scales_cost_little_more_than_one_scale(dev):
     x, scale = torch.randn(4096, 4096, device=dev).bfloat16(), torch.rand(4096, device=dev) + 0.5
 
