@@ -35,8 +35,13 @@ constexpr int kAmaxBlocks = 256;
 //   this                   4.2    4.5    6.1    7.4   11.4   34.1    131
 //   256 x 1024 threads     4.6    5.7    7.3    9.1   11.5   34.9    136
 //   up to 2048 x 256       4.3    4.7   11.3   24.6     94     97    154    (atomics on one word: 13 to 45 ns each)
+// An fp32 vector is 32 bytes, so four of them are as many bytes as eight of bf16; with eight, and with 1024 threads, fp32, us:
+//   elements              2^22   2^23   2^24   2^25   2^26   2^27
+//   four, 512 threads      7.5    9.5   17.1   30.8   59.7    118
+//   eight, 512 threads     7.9    9.4   18.3   33.8   66.7    134
+//   four, 1024 threads     7.8    8.9   17.2   32.0   61.9    123
 constexpr int kCastAmaxMaxThreads = 512;
-constexpr int kCastAmaxU = 8;
+constexpr int cast_amax_vectors(bool bf16_in) { return bf16_in ? 8 : 4; }
 constexpr int64_t kCastAmaxSmall = int64_t(1) << 21;  // elements
 
 // Block-level max of abs-value bit patterns, then one atomicMax per block.
@@ -1065,11 +1070,12 @@ struct CastAmaxShape {
   unsigned threads;
   int vectors;
 };
-inline CastAmaxShape cast_amax_shape(int sk, int64_t rows, int64_t vpr) {
+template <bool BF16_IN>
+CastAmaxShape cast_amax_shape(int sk, int64_t rows, int64_t vpr) {
   const bool small = rows * vpr * 8 <= kCastAmaxSmall;
   const unsigned threads = small ? kThreads : kCastAmaxMaxThreads;
-  if (sk == SK_SCALAR || sk == SK_FULL) return {threads, kCastAmaxU};
-  return {threads, small || vpr <= kCastAmaxMaxThreads ? 1 : (vpr <= 2 * kCastAmaxMaxThreads ? 2 : (vpr <= 4 * kCastAmaxMaxThreads ? 4 : kCastAmaxU))};
+  if (sk == SK_SCALAR || sk == SK_FULL) return {threads, cast_amax_vectors(BF16_IN)};
+  return {threads, small || vpr <= kCastAmaxMaxThreads ? 1 : (vpr <= 2 * kCastAmaxMaxThreads ? 2 : (vpr <= 4 * kCastAmaxMaxThreads ? 4 : cast_amax_vectors(BF16_IN)))};
 }
 
 template <bool BF16_IN, int FMT, bool AMAX, int U>
@@ -1083,7 +1089,7 @@ void launch_cast_to_rows(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, c
 template <bool BF16_IN, int FMT, bool AMAX>
 void launch_cast_to_vec(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, float sh, int is_dev, int64_t vpr,
                         int64_t bpr, int64_t total, int64_t mid, CastAmaxShape shape, uint32_t* amax, uint32_t* next) {
-  constexpr int U = AMAX ? kCastAmaxU : kCastU;
+  constexpr int U = AMAX ? cast_amax_vectors(BF16_IN) : kCastU;
   const unsigned T = AMAX ? shape.threads : kThreads;
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
   if (sk == SK_SCALAR) {
@@ -1115,7 +1121,7 @@ int cast_to_dispatch(const uint8_t* x, uint8_t* y, const float* scale, float sh,
     // In flat modes the row length need not be a multiple of 8: the tail goes
     // to the generic kernel.  In 2-D modes plan_vectors has required it.
     if (vpr > 0) {
-      const CastAmaxShape shape = cast_amax_shape(p.sk, p.rows, vpr);
+      const CastAmaxShape shape = cast_amax_shape<BF16_IN>(p.sk, p.rows, vpr);
       const int64_t per_block = amax ? (int64_t)shape.threads * shape.vectors : (int64_t)kThreads * kCastU;
       const int64_t bpr = (vpr + per_block - 1) / per_block;
       const int64_t total = bpr * p.rows;

@@ -10,7 +10,7 @@ import torch
 from helpers import E4
 
 pytestmark = pytest.mark.gpu
-SIZES = [1, 8, 4096, 16384, 16392, 2 ** 21, 2 ** 21 + 8, 2 ** 23, 2 ** 23 + 40, 2 ** 24 + 3]
+SIZES = [1, 8, 4096, 16384, 16392, 2 ** 21, 2 ** 21 + 8, 2 ** 22, 2 ** 22 + 8, 2 ** 23, 2 ** 23 + 40, 2 ** 24 + 3]
 
 
 @pytest.mark.parametrize("n", SIZES)
