@@ -133,7 +133,7 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
     const int64_t shortest = stream ? 512 : unit;  // part
     const bool in_parts = may_split && K >= (stream ? 2048 : 1792);
     const int64_t strips = (N + nb - 1) / nb, groups = strips * batch, units = (K + unit - 1) / unit;
-    const int64_t rows = M < 32 ? M : tile_rows;  // rows of sums that travel
+    const int64_t rows = M < 32 && tile_rows <= 32 ? M : tile_rows;  // rows of sums that travel (those of one row tile alone can be left out)
     const double width = (double)nb + (stream ? 0.0 : (double)tile_rows * (b_kmajor ? 0.25 : 0.5));
     for (int64_t parts = 1; parts <= 32 && parts <= units; ++parts) {
       if (parts > 1 && (!in_parts || groups > kMaxTickets || (double)(groups * parts) > 2.0 * cus)) break;

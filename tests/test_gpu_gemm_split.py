@@ -115,6 +115,16 @@ def test_short_products_stay_whole(pkg):
         assert 2 <= parts <= 8, (n, parts)
 
 
+def test_few_rows_of_an_mn_major_a_stay_whole_longer(pkg):
+    """A [K, M] runs on tiles of 128 rows, whose parts send all their sums: 16 x 1792 x 128 takes 12.0 us whole and 16.4 in parts."""
+    need = pkg.capi().mi355q_fp8_gemm_workspace_bytes
+    for k in (1792, 2048):
+        for n in (128, 1024, 4096, 14336):
+            for nk in (0, 1):
+                assert need(1, 16, nk, k if nk else n, 16, n, k, 1) == 0, (k, n, nk)
+    assert need(1, 16, 0, 1024, 16, 1024, 8192, 1) > 0
+
+
 @pytest.mark.timeout(600)
 def test_parts_of_k_meet_by_device_scope_accesses_in_order():
     """Sums stored (sc1), acknowledged, barrier, ticket, barrier, counter reset, sums read (sc1); nothing cache-wide."""
