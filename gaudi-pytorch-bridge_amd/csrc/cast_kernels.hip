@@ -81,11 +81,11 @@ __device__ __forceinline__ void block_amax_commit(uint32_t m, uint32_t* amax) {
 // load the compiler cannot tell that the previous iteration's load into the
 // same registers was consumed, and makes every load wait for all earlier ones.)
 template <bool BF16_IN, int FMT, int SK, bool AMAX, int U>
-__global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to_fp8_vec8(
+__device__ __forceinline__ void cast_to_fp8_vectors(
+    const int THREADS,
     const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
     float scale_host, int scale_is_dev, int64_t vec_per_row, int64_t blocks_per_row,
     int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
-  const int THREADS = AMAX ? (int)blockDim.x : kThreads;
   constexpr int IN_BYTES = BF16_IN ? 16 : 32;
   constexpr int kNt = 2;  // non-temporal
   uint32_t am = 0;
@@ -190,6 +190,22 @@ __global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to
     }
     block_amax_commit(am, amax);
   }
+}
+
+template <bool BF16_IN, int FMT, int SK, bool AMAX, int U>
+__global__ __launch_bounds__(AMAX ? kCastAmaxMaxThreads : kThreads) void cast_to_fp8_vec8(
+    const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale,
+    float scale_host, int scale_is_dev, int64_t vec_per_row, int64_t blocks_per_row,
+    int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
+  cast_to_fp8_vectors<BF16_IN, FMT, SK, AMAX, U>(AMAX ? (int)blockDim.x : kThreads, x, y, scale, scale_host, scale_is_dev, vec_per_row, blocks_per_row, total_blocks, mid, amax, next);
+}
+
+// With amax and rows that hold one or two vectors per thread (cast_amax_shape): less in flight per thread, by design.
+template <bool BF16_IN, int FMT, int SK, int U>
+__global__ __launch_bounds__(kCastAmaxMaxThreads) void cast_to_fp8_short_rows(
+    const uint8_t* __restrict__ x, uint8_t* __restrict__ y, const float* __restrict__ scale, int64_t vec_per_row, int64_t blocks_per_row,
+    int64_t total_blocks, int64_t mid, uint32_t* __restrict__ amax, uint32_t* __restrict__ next) {
+  cast_to_fp8_vectors<BF16_IN, FMT, SK, true, U>((int)blockDim.x, x, y, scale, 0.0f, 1, vec_per_row, blocks_per_row, total_blocks, mid, amax, next);
 }
 
 // Element by element, any alignment, any broadcast: tails and odd shapes.
@@ -1082,8 +1098,14 @@ template <bool BF16_IN, int FMT, bool AMAX, int U>
 void launch_cast_to_rows(int sk, hipStream_t st, const uint8_t* x, uint8_t* y, const float* scale, int64_t vpr, int64_t bpr,
                          int64_t total, int64_t mid, unsigned threads, uint32_t* amax, uint32_t* next) {
   const unsigned grid = (unsigned)(AMAX && total > kAmaxBlocks ? kAmaxBlocks : total);
-  if (sk == SK_ROW) cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
-  else cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
+  if constexpr (U < 4) {
+    if (sk == SK_ROW) cast_to_fp8_short_rows<BF16_IN, FMT, SK_ROW, U><<<grid, threads, 0, st>>>(x, y, scale, vpr, bpr, total, mid, amax, next);
+    else cast_to_fp8_short_rows<BF16_IN, FMT, SK_COL, U><<<grid, threads, 0, st>>>(x, y, scale, vpr, bpr, total, mid, amax, next);
+  } else if (sk == SK_ROW) {
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_ROW, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
+  } else {
+    cast_to_fp8_vec8<BF16_IN, FMT, SK_COL, AMAX, U><<<grid, threads, 0, st>>>(x, y, scale, 0.0f, 1, vpr, bpr, total, mid, amax, next);
+  }
 }
 
 template <bool BF16_IN, int FMT, bool AMAX>

@@ -165,7 +165,9 @@ def test_streaming_kernels_issue_their_loads_back_to_back():
     for name, seq in order.items():
         if "cast_to_fp8_vec8" in name or "cast_from_fp8_vec" in name:
             loads = 4                                   # U
-        elif "quantize_rows_kernel" in name:            # VPT is the last template argument
+        elif "cast_to_fp8_short_rows" in name:          # U is the last template argument
+            loads = int(name.split("ELi")[-1].split("E")[0])
+        elif "quantize_rows_kernel" in name:            # VPT is the last integer among the template arguments
             loads = int(name.split("ELi")[-1].split("E")[0]) * (2 if "silu_mul" in name else 1)
         else:
             continue
