@@ -17,7 +17,7 @@
 namespace mi355q {
 
 constexpr int kTicketStride = 16;                         // 32-bit words: one counter per 64-byte line
-constexpr size_t kTicketBytes = 64 * 1024;                // the counters' area, in front of the sums, the same for every shape
+constexpr size_t kTicketBytes = MI355Q_FP8_GEMM_COUNTER_BYTES;  // the counters' area, in front of the sums, the same for every shape
 constexpr int kMaxTickets = (int)(kTicketBytes / (kTicketStride * 4));
 
 enum class SplitTile { kStrip, k128x128, k256x128 };  // kStrip: the kernels for at most 128 rows

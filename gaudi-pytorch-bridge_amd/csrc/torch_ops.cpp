@@ -688,7 +688,7 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
 
   const size_t ws_bytes = mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
   const bool kept = ws_bytes == 0 || !stream_is_capturing();
-  Tensor ws = kept ? ticket_workspace(A, ws_bytes, kWsGemm) : captured_ticket_workspace(A, ws_bytes, 65536);
+  Tensor ws = kept ? ticket_workspace(A, ws_bytes, kWsGemm) : captured_ticket_workspace(A, ws_bytes, MI355Q_FP8_GEMM_COUNTER_BYTES);
   const int st =
       mi355q_fp8_gemm_ws(ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
                       bc_t.data_ptr(), to_mi355q_dtype(B.scalar_type()), tb ? 1 : 0, ldb,

@@ -266,11 +266,13 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda,
  * K is walked in parts by several workgroups whose fp32 sums meet through
  * `workspace` (device memory, 16-byte aligned, at least
  * mi355q_fp8_gemm_workspace_bytes() bytes; 0: the problem does not split).
- * It begins with 64 KiB of arrival counters (the same place for every shape):
+ * It begins with MI355Q_FP8_GEMM_COUNTER_BYTES of arrival counters (the same
+ * place for every shape; the rest need not be cleared):
  * zero-filled once before its first use, left zero by every call; calls that
  * may overlap in time need workspaces of their own.  NULL: the same result
  * (sums in another order) without the split.
  */
+#define MI355Q_FP8_GEMM_COUNTER_BYTES 65536
 size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb,
                                        int64_t M, int64_t N, int64_t K, int64_t batch);
 int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,

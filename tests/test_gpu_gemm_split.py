@@ -136,3 +136,50 @@ def test_parts_of_k_meet_by_device_scope_accesses_in_order():
         for name, seq in orders.items():
             assert "F" not in seq and seq.count("A") == 1, name
             assert re.search(r"S+W+BAW?BS?W?L+", seq), (name, seq)
+
+
+@pytest.mark.gpu
+def test_split_products_in_flight_on_two_streams(dev):
+    """Each stream has a workspace of its own: products of three kernels, interleaved without a wait."""
+    g = torch.Generator().manual_seed(8)
+    work = []
+    for m, k, n in ((1, 4096, 1024), (64, 14336, 256), (300, 8192, 1024)):
+        a, w = torch.randn(m, k, generator=g).to(E4).to(dev), torch.randn(k, n, generator=g).to(E4).to(dev)
+        work.append((a, w, torch.ops.hpu.fp8_gemm_v2(a, False, w, False, None, torch.float32)))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = []
+    for i in range(60):
+        with torch.cuda.stream(streams[i % 2]):
+            a, w, want = work[(i // 2 + i % 2) % 3]
+            got.append((torch.ops.hpu.fp8_gemm_v2(a, False, w, False, None, torch.float32), want))
+    torch.cuda.synchronize()
+    assert all(torch.equal(c, want) for c, want in got)
+
+
+@pytest.mark.gpu
+def test_workspaces_that_are_given_back(dev):
+    """More (stream, operator) pairs than buffers are kept: the least recently used one goes, and calls on its stream start
+    from a fresh one.  torch has 32 streams to hand out, so three operators with a workspace take part."""
+    g = torch.Generator().manual_seed(9)
+    a, w = torch.randn(1, 4096, generator=g).to(E4).to(dev), torch.randn(4096, 1024, generator=g).to(E4).to(dev)
+    x = torch.randn(8, 4096, generator=g).to(dev)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (4096, 64), generator=g, dtype=torch.int64).to(torch.int32).to(dev)
+    scale = (torch.rand(32, 512, generator=g) * 0.01).bfloat16().to(dev)
+
+    def run():
+        return (torch.ops.hpu.fp8_gemm_v2(a, False, w, False, None, torch.float32),
+                torch.ops.mi355q.w4a8_gemm(x.to(E4), packed, scale, None, False, torch.bfloat16, None, None),
+                torch.ops.mi355q.w4a16_gemm(x.bfloat16(), packed, scale, None, False, torch.bfloat16, None))
+
+    want = run()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(32)]
+    assert len({s.cuda_stream for s in streams}) * 3 > 64
+    got = []
+    for _ in range(3):
+        for s in streams:
+            with torch.cuda.stream(s):
+                got.append(run())
+    torch.cuda.synchronize()
+    assert all(torch.equal(c, r) for outs in got for c, r in zip(outs, want))

@@ -79,6 +79,39 @@ def test_graph_replays_of_a_ragged_product(dev):
         assert torch.equal(got, eager) and torch.equal(got.cpu(), a @ w8.cpu().float()), rep
 
 
+# one product per kernel that splits K: the stream kernel, the strip kernel, tiles that meet in pairs
+@pytest.mark.parametrize("M,K,N,name", [(1, 4096, 1024, b"split_stream"), (64, 14336, 256, b"split_strip"), (300, 8192, 1024, b"split_tile")])
+def test_graph_replays_of_split_products(pkg, dev, M, K, N, name):
+    """The arrival counters lie in a tensor of the graph's own, cleared by a fill kernel of the graph; here that memory is
+    full of ones when the allocator hands it out, in the capture and in every replay."""
+    assert pkg.capi().mi355q_fp8_gemm_ws_variant(0, K, 0, N, M, N, K, 1).startswith(name)
+    g = torch.Generator().manual_seed(M)
+    w8 = torch.randn(K, N, generator=g).to(E4).to(dev)
+    static_a = torch.zeros(M, K, dtype=E4, device=dev)
+    run = lambda a: ops.fp8_gemm_v2(a, False, w8, False, None, torch.float32)  # noqa: E731
+    run(static_a)
+    pool = torch.cuda.graph_pool_handle()
+    graphs, outs = [], []
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, pool=pool):
+            # freed at once: the memory of the allocations that follow, large ones and those of up to a MiB
+            ones = [torch.empty(n, dtype=torch.uint8, device=dev).fill_(255) for n in (48 << 20, 1 << 20, 1 << 20)]
+            del ones
+            outs.append(run(static_a))
+        graphs.append(graph)
+    for rep in range(4):
+        a = torch.randn(M, K, generator=g).to(E4).to(dev)
+        static_a.copy_(a)
+        want = run(a)
+        for graph, out in zip(graphs, outs):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), rep
+        assert torch.equal(run(a), want)
+
+
 def attention_like(q8, k8, sq, sk):
     """scores = q k^T in fp8, probabilities through softmax_fp8, their row sums through sum_fp8 (split: workspace)."""
     scores = ops.fp8_gemm_v2(q8, False, k8, True, None, torch.bfloat16, sq, sk, None, False)
