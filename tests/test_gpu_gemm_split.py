@@ -100,6 +100,49 @@ def test_one_workspace_serves_several_shapes(pkg, dev):
         assert int(ws[: 64 * 1024].count_nonzero()) == 0
 
 
+# per kernel that splits K: rows, K off the stages' 128, N off 16
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,name", [(1, 4112, 1000, b"split_stream"), (16, 4112, 16378, b"split_stream"), (40, 4112, 1000, b"split_strip"),
+                                        (128, 14352, 250, b"split_strip"), (300, 8208, 1000, b"split_tile128"), (2000, 14352, 1000, b"split_tile256")])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_what_lies_beside_the_operands_stays_out(pkg, dev, M, K, N, name, ta, tb):
+    """Operands in wider rows with NaN codes behind every row, and a row of NaN behind the last: exact results all the same.
+    Then an infinity and a NaN in the last k and the last column: they reach their own rows and columns and no others."""
+    lib = pkg.capi()
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator().manual_seed(M + N)
+    a, b = torch.randint(-2, 3, (M, K), generator=g).float(), torch.randint(-2, 3, (K, N), generator=g).float()
+
+    def beside(x):  # (rows rounded up to 16 for a transposed one, which is read in chunks of 16 along m or n)
+        rows, cols = x.shape
+        wide = torch.full((rows + 1, (cols + 15) // 16 * 16 + 32), float("nan"))
+        wide[:rows, :cols] = x
+        return wide
+
+    def product(a, b):
+        aw, bw = beside(a.t() if ta else a).to(E5).to(dev), beside(b.t() if tb else b).to(E5).to(dev)
+        lda, ldb = aw.shape[1], bw.shape[1]
+        variant = lib.mi355q_fp8_gemm_ws_variant(ta, lda, tb, ldb, M, N, K, 1)
+        assert variant.startswith(name) or (M <= 16 and (ta or tb) and b"strip_" in variant), variant
+        need = lib.mi355q_fp8_gemm_workspace_bytes(ta, lda, tb, ldb, M, N, K, 1)
+        ws = torch.full((need,), 255, dtype=torch.uint8, device=dev)  # NaN where the sums will lie
+        ws[: 64 * 1024] = 0
+        c = torch.full((M + 1, N), 7.0, device=dev)
+        assert lib.mi355q_fp8_gemm_ws(aw.data_ptr(), pkg.E5M2, ta, lda, bw.data_ptr(), pkg.E5M2, tb, ldb, c.data_ptr(), pkg.F32, N, M, N, K, None, 1.0,
+                                      pkg.GS_NONE, None, 1.0, pkg.GS_NONE, None, pkg.BIAS_NONE, 0, None, 0, 1, 0, 0, 0, 0, 0, ws.data_ptr(), need, st) == 0
+        assert bool((c[M] == 7.0).all())
+        return c[:M].cpu()
+
+    assert torch.equal(product(a, b), a @ b)
+    a[:, K - 1], b[K - 1, :] = 1.0, 1.0
+    want = a @ b
+    a[M - 1, K - 1] = float("inf")
+    b[K - 1, N - 1] = float("nan")
+    got = product(a, b)
+    assert bool(got[:, N - 1].isnan().all()) and bool((got[M - 1, : N - 1] == float("inf")).all())
+    assert torch.equal(got[: M - 1, : N - 1], want[: M - 1, : N - 1])
+
+
 def test_short_products_stay_whole(pkg):
     """K below which a product was slower in parts than whole, and longer ones that stay in parts; without a workspace none is."""
     need = pkg.capi().mi355q_fp8_gemm_workspace_bytes
@@ -129,8 +172,12 @@ def test_few_rows_of_an_mn_major_a_stay_whole_longer(pkg):
 def test_parts_of_k_meet_by_device_scope_accesses_in_order():
     """Sums stored (sc1), acknowledged, barrier, ticket, barrier, counter reset, sums read (sc1); nothing cache-wide."""
     import re
-    for src, least in (("gemm_stream.hip", 4), ("gemm_inst_kk.hip", 12)):
-        text = isa_check.compile_to_isa(src)
+    from concurrent.futures import ThreadPoolExecutor
+    # the strip kernel has three heights with an A [M, K] and one with an A [K, M], the tiles two sizes, four pairs of formats
+    sources = (("gemm_stream.hip", 4), ("gemm_inst_kk.hip", 20), ("gemm_inst_km.hip", 20), ("gemm_inst_mk.hip", 12), ("gemm_inst_mm.hip", 12))
+    with ThreadPoolExecutor(max_workers=4) as ex:
+        texts = list(ex.map(isa_check.compile_to_isa, [src for src, _ in sources]))
+    for (src, least), text in zip(sources, texts):
         orders = isa_check.exchange_order(text)
         assert len(orders) >= least and isa_check.scratch_bytes(text) == {}, src
         for name, seq in orders.items():

@@ -36,9 +36,9 @@ def test_silu_bits_on_every_bf16_value(oracle, pkg, dev):
 
 
 @pytest.mark.parametrize("cols", [2048, 8192])
-def test_table_kernel_on_every_bf16_value(oracle, pkg, dev, cols):
-    """Large calls (once a kernel of their own with a table of bf16(silu(gate)) in LDS): every one of the 65536 gate values, in every lane position, against the oracle (h_out, codes and
-    scales); rows of zeros and a ragged last workgroup share included."""
+def test_many_rows_of_every_bf16_value(oracle, pkg, dev, cols):
+    """Large calls: every one of the 65536 gate values, in every lane position, against the oracle (h_out, codes and scales);
+    rows of zeros included."""
     lib = pkg.capi()
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     rows = 2048 + 7
