@@ -121,11 +121,13 @@ int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
  *   then mi355q_quantize_rows of h (amax_r, scale_r = target / amax_r, cast,
  *   scale_out / scale_inv_out); h_out, when not NULL, receives h [rows, cols].
  * Between the reference's ops this step is left to aten (silu and mul on the
- * device, then cast_to_fp8_v2): there is no reference operator to cite.  The
- * exp is a fixed sequence of IEEE operations that the CPU oracle repeats
- * (ora_silu_mul_bf16), so results are bit-identical to it; against a correctly
- * rounded silu the bf16 value differs for 18 of the 65536 inputs, all below
- * -88, where the result (magnitude < 3.3e-37) is returned as -0.
+ * device, then cast_to_fp8_v2): there is no reference operator to cite.  silu
+ * is computed with the hardware's exp2 and reciprocal, accurately enough that
+ * its bf16 value is, for each of the 65536 inputs, the one of the CPU oracle's
+ * fixed sequence of IEEE operations (ora_silu_mul_bf16), so results are
+ * bit-identical to it; against a correctly rounded silu that value differs for
+ * 18 inputs, all below -88, where the result (magnitude < 3.3e-37) is returned
+ * as -0.
  * gate, up 16-byte aligned, cols and pitches multiples of 8, rows of up to 2048
  * 16-byte vectors; otherwise MI355Q_ERR_UNSUPPORTED.
  */
@@ -270,7 +272,10 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda,
  * place for every shape; the rest need not be cleared):
  * zero-filled once before its first use, left zero by every call; calls that
  * may overlap in time need workspaces of their own.  NULL: the same result
- * (sums in another order) without the split.
+ * (sums in another order) without the split.  With either entry the order of
+ * the fp32 sums depends on M, N, K, the batch and the layouts, so a row's last
+ * bits can differ between calls with different numbers of rows; one call gives
+ * the same bits on every run.
  */
 #define MI355Q_FP8_GEMM_COUNTER_BYTES 65536
 size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb,
