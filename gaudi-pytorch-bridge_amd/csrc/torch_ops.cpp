@@ -394,12 +394,13 @@ void cast_to_fp8_v2_boxed(const c10::OperatorHandle& op, c10::DispatchKeySet, to
       cs = resolve_cast_scale(scale, scale_shape, x);
     }
     if (chained) {
-      Tensor next = at::empty({}, words);
+      // (the memory alone, by the allocator that gave `out` its own: at::empty's way through the dispatcher is 0.5 us of the call)
+      c10::Storage next(c10::Storage::use_byte_size_t(), sizeof(float), out.storage().allocator(), /*resizable=*/true);
       check_status(mi355q_cast_to_fp8_amax_chain(x.data_ptr(), to_mi355q_dtype(x.scalar_type()), out.data_ptr(), to_mi355q_dtype(dst), cs.dev,
                                                  cs.host, cs.mode, cs.outer, cs.mid, cs.inner, amax.data_ptr<float>(), zeroed ? 1 : 0,
-                                                 next.data_ptr<float>(), current_stream(x)),
+                                                 static_cast<float*>(next.mutable_data()), current_stream(x)),
                    "mi355q_cast_to_fp8");
-      put_zero_word(x, next.storage());
+      put_zero_word(x, std::move(next));
     } else {
       check_status(launch_cast_to(x, out, cs, is_amax ? amax.data_ptr<float>() : nullptr, sr), "mi355q_cast_to_fp8");
     }

@@ -105,6 +105,7 @@ def test_amax_is_an_ordinary_tensor(dev):
         first, second = call(), call()
         assert inside.is_inference() and not first.is_inference()
         assert first.untyped_storage().nbytes() == 4 and first.storage_offset() == 0 and first._base is None
+        assert first.untyped_storage().device == x.device == first.device and first.untyped_storage().resizable()
         version = second._version
         first.mul_(2)  # refused for an inference tensor
         assert second._version == version
