@@ -24,6 +24,7 @@ lost 12 % that way, the cast with amax 23 %).  ``memory_order(text)`` lists, per
 order of loads (L), stores (S), full waits (W) and counted waits (w), so that a test can
 require the loads of a kernel to be issued back to back.
 """
+import functools
 import os
 import re
 import subprocess
@@ -192,8 +193,9 @@ def memory_order(text):
     return out
 
 
+@functools.lru_cache(maxsize=None)
 def compile_to_isa(source, extra_flags=()):
-    """Device-only assembly of one HIP source of csrc/ with the build's flags."""
+    """Device-only assembly of one HIP source of csrc/ with the build's flags (a source once per process: half a minute each)."""
     import importlib.util  # noqa: PLC0415
     spec = importlib.util.spec_from_file_location("_mi355q_build_flags", os.path.join(os.path.dirname(HERE), "gaudi-pytorch-bridge_amd", "build.py"))
     build = importlib.util.module_from_spec(spec)
