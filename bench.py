@@ -549,7 +549,7 @@ def bench_gemm_decode(ops, oracle, pkg, dev, steps, warmup):
                 lib_ms = None
         out.append(hbm_entry(f"fp8_gemm_v2_decode_M{M}",
                              f"C4 fp8_gemm_v2 M={M} K=8192 N=28672 per-token x per-channel scales -> bf16",
-                             nbytes, ms, steps, "fp8_gemm_stream_kernel" if M <= 16 else "fp8_gemm_skinny_kernel" if M <= 128 else "fp8_gemm_tile_kernel<256,128>",
+                             nbytes, ms, steps, "fp8_gemm_stream_kernel" if M <= 16 else "fp8_gemm_ring_kernel",
                              extra={"kernel_variant": pkg.capi().mi355q_fp8_gemm_ws_variant(0, K, 0, N, M, N, K, 1).decode(),
                                     "tflops": round(flop / (ms * 1e-3) / 1e12, 2), "library_gemm_ms_same_shape": lib_ms}))
     return out

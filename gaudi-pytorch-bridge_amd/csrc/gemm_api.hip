@@ -1,6 +1,7 @@
 // fp8_gemm_v2 C entry point: argument checks, kernel choice, and the any-shape
 // fallback kernel.  The MFMA tile kernels live in gemm_tile.h.
 #include <algorithm>
+#include <cmath>
 
 #include "gemm_dispatch.h"
 
@@ -73,109 +74,104 @@ inline bool tiled_ok(const void* A, int trans_a, int64_t lda, const void* B, int
   return M > 0 && N > 0 && K > 0;
 }
 
-// More than 128 rows: the tiles of gemm_tile_split.h, one workgroup per compute unit at most, where they are expected to beat
-// the uncut launch.  The estimates (us; `fill` is the share of the compute units that have a workgroup) are least-squares fits
-// to 590 products of 130 to 4000 rows, K from 1536 to 14336 and N from 64 to 8192, whole and in 2 to 16 parts, each timed with
-// the weights hot in the caches and cold and counted half and half, since a cut hides the cold weights' latency but costs the
-// same meeting when they are hot: 500 x 3072 x 2048 takes 13.2 / 23.8 whole, 14.8 / 18.4 in two parts, 20.9 / 21.1 in four.
-// Most are within 10 %.  The meeting costs more the fuller the chip is.  Beyond 16 parts nothing was faster.
-SplitPlan tile_split_plan(int64_t M, int64_t N, int64_t K, int64_t batch) {
-  SplitPlan best;
-  const int64_t cus = compute_units(), pairs = (K + 2 * kBK - 1) / (2 * kBK);
-  const TileChoice whole = N > 128 ? choose_tiles(M, N, K, batch) : TileChoice::k128x128;
-  if (whole == TileChoice::k256x256 && ((M + 255) / 256) * ((N + 255) / 256) * batch >= cus) return best;
-  auto tiles_of = [&](int64_t bm) { return ((M + bm - 1) / bm) * ((N + 127) / 128) * batch; };
-  const double all_stages = (double)((K + kBK - 1) / kBK);
-  double best_us = 0.85 * tile_us(whole, M, N, K, batch);
-  if (whole == TileChoice::k128x128) best_us = all_stages * (0.52 + 0.29 * (double)tiles_of(128) / (double)cus) + 2.7;
-  if (whole == TileChoice::k256x128) best_us = all_stages * 0.83 + 2.7 + (all_stages * 0.07 + 3.9) * (double)tiles_of(256) / (double)cus;
-  for (const int64_t bm : {128, 256}) {
-    const int64_t tiles = tiles_of(bm);
-    for (int64_t parts = 2; parts <= 16 && parts <= pairs && parts * tiles <= cus; ++parts) {
-      const double stages = 2.0 * (double)((pairs + parts - 1) / parts), levels = std::log2((double)parts);
-      const double fill = (double)(parts * tiles) / (double)cus;
-      const double us = bm == 128 ? stages * (0.51 + 0.13 * fill) + levels * (3.0 - 0.84 * fill) + 7.3 * fill + 2.9
-                                  : stages * (0.72 + 0.07 * fill) + levels * (5.8 - 0.82 * fill) + 9.1 * fill + 4.3;
-      if (us >= best_us) continue;
-      best_us = us;
-      best.tile = bm == 128 ? SplitTile::k128x128 : SplitTile::k256x128;
-      best.nb = 128;
-      best.strips = (int)(tiles / batch);
-      best.parts = (int)parts;
-      best.tile_rows = bm;
-      best.batch = batch;
-    }
-  }
-  return best;
-}
+// What a launch takes on the ring kernel, in microseconds.
+//  fixed          prologue, first loads, epilogue;
+//  stage, busy    a stage of 128 k alone on the chip, and what comes on top where every compute unit has a workgroup;
+//  round          the share of a stage that each further round of workgroups adds;
+//  meet, level, crowd   the parts' meeting: fixed, per doubling of the parts, and on a full chip.
+struct RingCost {
+  GemmKind kind;
+  int rows;
+  double fixed, stage, busy, meet, level, crowd, round;
+};
+// Least-squares fits to 480 products (1 to 4096 rows, K from 512 to 16384, N from 256 to 28672, both layouts of B, whole and
+// in 2 to 24 parts), each timed with the weights hot in the caches and cold and counted half and half.  The choice they make is
+// 1.8 % slower in the mean than the best one measured.  The line of the 256-row tile is lowered by a tenth, which costs nothing
+// over the sample and halves the reads of B where it decides.
+constexpr RingCost kRingCosts[] = {
+    {GemmKind::kRing16, 16, 2.84, 0.28, 0.44, 0.75, 0.83, 0.41, 1.10},
+    {GemmKind::kRing32, 32, 3.18, 0.29, 0.26, 0.61, 1.29, 1.25, 1.34},
+    {GemmKind::kRing64, 64, 3.99, 0.33, 0.16, -0.88, 2.86, 3.00, 1.35},
+    {GemmKind::kRing128, 128, 4.99, 0.37, 0.22, -0.85, 3.75, 4.13, 1.22},
+    {GemmKind::kRing256, 256, 6.59, 0.50, 0.19, -1.43, 5.03, 8.08, 1.19},
+};
 
-// The cut that is expected to take least.  More than 128 rows: tile_split_plan.  For fewer the figures (microseconds, bytes
-// per microsecond) are fits to 60 problems of 1 to 128 rows, K from 2048 to 14336 and N from 1024 to 38400, most of which
-// they meet within two microseconds:
-//  * a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where more of them run;
-//  * in the strip kernel A's tile travels along (a quarter of its bytes count with a K-major B, half with the shorter
-//    pieces of an MN-major one);
-//  * fixed costs, and with more than one part the meeting: each part's sums out, and all of them into the last one.
-// Short products stay whole where the meeting costs them more than the parts save.  Whole and in parts, us a launch,
-// weights hot in the caches / cold:
-//  * the strip kernel below K = 1792: 1 x 1280 x 512, B [N, K], 8.9 / 8.9 and 9.5 / 9.4; 8 x 1536 x 512 8.2 / 9.3 and 8.8 / 9.0
-//    (2048: 8 x 2048 x 512 9.5 / 10.7 and 9.1 / 9.5);
-//  * the stream kernel below K = 2048, against the strip kernel whole: 1 x 1024 x 2048 6.8 / 8.5 and 10.3 / 10.1;
-//  * no part of the stream kernel shorter than 512, two turns of its eight waves, since in a part of 256 a wave's first
-//    loads have none behind them: 8 x 2048 x 4096 in eight of those 12.1 / 12.0, in four parts on the strip kernel 10.0 / 10.2.
+// The kernel and the cut that are expected to take least.
+//  * Tiles of fewer than 128 rows exist for A [M, K]; up to 16 rows take the tile of 16, more of them none that is twice as high
+//    as the product.
+//  * At most one workgroup per compute unit where K is cut, parts of two stages at least, at most 16 of them.  Up to 128 rows
+//    short products stay whole: below K = 1792 a cut of few strips gains a microsecond at most (1 x 1600 x 1024: 7.3 whole, 6.3
+//    in four parts) and a cut of many loses as much; an A [K, M], whose tiles of 128 rows send all their sums, from 2304 on.
+//  * 256 x 256 tiles take 1.42 us a stage in every pass over the compute units.
+//  * Up to 16 rows against B [K, N] of more than 96 MiB: the stream kernel, whose 256-byte pieces of B come in at 5.5 TB/s
+//    against 5.0 for the ring's 128 (16 x 8192 x 28672: 43.4 / 46.4 us; 16 x 8192 x 14336, 112 MiB, 26.4 / 26.3; 13 x 14144 x
+//    5248, 71 MiB, 23.2 / 16.8).  Its cut: a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where
+//    more of them run; no part shorter than 512, two turns of its eight waves.
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
   SplitPlan best;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
-  if (M > 128) return may_split ? tile_split_plan(M, N, K, batch) : best;
-  const double cus = (double)compute_units();
-  double best_us = 0.0;
-  auto consider = [&](bool stream, int64_t nb, int64_t tile_rows, int64_t unit) {
-    const int64_t shortest = stream ? 512 : unit;  // part
-    const bool in_parts = may_split && K >= (stream ? 2048 : 1792);
-    const int64_t strips = (N + nb - 1) / nb, groups = strips * batch, units = (K + unit - 1) / unit;
-    const int64_t rows = M < 32 && tile_rows <= 32 ? M : tile_rows;  // rows of sums that travel (those of one row tile alone can be left out)
-    const double width = (double)nb + (stream ? 0.0 : (double)tile_rows * (b_kmajor ? 0.25 : 0.5));
-    for (int64_t parts = 1; parts <= 32 && parts <= units; ++parts) {
-      if (parts > 1 && (!in_parts || groups > kMaxTickets || (double)(groups * parts) > 2.0 * cus)) break;
-      if (parts > 1 && (units + parts - 1) / parts * unit < shortest) break;
-      const double wgs = (double)(groups * parts), rounds = std::ceil(wgs / cus);
-      const double rate = std::min(37e3, 6.5e6 / std::min(wgs, cus));
-      double us = rounds * (double)((units + parts - 1) / parts * unit) * width / rate + 4.5;
-      if (parts > 1)
-        us += stream ? 0.5 + 0.2 * (double)parts + (double)rows * (0.15 + 0.005 * (double)parts)
-                     : 2.0 + 0.25 * (double)parts + ((double)parts + 1.5) * (double)(rows * nb * 4) / 50e3;
-      if (best.nb != 0 && us >= best_us) continue;
-      best_us = us;
-      best.stream = stream;
-      best.nb = (int)nb;
-      best.strips = (int)strips;
-      best.parts = (int)parts;
-      best.tile_rows = tile_rows;
-      best.batch = batch;
-    }
-  };
+  const int64_t cus = compute_units(), stages = (K + kBK - 1) / kBK;
+  best.batch = batch;
   // (the stream kernel addresses an operand with 31-bit offsets)
-  if (a_kmajor && !b_kmajor && M <= 16 && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) consider(true, 256, 16, 256);
-  consider(false, 128, !a_kmajor ? 128 : (M <= 32 ? 32 : (M <= 64 ? 64 : 128)), kBK);
+  if (a_kmajor && !b_kmajor && M <= 16 && N * K > (96LL << 20) && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) {
+    best.kind = GemmKind::kStream;
+    best.nb = 256;
+    best.strips = (int)((N + 255) / 256);
+    best.tile_rows = 16;
+    const int64_t units = (K + 255) / 256, groups = best.strips * batch;
+    double best_us = 0.0;
+    for (int64_t parts = 1; parts <= 32 && (parts == 1 || (may_split && groups <= kMaxTickets && groups * parts <= 2 * cus && units / parts >= 2)); ++parts) {
+      const double wgs = (double)(groups * parts), rate = std::min(37e3, 6.5e6 / std::min(wgs, (double)cus));
+      double us = std::ceil(wgs / (double)cus) * (double)((units + parts - 1) / parts * 256) * 256.0 / rate;
+      if (parts > 1) us += 0.5 + 0.2 * (double)parts + (double)M * (0.15 + 0.005 * (double)parts);
+      if (parts > 1 && us >= best_us) continue;
+      best_us = us;
+      best.parts = (int)parts;
+    }
+    return best;
+  }
+  double best_us = 1e30;
+  if (M > 128 && N > 128) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256) * batch;
+    best_us = (double)((tiles + cus - 1) / cus) * (double)stages * 1.42 + 6.0;
+  }
+  for (const RingCost& c : kRingCosts) {
+    if (a_kmajor ? (c.rows == 16) != (M <= 16) || (c.rows > 32 && c.rows >= 2 * M) : c.rows < 128) continue;
+    const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + kRingBN - 1) / kRingBN);
+    const bool in_parts = may_split && (M > 128 || K >= (a_kmajor ? 1792 : 2304));
+    for (int64_t parts = 1; parts == 1 || (in_parts && parts <= 16 && parts * tiles * batch <= cus && 2 * parts <= stages); ++parts) {
+      const int64_t wgs = parts * tiles * batch, rounds = (wgs + cus - 1) / cus;
+      const double fill = (double)std::min(wgs, cus) / (double)cus;
+      double us = c.fixed + (double)((stages + parts - 1) / parts) * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round);
+      if (parts > 1) us += c.meet + c.level * std::log2((double)parts) + c.crowd * fill;
+      if (us >= best_us) continue;
+      best_us = us;
+      best.kind = c.kind;
+      best.nb = kRingBN;
+      best.strips = (int)tiles;
+      best.parts = (int)parts;
+      best.tile_rows = c.rows;
+    }
+  }
   return best;
 }
 
-// What launch_by_size and launch_gemm_stream run; may_split: the caller brings the workspace.
+// What launch_by_kind and launch_gemm_stream run; may_split: the caller brings the workspace.  A tile's extents (rows, columns,
+// bytes of K per stage) stand in falling order.
 const char* variant_name(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
   if (lda % 16 || ldb % 16 || lda > (1LL << 22) || ldb > (1LL << 22) || !k_chunks_ok(trans_a, trans_b, K)) return "simple";
   const SplitPlan p = split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, may_split);
-  if (M <= 128) {
-    if (p.stream) return p.parts > 1 ? "split_stream_Mx256_registers_mfma16x16" : "stream_Mx256_registers_mfma16x16";
-    return p.parts > 1 ? "split_strip_Mx128x128_ring_mfma32x32x64" : "strip_Mx128x128_ring_mfma32x32x64";
+  const bool cut = p.parts > 1;
+  if (p.kind == GemmKind::kStream) return cut ? "split_stream_Mx256_registers_mfma16x16" : "stream_Mx256_registers_mfma16x16";
+  if (p.kind == GemmKind::kRing16 && !trans_b && cut) return "split_stream_Mx128x128_ring_mfma16x16x128";
+  if (M <= 128) return cut ? "split_strip_Mx128x128_ring_mfma16x16x128" : "strip_Mx128x128_ring_mfma16x16x128";
+  switch (p.kind) {
+    case GemmKind::kRing32: return cut ? "split_tile128x128x32_ring_mfma16x16x128" : "tile128x128x32_ring_mfma16x16x128";
+    case GemmKind::kRing64: return cut ? "split_tile128x128x64_ring_mfma16x16x128" : "tile128x128x64_ring_mfma16x16x128";
+    case GemmKind::kRing128: return cut ? "split_tile128x128x128_ring_mfma16x16x128" : "tile128x128x128_ring_mfma16x16x128";
+    case GemmKind::kRing256: return cut ? "split_tile256x128x128_ring_mfma16x16x128" : "tile256x128x128_ring_mfma16x16x128";
+    default: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
   }
-  if (p.tile == SplitTile::k128x128) return "split_tile128x128x128_mfma32x32x64";
-  if (p.tile == SplitTile::k256x128) return "split_tile256x128x128_mfma32x32x64";
-  switch (N > 128 ? choose_tiles(M, N, K, batch) : TileChoice::k128x128) {
-    case TileChoice::k256x256: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
-    case TileChoice::k256x128: return "tile256x128x128_mfma32x32x64";
-    case TileChoice::k128x128: break;
-  }
-  return "tile128x128x128_mfma32x32x64";
 }
 
 }  // namespace mi355q
@@ -282,9 +278,9 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const
         if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;
         split.tickets = static_cast<uint32_t*>(workspace);
         split.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
-        split.tile = plan.tile;
       }
-      if (plan.stream) launch_gemm_stream(gb, fmt_a, fmt_b, plan, split, nb, st);
+      split.kind = plan.kind;
+      if (plan.kind == GemmKind::kStream) launch_gemm_stream(gb, fmt_a, fmt_b, plan, split, nb, st);
       else if (ak && bk) launch_gemm_kk(gb, split, fmt_a, fmt_b, nb, st);
       else if (ak) launch_gemm_km(gb, split, fmt_a, fmt_b, nb, st);
       else if (bk) launch_gemm_mk(gb, split, fmt_a, fmt_b, nb, st);

@@ -1,0 +1,484 @@
+// fp8 GEMM on tiles of 16 to 256 rows and 128 columns, for every product that does not fill the chip with 256 x 256 tiles:
+// one tile per workgroup, a ring of LDS stages of 128 k, v_mfma_f32_16x16x128_f8f6f4, K whole or in parts over workgroups.
+//
+// What bounds it.  A compute unit keeps about 32 KB of lines on their way, whatever asks for them (a loop that only loads, into
+// LDS or registers, 4 to 16 waves: 48 to 55 KB/us from HBM at 0.63 us a load, 150 to 200 KB/us from the XCD's L2): its intake is
+// what a stage costs, (rows + 128) x 128 bytes, and a wave that issues loads beyond that limit stalls.  Hence
+//  * four waves that only load and four that only multiply, one of each per SIMD, meeting at one barrier per stage: the
+//    loading waves' stalls hold up no MFMA, and the multiplying waves' loop is MFMAs, fragment reads and one addition per
+//    address register;
+//  * as many stages as the LDS holds (3 at 256 rows, 4, 6, 7, 7 below), counted waits, and load addresses without arithmetic;
+//  * low tiles where they fill the chip better, and K in parts only then (gemm_api.hip has the figures that choose);
+//  * plain loads for a B of at most 64 MiB: the nontemporal hint keeps a matrix out of the 256 MB memory-side cache, from
+//    which a second call would read it (64 x 8192 x 4096 warm: 40 us with the hint, 23 without; cold 0 to 10 % for it).
+// Measured against the strip, 128 x 128 and 256 x 128 kernels it replaces (us, weights [K, N] but where nk, three sets of them in
+// turn): 256 x 8192 x 28672 88.8 -> 68.3 (nk 93.3 -> 66.5; the load stream alone takes 64), 1000 x 3008 x 5000 29.3 -> 24.3, 669 x 8704 x
+// 7808 nk 54.8 -> 44.7, 64 x 14336 x 4096 25.0 -> 17.5, 83 x 6640 x 864 23.9 -> 11.0, 7 x 10816 x 704 nk 16.1 -> 9.7, 1 x 4096 x 4096
+// 12.2 -> 7.8; over 480 products of 1 to 4096 rows 26 % less time in the geometric mean warm, 23 % cold.
+#pragma once
+#include "gemm_split.h"
+#include "gemm_tile16.h"
+
+namespace mi355q {
+
+constexpr int kRingBN = 128;
+constexpr int kRingWaves = 4;                      // that multiply, and as many that load
+constexpr int kRingThreads = 2 * kRingWaves * 64;
+
+// Global -> LDS loader of a wave's share of one operand's stages (consecutive 1 KiB regions).  What a lane fetches does not
+// change from stage to stage, so its offsets are worked out once, with everything in them that the other loaders leave to
+// the descriptor or test per load: tile rows past the matrix read its last row (their products are never stored, and a
+// load that goes to memory retires in issue order, which the counted waits need), columns past it and, in a ragged last
+// stage, k past K read as zero through an offset that no descriptor covers.  A step along K is one 64-bit scalar addition,
+// whatever the operand's size.
+template <bool KMAJOR, int EXT>
+struct RingLoader {
+  using G = TileGeom<KMAJOR, KMAJOR ? EXT : kBK, KMAJOR ? kBK : EXT, 1>;
+  static constexpr int kCPR = G::kChunksPerRow, kRowsPerRegion = 64 / kCPR;
+  static constexpr int kPerWave = G::kChunks / 64 / kRingWaves;
+  static_assert(kPerWave * kRingWaves * 64 == G::kChunks, "tile does not split over the waves");
+  static constexpr int kNowhere = 0x7fffffff;
+  uint64_t base;  // the next stage to load
+  int64_t step;
+  int at[kPerWave], limit[kPerWave];  // a lane's offsets in a stage, lowered by issue()'s immediate, and their k in it
+  int cur[kPerWave];                  // those of the next stage's loads
+  int wave;
+
+  // p: the operand at the tile's first row (column) and the workgroup's first k; valid: rows (columns) from there to the edge
+  __device__ __forceinline__ void init(const uint8_t* p, int64_t ld, int valid, int wave_) {
+    wave = wave_;
+    const uint64_t b = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+    base = ((uint64_t)hi << 32) | lo;
+    step = KMAJOR ? kBK : (int64_t)kBK * ld;
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int row = (wave * kPerWave + i) * kRowsPerRegion + lane / kCPR;
+      const int c16 = ((lane % kCPR) ^ G::swizzle(row)) * 16;
+      int v;
+      if constexpr (KMAJOR) v = (row < valid ? row : valid - 1) * (int)ld + c16;
+      else v = c16 < ((valid + 15) & ~15) ? row * (int)ld + c16 : kNowhere;  // (the chunk that straddles the edge lies in the row's padding)
+      at[i] = v - (i & 3) * 1024;
+      limit[i] = KMAJOR ? c16 : row;
+      cur[i] = at[i];
+    }
+  }
+  // The next stage's loads read zeros from its k `valid_k` on (kBK: all of it is inside K).
+  __device__ __forceinline__ void select(int valid_k) {
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) cur[i] = limit[i] < valid_k ? at[i] : kNowhere - (i & 3) * 1024;
+  }
+  // Load I of the next stage into the operand's tile at LDS address `tile`.  Four loads in a row share a write of m0 (see
+  // DmaLoader::issue_one); NT: the operand is read once.
+  template <int I, bool NT>
+  __device__ __forceinline__ void issue(uint32_t tile) const {
+    constexpr int r = I & 3;
+    const i32x4 rsrc = {(int)(uint32_t)base, (int)((uint32_t)(base >> 32) & 0xffffu), 0x7ffffff0, 0x00020000};
+    if constexpr (r == 0) {
+      const uint32_t dst = tile + (uint32_t)((wave * kPerWave + I) * 1024);
+      if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" : : "s"(dst), "v"(cur[I]), "s"(rsrc) : "memory", "m0");
+      else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(dst), "v"(cur[I]), "s"(rsrc) : "memory", "m0");
+    } else {
+      if constexpr (NT) asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 nt lds" : : "v"(cur[I]), "s"(rsrc), "n"(r * 1024) : "memory");
+      else asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(cur[I]), "s"(rsrc), "n"(r * 1024) : "memory");
+    }
+  }
+};
+
+// Fragment reads of FragReader16 from a ring position that is not a compile-time constant: one addition per address
+// register and stage.
+template <bool KMAJOR, int EXT, int TILES>
+struct RingReader : FragReader16<KMAJOR, EXT, TILES> {
+  using Base = FragReader16<KMAJOR, EXT, TILES>;
+  __device__ __forceinline__ void move(int bytes) {
+#pragma unroll
+    for (int i = 0; i < Base::kRegs; ++i) this->addr[i] += (uint32_t)bytes;
+  }
+};
+
+// A wave's scales and bias (ScaleStager's layout), then room for its rows: 16 MT x 16 NT results leave through LDS.
+constexpr int kRingScaleBytes = kStagedBytes;
+
+// The fast bf16 epilogue (see epilogue_fast_ok) for wave tiles of 16 MT x 16 NT: epilogue16_bf16_fast with rows of 32 NT bytes.
+// Write cycles (16 rows, two neighbouring 8-byte slots) and read cycles (whole rows, 16-byte chunks) touch distinct banks.
+template <int MT, int NT, bool PER_COL, bool HAS_BIAS>
+__device__ __forceinline__ void ring_epilogue_fast(const GemmArgs& g, int64_t batch, f32x4 (&acc)[MT][NT], int m_wave, int n_wave,
+                                                   const uint8_t* staged_p, uint8_t* rows_p, ScalarScales scalars) {
+  static_assert(NT == 2 || NT == 4, "64- or 128-byte rows");
+  constexpr int kRow = 32 * NT, kShift = NT == 4 ? 1 : 2, kMask = 2 * NT - 1;
+  constexpr int kLanesPerRow = 2 * NT, kRowsPerPass = 64 / kLanesPerRow, kPasses = 16 / kRowsPerPass;
+  LDS_AS const uint8_t* staged = (LDS_AS const uint8_t*)staged_p;
+  LDS_AS uint8_t* out = (LDS_AS uint8_t*)rows_p;
+  const int lane = threadIdx.x & 63, r = lane & 15, gq = lane >> 4;
+  float cs[PER_COL ? NT : 1][4], cb[HAS_BIAS ? NT : 1][4];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int col = 16 * j + 4 * gq;
+    if constexpr (PER_COL) {
+      const f32x4 v = *reinterpret_cast<LDS_AS const f32x4*>(staged + kStagedColScale + col * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) cs[j][e] = v[e];
+    }
+    if constexpr (HAS_BIAS) {
+      const u32x2 v = *reinterpret_cast<LDS_AS const u32x2*>(staged + kStagedBias + col * 2);
+      cb[j][0] = __uint_as_float(v[0] << 16);
+      cb[j][1] = __uint_as_float(v[0] & 0xffff0000u);
+      cb[j][2] = __uint_as_float(v[1] << 16);
+      cb[j][3] = __uint_as_float(v[1] & 0xffff0000u);
+    }
+  }
+  const int rows = g.M - m_wave < 16 * MT ? g.M - m_wave : 16 * MT;
+  uint16_t* cbase = reinterpret_cast<uint16_t*>(g.C) + batch * g.stride_c + (int64_t)m_wave * g.ldc;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(cbase, 0, rows > 0 ? rows * (int)g.ldc * 2 : 0, 0x00020000);
+  const int row_in_pass = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
+  const int n_out = n_wave + 8 * chunk, pitch = (int)g.ldc * 2;
+  const int voff0 = n_out < g.N ? row_in_pass * pitch + n_out * 2 : 0x7fffffff;
+  const int pass_step = n_out < g.N ? kRowsPerPass * pitch : 0;
+  static_for<MT>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const float staged_ra = *reinterpret_cast<LDS_AS const float*>(staged + kStagedRowScale + (16 * i + r) * 4);
+    float ra = g.sa_mode == MI355Q_GS_PER_ROW ? staged_ra : scalars.sa;
+    if (!PER_COL) ra *= scalars.sb;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float b = HAS_BIAS ? cb[j][e] : 0.0f;
+        if constexpr (PER_COL) v[e] = __builtin_fmaf(acc[i][j][e] * ra, cs[j][e], b);
+        else v[e] = __builtin_fmaf(acc[i][j][e], ra, b);
+      }
+      const int slot = (4 * j + gq) ^ (2 * ((r >> kShift) & kMask));
+      *reinterpret_cast<LDS_AS u32x2*>(out + i * 16 * kRow + r * kRow + slot * 8) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+  });
+  // (a wave reads only what it wrote itself, and its LDS instructions execute in order)
+  static_for<MT>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int row = p * kRowsPerPass + row_in_pass;
+      const u32x4 o = *reinterpret_cast<LDS_AS const u32x4*>(out + i * 16 * kRow + row * kRow + ((chunk ^ ((row >> kShift) & kMask)) << 4));
+      __builtin_amdgcn_raw_buffer_store_b128(o, rsrc, voff0 + (i * kPasses + p) * pass_step, 0, 2);  // aux 2: nontemporal
+    }
+  });
+}
+
+// Every other form (fp32 output, accumulate input, full bias, scales per column of A or row of B, rows of C at any
+// alignment): the wave's sums go to LDS as they are, then a rolled loop takes four columns of a row per lane.
+template <int MT, int NT>
+__device__ __forceinline__ void ring_epilogue_any(const GemmArgs& g, int64_t batch, f32x4 (&acc)[MT][NT], int m_wave, int n_wave,
+                                                  float* rows, ScalarScales scalars) {
+  constexpr int kPitch = 16 * NT + 4, kLanesPerRow = 4 * NT, kRowsPerPass = 64 / kLanesPerRow;
+  const int lane = threadIdx.x & 63, r = lane & 15, gq = lane >> 4;
+  static_for<MT>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4*>(rows + (16 * i + r) * kPitch + 16 * j + 4 * gq) = acc[i][j];
+  });
+  const int es = g.out_bf16 ? 2 : 4;
+  uint8_t* C = g.C + batch * g.stride_c * es;
+  const uint8_t* D = g.D ? g.D + batch * g.stride_d * es : nullptr;
+  const uint8_t* bias = g.bias ? g.bias + batch * g.stride_bias * es : nullptr;
+  const int n = n_wave + (lane % kLanesPerRow) * 4;
+  if (n >= g.N) return;
+  float sa_c[4], sb_c[4], bias_c[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int ne = n + e < g.N ? n + e : g.N - 1;
+    sa_c[e] = g.sa_mode == MI355Q_GS_PER_COL ? g.sa[ne] : scalars.sa;
+    sb_c[e] = g.sb_mode == MI355Q_GS_PER_COL ? g.sb[ne] : scalars.sb;
+    bias_c[e] = g.bias_mode == MI355Q_BIAS_ROW_VECTOR ? load_out_as_f32(bias, ne, g.out_bf16) : 0.0f;
+  }
+  const bool vec_ok = (n + 3 < g.N) && ((g.ldc * es) % (4 * es) == 0) && ((reinterpret_cast<uintptr_t>(C) + (size_t)n * es) % (4 * es) == 0);
+  const bool a_rows = g.sa_mode == MI355Q_GS_PER_ROW, b_rows = g.sb_mode == MI355Q_GS_PER_ROW, full = g.bias_mode == MI355Q_BIAS_FULL;
+  const int last = g.M - m_wave < 16 * MT ? g.M - m_wave : 16 * MT;
+#pragma unroll 4
+  for (int row = lane / kLanesPerRow; row < last; row += kRowsPerPass) {
+    const int m = m_wave + row;
+    const f32x4 a = *reinterpret_cast<const f32x4*>(rows + row * kPitch + (lane % kLanesPerRow) * 4);
+    const float ra = a_rows ? g.sa[m] : 1.0f, rb = b_rows ? g.sb[m] : 1.0f;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // (one of ra and sa_c is exactly 1, likewise rb and sb_c)
+      float t = a[e] * (a_rows ? ra : sa_c[e]);
+      t = t * (b_rows ? rb : sb_c[e]);
+      v[e] = t + bias_c[e];
+    }
+    if (full || D) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int ne = n + e < g.N ? n + e : g.N - 1;
+        if (full) v[e] += load_out_as_f32(bias, (int64_t)m * g.ldbias + ne, g.out_bf16);
+        if (D) v[e] += load_out_as_f32(D, (int64_t)m * g.ldd + ne, g.out_bf16);
+      }
+    }
+    uint8_t* const to = C + ((int64_t)m * g.ldc + n) * es;
+    if (g.out_bf16) {
+      const uint32_t w0 = pack_bf16x2(v[0], v[1]), w1 = pack_bf16x2(v[2], v[3]);
+      uint16_t* c16 = reinterpret_cast<uint16_t*>(to);
+      if (vec_ok) {
+        *reinterpret_cast<u32x2*>(to) = u32x2{w0, w1};
+      } else {
+        c16[0] = (uint16_t)w0;
+        if (n + 1 < g.N) c16[1] = (uint16_t)(w0 >> 16);
+        if (n + 2 < g.N) c16[2] = (uint16_t)w1;
+        if (n + 3 < g.N) c16[3] = (uint16_t)(w1 >> 16);
+      }
+    } else if (vec_ok) {
+      *reinterpret_cast<f32x4*>(to) = f32x4{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < g.N) reinterpret_cast<float*>(to)[e] = v[e];
+    }
+  }
+}
+
+// BM = 16: one row tile, in LDS with 16 more rows that nothing reads (each of the four loading waves brings a whole region).
+template <int BM>
+struct RingShape {
+  static constexpr int kRows = BM < 32 ? 32 : BM;  // of A in LDS
+  static constexpr int kWavesM = BM >= 128 ? 2 : 1, kWavesN = kRingWaves / kWavesM;
+  static constexpr int MT = BM / kWavesM / 16, NT = kRingBN / kWavesN / 16;
+  static constexpr int kStage = (kRows + kRingBN) * kBK, kOffB = kRows * kBK;
+  static constexpr int kFit = (160 * 1024 - kRingWaves * kRingScaleBytes - 64) / kStage;
+  static constexpr int kStages = kFit < 7 ? kFit : 7;
+};
+
+// The load side of a workgroup: four waves that do nothing else.
+template <int BM, bool A_KMAJOR, bool B_KMAJOR>
+struct RingProducer {
+  using Shape = RingShape<BM>;
+  static constexpr int R = Shape::kStages, kStage = Shape::kStage, kOffB = Shape::kOffB;
+  using LoaderA = RingLoader<A_KMAJOR, Shape::kRows>;
+  using LoaderB = RingLoader<B_KMAJOR, kRingBN>;
+  static constexpr int kOps = LoaderA::kPerWave + LoaderB::kPerWave;
+  static_assert((R - 1) * kOps <= 63, "vmcnt holds 6 bits");
+  LoaderA la;
+  LoaderB lb;
+  uint32_t slot, ring;  // LDS addresses of the next stage's slot and of the ring
+  int next, stages;     // the stage of K the loaders point at, and their number
+  int last_k;           // k in the last stage of K
+
+  __device__ __forceinline__ void select() {
+    const int valid = next == stages - 1 ? last_k : kBK;
+    la.select(valid);
+    lb.select(valid);
+  }
+  // The next stage's loads; then the loaders move on (after the last stage of K comes the first).
+  template <bool NT_B>
+  __device__ __forceinline__ void issue_stage() {
+    static_for<LoaderA::kPerWave>([&](auto ic) { la.template issue<decltype(ic)::value, false>(slot); });
+    static_for<LoaderB::kPerWave>([&](auto ic) { lb.template issue<decltype(ic)::value, NT_B>(slot + kOffB); });
+    slot = slot + kStage == ring + R * kStage ? ring : slot + kStage;
+    la.base += (uint64_t)la.step;
+    lb.base += (uint64_t)lb.step;
+    const bool was_last = next == stages - 1;
+    if (++next == stages) {
+      next = 0;
+      la.base -= (uint64_t)(la.step * stages);
+      lb.base -= (uint64_t)(lb.step * stages);
+    }
+    if (last_k != kBK && (was_last || next == stages - 1)) select();
+  }
+  // Until at most `left` stages' loads of this wave are outstanding.
+  __device__ __forceinline__ static void wait_upto(int left) {
+    static_for<R>([&](auto nc) {
+      constexpr int n = decltype(nc)::value, ops = n * kOps;
+      if (left == n || (n == 0 && left < 0)) __builtin_amdgcn_s_waitcnt((ops & 15) | ((ops >> 4) << 14) | 0x0f70);
+    });
+  }
+};
+
+// The multiply side.  Fragments are single-buffered as in gemm_tile16.h: those of the next stage replace this stage's as
+// they die, so the barrier early in a stage finds every wave done with the stage's ring slot, and the next stage landed.
+template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
+struct RingConsumer {
+  using Shape = RingShape<BM>;
+  static constexpr int MT = Shape::MT, NT = Shape::NT, R = Shape::kStages, kStage = Shape::kStage;
+  using ReaderA = RingReader<A_KMAJOR, Shape::kRows, MT>;
+  using ReaderB = RingReader<B_KMAJOR, kRingBN, NT>;
+  static constexpr int kBarrierAt = MT == 1 ? 0 : NT - 1;  // the stage's barrier stands in front of this MFMA, the first after which a fragment is dead
+  f32x4 acc[MT][NT];
+  i32x8 fa[MT], fb[NT];
+  ReaderA ra;
+  ReaderB rb;
+  int rd;  // the ring slot the readers point at, in bytes
+
+  template <int I>
+  __device__ __forceinline__ void read_a() {
+    static_for<ReaderA::kParts>([&](auto pc) { ra.template read<I, decltype(pc)::value, 0>(fa[I]); });
+  }
+  template <int J>
+  __device__ __forceinline__ void read_b() {
+    static_for<ReaderB::kParts>([&](auto pc) { rb.template read<J, decltype(pc)::value, 0>(fb[J]); });
+  }
+  __device__ __forceinline__ void first_fragments() {
+    static_for<MT>([&](auto ic) { read_a<decltype(ic)::value>(); });
+    static_for<NT>([&](auto jc) { read_b<decltype(jc)::value>(); });
+  }
+  // (after the last stage the reads fetch a slot whose contents are not used)
+  __device__ __forceinline__ void stage() {
+    static_for<MT * NT>([&](auto gc) {
+      constexpr int gi = decltype(gc)::value, i = gi / NT, j = gi % NT;
+      if constexpr (gi == kBarrierAt) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's reads of the stage are done
+        __syncthreads();
+        const int d = rd + kStage == R * kStage ? -(R - 1) * kStage : kStage;
+        rd += d;
+        ra.move(d);
+        rb.move(d);
+      }
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[j], fa[i], acc[i][j], mfma_code<FMT_B>(), mfma_code<FMT_A>(), 0, 0, 0, 0);
+      if constexpr (j == NT - 1) read_a<i>();
+      if constexpr (i == MT - 1) read_b<j>();
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+};
+
+// NT_B: every byte of B is read by one workgroup alone (one row of tiles).
+template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B, bool NT_B>
+__global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g, SplitArgs split) {
+  using Producer = RingProducer<BM, A_KMAJOR, B_KMAJOR>;
+  using Consumer = RingConsumer<BM, A_KMAJOR, B_KMAJOR, FMT_A, FMT_B>;
+  using Shape = RingShape<BM>;
+  constexpr int MT = Shape::MT, NT = Shape::NT, R = Shape::kStages;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds_ring[R * Shape::kStage];
+  __shared__ __attribute__((aligned(16))) uint8_t lds_scales[kRingWaves * kRingScaleBytes];
+  static_assert(kRingWaves * 16 * MT * (16 * NT + 4) * 4 <= R * Shape::kStage, "the epilogue's rows overlay the ring");
+
+  // this workgroup's tile and part of K (whole stages)
+  int tile_m = 0, tile_n, part = 0, tile;
+  const int tiles = g.tiles_m * g.tiles_n;
+  if (g.tiles_m == 1) {
+    tile = blockIdx.x;
+    if (split.parts > 1) {
+      part = blockIdx.x / (unsigned)tiles;
+      tile = blockIdx.x - part * tiles;
+    }
+    tile_n = tile;
+  } else {
+    // each XCD takes a contiguous range of (part, tile), so that the panels its workgroups share come out of its L2
+    const int bid = blockIdx.x, units = gridDim.x;
+    const int xcd = bid & 7, per = units >> 3, rem = units & 7;
+    const int unit = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (bid >> 3);
+    part = split.parts > 1 ? unit / (unsigned)tiles : 0;
+    tile = unit - part * tiles;
+    tile_coords(tile, g.tiles_m, g.tiles_n, &tile_m, &tile_n);
+  }
+  if (split.parts > 1) {
+    const unsigned all = (g.K + kBK - 1) / kBK;
+    const int s0 = (int)(part * all / (unsigned)split.parts), s1 = (int)((part + 1) * all / (unsigned)split.parts);
+    g.K = (g.K < s1 * kBK ? g.K : s1 * kBK) - s0 * kBK;
+    g.A += (int64_t)s0 * kBK * (A_KMAJOR ? 1 : g.lda);
+    g.B += (int64_t)s0 * kBK * (B_KMAJOR ? 1 : g.ldb);
+  }
+  const int m0 = tile_m * BM, n0 = tile_n * kRingBN;
+  const int64_t batch = blockIdx.y;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int stages = (g.K + kBK - 1) / kBK;
+
+  if (wave >= kRingWaves) {
+    Producer p;
+    p.slot = p.ring = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_ring;
+    p.stages = stages;
+    p.last_k = g.K - (stages - 1) * kBK;
+    p.next = 0;
+    p.la.init(g.A + batch * g.stride_a + (int64_t)m0 * (A_KMAJOR ? g.lda : 1), g.lda, g.M - m0, wave - kRingWaves);
+    p.lb.init(g.B + batch * g.stride_b + (int64_t)n0 * (B_KMAJOR ? g.ldb : 1), g.ldb, g.N - n0, wave - kRingWaves);
+    // With a K-major B in one row of tiles each strip walks K from a stage of its own and wraps around: strips in step send
+    // requests that differ only in high address bits to the same few memory channels.  (An MN-major operand's ragged stage
+    // has loads that go nowhere, which may retire ahead of older ones: it has to be the last, and nothing is counted then.)
+    const bool tail_goes_nowhere = (!A_KMAJOR || !B_KMAJOR) && p.last_k != kBK;
+    if (B_KMAJOR && g.tiles_m == 1 && !tail_goes_nowhere) {
+      p.next = (int)((unsigned)tile_n * (unsigned)stages / (unsigned)g.tiles_n);
+      p.la.base += (uint64_t)(p.la.step * p.next);
+      p.lb.base += (uint64_t)(p.lb.step * p.next);
+    }
+    p.select();
+    for (int s = 0; s < R && s < stages; ++s) p.template issue_stage<NT_B>();
+    Producer::wait_upto(tail_goes_nowhere && stages <= R ? 0 : (stages < R ? stages : R) - 1);
+    __syncthreads();  // the first stage is in LDS
+    for (int s = 0; s < stages; ++s) {
+      const bool more = s + R < stages;
+      Producer::wait_upto(more ? R - 2 : (tail_goes_nowhere ? 0 : stages - 2 - s));
+      __syncthreads();  // stage s + 1 is in LDS, and stage s in the consumers' registers
+      if (more) p.template issue_stage<NT_B>();
+    }
+    return;
+  }
+
+  Consumer c;
+  const int wm = (wave / Shape::kWavesN) * (16 * MT), wn = (wave % Shape::kWavesN) * (16 * NT);
+  if (g.fast_epi) ScaleStager::issue<(MT + 1) / 2, NT / 2>(g, batch, m0 + wm, n0 + wn, reinterpret_cast<float*>(lds_scales + wave * kRingScaleBytes));
+  const ScalarScales scalars = load_scalar_scales(g);
+  const uint32_t ring = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_ring;
+  c.ra.init(ring, wm);
+  c.rb.init(ring + Producer::kOffB, wn);
+  c.rd = 0;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) c.acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  c.first_fragments();
+  for (int s = 0; s < stages; ++s) c.stage();
+
+  // the producers have ended, and every load has landed; the ring is idle once the other consumers have read their last
+  const int slot = (int)batch * tiles + tile, slots = tiles * gridDim.y;
+  constexpr bool kPairs = BM >= 128;
+  const uint32_t seen = !kPairs && split.parts > 1 ? split_look(split, slot) : 0;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (split.parts > 1) {
+    uint32_t* word = reinterpret_cast<uint32_t*>(lds_ring);
+    if constexpr (kPairs) {
+      if (!meet_in_pairs<4 * MT * NT, kRingWaves * 64>(
+              split, slot, slots, part, word,
+              [&](auto jc) { constexpr int j = decltype(jc)::value; return c.acc[j / (4 * NT)][j / 4 % NT][j % 4]; },
+              [&](auto jc, float v) { constexpr int j = decltype(jc)::value; c.acc[j / (4 * NT)][j / 4 % NT][j % 4] = v; }))
+        return;
+    } else {
+      if (threadIdx.x == 0) *word = seen;
+      __syncthreads();
+      const bool others_in = *word == (uint32_t)split.parts - 1;
+      __syncthreads();
+      if (!split_exchange<4 * MT * NT, kRingWaves * 64>(
+              split, slot, slots, part, true, others_in, word, [&](int j) { return c.acc[j / (4 * NT)][j / 4 % NT][j % 4]; },
+              [&](int j, float v) { c.acc[j / (4 * NT)][j / 4 % NT][j % 4] = v; }))
+        return;
+    }
+    __syncthreads();  // the word has been read
+  }
+  if (g.fast_epi && g.D == nullptr) {
+    const uint8_t* staged = lds_scales + wave * kRingScaleBytes;
+    uint8_t* rows = lds_ring + wave * (16 * MT * 32 * NT);
+    const bool per_col = g.sb_mode == MI355Q_GS_PER_COL, bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR;
+    if (per_col && bias) ring_epilogue_fast<MT, NT, true, true>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
+    else if (per_col) ring_epilogue_fast<MT, NT, true, false>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
+    else if (bias) ring_epilogue_fast<MT, NT, false, true>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
+    else ring_epilogue_fast<MT, NT, false, false>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
+  } else {
+    ring_epilogue_any<MT, NT>(g, batch, c.acc, m0 + wm, n0 + wn, reinterpret_cast<float*>(lds_ring) + wave * 16 * MT * (16 * NT + 4), scalars);
+  }
+}
+
+// B larger than this and read once is loaded past the caches (the nontemporal hint).
+constexpr int64_t kRingStreamBytes = 64LL << 20;
+
+template <int BM, bool AK, bool BK_, int FA, int FB>
+void launch_ring(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
+  GemmArgs a = g;
+  a.tiles_m = (g.M + BM - 1) / BM;
+  a.tiles_n = (g.N + kRingBN - 1) / kRingBN;
+  dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (split.parts > 1 ? split.parts : 1)), (unsigned)batch);
+  if (a.tiles_m == 1 && (int64_t)g.N * g.K > kRingStreamBytes) fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, true><<<grid, kRingThreads, 0, st>>>(a, split);
+  else fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, false><<<grid, kRingThreads, 0, st>>>(a, split);
+}
+
+}  // namespace mi355q

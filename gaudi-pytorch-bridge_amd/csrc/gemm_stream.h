@@ -15,10 +15,9 @@
 // Strips of 256 columns because 256-byte pieces of such a matrix stream at 6.65 TB/s and 128-byte ones at 5.8 (strip
 // reads alone, 235 MB: 35.3 against 40.3 us); with 8-byte loads (strips of 128 columns here) it was 5.0.  Measured at
 // 16 x 8192 x 28672: 38.9 us for the stream, 1.8 for the sum over the waves and the epilogue, 2.2 for the meeting of
-// the two parts of K: 43 us (strip kernel of gemm_skinny.h: 45.5).  1 x 14336 x 4096: 17.6 us in 16 parts (56 as 32
-// strips of 128 columns with K in one piece).  A second row tile (M <= 32) leaves room for half the loads in flight and
-// loses to the strip kernel (48 against 46.5 us); a K-major B, loaded in 64-byte pieces per row, does so as well
-// (52 against 40).
+// the two parts of K: 43 us (ring kernel of gemm_ring.h: 46.4).  Below about 100 MB of B the ring kernel's shorter start
+// and end win (16 x 8192 x 8192: 18.9 against 15.1 us).  A second row tile (M <= 32) leaves room for half the loads in flight
+// and loses as well (48 against 46.5 us), and so does a K-major B, loaded in 64-byte pieces per row (52 against 40).
 #pragma once
 #include "gemm_split.h"
 

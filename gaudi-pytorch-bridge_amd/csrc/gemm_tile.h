@@ -132,7 +132,7 @@ struct TileGeom {
     if constexpr (KMAJOR && ROW_BYTES == 128) return V == 1 ? (((row >> 2) & 1) | (row & 2) | ((row >> 1) & 4)) : ((row >> 1) & 7);
     else if constexpr (KMAJOR) return (row >> 2) & 3;
     else if constexpr (ROW_BYTES == 256) return V == 1 ? (((row & 7) << 1) | ((row >> 5) & 1)) : ((row & 7) << 1);
-    else return ((row >> 1) & 3) << 1;
+    else return V == 1 ? (((row >> 1) & 3) | ((row >> 3) & 4)) : (((row >> 1) & 3) << 1);
   }
   __device__ static __forceinline__ int lds_offset(int row, int chunk) {
     return row * ROW_BYTES + ((chunk ^ swizzle(row)) << 4);
@@ -269,18 +269,16 @@ struct DmaLoader {
 
   // Issues load I of this wave's share of the stage the descriptor points at,
   // which starts at k0.
-  // NT: the nontemporal hint, for an operand that is read once (the weights of a decode-shaped call): a strip
-  // read of a 235 MB matrix runs 8 % faster with it (41 against 45 us), through registers or into LDS alike.
   // K_CHECK false: the caller's K is a whole number of the stages it walks, no lane is ever past K, and the
   // operand is narrow (see advance_narrow()).  Then (and without CLAMP_ROWS) a lane's offset does not depend on the
   // stage, the descriptor stays where set_tile() put it and the stage is the instruction's scalar offset; and four
   // loads in a row share one write of m0: the instruction's immediate offset moves the LDS address and the memory
   // address alike, so region I takes the m0 of region I - I % 4, the immediate (I % 4) KiB, and a lane offset
   // lowered by as much.  The caller issues the regions of a group in order with nothing between them that writes m0.
-  template <int I, bool CLAMP_ROWS = false, bool NT = false, bool K_CHECK = true>
+  template <int I, bool CLAMP_ROWS = false, bool K_CHECK = true>
   __device__ __forceinline__ void issue_one(uint8_t* lds_tile, int k0, int K) const {
     const uint32_t lds_base = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_tile;
-    if constexpr (!K_CHECK && !CLAMP_ROWS && !NT && kPerWave % 4 == 0) {
+    if constexpr (!K_CHECK && !CLAMP_ROWS && kPerWave % 4 == 0) {
       constexpr int i = I, r = I % 4;
       const int vo = voff[i % kStored] + (i / kStored) * region_step - r * 1024;
       if constexpr (r == 0) {
@@ -305,36 +303,15 @@ struct DmaLoader {
       // Written as asm so that the compiler, which would otherwise make every later
       // LDS read wait for all outstanding global->LDS loads, leaves the waiting to
       // the explicit vmcnt drain before each barrier.
-      if constexpr (NT) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
-                     :
-                     : "s"(dst), "v"(vo), "s"(rsrc)
-                     : "memory", "m0");
-      } else {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     :
-                     : "s"(dst), "v"(vo), "s"(rsrc)
-                     : "memory", "m0");
-      }
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                   :
+                   : "s"(dst), "v"(vo), "s"(rsrc)
+                   : "memory", "m0");
     }
   }
 
   __device__ __forceinline__ void issue(uint8_t* lds_tile, int k0, int K) const {
     static_for<kPerWave>([&](auto ic) { issue_one<decltype(ic)::value>(lds_tile, k0, K); });
-  }
-
-  // Points the descriptor at K stage `stage` of the tile set_tile() chose, which
-  // has to be the most recent call (it leaves the descriptor at stage 0 and
-  // this walks from wherever advance() has taken it).  Stages at or beyond K
-  // are entirely out of range.
-  __device__ __forceinline__ void seek(int from_stage, int to_stage) {
-    const int64_t d = (int64_t)(to_stage - from_stage) * step;
-    uint64_t b = ((uint64_t)(uint32_t)rsrc[1] << 32) | (uint32_t)rsrc[0];
-    b += (uint64_t)d;
-    rsrc[0] = (int)(uint32_t)b;
-    rsrc[1] = (int)(uint32_t)(b >> 32);
-    remaining -= d;
-    set_records();
   }
 
   // advance() for an operand whose whole extent, from its first byte to the last one the launch may address, is
@@ -691,20 +668,17 @@ constexpr int fast_epilogue_stores() { return MT * 2 * NT; }
 // columns past N are dropped by the store's range check instead of by branches
 // (with branches in it the register allocator copies every accumulator out of
 // the accumulation registers at once and spills).
-// STAGED: the scale and bias values of the wave's rows and columns already sit
-// in its staging area (ScaleStager, below) and the scalar scales come as
-// arguments, so that the epilogue loads nothing from global memory: a wait for
-// such a load would also wait for every global->LDS load issued before it,
-// that is for the next tile's first stages.
+// The scale and bias values of the wave's rows and columns already sit in its staging area (ScaleStager, below) and the
+// scalar scales come as arguments, so that the epilogue loads nothing from global memory: a wait for such a load would
+// also wait for every global->LDS load issued before it, that is for the next tile's first stages.
 // Layout of the staged values in a wave's staging area (bytes): B scales of its
 // 32 NT columns (fp32), bias of the same columns (bf16), A scales of its 32 MT
 // rows (fp32).  Values of a kind the problem does not have are zeros.
 constexpr int kStagedColScale = 0, kStagedBias = 512, kStagedRowScale = 768, kStagedBytes = 1280;
 
-template <int MT, int NT, bool PER_COL, bool HAS_BIAS, bool STAGED = false, bool HAS_D = false>
+template <int MT, int NT, bool PER_COL, bool HAS_BIAS, bool HAS_D = false>
 __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t batch, f32x16 (&acc)[MT][NT],
-                                                   int m_wave, int n_wave, float* stage_f,
-                                                   ScalarScales scalars = ScalarScales{1.0f, 1.0f}) {
+                                                   int m_wave, int n_wave, float* stage_f, ScalarScales scalars) {
   static_assert(MT <= 4 && NT <= 4, "staged layout");
   constexpr int kRowBytes = 64 * NT;
   constexpr int kSlotMask = 8 * NT - 1;
@@ -717,31 +691,24 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
   const int lane = lane_id_here();
   const int r = lane & 31, h = lane >> 5;
 
-  if constexpr (!STAGED) scalars = load_scalar_scales(g);
   const float sa_s = scalars.sa, sb_s = scalars.sb;
 
-  // Per-column values of the columns this lane holds in the accumulator layout
-  // (columns at or beyond N read the last four: their results are not stored).
+  // Per-column values of the columns this lane holds in the accumulator layout.
   // A scalar B scale is folded into the row factor instead, which leaves one
   // fused multiply-add per element.
   float cs[PER_COL ? NT : 1][4][4], cb[HAS_BIAS ? NT : 1][4][4];
-  const uint16_t* bias = reinterpret_cast<const uint16_t*>(g.bias) + (HAS_BIAS ? batch * g.stride_bias : 0);
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int col = 32 * j + 8 * q + 4 * h;  // inside the wave's tile
-      int n = n_wave + col;
-      n = n < g.N - 4 ? n : g.N - 4;
       if constexpr (PER_COL) {
-        const f32x4 v = STAGED ? *reinterpret_cast<LDS_AS const f32x4*>(stage + kStagedColScale + col * 4)
-                               : *reinterpret_cast<const f32x4*>(g.sb + n);
+        const f32x4 v = *reinterpret_cast<LDS_AS const f32x4*>(stage + kStagedColScale + col * 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) cs[j][q][e] = v[e];
       }
       if constexpr (HAS_BIAS) {
-        const u32x2 v = STAGED ? *reinterpret_cast<LDS_AS const u32x2*>(stage + kStagedBias + col * 2)
-                               : *reinterpret_cast<const u32x2*>(bias + n);
+        const u32x2 v = *reinterpret_cast<LDS_AS const u32x2*>(stage + kStagedBias + col * 2);
         cb[j][q][0] = __uint_as_float(v[0] << 16);
         cb[j][q][1] = __uint_as_float(v[0] & 0xffff0000u);
         cb[j][q][2] = __uint_as_float(v[1] << 16);
@@ -751,14 +718,8 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
   float ra[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    const int m = m_wave + 32 * i + r;
-    if constexpr (STAGED) {
-      const float staged = *reinterpret_cast<LDS_AS const float*>(stage + kStagedRowScale + (32 * i + r) * 4);
-      ra[i] = g.sa_mode == MI355Q_GS_PER_ROW ? staged : sa_s;
-    } else {
-      ra[i] = sa_s;
-      if (g.sa_mode == MI355Q_GS_PER_ROW) ra[i] = g.sa[m < g.M ? m : g.M - 1];
-    }
+    const float staged = *reinterpret_cast<LDS_AS const float*>(stage + kStagedRowScale + (32 * i + r) * 4);
+    ra[i] = g.sa_mode == MI355Q_GS_PER_ROW ? staged : sa_s;
     if (!PER_COL) ra[i] *= sb_s;
   }
 
@@ -861,22 +822,21 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
 // ALLOW_D false: the caller guarantees there is no accumulate input (the
 // kernel with 256 accumulator registers per lane keeps its epilogue to four
 // variants; with more, the compiler copies accumulators to scratch memory).
-template <int MT, int NT, bool STAGED = false, bool ALLOW_D = true>
+template <int MT, int NT, bool ALLOW_D = true>
 __device__ __forceinline__ void epilogue_bf16_fast_any(const GemmArgs& g, int64_t batch, f32x16 (&acc)[MT][NT],
-                                                       int m_wave, int n_wave, float* stage,
-                                                       ScalarScales scalars = ScalarScales{1.0f, 1.0f}) {
+                                                       int m_wave, int n_wave, float* stage, ScalarScales scalars) {
   const bool per_col = g.sb_mode == MI355Q_GS_PER_COL, bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR;
   if (ALLOW_D && g.D != nullptr) {
-    if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true, STAGED, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else if (per_col) epilogue_bf16_fast<MT, NT, true, false, STAGED, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else if (bias) epilogue_bf16_fast<MT, NT, false, true, STAGED, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else epilogue_bf16_fast<MT, NT, false, false, STAGED, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+    if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+    else if (per_col) epilogue_bf16_fast<MT, NT, true, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+    else if (bias) epilogue_bf16_fast<MT, NT, false, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+    else epilogue_bf16_fast<MT, NT, false, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
     return;
   }
-  if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true, STAGED>(g, batch, acc, m_wave, n_wave, stage, scalars);
-  else if (per_col) epilogue_bf16_fast<MT, NT, true, false, STAGED>(g, batch, acc, m_wave, n_wave, stage, scalars);
-  else if (bias) epilogue_bf16_fast<MT, NT, false, true, STAGED>(g, batch, acc, m_wave, n_wave, stage, scalars);
-  else epilogue_bf16_fast<MT, NT, false, false, STAGED>(g, batch, acc, m_wave, n_wave, stage, scalars);
+  if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+  else if (per_col) epilogue_bf16_fast<MT, NT, true, false>(g, batch, acc, m_wave, n_wave, stage, scalars);
+  else if (bias) epilogue_bf16_fast<MT, NT, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
+  else epilogue_bf16_fast<MT, NT, false, false>(g, batch, acc, m_wave, n_wave, stage, scalars);
 }
 
 // Brings the scale and bias values the fast epilogue of one wave tile needs
@@ -1166,7 +1126,7 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
     k_step(std::true_type{}, 0);
     for (int kt = 2; kt < KT2; kt += 2) k_step(std::false_type{}, kt);
     if (FAST_ONLY || g.fast_epi) {
-      epilogue_bf16_fast_any<MT, NT, true, !FAST_ONLY>(g, batch, core.acc, m0 + wm, n0 + wn, stage, scalars);
+      epilogue_bf16_fast_any<MT, NT, !FAST_ONLY>(g, batch, core.acc, m0 + wm, n0 + wn, stage, scalars);
       // A store whose lanes are all past M or N completes at once and must not be counted as
       // outstanding: after a tile on the matrix edge the next tile waits for everything.
       stores_pending = m0 + BM <= g.M && n0 + BN <= g.N;
@@ -1183,15 +1143,13 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
 // WN: waves along n (the workgroup has 2 x WN); FAST_ONLY: the kernel carries
 // the fast bf16 epilogue alone, without an accumulate input: the launch must
 // satisfy epilogue_fast_ok() and have no D.
-// WGS_PER_CU: workgroups of the persistent grid per compute unit (2 where the
-// kernel's LDS and registers let two be resident).
-template <int BM, int BN, int WN, bool FAST_ONLY, bool AK, bool BK_, int FA, int FB, int WGS_PER_CU = 1>
+template <int BM, int BN, int WN, bool FAST_ONLY, bool AK, bool BK_, int FA, int FB>
 void launch_tile(const GemmArgs& g, int64_t batch, hipStream_t st) {
   GemmArgs a = g;
   a.tiles_m = (g.M + BM - 1) / BM;
   a.tiles_n = (g.N + BN - 1) / BN;
   const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
-  const int cus = compute_units() * WGS_PER_CU;
+  const int cus = compute_units();
   dim3 grid((unsigned)(tiles < cus ? tiles : cus), (unsigned)batch);
   fp8_gemm_tile_kernel<BM, BN, WN, AK, BK_, FA, FB, FAST_ONLY><<<grid, kWavesM * WN * 64, 0, st>>>(a);
 }

@@ -226,8 +226,8 @@ struct TileCore16 {
   template <int OP, int STAGE>
   __device__ __forceinline__ void dma_op(int kt) {
     constexpr int na = LoaderA::kPerWave;
-    if constexpr (OP < na) la.template issue_one<OP, false, false, !LEAN>(ring + STAGE * kStageA, kt * kBK, K);
-    else lb.template issue_one<OP - na, false, false, !LEAN>(ring + 2 * kStageA + STAGE * kStageB, kt * kBK, K);
+    if constexpr (OP < na) la.template issue_one<OP, false, !LEAN>(ring + STAGE * kStageA, kt * kBK, K);
+    else lb.template issue_one<OP - na, false, !LEAN>(ring + 2 * kStageA + STAGE * kStageB, kt * kBK, K);
   }
   __device__ __forceinline__ void step_descriptors() {
     if constexpr (LEAN) {

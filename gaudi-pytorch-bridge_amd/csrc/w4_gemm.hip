@@ -26,7 +26,7 @@
 // Relative to an fp8 operand whose lane holds k = 32 h + j in byte j (h = lane / 32), the fp4 operand of the
 // 32x32x64 MFMA holds k = 16 h + j in nibble j < 16 and k = 32 + 16 h + (j - 16) in nibble j >= 16.
 //
-// Two kernels.  The first, below, is shaped like the strip kernel of gemm_skinny.h (the second, for groups of
+// Two kernels.  The first, below, has strips of 128 columns (the second, for groups of
 // 128 with bf16 scales, follows it: 256-column strips, K split over workgroups): the weights stream once through a deep LDS
 // ring, one workgroup per 128 columns; rows of A beyond 64 run as further row blocks that
 // stream the weights again, which suits decode and small prefill batches, the shapes
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kW4Threads) void w4a8_gemm_kernel(W4Args a) {
     int wr_off = (S - 1) * kStage;
     for (int kt = 0; kt < KT; ++kt) {
       // The loads of stage kt have landed once only those of later stages are outstanding; the
-      // zero-fill loads past K complete at once and are not counted (see gemm_skinny.h).
+      // zero-fill loads past K complete at once and are not counted.
       wait_for_stage(KT - 1 - kt);
       // stage kt is in LDS for the consumers, who are done with stage kt - 1, whose room the next loads take
       __syncthreads();

@@ -1,0 +1,49 @@
+"""The ring kernel (gemm_ring.h) at the edges of its tiles: rows and columns beside the tile heights and strips, K of less than a
+stage, of a ragged last stage and of more and fewer stages than the ring holds, each height whole and in parts, all layouts.
+Operands are small integers and scales powers of two, so that every fp32 sum is exact in any order and the result must match
+bit for bit."""
+import pytest
+import torch
+
+from helpers import E4, E5
+
+CASES = [  # M, K, N, trans_a, trans_b
+    (16, 144, 130, 0, 0), (1, 16, 256, 0, 1), (3, 8176, 8210, 0, 1), (16, 2064, 129, 0, 0), (1, 8192, 8208, 0, 1),     # 16 rows
+    (17, 128, 128, 0, 0), (32, 2064, 130, 0, 1), (33, 400, 1000, 0, 0), (49, 896, 384, 0, 1),                          # 32
+    (64, 4112, 4100, 0, 0), (100, 8192, 11264, 0, 0), (128, 1168, 13000, 0, 1), (65, 768, 9000, 0, 0),                 # 64
+    (257, 272, 8200, 0, 1), (129, 512, 12000, 0, 0), (300, 7168, 7168, 0, 0),                                          # 128
+    (129, 1040, 20000, 0, 0), (513, 2576, 7168, 0, 1), (700, 8208, 4090, 0, 0),                                        # 256
+    (65, 2576, 250, 1, 0), (144, 1040, 5000, 1, 1), (600, 1303, 3000, 1, 0), (16, 4096, 256, 1, 1), (1000, 4096, 4096, 1, 0),  # A [K, M]
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,ta,tb", CASES)
+def test_ring_tiles_are_exact(M, K, N, ta, tb, dev):
+    g = torch.Generator().manual_seed(M * 5 + K * 3 + N)
+    a, b = torch.randint(-2, 3, (M, K), generator=g).float(), torch.randint(-2, 3, (K, N), generator=g).float()
+    fa, fb = ((E4, E4), (E4, E5), (E5, E4), (E5, E5))[(M + K + N) % 4]
+    a8, b8 = (a.t().contiguous() if ta else a).to(fa).to(dev), (b.t().contiguous() if tb else b).to(fb).to(dev)
+    gemm = torch.ops.hpu.fp8_gemm_v2
+    p = (a.to(dev) @ b.to(dev)).cpu()  # (small integers: exact in fp32)
+    sa, sb = (torch.arange(M) % 3 - 1.0).exp2(), (torch.arange(N) % 2 - 1.0).exp2()
+    bias = (torch.arange(N) % 5 - 2).float()
+    ref = (p * sa[:, None]) * sb[None] + bias
+    for out in (torch.float32, torch.bfloat16):
+        for _ in range(2):
+            c = gemm(a8, bool(ta), b8, bool(tb), None, out, sa[:, None].to(dev), sb.to(dev), bias.to(out).to(dev), False, [1, N])
+            assert torch.equal(c.cpu(), ref.to(out))
+    d = torch.randint(-4, 5, (M, N), generator=g).bfloat16()
+    half, two = torch.tensor(0.5).to(dev), torch.tensor(2.0).to(dev)
+    assert torch.equal(gemm(a8, bool(ta), b8, bool(tb), d.to(dev), torch.bfloat16, half, two, None, True).cpu(), (p + d.float()).bfloat16())
+    assert torch.equal(gemm(a8, bool(ta), b8, bool(tb), None, torch.bfloat16, half, two, bias.bfloat16().to(dev), False).cpu(), (p + bias).bfloat16())
+
+
+def test_every_height_is_reached(pkg):
+    """The cases above run on every tile height, whole and in parts."""
+    name = pkg.capi().mi355q_fp8_gemm_ws_variant
+    up = lambda x: (x + 15) // 16 * 16  # noqa: E731
+    # (A [K, M] with a ragged K is the one form whose K is not rounded up before the launch)
+    got = {name(ta, up(M if ta else K), tb, up(K if tb else N), M, N, K if ta and not tb else up(K), 1).decode().split("_ring")[0] for M, K, N, ta, tb in CASES}
+    want = {"strip_Mx128x128", "split_strip_Mx128x128", "split_stream_Mx128x128", "tile128x128x128", "tile256x128x128", "split_tile256x128x128"}
+    assert want <= got, want - got
