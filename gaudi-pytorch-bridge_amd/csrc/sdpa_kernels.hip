@@ -54,12 +54,13 @@ struct SdpaArgs {
   int64_t ldq, ldk, ldv, ldm, ldo;
   int L, S, Dk, Dv;
   int mask_kind, causal, out_fp8;
-  int vec_q, vec_k, vec_v, vec_o;  // 16-byte (q, k, v) / 4-element (out) accesses are possible
+  int vec_q, vec_k, vec_v, vec_o;  // 16-byte (q, k, v) / 4-element (out; 2: 8-element) accesses are possible
   int dma;                         // k and v go global -> LDS directly
   int nqb;                         // query blocks per (batch, head)
   float scale;
   const float* sc_dev[6];  // d_scale_q, d_scale_k, d_scale_v, q_scale_s, q_scale_o, d_scale_s
   float sc_host[6];        // used where sc_dev is null; 0 = absent
+  int any_dev;             // some sc_dev is not null; otherwise every sc_host but the fifth holds the value to use
   float* amax_s;
   float* amax_o;
   // the few-queries kernel only
@@ -77,6 +78,39 @@ struct SdpaArgs {
 __device__ __forceinline__ float sdpa_scale(const SdpaArgs& a, int i, float absent) {
   if (a.sc_dev[i] != nullptr) return *a.sc_dev[i];
   return a.sc_host[i] != 0.0f ? a.sc_host[i] : absent;
+}
+
+// The scales of a launch.  Without device pointers they are read as they stand: five pointer tests, each with a branch and a
+// load behind it, took half a microsecond of a workgroup's start.
+struct SdpaScales {
+  float dq, dk, qs;
+  __device__ __forceinline__ void load(const SdpaArgs& a) {
+    if (__builtin_expect(a.any_dev == 0, 1)) {
+      dq = a.sc_host[0];
+      dk = a.sc_host[1];
+      qs = a.sc_host[3];
+    } else {
+      dq = sdpa_scale(a, 0, 1.0f);
+      dk = sdpa_scale(a, 1, 1.0f);
+      qs = sdpa_scale(a, 3, 1.0f);
+    }
+  }
+};
+__device__ __forceinline__ float uniform_f32(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+// d_scale_s d_scale_v, read where the rows are stored
+__device__ __forceinline__ float sdpa_out_scale(const SdpaArgs& a, float qs) {
+  if (__builtin_expect(a.any_dev == 0, 1)) return a.sc_host[5] * a.sc_host[2];
+  return sdpa_scale(a, 5, 1.0f / qs) * sdpa_scale(a, 2, 1.0f);
+}
+
+// The batch index along dimension d, the higher dimensions left in `rest`.  (32 bits: a launch has fewer workgroups than that,
+// and the 64-bit division that stood here costs 150 instructions each time.)
+__device__ __forceinline__ int64_t sdpa_batch_index(const SdpaArgs& a, int d, uint32_t& rest) {
+  const uint32_t n = (uint32_t)a.bdim[d];
+  if (n == 1) return 0;
+  const uint32_t q = rest / n, b = rest - q * n;
+  rest = q;
+  return b;
 }
 
 // LDS offset of 16-byte chunk `chunk` of K row `row` (ROW_BYTES per row).  The 16 lanes of one
@@ -175,10 +209,12 @@ __global__ void sdpa_clear_amax_kernel(float* a, float* b) {
 
 // One block of 64 keys for a wave's 32 query rows: S^T = K Q^T from the K tile at kb, masks, the
 // online-softmax update of (m_run, l_run, o), and O^T += V^T P^T from the V tile at vb.  qpos is the
-// lane's query position (for the causal comparison), mrow its row of the mask; `edge` says that some
-// score of the block may need masking (wave-uniform), otherwise the cheap path runs.
-template <int DKC, int DVT, int FMT, bool QL = false>
-__device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb, const uint8_t* vb, int kv0, bool edge, int qpos,
+// lane's query position (for the causal comparison), mrow its row of the mask.  Wave-uniform: `edge` says that some score of
+// the block may lie behind the last key, `general` that there is a mask, a first key, or a scale that is not positive; PLAIN:
+// neither, at compile time.  (The kernels walk their plain blocks in a loop of its own: with the other forms in the same
+// loop the compiler copies all 32 scores on the way to where the paths meet, 5 % of the prefill.)
+template <int DKC, int DVT, int FMT, bool QL, bool PLAIN>
+__device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb, const uint8_t* vb, int kv0, bool edge, bool general, int qpos,
                                            bool q_ok, const uint8_t* mrow, const i32x8 (&qf)[DKC], float sc2, float lqs, bool clamp_p,
                                            f32x16 (&o)[DVT], float& m_run, float& l_run, const uint8_t* qbase = nullptr,
                                            int klo = 0, int khi = 0x7fffffff) {
@@ -248,9 +284,19 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
 #endif
   }
 
-  // scores in units of log2, masks applied
+  // Scores in units of log2, masks applied.  Where only a last key is set (the causal rule, the end of the keys), a lane
+  // knows how many of the block's keys it may see and the scores stay as the MFMA left them.
   float mx = -__builtin_inff();
-  if (!edge && sc2 >= 0.0f) {
+  if (PLAIN || !general) {
+    if (!PLAIN && edge) {
+      int last = khi < a.S ? khi : a.S;
+      if (a.causal && qpos < last) last = qpos + 1;
+      const int left = last - kv0 - 4 * h;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[t][r] = 32 * t + 8 * (r >> 2) + (r & 3) < left ? s[t][r] : -__builtin_inff();
+    }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -288,9 +334,9 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   float psum = 0.0f;
   i32x8 pf = {0, 0, 0, 0, 0, 0, 0, 0};
   // p = 2^(x + shift) for this lane's 32 scores, their sum, and the fp8 codes packed in register
-  // order.  RAW: s still holds the unscaled products (x = s * sc2); CLAMP: q_scale_s exceeds the
-  // format's range.  Compile-time variants, so that the common one is a multiply-add, an exp2 and an
-  // add per score.
+  // order.  RAW: s still holds the unscaled products (x = s * sc2); CLAMP: q_scale_s may exceed the
+  // format's range (it changes nothing where it does not).  Compile-time variants, so that the common one
+  // is a multiply-add, an exp2 and an add per score.
   auto exponentials = [&](auto rawc, auto clampc) {
     constexpr bool RAW = decltype(rawc)::value, CLAMP = decltype(clampc)::value;
 #pragma unroll
@@ -321,10 +367,8 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
         pf[4 * t + j] = w;
       }
   };
-  const bool raw = !edge && sc2 >= 0.0f;  // s still holds the unscaled products
-  if (raw && !clamp_p) exponentials(std::true_type{}, std::false_type{});
-  else if (raw) exponentials(std::true_type{}, std::true_type{});
-  else if (!clamp_p) exponentials(std::false_type{}, std::false_type{});
+  if ((PLAIN || !general) && !clamp_p) exponentials(std::true_type{}, std::false_type{});
+  else if (PLAIN || !general) exponentials(std::true_type{}, std::true_type{});
   else exponentials(std::false_type{}, std::true_type{});
   l_run = l_run * alpha + psum;
 
@@ -430,14 +474,14 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   int id = blockIdx.x;
   const int total = gridDim.x;
   if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-  int64_t bi = id / a.nqb;
+  uint32_t bi = (uint32_t)id / (uint32_t)a.nqb;
   const int qb = a.nqb - 1 - (id - (int)bi * a.nqb);  // under a causal mask the long rows start first
   int64_t q_off = 0, k_off = 0, v_off = 0, m_off = 0, o_off = 0;
   int64_t b_valid = 0;
 #pragma unroll
   for (int d = 2; d >= 0; --d) {
-    const int64_t b = bi % a.bdim[d];
-    bi /= a.bdim[d];
+    const int64_t b = sdpa_batch_index(a, d, bi);
+    if (b == 0) continue;
     q_off += b * a.q_bs[d];
     k_off += b * a.k_bs[d];
     v_off += b * a.v_bs[d];
@@ -463,11 +507,11 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   const int qrow = wq0 + lq;
   const bool q_ok = qrow < a.L;
 
-  const float dq = sdpa_scale(a, 0, 1.0f), dk = sdpa_scale(a, 1, 1.0f), dv = sdpa_scale(a, 2, 1.0f);
-  const float qs = sdpa_scale(a, 3, 1.0f);
-  const float ds = sdpa_scale(a, 5, 1.0f / qs);
-  const float sc2 = a.scale * dq * dk * kLog2e;
-  const float lqs = __builtin_log2f(qs);
+  SdpaScales sc;
+  sc.load(a);
+  const float qs = uniform_f32(sc.qs);  // (the same in every lane, and known to be: they need no vector registers)
+  const float sc2 = uniform_f32(a.scale * sc.dq * sc.dk * kLog2e);
+  const float lqs = uniform_f32(__builtin_log2f(qs));
   constexpr float kMax8 = FMT == MI355Q_E5M2 ? 57344.0f : 448.0f;
   const bool clamp_p = !(qs <= kMax8);
 
@@ -480,24 +524,6 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
     const u32x4 hi = load_chunk(rp, q_ok, 64 * c + 32 * h + 16, a.Dk, a.vec_q);
     qf[c] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
   }
-  // The fragments are first used by an MFMA inside the block loop, and the wait for their loads would be placed
-  // there: a vmcnt(0) in every pass, which also waits for the K / V blocks just requested.  Naming them here
-  // puts that wait in front of the loop.
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass, which compiles this body for the launch stub, knows no "v"
-#pragma unroll
-  for (int c = 0; c < DKC; ++c) asm volatile("" : : "v"(qf[c]));
-#endif
-  const uint8_t* qbase = qlds + (kQLds ? wave * 4096 + h * 512 + lq * 16 : 0);
-  if constexpr (kQLds) {
-#pragma unroll
-    for (int c = 0; c < DKC; ++c) {
-      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2) * 1024 + h * 512 + lq * 16) =
-          u32x4{(uint32_t)qf[c][0], (uint32_t)qf[c][1], (uint32_t)qf[c][2], (uint32_t)qf[c][3]};
-      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2 + 1) * 1024 + h * 512 + lq * 16) =
-          u32x4{(uint32_t)qf[c][4], (uint32_t)qf[c][5], (uint32_t)qf[c][6], (uint32_t)qf[c][7]};
-    }
-  }
-
   // blocks blk0 .. nblk - 1 hold the keys of the window
   int nblk = (khi + kSdpaBN - 1) / kSdpaBN;
   if (a.causal) {
@@ -587,16 +613,31 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   float l_run = 0.0f;               // this half-wave's share of the running sum (times q_scale_s)
 
   const uint8_t* mrow = a.mask + (m_off + (int64_t)qrow * a.ldm) * (a.mask_kind == kMaskBool ? 1 : a.mask_kind == kMaskBf16 ? 2 : 4);
-  // ring positions count from the window's first block
+  // The first blocks (ring positions count from the window's first one) are requested behind the query fragments, and the
+  // wait for those covers them: one trip to memory at the start instead of two.
+  if constexpr (DMA) {
+    for (int b = 0; b < kStages - 1 && blk0 + b < nblk; ++b) issue_block(b);
+  }
+  // The fragments are first used by an MFMA inside the block loop, and the wait for their loads would be placed
+  // there: a vmcnt(0) in every pass, which also waits for the K / V blocks just requested.  Naming them here
+  // puts that wait in front of the loop.
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass, which compiles this body for the launch stub, knows no "v"
+#pragma unroll
+  for (int c = 0; c < DKC; ++c) asm volatile("" : : "v"(qf[c]));
+#endif
+  const uint8_t* qbase = qlds + (kQLds ? wave * 4096 + h * 512 + lq * 16 : 0);
+  if constexpr (kQLds) {
+#pragma unroll
+    for (int c = 0; c < DKC; ++c) {
+      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2) * 1024 + h * 512 + lq * 16) =
+          u32x4{(uint32_t)qf[c][0], (uint32_t)qf[c][1], (uint32_t)qf[c][2], (uint32_t)qf[c][3]};
+      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2 + 1) * 1024 + h * 512 + lq * 16) =
+          u32x4{(uint32_t)qf[c][4], (uint32_t)qf[c][5], (uint32_t)qf[c][6], (uint32_t)qf[c][7]};
+    }
+  }
   if (nblk > blk0) {
     if constexpr (DMA) {
-      for (int b = 0; b < kStages - 1 && blk0 + b < nblk; ++b) issue_block(b);
-      if (nblk - blk0 >= kStages - 1 && (blk0 + kStages - 1) * kSdpaBN <= a.S) {
-        constexpr int cnt = (kStages - 2) * (KREG + VREG);
-        __builtin_amdgcn_s_waitcnt((cnt & 15) | ((cnt >> 4) << 14) | 0x0f70);  // the first block has landed
-      } else {
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     } else {
       fetch(blk0);
       commit(0);
@@ -604,7 +645,9 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   }
   __syncthreads();
 
-  for (int blk = blk0; blk < nblk; ++blk) {
+  const bool masked = a.mask_kind != kMaskNone || !(sc2 > 0.0f);
+  auto step = [&](auto pc, int blk) {
+    constexpr bool PLAIN = decltype(pc)::value;
     const int kv0 = blk * kSdpaBN;
     const int pos = blk - blk0;
     if constexpr (DMA) {
@@ -616,10 +659,10 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
     const uint8_t* vb = kb + KBYTES;
 
     // a wave whose 32 rows all lie above this block's first key has nothing to add
-    const bool active = !(a.causal && kv0 > wq0 + 31);
-    if (active) {
-      const bool edge = (a.causal && kv0 + kSdpaBN - 1 > wq0) || kv0 + kSdpaBN > khi || kv0 < klo || a.mask_kind != kMaskNone;
-      sdpa_block<DKC, DVT, FMT, kQLds>(a, kb, vb, kv0, edge, qrow, q_ok, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run, qbase, klo, khi);
+    if (PLAIN || !(a.causal && kv0 > wq0 + 31)) {
+      const bool edge = (a.causal && kv0 + kSdpaBN - 1 > wq0) || kv0 + kSdpaBN > khi;
+      sdpa_block<DKC, DVT, FMT, kQLds, PLAIN>(a, kb, vb, kv0, edge, masked || kv0 < klo, qrow, q_ok, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run,
+                                              qbase, klo, khi);
     }
 
     if constexpr (DMA) {
@@ -637,58 +680,91 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
       if (blk + 1 < nblk) commit((pos + 1) & 1);
     }
     __syncthreads();
+  };
+  // the leading blocks that every row of the workgroup sees whole
+  int plain = khi / kSdpaBN;
+  if (a.causal && (q0 + 1) / kSdpaBN < plain) plain = (q0 + 1) / kSdpaBN;
+  if (masked || klo > 0) plain = 0;
+  int blk = blk0;
+  if constexpr (DVT <= 4 || DMA) {  // (through registers a second loop does not fit at head dimension 256)
+    for (; blk < plain; ++blk) step(std::true_type{}, blk);
   }
+  for (; blk < nblk; ++blk) step(std::false_type{}, blk);
 
   // out = O * d_scale_s * d_scale_v / l.  l_run carries the factor q_scale_s that p did.
   const float l_tot = (l_run + __shfl_xor(l_run, 32, 64)) / qs;
   const float inv_l = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  const float f = inv_l * (ds * dv);
-  const float qo = a.out_fp8 ? sdpa_scale(a, 4, 1.0f) : 1.0f;
-  float amax_o = 0.0f;
-  uint8_t* orow = a.out + (o_off + (int64_t)qrow * a.ldo) * (a.out_fp8 ? 1 : 2);
+  const float f = inv_l * sdpa_out_scale(a, qs);
+  if (a.vec_o == 2 && !a.out_fp8 && a.Dv == 32 * DVT && a.amax_o == nullptr) {
+    // whole rows in bf16: neighbouring groups of four columns of the two half-waves change places, so that a lane has eight
+    // consecutive columns, and leave as 16 bytes.  (The general form below is 12 KB of straight-line code at head dimension
+    // 128: a workgroup spent 3.2 us fetching it, 6 us at 256.)
+    if (q_ok) {
+      uint16_t* to = reinterpret_cast<uint16_t*>(a.out) + o_off + (int64_t)qrow * a.ldo + 8 * h;
 #pragma unroll
-  for (int t = 0; t < DVT; ++t)
+      for (int t = 0; t < DVT; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d0 = 32 * t + 8 * j + 4 * h;
-      float val[4];
+        for (int j = 0; j < 4; j += 2) {
+          typedef unsigned u32x2v __attribute__((ext_vector_type(2)));
+          u32x4 w;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        val[i] = o[t][4 * j + i] * f;
-        if (q_ok && d0 + i < a.Dv) amax_o = __builtin_fmaxf(amax_o, __builtin_fabsf(val[i]));
-      }
-      if (!q_ok || d0 >= a.Dv) continue;
-      if (a.out_fp8) {
-        const uint32_t w = cvt_fp8x4<MI355Q_E4M3FN>(val[0] * qo, val[1] * qo, val[2] * qo, val[3] * qo);
-        if (a.vec_o) {
-          *reinterpret_cast<uint32_t*>(orow + d0) = w;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (d0 + i < a.Dv) orow[d0 + i] = (uint8_t)(w >> (8 * i));
+          for (int i = 0; i < 2; ++i) {
+            const u32x2v sw = __builtin_amdgcn_permlane32_swap(pack_bf16x2(o[t][4 * j + 2 * i] * f, o[t][4 * j + 2 * i + 1] * f),
+                                                               pack_bf16x2(o[t][4 * j + 4 + 2 * i] * f, o[t][4 * j + 5 + 2 * i] * f), false, false);
+            w[i] = sw[0];
+            w[2 + i] = sw[1];
+          }
+          *reinterpret_cast<u32x4*>(to + 32 * t + 8 * j) = w;
         }
-      } else {
-        const uint32_t w0 = pack_bf16x2(val[0], val[1]), w1 = pack_bf16x2(val[2], val[3]);
-        if (a.vec_o) {
-          *reinterpret_cast<u32x2*>(orow + 2 * d0) = u32x2{w0, w1};
-        } else {
-          uint16_t* o16 = reinterpret_cast<uint16_t*>(orow);
-          const uint32_t ws[2] = {w0, w1};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (d0 + i < a.Dv) o16[d0 + i] = (uint16_t)(ws[i >> 1] >> (16 * (i & 1)));
-        }
-      }
     }
+  } else {
+    const float qo = a.out_fp8 ? sdpa_scale(a, 4, 1.0f) : 1.0f;
+    float amax_o = 0.0f;
+    uint8_t* orow = a.out + (o_off + (int64_t)qrow * a.ldo) * (a.out_fp8 ? 1 : 2);
+#pragma unroll
+    for (int t = 0; t < DVT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int d0 = 32 * t + 8 * j + 4 * h;
+        float val[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          val[i] = o[t][4 * j + i] * f;
+          if (q_ok && d0 + i < a.Dv) amax_o = __builtin_fmaxf(amax_o, __builtin_fabsf(val[i]));
+        }
+        if (!q_ok || d0 >= a.Dv) continue;
+        if (a.out_fp8) {
+          const uint32_t w = cvt_fp8x4<MI355Q_E4M3FN>(val[0] * qo, val[1] * qo, val[2] * qo, val[3] * qo);
+          if (a.vec_o) {
+            *reinterpret_cast<uint32_t*>(orow + d0) = w;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (d0 + i < a.Dv) orow[d0 + i] = (uint8_t)(w >> (8 * i));
+          }
+        } else {
+          const uint32_t w0 = pack_bf16x2(val[0], val[1]), w1 = pack_bf16x2(val[2], val[3]);
+          if (a.vec_o) {
+            *reinterpret_cast<u32x2*>(orow + 2 * d0) = u32x2{w0, w1};
+          } else {
+            uint16_t* o16 = reinterpret_cast<uint16_t*>(orow);
+            const uint32_t ws[2] = {w0, w1};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (d0 + i < a.Dv) o16[d0 + i] = (uint16_t)(ws[i >> 1] >> (16 * (i & 1)));
+          }
+        }
+      }
+    if (a.amax_o != nullptr) {
+      const uint32_t m = wave_max_u32(__float_as_uint(amax_o));
+      if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), m);
+    }
+  }
 
   if (a.amax_s != nullptr) {
     // the largest probability of a row is the one at the row maximum: 1 / l
     const uint32_t m = wave_max_u32(__float_as_uint(q_ok ? inv_l : 0.0f));
     if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_s), m);
-  }
-  if (a.amax_o != nullptr) {
-    const uint32_t m = wave_max_u32(__float_as_uint(amax_o));
-    if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), m);
   }
 }
 
@@ -800,18 +876,17 @@ __device__ __forceinline__ void sdpa_decode_finish(const SdpaArgs& a, uint8_t* l
     }
   }
   // normalise (0 for a row with nothing to attend to), scale, round and store; the amax updates
-  const float lsum = L / qs;
+  const float lsum = L / qs, out_scale = sdpa_out_scale(a, qs);
   const float inv_l = lsum > 0.0f ? 1.0f / lsum : 0.0f;
   const bool row_ok = row < a.rows;
   const int rin = a.pack ? row / a.L : 0, rq = a.pack ? row - rin * a.L : row;
   uint8_t* orow = a.out + (o_off + (int64_t)rin * a.o_bs[2] + (int64_t)rq * a.ldo) * (a.out_fp8 ? 1 : 2);
-  const float dv = sdpa_scale(a, 2, 1.0f), ds = sdpa_scale(a, 5, 1.0f / qs);
   const float qo = a.out_fp8 ? sdpa_scale(a, 4, 1.0f) : 1.0f;
   float amax_o = 0.0f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int d = dv0 + i * STEP;
-    const float x = val[i] * inv_l * (ds * dv);
+    const float x = val[i] * inv_l * out_scale;
     if (row_ok && d < a.Dv) {
       amax_o = __builtin_fmaxf(amax_o, __builtin_fabsf(x));
       if (a.out_fp8) orow[d] = (uint8_t)(cvt_fp8x4<MI355Q_E4M3FN>(x * qo, 0.f, 0.f, 0.f) & 0xffu);
@@ -830,14 +905,14 @@ __device__ __forceinline__ void sdpa_decode_finish(const SdpaArgs& a, uint8_t* l
 }
 
 // offsets of workgroup `g`'s tensors; with `pack` the innermost batch dimension stays inside the tile
-__device__ __forceinline__ void sdpa_group_offsets(const SdpaArgs& a, int64_t g, int64_t& q_off, int64_t& k_off, int64_t& v_off,
+__device__ __forceinline__ void sdpa_group_offsets(const SdpaArgs& a, uint32_t g, int64_t& q_off, int64_t& k_off, int64_t& v_off,
                                                    int64_t& m_off, int64_t& o_off) {
   q_off = k_off = v_off = m_off = o_off = 0;
 #pragma unroll
   for (int d = 2; d >= 0; --d) {
     if (d == 2 && a.pack) continue;
-    const int64_t b = g % a.bdim[d];
-    g /= a.bdim[d];
+    const int64_t b = sdpa_batch_index(a, d, g);
+    if (b == 0) continue;
     q_off += b * a.q_bs[d];
     k_off += b * a.k_bs[d];
     v_off += b * a.v_bs[d];
@@ -863,8 +938,8 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lq = lane & 31, h = lane >> 5;
-  const int64_t grp = blockIdx.x / a.nsplit;
-  const int split = blockIdx.x - (int)grp * a.nsplit;
+  const uint32_t grp = blockIdx.x / (uint32_t)a.nsplit;
+  const int split = (int)(blockIdx.x - grp * (uint32_t)a.nsplit);
   int64_t q_off, k_off, v_off, m_off, o_off;
   sdpa_group_offsets(a, grp, q_off, k_off, v_off, m_off, o_off);
 
@@ -875,10 +950,11 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
   const uint8_t* mrow = a.mask + (m_off + (int64_t)inner * a.m_bs[2] + (int64_t)qpos * a.ldm) *
                                      (a.mask_kind == kMaskBool ? 1 : a.mask_kind == kMaskBf16 ? 2 : 4);
 
-  const float dq = sdpa_scale(a, 0, 1.0f), dk = sdpa_scale(a, 1, 1.0f);
-  const float qs = sdpa_scale(a, 3, 1.0f);
-  const float sc2 = a.scale * dq * dk * kLog2e;
-  const float lqs = __builtin_log2f(qs);
+  SdpaScales sc;
+  sc.load(a);
+  const float qs = uniform_f32(sc.qs);  // (the same in every lane, and known to be: they need no vector registers)
+  const float sc2 = uniform_f32(a.scale * sc.dq * sc.dk * kLog2e);
+  const float lqs = uniform_f32(__builtin_log2f(qs));
   constexpr float kMax8 = FMT == MI355Q_E5M2 ? 57344.0f : 448.0f;
   const bool clamp_p = !(qs <= kMax8);
 
@@ -941,7 +1017,8 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
 
   int buf = 0;
   if (b0 + wave < b1) issue_block(0);
-  for (int blk = b0 + wave; blk < b1; blk += 4) {
+  const bool masked = a.mask_kind != kMaskNone || !(sc2 > 0.0f);
+  auto step = [&](auto pc, int blk) {
     const int kv0 = blk * kSdpaBN;
     const bool more = blk + 4 < b1;
     if (more) issue_block(buf ^ 1);
@@ -956,10 +1033,15 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
       __builtin_amdgcn_s_waitcnt(0x0f70);
     }
     const uint8_t* kb = mine + buf * kStage;
-    const bool edge = a.causal || kv0 + kSdpaBN > a.S || a.mask_kind != kMaskNone;
-    sdpa_block<DKC, DVT, FMT>(a, kb, kb + KBYTES, kv0, edge, qpos, q_ok, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run);
+    sdpa_block<DKC, DVT, FMT, false, decltype(pc)::value>(a, kb, kb + KBYTES, kv0, a.causal || kv0 + kSdpaBN > a.S, masked, qpos, q_ok, mrow, qf, sc2,
+                                                          lqs, clamp_p, o, m_run, l_run);
     buf ^= 1;
-  }
+  };
+  int plain = a.S / kSdpaBN < b1 ? a.S / kSdpaBN : b1;
+  if (masked || a.causal) plain = 0;
+  int blk = b0 + wave;
+  for (; blk < plain; blk += 4) step(std::true_type{}, blk);
+  for (; blk < b1; blk += 4) step(std::false_type{}, blk);
 
   // ---- merge the four waves: each leaves O^T [dv][row], m[row], l[row] in LDS
   __builtin_amdgcn_s_waitcnt(0x0f70);
@@ -1118,6 +1200,7 @@ int mi355q_fp8_sdpa_fwd(const void* q, const void* k, const void* v, int fp8_fmt
   bool vv = aligned_to(v, 16) && d->head_dim_v % 16 == 0 && d->ldv % 16 == 0;
   const size_t oel = out_dtype == MI355Q_BF16 ? 2 : 1;
   bool vo = aligned_to(out, 4 * oel) && d->head_dim_v % 4 == 0 && d->ldo % 4 == 0;
+  bool vo8 = aligned_to(out, 8 * oel) && d->head_dim_v % 8 == 0 && d->ldo % 8 == 0;
   for (int i = 0; i < 3; ++i) {
     a.bdim[i] = d->batch[i];
     a.q_bs[i] = d->q_bstride[i];
@@ -1129,13 +1212,14 @@ int mi355q_fp8_sdpa_fwd(const void* q, const void* k, const void* v, int fp8_fmt
     vk = vk && d->k_bstride[i] % 16 == 0;
     vv = vv && d->v_bstride[i] % 16 == 0;
     vo = vo && d->out_bstride[i] % 4 == 0;
+    vo8 = vo8 && d->out_bstride[i] % 8 == 0;
   }
   a.ldq = d->ldq; a.ldk = d->ldk; a.ldv = d->ldv; a.ldm = d->ldmask; a.ldo = d->ldo;
   a.L = (int)d->q_len; a.S = (int)d->kv_len; a.Dk = (int)d->head_dim_qk; a.Dv = (int)d->head_dim_v;
   a.mask_kind = mask_kind;
   a.causal = is_causal != 0;
   a.out_fp8 = out_dtype == MI355Q_E4M3FN;
-  a.vec_q = vq; a.vec_k = vk; a.vec_v = vv; a.vec_o = vo;
+  a.vec_q = vq; a.vec_k = vk; a.vec_v = vv; a.vec_o = vo8 ? 2 : vo;
   // direct loads address a block's rows with 32-bit offsets from a base that moves with the block
   a.dma = vk && vv && d->ldk < (1 << 24) && d->ldv < (1 << 24);
   a.nqb = (int)nqb;
@@ -1143,6 +1227,12 @@ int mi355q_fp8_sdpa_fwd(const void* q, const void* k, const void* v, int fp8_fmt
   for (int i = 0; i < 6; ++i) {
     a.sc_dev[i] = scale_dev != nullptr ? scale_dev[i] : nullptr;
     a.sc_host[i] = scale_host != nullptr ? scale_host[i] : 0.0f;
+    a.any_dev = a.any_dev || a.sc_dev[i] != nullptr;
+  }
+  if (!a.any_dev) {  // the defaults that sdpa_scale() would put in
+    for (int i = 0; i < 4; ++i)
+      if (a.sc_host[i] == 0.0f) a.sc_host[i] = 1.0f;
+    if (a.sc_host[5] == 0.0f) a.sc_host[5] = 1.0f / a.sc_host[3];
   }
   a.amax_s = amax_s;
   a.amax_o = amax_o;

@@ -624,3 +624,34 @@ def test_fp8_sdpa_fwd_measurement_pass_and_checks(dev):
     assert torch.allclose(out.float(), w @ v.float(), atol=3e-2) and abs(float(amax_s) - float(w.max())) < 1e-3
     with pytest.raises(RuntimeError, match="dropout is not implemented"):
         torch.ops.hpu.fp8_sdpa_fwd(q, k, v, None, 0.1, 0.2, True, "None", *NONE6, False, None, "left")
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("scale", [0.09, 0.0, -0.2])
+@pytest.mark.parametrize("L,S", [(1, 1), (63, 64), (64, 65), (65, 128), (127, 129), (130, 191), (192, 192)])
+def test_block_edges_and_signs_of_the_scale(oracle, dev, D, scale, L, S):
+    """Blocks that every row sees whole, blocks with a last key and blocks beyond it, causal or not; scales that are not
+    positive take the general form of the block."""
+    gen = torch.Generator().manual_seed(D + L + S)
+    q, k, v = make_qkv(gen, (2, L, D), (2, S, D), (2, S, D))
+    for causal in (False, True):
+        out = run_op(dev, q, k, v, causal=causal, scale=scale)[0]
+        ref, _, _ = oracle.torch_fp8_sdpa(q, k, v, scale=scale, is_causal=causal)
+        check_bf16(out, ref, f"{L} x {S}, D {D}, scale {scale}, causal {causal}")
+
+
+@pytest.mark.parametrize("pitch", [0, 8, 4, 1])
+def test_rows_of_the_output_at_any_pitch(oracle, pkg, dev, pitch):
+    """Output rows that take 16-byte, 8-byte and single stores: the same values, and nothing beside them."""
+    gen = torch.Generator().manual_seed(77)
+    B, L, S, D = 3, 70, 100, 128
+    q, k, v = make_qkv(gen, (B, L, D), (B, S, D), (B, S, D))
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    ldo = D + pitch
+    out = torch.full((B, L, ldo), 7.0, dtype=torch.bfloat16, device=dev)
+    desc = (ctypes.c_int64 * 29)(1, 1, B, 0, 0, L * D, 0, 0, S * D, 0, 0, S * D, 0, 0, 0, 0, 0, L * ldo, L, S, D, D, D, D, D, 0, ldo)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert pkg.capi().mi355q_fp8_sdpa_fwd(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), pkg.E4M3FN, None, 0, out.data_ptr(), pkg.BF16, desc,
+                                          1 / math.sqrt(D), 0, None, None, None, None, None, 0, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out[..., :D], run_op(dev, q, k, v)[0]) and bool((out[..., D:] == 7.0).all())
