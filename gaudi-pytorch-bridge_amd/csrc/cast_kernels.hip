@@ -1229,7 +1229,9 @@ inline bool scale_args_ok(const float* scale, int mode, int64_t outer, int64_t m
 // Few rows leave compute units idle, and a row's time is that of its slowest thread: one vector per thread, two where
 // 1024 threads do not suffice.  With many rows four vectors per thread keep more loads in flight and several
 // workgroups on a compute unit (three, five or seven: 3 to 10 % slower at 1024 x 14336 and 2048 x 5632; at 512 rows
-// the two forms cross).
+// the two forms cross).  Rows of more than 2048 vectors (the inner width of a 70B-class MLP) have four per thread at any
+// number of rows; as separate operations (aten's silu and mul, row maxima, a division, a cast, a reciprocal) 4 x 19904
+// took nine launches, and the whole MLP of 4 x 7488 / 19904 114 us against 98 with one kernel.
 constexpr int64_t kFewRows = 512;
 constexpr int kBulkVectors = 4;
 struct RowShape {
@@ -1237,10 +1239,10 @@ struct RowShape {
   unsigned threads;
 };
 inline RowShape row_shape(int64_t rows, int64_t vpr) {
-  const int vpt = rows < kFewRows ? (vpr <= kMaxRowThreads ? 1 : 2) : kBulkVectors;
+  const int vpt = rows < kFewRows && vpr <= 2 * kMaxRowThreads ? (vpr <= kMaxRowThreads ? 1 : 2) : kBulkVectors;
   return {vpt, (unsigned)(((vpr + vpt - 1) / vpt + 63) / 64 * 64)};
 }
-constexpr int64_t kMaxRowVectors = 2 * kMaxRowThreads;
+constexpr int64_t kMaxRowVectors = kBulkVectors * kMaxRowThreads, kMaxRaggedVectors = 2 * kMaxRowThreads;
 
 // Calls f(vectors per thread, saturate, threads); false: the row does not fit a workgroup.
 template <int FMT, typename F>
@@ -1429,7 +1431,7 @@ int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
   const uint8_t* xb = static_cast<const uint8_t*>(x);
   uint8_t* yb = static_cast<uint8_t*>(y);
   if (cols % epv != 0 || !aligned(x, 16) || !aligned(y, epv)) {
-    if (vpr > kMaxRowVectors || !aligned(x, epv == 8 ? 2 : 4)) return MI355Q_ERR_UNSUPPORTED;
+    if (vpr > kMaxRaggedVectors || !aligned(x, epv == 8 ? 2 : 4)) return MI355Q_ERR_UNSUPPORTED;
     const unsigned grid = (unsigned)rows, threads = (unsigned)(((vpr + 1) / 2 + 63) / 64 * 64);
     if (x_dtype == MI355Q_BF16) {
       if (fp8_fmt == MI355Q_E4M3FN) quantize_ragged_rows_kernel<true, MI355Q_E4M3FN><<<grid, threads, 0, st>>>(xb, yb, (int)cols, target, scale_out, scale_inv_out);

@@ -104,10 +104,11 @@ int mi355q_rowwise_amax(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * mi355q_cast_to_fp8 with MI355Q_SCALE_MID, which it replaces when a caller
  * quantises activations on the fly.  The reference has no such op
  * (fp8_ops.cpp:170-178: its amax is one scalar and the scale is computed by
- * the caller).  Rows of up to 2048 16-byte vectors (16384 bf16 / 8192 fp32
- * elements), x aligned to its elements; fastest where x is 16-byte aligned and
- * cols a multiple of 8 (bf16) or 4 (fp32).  Longer rows:
- * MI355Q_ERR_UNSUPPORTED, and the caller takes the three-step route.
+ * the caller).  Rows of up to 4096 16-byte vectors (32768 bf16 / 16384 fp32
+ * elements) where x is 16-byte aligned and cols a multiple of 8 (bf16) or 4
+ * (fp32), which is also the fastest; otherwise x aligned to its elements and up
+ * to 2048 vectors.  Longer rows: MI355Q_ERR_UNSUPPORTED, and the caller takes
+ * the three-step route.
  */
 int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
                          void* y, int fp8_fmt, float target,
@@ -128,7 +129,7 @@ int mi355q_quantize_rows(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * bit-identical to it; against a correctly rounded silu that value differs for
  * 18 inputs, all below -88, where the result (magnitude < 3.3e-37) is returned
  * as -0.
- * gate, up 16-byte aligned, cols and pitches multiples of 8, rows of up to 2048
+ * gate, up 16-byte aligned, cols and pitches multiples of 8, rows of up to 4096
  * 16-byte vectors; otherwise MI355Q_ERR_UNSUPPORTED.
  */
 int mi355q_silu_mul_quantize_rows(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up,

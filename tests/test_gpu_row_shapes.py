@@ -25,6 +25,25 @@ def test_rows_of_every_shape(oracle, dev, rows, cols, fmt):
     assert torch.equal(h.cpu().view(torch.uint8), h_ref.view(torch.uint8)) and torch.equal(h_inv.cpu(), h_inv_ref)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 16392), (511, 16448), (600, 20808), (3, 32768), (2, 32776)])  # the last: three steps again
+def test_rows_of_more_than_two_vectors_per_thread(oracle, dev, rows, cols):
+    g = torch.Generator().manual_seed(rows + cols)
+    gate = (torch.randn(rows, cols, generator=g) * 3).bfloat16()
+    own = torch.ops.mi355q
+    for x in (gate, gate[:, : cols // 2].float()):
+        y, inv = own.quantize_rows(x.to(dev), E4)
+        y_ref, inv_ref = oracle.quantize_rows(x, E4)
+        assert torch.equal(y.cpu().view(torch.uint8), y_ref.view(torch.uint8)) and torch.equal(inv.cpu(), inv_ref)
+    if cols > 32768:
+        return  # aten's silu there
+    up = torch.randn(rows, cols, generator=g).bfloat16()
+    up[-1, 5] = float("inf")  # the row's scale is 0 and its codes as the oracle has them
+    h, h_inv = own.silu_mul_quantize_rows(gate.to(dev), up.to(dev), E5)
+    h_ref, h_inv_ref = oracle.quantize_rows(oracle.c_silu_mul_bf16(gate, up), E5)
+    assert_fp8_equal(h, h_ref, E5, f"{rows} x {cols}")
+    assert torch.equal(h_inv.cpu(), h_inv_ref)
+
+
 def test_target_past_the_largest_code_saturates(pkg, dev):
     lib = pkg.capi()
     x = torch.tensor([[1.0, -2.0, 3.0, 4.0, -4.0, 0.5, 0.0, 1.5]]).bfloat16().to(dev)
