@@ -59,6 +59,7 @@ void launch_by_kind(const GemmArgs& g, const SplitArgs& split, int64_t batch, hi
     if (split.kind == GemmKind::kRing16) return launch_ring<16, AK, BK_, FA, FB>(g, split, batch, st);
     if (split.kind == GemmKind::kRing32) return launch_ring<32, AK, BK_, FA, FB>(g, split, batch, st);
     if (split.kind == GemmKind::kRing64) return launch_ring<64, AK, BK_, FA, FB>(g, split, batch, st);
+    if (split.kind == GemmKind::kRing192) return launch_ring<192, AK, BK_, FA, FB>(g, split, batch, st);
   }
   if (split.kind == GemmKind::kRing128) return launch_ring<128, AK, BK_, FA, FB>(g, split, batch, st);
   if (split.kind == GemmKind::kRing256) return launch_ring<256, AK, BK_, FA, FB>(g, split, batch, st);

@@ -7,14 +7,16 @@
 //  * four waves that only load and four that only multiply, one of each per SIMD, meeting at one barrier per stage: the
 //    loading waves' stalls hold up no MFMA, and the multiplying waves' loop is MFMAs, fragment reads and one addition per
 //    address register;
-//  * as many stages as the LDS holds (3 at 256 rows, 4, 6, 7, 7 below), counted waits, and load addresses without arithmetic;
+//  * as many stages as the LDS holds (3 at 256 and 192 rows, 4, 6, 7, 7 below), counted waits, and load addresses without arithmetic;
 //  * low tiles where they fill the chip better, and K in parts only then (gemm_api.hip has the figures that choose);
 //  * plain loads for a B of at most 64 MiB: the nontemporal hint keeps a matrix out of the 256 MB memory-side cache, from
 //    which a second call would read it (64 x 8192 x 4096 warm: 40 us with the hint, 23 without; cold 0 to 10 % for it).
 // Measured against the strip, 128 x 128 and 256 x 128 kernels it replaces (us, weights [K, N] but where nk, three sets of them in
 // turn): 256 x 8192 x 28672 88.8 -> 68.3 (nk 93.3 -> 66.5; the load stream alone takes 64), 1000 x 3008 x 5000 29.3 -> 24.3, 669 x 8704 x
 // 7808 nk 54.8 -> 44.7, 64 x 14336 x 4096 25.0 -> 17.5, 83 x 6640 x 864 23.9 -> 11.0, 7 x 10816 x 704 nk 16.1 -> 9.7, 1 x 4096 x 4096
-// 12.2 -> 7.8; over 480 products of 1 to 4096 rows 26 % less time in the geometric mean warm, 23 % cold.
+// 12.2 -> 7.8.  192 rows, for A [M, K] (a K-major tile's LDS rows are 128 bytes at any height, an MN-major one's would be no power
+// of two): 24 stages of 240 tiles against 160 of 256 rows, 1000 x 3008 x 5000 32.3 -> 30.6; 267 x 4736 x 28544 on tiles of 192 rows against
+// 256 x 256 60.4 -> 51.9, 268 x 5296 x 13328 40.8 -> 34.4; over 480 products of 1 to 4096 rows 26 % less time in the geometric mean warm, 23 % cold.
 #pragma once
 #include "gemm_split.h"
 #include "gemm_tile16.h"

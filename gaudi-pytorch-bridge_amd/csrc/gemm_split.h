@@ -22,7 +22,7 @@ constexpr int kMaxTickets = (int)(kTicketBytes / (kTicketStride * 4));
 
 // The kernel of a product: 256 x 256 tiles (gemm_tile16.h, gemm_tile.h), rows of a ring tile (gemm_ring.h), or B streamed into
 // registers (gemm_stream.h).
-enum class GemmKind { kTile256, kRing16, kRing32, kRing64, kRing128, kRing256, kStream };
+enum class GemmKind { kTile256, kRing16, kRing32, kRing64, kRing128, kRing192, kRing256, kStream };
 
 struct SplitArgs {
   int parts;           // workgroups that share a strip or tile of C, one part of K each
