@@ -40,6 +40,8 @@
 // MFMAs: keeping each role's loop short is what the split is for.  The roles meet at one
 // barrier per K stage of 128.  At the end of a group of K the group's scales multiply the
 // partial sums into the totals, in fp32.
+#include <algorithm>
+
 #include "gemm_tile.h"
 
 namespace mi355q {
@@ -496,9 +498,9 @@ __global__ __launch_bounds__(kW4Threads) void w4a8_gemm_kernel(W4Args a) {
 // at about 3.2 TB/s, whole lines at 4.3), and K is cut into `ksplit` parts walked by as many
 // workgroups, so that a launch fills the chip whatever N is.  The parts of a strip meet through
 // memory: every workgroup stores its partial sums (already scaled by the groups' scales, fp32, in
-// register order), and the one that draws the last ticket of the strip adds them up in the order
-// of the parts, whoever came last, and runs the epilogue.  The last one also returns the ticket
-// counter to zero for the next launch.
+// register order).  Up to 32 rows the one that draws the last ticket of the strip adds them up in the order
+// of the parts, whoever came last, and runs the epilogue; it also returns the ticket
+// counter to zero for the next launch.  Above that a second launch does (w4_finish_kernel).
 //
 // Roles and the stage pipeline are those of the kernel above, with eight consumer waves of 32
 // columns and four producers.  The 16-byte slots of a packed row in LDS are XORed with
@@ -554,6 +556,36 @@ template <int FMT_A>
 __device__ __forceinline__ f32x4 w4_mfma16(const u32x4& plane, const i32x8& fa, const f32x4& c, int e) {
   const i32x8 b = {(int)plane[0], (int)plane[1], (int)plane[2], (int)plane[3], 0, 0, 0, 0};
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, fa, c, 4, mfma_code<FMT_A>(), 0, e, 0, 127);
+}
+
+// The epilogue of four columns of a row: N is a multiple of 32, so they are inside or outside together.
+__device__ __forceinline__ void w4_store4(const GemmArgs& g, const ScalarScales& scalars, int m, int n, const f32x4& sums) {
+  if (m >= g.M || n >= g.N) return;
+  const int es = g.out_bf16 ? 2 : 4;
+  const float sa = g.sa_mode == MI355Q_GS_PER_ROW ? g.sa[m] : scalars.sa;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR ? load_out_as_f32(g.bias, n + e, g.out_bf16) : 0.0f;
+    v[e] = __fmul_rn(sums[e], sa) + bias;  // rounded as the other epilogues round
+  }
+  uint8_t* cp = g.C + ((int64_t)m * g.ldc + n) * es;
+  const bool vec_ok = (reinterpret_cast<uintptr_t>(cp) % (4 * es)) == 0;
+  if (g.out_bf16) {
+    if (vec_ok) {
+      *reinterpret_cast<u32x2*>(cp) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) reinterpret_cast<uint16_t*>(cp)[e] = (uint16_t)(pack_bf16x2(v[e], v[e]) & 0xffffu);
+    }
+  } else {
+    if (vec_ok) {
+      *reinterpret_cast<f32x4*>(cp) = f32x4{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) reinterpret_cast<float*>(cp)[e] = v[e];
+    }
+  }
 }
 
 // ROWS: 16 (one row tile; a product is folded one stage late), or 32, 64, 128 (ROWS / 16 row tiles; row blocks of
@@ -962,7 +994,19 @@ __global__ __launch_bounds__(kW4WideThreads) void w4a8_wide_kernel(W4Args a) {
   }
   __syncthreads();  // every load has landed and every stage is consumed: the ring is idle
 
-  if (a.ksplit > 1) {
+  if constexpr (ROWS >= 64) {
+    if (a.ksplit > 1) {  // w4_finish_kernel adds the parts up
+      const int strips = (int)gridDim.x / a.ksplit;
+      f32x4* to = reinterpret_cast<f32x4*>(a.partials) +
+                  ((int64_t)(part * strips * (int)gridDim.y + (int)blockIdx.y * strips + strip) * kConsumers + wq) * 2 * RT * 64 + lane;
+      if (!producer) {
+#pragma unroll
+        for (int j = 0; j < 2 * RT; ++j)
+          if (16 * (j >> 1) < g.M) to[j * 64] = f32x4{total[4 * j], total[4 * j + 1], total[4 * j + 2], total[4 * j + 3]};
+      }
+      return;
+    }
+  } else if (a.ksplit > 1) {
     // Partial sums in register order: 64-bit word number h 64 + lane (h < NV / 2) of consumer wave wq.  They are
     // written and read with device-scope atomic accesses, which go past the caches of this XCD to where the other
     // XCDs see them: no cache has to be written back or invalidated as a whole, which a fence would do (and
@@ -1016,43 +1060,47 @@ __global__ __launch_bounds__(kW4WideThreads) void w4a8_wide_kernel(W4Args a) {
     }
   }
   if (producer) return;
-  {
-    // C[m, n .. n + 3] for this lane's rows (one per row tile) and its two sets of four columns
-    const int gk = lane >> 4;
-    const ScalarScales scalars = load_scalar_scales(g);
-    const int es = g.out_bf16 ? 2 : 4;
+  // C[m, n .. n + 3] for this lane's rows (one per row tile) and its two sets of four columns
+  const int gk = lane >> 4;
+  const ScalarScales scalars = load_scalar_scales(g);
 #pragma unroll
-    for (int j = 0; j < 2 * RT; ++j) {
-      const int t = j & 1, m = 16 * (j >> 1) + (lane & 15);
-      if (m >= g.M) continue;
-      const float sa = g.sa_mode == MI355Q_GS_PER_ROW ? g.sa[m] : scalars.sa;
-      const int n = n0 + wq * 32 + 16 * t + 4 * gk;
-      if (n >= g.N) continue;  // N is a multiple of 32: the four columns are inside or outside together
-      float v[4];
+  for (int j = 0; j < 2 * RT; ++j)
+    w4_store4(g, scalars, 16 * (j >> 1) + (lane & 15), n0 + wq * 32 + 16 * (j & 1) + 4 * gk, f32x4{total[4 * j], total[4 * j + 1], total[4 * j + 2], total[4 * j + 3]});
+}
+
+// The parts of K of tiles of 64 or 128 rows, added up in their order, and the epilogue: a wave per row tile and 32 columns.
+// Such a tile's sums are 64 or 128 KiB a part, which one workgroup takes in at 50 KB/us however they are ordered (added up by
+// the workgroup that came last, or in pairs): 20 us for eight parts of 128 rows.  As a launch of its own all compute units
+// read them: 100 x 9472 x 1664 41 -> 22 us, 173 x 8192 x 7808 45 -> 35, 48 x 8192 x 7808 28 -> 24; two fp8 planes, 490 x 4096 x 3648
+// 42 -> 34.
+template <int RT>
+__global__ __launch_bounds__(256) void w4_finish_kernel(W4Args a, int strips) {
+  const int lane = lane_id_here();
+  const int unit = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // (strip of a row block, consumer wave, row tile)
+  const int i = unit % RT, wq = unit / RT % kW4WideConsumers, strip_rb = unit / RT / kW4WideConsumers;
+  const int strip = strip_rb % strips, m_tile = strip_rb / strips * (16 * RT) + 16 * i;
+  if (m_tile >= a.g.M) return;
+  const int tiles = (int)gridDim.x / (2 * RT);  // strips of all row blocks
+  const f32x4* from = reinterpret_cast<const f32x4*>(a.partials) + ((int64_t)(strip_rb * kW4WideConsumers + wq) * 2 * RT + 2 * i) * 64 + lane;
+  const int64_t part_stride = (int64_t)tiles * kW4WideConsumers * 2 * RT * 64;
+  f32x4 total[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  constexpr int kAhead = 4;  // parts whose loads are in flight together
+  for (int p = 0; p < a.ksplit; p += kAhead) {
+    f32x4 v[kAhead][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR ? load_out_as_f32(g.bias, n + e, g.out_bf16) : 0.0f;
-        v[e] = __fmul_rn(total[4 * j + e], sa) + bias;  // rounded as the other epilogues round
-      }
-      uint8_t* cp = g.C + ((int64_t)m * g.ldc + n) * es;
-      const bool vec_ok = (reinterpret_cast<uintptr_t>(cp) % (4 * es)) == 0;
-      if (g.out_bf16) {
-        if (vec_ok) {
-          *reinterpret_cast<u32x2*>(cp) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        } else {
+    for (int q = 0; q < kAhead; ++q)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) reinterpret_cast<uint16_t*>(cp)[e] = (uint16_t)(pack_bf16x2(v[e], v[e]) & 0xffffu);
-        }
-      } else {
-        if (vec_ok) {
-          *reinterpret_cast<f32x4*>(cp) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
+      for (int t = 0; t < 2; ++t) v[q][t] = from[(p + q < a.ksplit ? p + q : p) * part_stride + 64 * t];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) reinterpret_cast<float*>(cp)[e] = v[e];
-        }
-      }
-    }
+    for (int q = 0; q < kAhead; ++q)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[t][e] += p + q < a.ksplit ? v[q][t][e] : 0.0f;
   }
+  const ScalarScales scalars = load_scalar_scales(a.g);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) w4_store4(a.g, scalars, m_tile + (lane & 15), strip * kW4WideBN + wq * 32 + 16 * t + 4 * (lane >> 4), total[t]);
 }
 
 // How the wide kernel takes a problem: rows per workgroup (16 rows sit in a 32-row tile of LDS), row
@@ -1068,20 +1116,39 @@ struct W4WidePlan {
     return parts < 2 ? 0 : ticket_bytes() + (size_t)parts * strips * row_blocks * w4_wide_partial_bytes(tile_rows());
   }
 };
-inline W4WidePlan w4a8_wide_plan(int64_t M, int64_t N, int64_t K, int64_t group, int scale_f32) {
+// What a part of K costs, in microseconds: a stage of a tile, the parts' meeting, what each part adds to it and what a full chip
+// does.  From products of 7 to 490 rows, K from 1408 to 12288 and N from 1312 to 28672, timed in one to 24 parts: 7 x 1408 x 1664 with
+// two planes takes 14.9 us whole, 12.2 in four parts and 13.6 in eleven, 48 rows 20.4, 14.0 and 13.9.  fp8 activations: parts of
+// eight stages at least (a part more of short products gained a microsecond at most up to 32 rows).
+struct W4Cost {
+  double stage, meet, part, crowd;
+};
+inline W4WidePlan w4_wide_plan(int64_t M, int64_t N, int64_t K, int64_t group, int scale_f32, bool a16) {
   W4WidePlan p{0, 0, 0, 0};
   if (group != kBK || scale_f32 || K <= 0 || M <= 0 || N <= 0) return p;
   p.rows = M <= 16 ? 16 : (M <= 32 ? 32 : (M <= 64 ? 64 : 128));
   p.row_blocks = (int)((M + p.tile_rows() - 1) / p.tile_rows());
   p.strips = (int)((N + kW4WideBN - 1) / kW4WideBN);
   const int64_t kt = (K + kBK - 1) / kBK, groups = (int64_t)p.strips * p.row_blocks;
-  int64_t parts = 256 / groups;
-  if (parts > kt / 8) parts = kt / 8;
-  // too few workgroups for the chip even so: the 128-column strips have twice as many
-  if (parts < 2) parts = groups >= 100 ? 1 : 0;
-  if (p.row_blocks > 65535) parts = 0;
-  if (parts >= 2 && (size_t)groups * 4 > W4WidePlan::ticket_bytes()) parts = 1;  // (cannot happen: 256 / groups >= 2)
-  p.parts = (int)parts;
+  // at most one workgroup per compute unit
+  const int64_t most = std::min<int64_t>(256 / groups, kt / (a16 ? 2 : 8));
+  const W4Cost c = p.rows == 16   ? W4Cost{0.57, 1.0, 0.40, 0.5}
+                   : p.rows == 32 ? W4Cost{0.63, 1.0, 0.50, 2.0}
+                   : p.rows == 64 ? W4Cost{a16 ? 0.98 : 0.70, 1.0, 0.25, 6.0}
+                                  : W4Cost{a16 ? 1.65 : 1.15, 1.0, 0.25, 9.0};
+  double best = (double)kt * c.stage;
+  p.parts = 1;
+  for (int64_t n = 2; n <= most; ++n) {
+    const double us = (double)((kt + n - 1) / n) * c.stage + c.meet + c.part * (double)n + c.crowd * (double)(groups * n) / 256.0;
+    if (us >= best) continue;
+    best = us;
+    p.parts = (int)n;
+  }
+  // too few workgroups for the chip even so: the 128-column strips have twice as many (and, where there are more of them than the
+  // chip holds, half the rounding error: 100 x 1408 x 17280 took 23 us here against 30, with 2.9e-5 against 1.4e-5 in fp32)
+  if (p.parts < 2 && groups < 100) p.parts = 0;
+  if (p.row_blocks > 65535) p.parts = 0;
+  if (p.parts >= 2 && (size_t)groups * 4 > W4WidePlan::ticket_bytes()) p.parts = 1;  // (cannot happen: 256 / groups >= 2)
   return p;
 }
 
@@ -1094,58 +1161,30 @@ void w4a8_launch(const W4Args& a, hipStream_t st) {
   else w4a8_gemm_kernel<BM, FMT_A, true, 2><<<grid, kW4Threads, 0, st>>>(a);
 }
 
-template <int FMT_A>
-void w4a8_launch_by_m(const W4Args& a, hipStream_t st) {
-  if (a.ksplit > 0) {
-    const bool z = a.zp != nullptr || a.is_signed;
-    const unsigned strips = (unsigned)((a.g.N + kW4WideBN - 1) / kW4WideBN);
-    if (a.g.M <= 16) {
-      const dim3 grid(strips * (unsigned)a.ksplit);
-      if (z) w4a8_wide_kernel<FMT_A, true, 16><<<grid, kW4WideThreads, 0, st>>>(a);
-      else w4a8_wide_kernel<FMT_A, false, 16><<<grid, kW4WideThreads, 0, st>>>(a);
-    } else if (a.g.M <= 32) {
-      const dim3 grid(strips * (unsigned)a.ksplit);
-      if (z) w4a8_wide_kernel<FMT_A, true, 32><<<grid, kW4WideThreads, 0, st>>>(a);
-      else w4a8_wide_kernel<FMT_A, false, 32><<<grid, kW4WideThreads, 0, st>>>(a);
-    } else if (a.g.M <= 64) {
-      const dim3 grid(strips * (unsigned)a.ksplit);
-      if (z) w4a8_wide_kernel<FMT_A, true, 64><<<grid, kW4WideThreads, 0, st>>>(a);
-      else w4a8_wide_kernel<FMT_A, false, 64><<<grid, kW4WideThreads, 0, st>>>(a);
-    } else {
-      const dim3 grid(strips * (unsigned)a.ksplit, (unsigned)((a.g.M + 127) / 128));
-      if (z) w4a8_wide_kernel<FMT_A, true, 128><<<grid, kW4WideThreads, 0, st>>>(a);
-      else w4a8_wide_kernel<FMT_A, false, 128><<<grid, kW4WideThreads, 0, st>>>(a);
-    }
-  } else if (a.g.M <= 32) {
-    w4a8_launch<32, FMT_A>(a, st);
-  } else {
-    w4a8_launch<64, FMT_A>(a, st);
+template <int FMT_A, bool A16, int ROWS>
+void w4_wide_launch_rows(const W4Args& a, hipStream_t st) {
+  const unsigned strips = (unsigned)((a.g.N + kW4WideBN - 1) / kW4WideBN), blocks = ROWS < 128 ? 1u : (unsigned)((a.g.M + 127) / 128);
+  const dim3 grid(strips * (unsigned)a.ksplit, blocks);
+  if (a.zp != nullptr || a.is_signed) w4a8_wide_kernel<FMT_A, true, ROWS, A16><<<grid, kW4WideThreads, 0, st>>>(a);
+  else w4a8_wide_kernel<FMT_A, false, ROWS, A16><<<grid, kW4WideThreads, 0, st>>>(a);
+  if constexpr (ROWS >= 64) {
+    if (a.ksplit > 1) w4_finish_kernel<ROWS / 16><<<strips * blocks * (2 * ROWS / 16), 256, 0, st>>>(a, (int)strips);
   }
 }
+// A16: on two fp8 planes of 16-bit activations.
+template <int FMT_A, bool A16>
+void w4_wide_launch(const W4Args& a, hipStream_t st) {
+  if (a.g.M <= 16) w4_wide_launch_rows<FMT_A, A16, 16>(a, st);
+  else if (a.g.M <= 32) w4_wide_launch_rows<FMT_A, A16, 32>(a, st);
+  else if (a.g.M <= 64) w4_wide_launch_rows<FMT_A, A16, 64>(a, st);
+  else w4_wide_launch_rows<FMT_A, A16, 128>(a, st);
+}
 
-// The wide kernel on two fp8 planes of 16-bit activations (always this kernel: K in one part where the plan would
-// rather use the 128-column strips, which have no two-plane form).
-inline void w4a16_launch(const W4Args& a, hipStream_t st) {
-  const bool z = a.zp != nullptr || a.is_signed;
-  const unsigned strips = (unsigned)((a.g.N + kW4WideBN - 1) / kW4WideBN);
-  constexpr int F = MI355Q_E4M3FN;
-  if (a.g.M <= 16) {
-    const dim3 grid(strips * (unsigned)a.ksplit);
-    if (z) w4a8_wide_kernel<F, true, 16, true><<<grid, kW4WideThreads, 0, st>>>(a);
-    else w4a8_wide_kernel<F, false, 16, true><<<grid, kW4WideThreads, 0, st>>>(a);
-  } else if (a.g.M <= 32) {
-    const dim3 grid(strips * (unsigned)a.ksplit);
-    if (z) w4a8_wide_kernel<F, true, 32, true><<<grid, kW4WideThreads, 0, st>>>(a);
-    else w4a8_wide_kernel<F, false, 32, true><<<grid, kW4WideThreads, 0, st>>>(a);
-  } else if (a.g.M <= 64) {
-    const dim3 grid(strips * (unsigned)a.ksplit);
-    if (z) w4a8_wide_kernel<F, true, 64, true><<<grid, kW4WideThreads, 0, st>>>(a);
-    else w4a8_wide_kernel<F, false, 64, true><<<grid, kW4WideThreads, 0, st>>>(a);
-  } else {
-    const dim3 grid(strips * (unsigned)a.ksplit, (unsigned)((a.g.M + 127) / 128));
-    if (z) w4a8_wide_kernel<F, true, 128, true><<<grid, kW4WideThreads, 0, st>>>(a);
-    else w4a8_wide_kernel<F, false, 128, true><<<grid, kW4WideThreads, 0, st>>>(a);
-  }
+template <int FMT_A>
+void w4a8_launch_by_m(const W4Args& a, hipStream_t st) {
+  if (a.ksplit > 0) w4_wide_launch<FMT_A, false>(a, st);
+  else if (a.g.M <= 32) w4a8_launch<32, FMT_A>(a, st);
+  else w4a8_launch<64, FMT_A>(a, st);
 }
 
 // Workspace of mi355q_w4a16_gemm: [arrival counters and partial sums of the K split, as for W4A8][plane 1][plane 2]
@@ -1157,7 +1196,7 @@ struct W4A16Layout {
 inline W4A16Layout w4a16_layout(int64_t M, int64_t N, int64_t K, int64_t group, int scale_f32) {
   const auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   W4A16Layout l{};
-  const W4WidePlan plan = w4a8_wide_plan(M, N, K, group, scale_f32);
+  const W4WidePlan plan = w4_wide_plan(M, N, K, group, scale_f32, true);
   // the arrival counters' KiB is set aside whether this shape splits K or not: a buffer that serves calls of several
   // shapes must not find the planes of one call where the next one keeps its counters
   l.split_bytes = plan.parts >= 2 ? plan.workspace_bytes() : W4WidePlan::ticket_bytes();
@@ -1227,19 +1266,20 @@ extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const 
   a.scale_f32 = 0;
   a.is_signed = is_signed != 0;
   a.stages_per_group = 1;
-  const W4WidePlan plan = w4a8_wide_plan(M, N, K, group, 0);
+  const W4WidePlan plan = w4_wide_plan(M, N, K, group, 0, true);
   a.ksplit = 1;
   if (plan.parts >= 2 && split_k) {
     a.ksplit = plan.parts;
     a.tickets = reinterpret_cast<uint32_t*>(ws);
     a.partials = reinterpret_cast<float*>(ws + plan.ticket_bytes());
   }
-  w4a16_launch(a, st);
+  // (always the wide kernel: K in one part where the plan would rather use the 128-column strips, which have no two-plane form)
+  w4_wide_launch<MI355Q_E4M3FN, true>(a, st);
   return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;
 }
 
 extern "C" size_t mi355q_w4a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int scale_dtype) {
-  return w4a8_wide_plan(M, N, K, group, scale_dtype == MI355Q_F32).workspace_bytes();
+  return w4_wide_plan(M, N, K, group, scale_dtype == MI355Q_F32, false).workspace_bytes();
 }
 
 extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int32_t* packed, int64_t ld_packed,
@@ -1287,7 +1327,7 @@ extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int
   a.is_signed = is_signed != 0;
   a.stages_per_group = (int)(group / kBK);
   // the wide kernel where it applies: K in parts if the caller brought the room for the partial sums
-  const W4WidePlan plan = w4a8_wide_plan(M, N, K, group, a.scale_f32);
+  const W4WidePlan plan = w4_wide_plan(M, N, K, group, a.scale_f32, false);
   if (plan.parts >= 2 && workspace != nullptr) {
     if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;
     a.ksplit = plan.parts;

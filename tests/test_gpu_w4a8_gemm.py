@@ -269,3 +269,49 @@ def test_exact_at_the_benchmark_shape(oracle, dev, M):
     assert torch.equal(out.cpu().double(), expect)
     out2 = torch.ops.mi355q.w4a8_gemm(a.to(E4).to(dev), pk.to(dev), s.to(dev), pz.to(dev), False, torch.float32, sa.to(dev), None)
     assert torch.equal(out2, out)
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 2048, 288), (64, 9472, 1664), (65, 4096, 160), (128, 2048, 256), (145, 4224, 1056), (100, 1408, 17280)])
+def test_parts_of_high_tiles_are_exact(oracle, dev, M, K, N):
+    """Tiles of 64 and 128 rows whose parts of K are added up by a second launch: first and last rows of a tile, a second row
+    block, a last strip of 32 columns, with one plane and with two (which takes more parts), and rows that start at odd elements."""
+    gen = torch.Generator().manual_seed(M + K + N)
+    q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
+    a = torch.randint(-4, 5, (M, K), generator=gen).float()
+    sa = torch.exp2(torch.randint(-2, 3, (M, 1), generator=gen).float())
+    bias = torch.randint(-8, 9, (N,), generator=gen).float()
+    w = (q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0)
+    p = a.double() @ w
+    assert p.abs().max() < 2 ** 20
+    own, d = torch.ops.mi355q, lambda t: t.to(dev)  # noqa: E731
+    for out in (torch.float32, torch.bfloat16):
+        for _ in range(2):
+            y = own.w4a8_gemm(d(a.to(E4)), d(pk), d(s), d(pz), False, out, d(sa), d(bias.to(out)))
+            assert torch.equal(y.cpu(), (p * sa.double() + bias.double()).float().to(out))
+            y = own.w4a16_gemm(d(a.bfloat16()), d(pk), d(s), d(pz), False, out, d(bias.to(out)))
+            assert torch.equal(y.cpu(), (p + bias.double()).float().to(out))
+
+
+def test_two_threads_on_a_stream_keep_their_parts_apart(oracle, dev):
+    """Calls of two launches each from two threads on one stream, which share its workspace."""
+    import threading
+    M, K, N = 100, 4096, 512
+    jobs = []
+    for seed in (1, 2):
+        gen = torch.Generator().manual_seed(seed)
+        q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
+        a = torch.randint(-4, 5, (M, K), generator=gen).float()
+        w = (q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0)
+        jobs.append((a.to(E4).to(dev), pk.to(dev), s.to(dev), pz.to(dev), (a.double() @ w).float().to(dev)))
+    stream, wrong = torch.cuda.current_stream(), []
+
+    def work(a, pk, s, pz, ref):
+        with torch.cuda.stream(stream):
+            for op, x in ((torch.ops.mi355q.w4a8_gemm, a), (torch.ops.mi355q.w4a16_gemm, a.bfloat16())):
+                ys = [op(x, pk, s, pz, False, torch.float32) for _ in range(60)]
+                wrong.extend(1 for y in ys if not torch.equal(y, ref))
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
