@@ -99,6 +99,13 @@ constexpr RingCost kRingCosts[] = {
     {GemmKind::kRing256, 256, 6.59, 0.50, 0.19, -1.43, 5.03, 8.08, 1.19},
 };
 
+constexpr int kMostParts = 16;
+// log2 of a number of parts.  (The choice is made twice on a call; with log2 and 64-bit divisions in the loop over the parts it
+// took 1.1 us for 100 x 16384 x 256, without 0.33.)
+constexpr double kLog2[kMostParts + 1] = {0.0, 0.0, 1.0, 1.5849625007211562, 2.0, 2.321928094887362, 2.584962500721156, 2.807354922057604, 3.0,
+                                          3.169925001442312, 3.321928094887362, 3.4594316186372973, 3.584962500721156, 3.700439718141092,
+                                          3.807354922057604, 3.9068905956085187, 4.0};
+
 // The kernel and the cut that are expected to take least.
 //  * Tiles of fewer than 128 rows exist for A [M, K]; up to 16 rows take the tile of 16, more of them none that is twice as high
 //    as the product.
@@ -138,21 +145,25 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256) * batch;
     best_us = (double)((tiles + cus - 1) / cus) * (double)stages * 1.42 + 6.0;
   }
+  const double per_cu = 1.0 / (double)cus;
   for (const RingCost& c : kRingCosts) {
     if (a_kmajor ? (c.rows == 16) != (M <= 16) || (c.rows > 32 && c.rows >= 2 * M) : c.rows != 128 && c.rows != 256) continue;
-    const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + kRingBN - 1) / kRingBN);
+    const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + kRingBN - 1) / kRingBN), wgs = tiles * batch, rounds = (wgs + cus - 1) / cus;
+    double fill = (double)std::min(wgs, cus) * per_cu;
+    double us = c.fixed + (double)stages * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round);
     const bool in_parts = may_split && (M > 128 || K >= (a_kmajor ? 1792 : 2304));
-    for (int64_t parts = 1; parts == 1 || (in_parts && parts <= 16 && parts * tiles * batch <= cus && 2 * parts <= stages); ++parts) {
-      const int64_t wgs = parts * tiles * batch, rounds = (wgs + cus - 1) / cus;
-      const double fill = (double)std::min(wgs, cus) / (double)cus;
-      double us = c.fixed + (double)((stages + parts - 1) / parts) * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round);
-      if (parts > 1) us += c.meet + c.level * std::log2((double)parts) + c.crowd * fill;
+    const int most = in_parts && stages >= 4 && rounds == 1 ? (int)std::min<int64_t>({cus / wgs, stages / 2, kMostParts}) : 1;
+    for (int parts = 1; parts <= most; ++parts) {
+      if (parts > 1) {
+        fill = (double)(parts * (int)wgs) * per_cu;
+        us = c.fixed + (double)(((unsigned)stages + (unsigned)parts - 1) / (unsigned)parts) * (c.stage + c.busy * fill) + c.meet + c.level * kLog2[parts] + c.crowd * fill;
+      }
       if (us >= best_us) continue;
       best_us = us;
       best.kind = c.kind;
       best.nb = kRingBN;
       best.strips = (int)tiles;
-      best.parts = (int)parts;
+      best.parts = parts;
       best.tile_rows = c.rows;
     }
   }
