@@ -558,17 +558,31 @@ __device__ __forceinline__ f32x4 w4_mfma16(const u32x4& plane, const i32x8& fa, 
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, fa, c, 4, mfma_code<FMT_A>(), 0, e, 0, 127);
 }
 
+// What the epilogue multiplies a row by and adds to its columns.  Loaded for all of a lane's results before the first is stored: a
+// load behind a store waits for a trip to the L2 of its own, and a lane of a 128-row tile has
+// sixteen (uint4, us, before and after: 512 x 4096 x 16384 54.5 -> 51.8, two planes 74.5 -> 70.9; 60 x 4096 x 40960 36.3 -> 34.7,
+// 41.7 -> 40.5; 133 x 10112 x 21696 two planes 140.5 -> 135.5; parts added up by a second launch +- 0).  (Rows and columns past the
+// edge read the last ones; they are not stored.)
+__device__ __forceinline__ float w4_row_scale(const GemmArgs& g, const ScalarScales& scalars, int m) {
+  return g.sa_mode == MI355Q_GS_PER_ROW ? g.sa[m < g.M ? m : g.M - 1] : scalars.sa;
+}
+__device__ __forceinline__ f32x4 w4_bias4(const GemmArgs& g, int n) {
+  f32x4 b = {0.f, 0.f, 0.f, 0.f};
+  if (g.bias_mode == MI355Q_BIAS_ROW_VECTOR) {
+    const int from = n < g.N ? n : g.N - 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = load_out_as_f32(g.bias, from + e, g.out_bf16);
+  }
+  return b;
+}
+
 // The epilogue of four columns of a row: N is a multiple of 32, so they are inside or outside together.
-__device__ __forceinline__ void w4_store4(const GemmArgs& g, const ScalarScales& scalars, int m, int n, const f32x4& sums) {
+__device__ __forceinline__ void w4_store4(const GemmArgs& g, int m, int n, const f32x4& sums, float sa, const f32x4& bias) {
   if (m >= g.M || n >= g.N) return;
   const int es = g.out_bf16 ? 2 : 4;
-  const float sa = g.sa_mode == MI355Q_GS_PER_ROW ? g.sa[m] : scalars.sa;
   float v[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR ? load_out_as_f32(g.bias, n + e, g.out_bf16) : 0.0f;
-    v[e] = __fmul_rn(sums[e], sa) + bias;  // rounded as the other epilogues round
-  }
+  for (int e = 0; e < 4; ++e) v[e] = __fmul_rn(sums[e], sa) + bias[e];  // rounded as the other epilogues round
   uint8_t* cp = g.C + ((int64_t)m * g.ldc + n) * es;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(cp) % (4 * es)) == 0;
   if (g.out_bf16) {
@@ -1063,9 +1077,16 @@ __global__ __launch_bounds__(kW4WideThreads) void w4a8_wide_kernel(W4Args a) {
   // C[m, n .. n + 3] for this lane's rows (one per row tile) and its two sets of four columns
   const int gk = lane >> 4;
   const ScalarScales scalars = load_scalar_scales(g);
+  float sa[RT];
+  f32x4 bias[2];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) sa[i] = w4_row_scale(g, scalars, 16 * i + (lane & 15));
+#pragma unroll
+  for (int t = 0; t < 2; ++t) bias[t] = w4_bias4(g, n0 + wq * 32 + 16 * t + 4 * gk);
 #pragma unroll
   for (int j = 0; j < 2 * RT; ++j)
-    w4_store4(g, scalars, 16 * (j >> 1) + (lane & 15), n0 + wq * 32 + 16 * (j & 1) + 4 * gk, f32x4{total[4 * j], total[4 * j + 1], total[4 * j + 2], total[4 * j + 3]});
+    w4_store4(g, 16 * (j >> 1) + (lane & 15), n0 + wq * 32 + 16 * (j & 1) + 4 * gk, f32x4{total[4 * j], total[4 * j + 1], total[4 * j + 2], total[4 * j + 3]},
+              sa[j >> 1], bias[j & 1]);
 }
 
 // The parts of K of tiles of 64 or 128 rows, added up in their order, and the epilogue: a wave per row tile and 32 columns.
@@ -1083,6 +1104,9 @@ __global__ __launch_bounds__(256) void w4_finish_kernel(W4Args a, int strips) {
   const int tiles = (int)gridDim.x / (2 * RT);  // strips of all row blocks
   const f32x4* from = reinterpret_cast<const f32x4*>(a.partials) + ((int64_t)(strip_rb * kW4WideConsumers + wq) * 2 * RT + 2 * i) * 64 + lane;
   const int64_t part_stride = (int64_t)tiles * kW4WideConsumers * 2 * RT * 64;
+  const int m = m_tile + (lane & 15), n = strip * kW4WideBN + wq * 32 + 4 * (lane >> 4);
+  const float sa = w4_row_scale(a.g, load_scalar_scales(a.g), m);
+  const f32x4 bias[2] = {w4_bias4(a.g, n), w4_bias4(a.g, n + 16)};
   f32x4 total[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   constexpr int kAhead = 4;  // parts whose loads are in flight together
   for (int p = 0; p < a.ksplit; p += kAhead) {
@@ -1098,9 +1122,8 @@ __global__ __launch_bounds__(256) void w4_finish_kernel(W4Args a, int strips) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) total[t][e] += p + q < a.ksplit ? v[q][t][e] : 0.0f;
   }
-  const ScalarScales scalars = load_scalar_scales(a.g);
 #pragma unroll
-  for (int t = 0; t < 2; ++t) w4_store4(a.g, scalars, m_tile + (lane & 15), strip * kW4WideBN + wq * 32 + 16 * t + 4 * (lane >> 4), total[t]);
+  for (int t = 0; t < 2; ++t) w4_store4(a.g, m, n + 16 * t, total[t], sa, bias[t]);
 }
 
 // How the wide kernel takes a problem: rows per workgroup (16 rows sit in a 32-row tile of LDS), row
