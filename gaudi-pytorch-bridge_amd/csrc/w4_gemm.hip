@@ -498,9 +498,9 @@ __global__ __launch_bounds__(kW4Threads) void w4a8_gemm_kernel(W4Args a) {
 // at about 3.2 TB/s, whole lines at 4.3), and K is cut into `ksplit` parts walked by as many
 // workgroups, so that a launch fills the chip whatever N is.  The parts of a strip meet through
 // memory: every workgroup stores its partial sums (already scaled by the groups' scales, fp32, in
-// register order).  Up to 32 rows the one that draws the last ticket of the strip adds them up in the order
+// register order).  Up to 32 rows, and where two parts of 64 rows meet, the one that draws the last ticket of the strip adds them up in the order
 // of the parts, whoever came last, and runs the epilogue; it also returns the ticket
-// counter to zero for the next launch.  Above that a second launch does (w4_finish_kernel).
+// counter to zero for the next launch.  Else a second launch does (w4_finish_kernel).
 //
 // Roles and the stage pipeline are those of the kernel above, with eight consumer waves of 32
 // columns and four producers.  The 16-byte slots of a packed row in LDS are XORed with
@@ -600,6 +600,14 @@ __device__ __forceinline__ void w4_store4(const GemmArgs& g, int m, int n, const
       for (int e = 0; e < 4; ++e) reinterpret_cast<float*>(cp)[e] = v[e];
     }
   }
+}
+
+// Whether the parts are added up by w4_finish_kernel.  Two parts of 64 rows are not: there the launch costs more than the one
+// part that the last workgroup reads (64 x 8192 x 28672, two planes: 46.4 us with it, 42.9 without; 50 x 8192 x 24000 51.3 and 47.2;
+// in three parts, 64 x 8192 x 20480, 41.4 either way).
+template <int ROWS>
+__host__ __device__ constexpr bool w4_parts_meet_later(int parts) {
+  return ROWS == 128 ? parts > 1 : ROWS == 64 && parts > 2;
 }
 
 // ROWS: 16 (one row tile; a product is folded one stage late), or 32, 64, 128 (ROWS / 16 row tiles; row blocks of
@@ -1009,7 +1017,7 @@ __global__ __launch_bounds__(kW4WideThreads) void w4a8_wide_kernel(W4Args a) {
   __syncthreads();  // every load has landed and every stage is consumed: the ring is idle
 
   if constexpr (ROWS >= 64) {
-    if (a.ksplit > 1) {  // w4_finish_kernel adds the parts up
+    if (w4_parts_meet_later<ROWS>(a.ksplit)) {  // w4_finish_kernel adds the parts up
       const int strips = (int)gridDim.x / a.ksplit;
       f32x4* to = reinterpret_cast<f32x4*>(a.partials) +
                   ((int64_t)(part * strips * (int)gridDim.y + (int)blockIdx.y * strips + strip) * kConsumers + wq) * 2 * RT * 64 + lane;
@@ -1020,7 +1028,8 @@ __global__ __launch_bounds__(kW4WideThreads) void w4a8_wide_kernel(W4Args a) {
       }
       return;
     }
-  } else if (a.ksplit > 1) {
+  }
+  if (ROWS < 128 && a.ksplit > 1) {
     // Partial sums in register order: 64-bit word number h 64 + lane (h < NV / 2) of consumer wave wq.  They are
     // written and read with device-scope atomic accesses, which go past the caches of this XCD to where the other
     // XCDs see them: no cache has to be written back or invalidated as a whole, which a fence would do (and
@@ -1191,7 +1200,7 @@ void w4_wide_launch_rows(const W4Args& a, hipStream_t st) {
   if (a.zp != nullptr || a.is_signed) w4a8_wide_kernel<FMT_A, true, ROWS, A16><<<grid, kW4WideThreads, 0, st>>>(a);
   else w4a8_wide_kernel<FMT_A, false, ROWS, A16><<<grid, kW4WideThreads, 0, st>>>(a);
   if constexpr (ROWS >= 64) {
-    if (a.ksplit > 1) w4_finish_kernel<ROWS / 16><<<strips * blocks * (2 * ROWS / 16), 256, 0, st>>>(a, (int)strips);
+    if (w4_parts_meet_later<ROWS>(a.ksplit)) w4_finish_kernel<ROWS / 16><<<strips * blocks * (2 * ROWS / 16), 256, 0, st>>>(a, (int)strips);
   }
 }
 // A16: on two fp8 planes of 16-bit activations.

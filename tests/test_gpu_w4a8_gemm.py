@@ -271,10 +271,12 @@ def test_exact_at_the_benchmark_shape(oracle, dev, M):
     assert torch.equal(out2, out)
 
 
-@pytest.mark.parametrize("M,K,N", [(33, 2048, 288), (64, 9472, 1664), (65, 4096, 160), (128, 2048, 256), (145, 4224, 1056), (100, 1408, 17280)])
+@pytest.mark.parametrize("M,K,N", [(33, 2048, 288), (64, 9472, 1664), (65, 4096, 160), (128, 2048, 256), (145, 4224, 1056), (100, 1408, 17280),
+                                   (49, 2048, 22016), (64, 2176, 28672)])
 def test_parts_of_high_tiles_are_exact(oracle, dev, M, K, N):
     """Tiles of 64 and 128 rows whose parts of K are added up by a second launch: first and last rows of a tile, a second row
-    block, a last strip of 32 columns, with one plane and with two (which takes more parts), and rows that start at odd elements."""
+    block, a last strip of 32 columns, with one plane and with two (which takes more parts), and rows that start at odd elements.
+    The last two: two parts of 64 rows, added up by the workgroup that comes last."""
     gen = torch.Generator().manual_seed(M + K + N)
     q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
     a = torch.randint(-4, 5, (M, K), generator=gen).float()
