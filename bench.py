@@ -52,8 +52,8 @@ MEASURED_TRAFFIC = {
     "fp8_gemm_v2": 939.89e6,
     "fp8_gemm_v2_B_NK": 939.33e6,
     "fp8_gemm_v2_decode_M16": 236.92e6,
-    "fp8_gemm_v2_decode_M64": 243.07e6,
-    "fp8_gemm_v2_decode_M256": 266.45e6,
+    "fp8_gemm_v2_decode_M64": 242.92e6,
+    "fp8_gemm_v2_decode_M256": 266.37e6,
     "w4a8_gemm_M16": 130.86e6,      # the partial sums of the two K parts on top of the 124 MB of operands
     "w4a8_gemm_M32": 139.63e6,
     "w4a8_gemm_M64": 157.22e6,

@@ -1,4 +1,4 @@
-"""Products of more than 128 rows with K in parts over workgroups (gemm_tile_split.h), and the choice of tiles for them.
+"""Products of more than 128 rows with K in parts over workgroups (gemm_ring.h), and the choice of tiles for them.
 Operands are small integers and scales powers of two, so that every fp32 sum is exact in any order and the result must
 match bit for bit."""
 import pytest
