@@ -141,17 +141,13 @@ __device__ __forceinline__ void ring_epilogue_fast(const GemmArgs& g, int64_t ba
   static_for<MT>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     const float staged_ra = *reinterpret_cast<LDS_AS const float*>(staged + kStagedRowScale + (16 * i + r) * 4);
-    float ra = g.sa_mode == MI355Q_GS_PER_ROW ? staged_ra : scalars.sa;
-    if (!PER_COL) ra *= scalars.sb;
+    const float ra = g.sa_mode == MI355Q_GS_PER_ROW ? staged_ra : scalars.sa;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       float v[4];
+      // (one scale after the other: their product can leave fp32's range where neither sums nor results do)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float b = HAS_BIAS ? cb[j][e] : 0.0f;
-        if constexpr (PER_COL) v[e] = __builtin_fmaf(acc[i][j][e] * ra, cs[j][e], b);
-        else v[e] = __builtin_fmaf(acc[i][j][e], ra, b);
-      }
+      for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[i][j][e] * ra, PER_COL ? cs[PER_COL ? j : 0][e] : scalars.sb, HAS_BIAS ? cb[HAS_BIAS ? j : 0][e] : 0.0f);
       const int slot = (4 * j + gq) ^ (2 * ((r >> kShift) & kMask));
       *reinterpret_cast<LDS_AS u32x2*>(out + i * 16 * kRow + r * kRow + slot * 8) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }

@@ -47,8 +47,9 @@ def test_split_products_are_exact(M, K, N, trans_b, dev):
 @pytest.mark.parametrize("exponent", [70, -72])
 @pytest.mark.parametrize("kind_a", ["scalar", "row", "col"])
 @pytest.mark.parametrize("kind_b", ["scalar", "row", "col"])
-def test_scales_are_applied_one_after_the_other(M, exponent, kind_a, kind_b, dev):
-    """fp32 results whose scales multiply to something outside fp32's range, while sums and results lie inside it: 2^140
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+def test_scales_are_applied_one_after_the_other(M, exponent, kind_a, kind_b, out, dev):
+    """Results whose scales multiply to something outside fp32's range, while sums and results lie inside it: 2^140
     is infinite and 2^-144 has five bits left of a scale with seven."""
     K = N = 4096
     unit = 2.0 ** -14 if exponent > 0 else 2.0 ** 9
@@ -66,12 +67,14 @@ def test_scales_are_applied_one_after_the_other(M, exponent, kind_a, kind_b, dev
         return s if kind == "scalar" else (s * (1.0 - 0.25 * (torch.arange(N) % 2)))[None]
 
     sa, sb = scale(kind_a, 1.0 + 2.0 ** -6), scale(kind_b, 1.0)
-    c = torch.ops.hpu.fp8_gemm_v2(a.to(E5).to(dev), False, b.to(E5).to(dev), False, None, torch.float32, sa.to(dev), sb.to(dev), None, False,
+    c = torch.ops.hpu.fp8_gemm_v2(a.to(E5).to(dev), False, b.to(E5).to(dev), False, None, out, sa.to(dev), sb.to(dev), None, False,
                                   list(sb.shape) if kind_b != "scalar" else None)
     ref = (sums * sa.double() * sb.double()).float()
     assert bool(ref.isfinite().all()) and int((ref == 0).sum()) == M
-    # (results below 2^-126 are rounded to a whole number of 2^-149)
-    assert torch.allclose(c.cpu(), ref, rtol=2.0 ** -22, atol=2.0 ** -149)
+    # results below 2^-126 are rounded to a whole number of 2^-149 (bf16: 2^-133); of 1 + 2^-6 and its 0.75 and 0.5625, bf16's eight
+    # bits hold the first two, and the third is half a unit off at most
+    rtol, atol = (2.0 ** -22, 2.0 ** -149) if out == torch.float32 else (2.0 ** -8, 2.0 ** -133)
+    assert torch.allclose(c.float().cpu(), ref, rtol=rtol, atol=atol)
 
 
 @pytest.mark.gpu
