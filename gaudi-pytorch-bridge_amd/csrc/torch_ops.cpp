@@ -220,7 +220,7 @@ int launch_cast_to(const Tensor& x, Tensor& out, const CastScale& cs, float* ama
 // key splits of the attention kernel for few queries) keep arrival counters in their workspace, which have to be zero
 // when a call starts and are left zero by every call: one zero-filled buffer per (device, stream, op) is kept here and
 // grown on demand, so that no launch has to clear them.  Calls on one stream run in order, which is
-// all the sharing the buffer allows (calls of several launches: WorkspaceTurn); the ops lay their counters out differently and do not share.  At most
+// all the sharing the buffer allows (calls of several launches keep them together themselves); the ops lay their counters out differently and do not share.  At most
 // kKeptWorkspaces buffers are kept: past that the one that was used least recently is given back (to the caching
 // allocator, which hands it out again only to work queued behind what still uses it).  While a stream is being captured into a graph no kept
 // buffer is handed out (its memory would belong to the graph's pool, and replays of two graphs could overlap): the
@@ -232,7 +232,6 @@ struct TicketWorkspaceCache {
   struct Entry {
     Tensor buffer;
     uint64_t used = 0;
-    std::shared_ptr<std::mutex> launching = std::make_shared<std::mutex>();
   };
   std::mutex mu;
   uint64_t clock = 0;
@@ -264,22 +263,6 @@ Tensor ticket_workspace(const Tensor& like, size_t bytes, TicketWorkspaceOp op) 
   if (c.map.size() > kKeptWorkspaces) drop_least_recent(c.map);
   return t;
 }
-// Held by a call of several launches (the 4-bit GEMMs) from its first to its last, so that two threads' launches on a stream do
-// not mix: the second launch of one call would read what the first of the other has written.
-struct WorkspaceTurn {
-  std::shared_ptr<std::mutex> order;
-  std::unique_lock<std::mutex> lock;
-  WorkspaceTurn(const Tensor& like, TicketWorkspaceOp op) {
-    TicketWorkspaceCache& c = ticket_workspace_cache();
-    {
-      std::lock_guard<std::mutex> cache_lock(c.mu);
-      const auto it = c.map.find(std::make_tuple((int)like.device().index(), current_stream(like), (int)op));
-      if (it == c.map.end()) return;  // given back meanwhile: the buffer is this call's alone
-      order = it->second.launching;
-    }
-    lock = std::unique_lock<std::mutex>(*order);
-  }
-};
 // While the stream is being captured: a buffer out of the graph's pool, its counters (the first `counters` bytes)
 // zeroed by a small fill kernel, which every replay runs again; the rest (partial sums that are written before they
 // are read) as it comes.
@@ -971,8 +954,6 @@ Tensor w4a8_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, con
   const size_t ws_bytes = mi355q_w4a8_gemm_workspace_bytes(M, N, K, group, to_mi355q_dtype(s.scalar_type()));
   const bool kept = !stream_is_capturing();
   Tensor ws = kept ? ticket_workspace(a, ws_bytes, kWsW4a8) : (ws_bytes ? captured_ticket_workspace(a, ws_bytes, 1024) : Tensor());
-  c10::optional<WorkspaceTurn> turn;
-  if (kept && ws_bytes) turn.emplace(a, kWsW4a8);
   const int st = mi355q_w4a8_gemm(a.data_ptr(), to_mi355q_dtype(a.scalar_type()), K, w.data_ptr<int32_t>(), N / 8, s.data_ptr(),
                                   to_mi355q_dtype(s.scalar_type()), has_zp ? z.data_ptr<int32_t>() : nullptr, is_signed ? 1 : 0,
                                   group, out.data_ptr(), to_mi355q_dtype(out_dtype), N, M, N, K, sa_dev, 1.0f, sa_mode,
@@ -1029,8 +1010,6 @@ Tensor w4a16_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, co
   // graph's own with its counters cleared
   const bool kept = !stream_is_capturing();
   Tensor ws = kept ? ticket_workspace(a, bytes, kWsW4a16) : captured_ticket_workspace(a, bytes, 1024);
-  c10::optional<WorkspaceTurn> turn;
-  if (kept) turn.emplace(a, kWsW4a16);
   const int st = mi355q_w4a16_gemm(a.data_ptr(), MI355Q_BF16, K, w.data_ptr<int32_t>(), N / 8, s.data_ptr(),
                                    to_mi355q_dtype(s.scalar_type()), has_zp ? z.data_ptr<int32_t>() : nullptr, is_signed ? 1 : 0, group,
                                    out.data_ptr(), to_mi355q_dtype(out_dtype), N, M, N, K, has_bias ? b.data_ptr() : nullptr,

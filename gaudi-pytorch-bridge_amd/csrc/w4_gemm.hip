@@ -41,6 +41,7 @@
 // barrier per K stage of 128.  At the end of a group of K the group's scales multiply the
 // partial sums into the totals, in fp32.
 #include <algorithm>
+#include <mutex>
 
 #include "gemm_tile.h"
 
@@ -1219,6 +1220,14 @@ void w4a8_launch_by_m(const W4Args& a, hipStream_t st) {
   else w4a8_launch<64, FMT_A>(a, st);
 }
 
+// Held by a call that uses a workspace from its first launch to its last (planes, product, sum of the parts), so that threads
+// that queue calls on one stream with one workspace do not mix them: a launch would read what another call's has written.  A
+// mutex per group of workspaces, for nothing has to be looked up or kept (20 ns where nobody waits).
+inline std::mutex& w4_launch_order(const void* workspace) {
+  static std::mutex order[64];
+  return order[(reinterpret_cast<uintptr_t>(workspace) >> 8) % 64];
+}
+
 // Workspace of mi355q_w4a16_gemm: [arrival counters and partial sums of the K split, as for W4A8][plane 1][plane 2]
 // [1 / row scale], each part 256-byte aligned.
 struct W4A16Layout {
@@ -1272,6 +1281,7 @@ extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const 
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   float* sx_inv = reinterpret_cast<float*>(ws + l.scale_off);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const std::lock_guard<std::mutex> in_order(w4_launch_order(workspace));
   const int sp = mi355q_split_rows_fp8x2(A, a_dtype, lda, M, K, ws + l.plane_off, ws + l.lo_off, l.ld, sx_inv, stream);
   if (sp != MI355Q_OK) return sp;
   W4Args a{};
@@ -1373,6 +1383,8 @@ extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int
     // an empty sum: bias (or zero) through the same epilogue, with no stage to walk
     a.stages_per_group = 1;
   }
+  std::unique_lock<std::mutex> in_order;
+  if (a.partials != nullptr) in_order = std::unique_lock<std::mutex>(w4_launch_order(workspace));
   if (fmt_a == MI355Q_E4M3FN) w4a8_launch_by_m<MI355Q_E4M3FN>(a, st);
   else w4a8_launch_by_m<MI355Q_E5M2>(a, st);
   return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;

@@ -318,8 +318,8 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
  * and no workspace is read).  Its first KiB holds arrival counters (whatever the shape): they have
  * to be zero when a call starts and every call leaves them zero, so a workspace is zero-filled
  * once, when it is allocated, and then reused, also for other shapes it is large enough for.  Calls
- * that share a workspace must not overlap (one stream, or an order between the streams), nor may threads
- * that share one mix their launches: above 32 rows a call in parts can be two.  NULL is allowed: the
+ * that share a workspace must not overlap (one stream, or an order between the streams); threads may
+ * queue theirs side by side, a call's launches (above 32 rows there can be two) stay together.  NULL is allowed: the
  * call then runs without the split, slower for these shapes.  Too small or misaligned:
  * MI355Q_ERR_WORKSPACE.  The parts are added in a fixed order: a result does not depend on which
  * workgroup finished last.

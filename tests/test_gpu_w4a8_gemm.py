@@ -317,3 +317,42 @@ def test_two_threads_on_a_stream_keep_their_parts_apart(oracle, dev):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not wrong
+
+
+@pytest.mark.parametrize("M", [16, 48, 100])
+def test_two_threads_share_a_workspace_of_the_c_entries(oracle, pkg, dev, M):
+    """The same through the C entries: calls of one, two and three launches that two threads queue on one stream with one
+    workspace, each call's launches together."""
+    import ctypes
+    import threading
+    lib, (K, N) = pkg.capi(), (4096, 512)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    need8, need16 = lib.mi355q_w4a8_gemm_workspace_bytes(M, N, K, 128, pkg.BF16), lib.mi355q_w4a16_gemm_workspace_bytes(M, N, K, 128, pkg.BF16)
+    assert need8 > 1024 and need16 > need8
+    ws = torch.zeros(max(need8, need16), dtype=torch.uint8, device=dev)
+    jobs, calls = [], 60
+    for seed in (1, 2):
+        gen = torch.Generator().manual_seed(seed)
+        q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
+        a = torch.randint(-4, 5, (M, K), generator=gen).float()
+        w = (q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0)
+        jobs.append((a.to(E4).to(dev), a.bfloat16().to(dev), pk.to(dev), s.to(dev), pz.to(dev),
+                     [torch.empty(M, N, device=dev) for _ in range(2 * calls)], (a.double() @ w).float()))
+    failed = []
+
+    def work(a8, a16, pk, s, pz, ys, ref):
+        for i, y in enumerate(ys):
+            tail = (K, pk.data_ptr(), N // 8, s.data_ptr(), pkg.BF16, pz.data_ptr(), 0, 128, y.data_ptr(), pkg.F32, N, M, N, K)
+            if i % 2:
+                r = lib.mi355q_w4a16_gemm(a16.data_ptr(), pkg.BF16, *tail, None, ws.data_ptr(), ws.numel(), 1, st)
+            else:
+                r = lib.mi355q_w4a8_gemm(a8.data_ptr(), pkg.E4M3FN, *tail, None, 1.0, pkg.GS_NONE, None, ws.data_ptr(), ws.numel(), st)
+            failed.extend([r] if r else [])
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    assert not failed and all(torch.equal(y.cpu(), j[-1]) for j in jobs for y in j[-2])
+    assert int(ws[:1024].count_nonzero()) == 0
