@@ -164,8 +164,106 @@ __device__ __forceinline__ void ring_epilogue_fast(const GemmArgs& g, int64_t ba
   });
 }
 
-// Every other form (fp32 output, accumulate input, full bias, scales per column of A or row of B, rows of C at any
-// alignment): the wave's sums go to LDS as they are, then a rolled loop takes four columns of a row per lane.
+// The kernel's epilogues, GemmArgs::fast_epi of its launch.
+enum RingEpilogue { kRingAny = 0, kRingFast = 1, kRingRows = 2 };
+
+// Whether ring_epilogue_rows serves a launch: rows of C and of the accumulate input in aligned pieces of four, at offsets
+// below 2^30 from a tile's first row.
+inline bool ring_rows_ok(const GemmArgs& g, int64_t batches) {
+  const int64_t es = g.out_bf16 ? 2 : 4;
+  const auto pieces = [&](const void* p, int64_t ld, int64_t stride) {
+    return reinterpret_cast<uintptr_t>(p) % (size_t)(4 * es) == 0 && ld >= 0 && ld % 4 == 0 && ld <= (int64_t(1) << 21) && (batches == 1 || stride % 4 == 0);
+  };
+  return g.N % 4 == 0 && g.N <= (1 << 21) && g.bias_mode != MI355Q_BIAS_FULL && pieces(g.C, g.ldc, g.stride_c) && (g.D == nullptr || pieces(g.D, g.ldd, g.stride_d));
+}
+
+// fp32 output, an accumulate input (or a full bias in its place), scales per column of A or row of B: the wave's sums go to LDS as
+// they are, with the scales of a row behind it, and come back with a lane owning four columns of a row, whose accumulate input it
+// has requested eight rows ahead.  Bound by the rows of C and D.  Column by column, each with a test and an address of its own as
+// in ring_epilogue_any, the input cost a tile of 256 rows 33 us (us a product, that form -> this one: 4096 x 4096 x 14336 with an
+// accumulate input 436 -> 213, fp32 258 -> 213, both 464 -> 244; 192 x 4096 x 14336 42.1 -> 22.7, 27.5 -> 21.7, 42.3 -> 23.2;
+// 16 x 4096 x 4096 8.7 -> 7.4, 7.6 -> 7.4, 8.8 -> 7.6).
+template <int MT, int NT, bool F32, bool HAS_D>
+__device__ __forceinline__ void ring_epilogue_rows(const GemmArgs& g, int64_t batch, f32x4 (&acc)[MT][NT], int m_wave, int n_wave,
+                                                   float* rows_p, ScalarScales scalars) {
+  constexpr int kPitch = 16 * NT + 4, kLanesPerRow = 4 * NT, kRowsPerPass = 64 / kLanesPerRow, kPasses = 16 * MT / kRowsPerPass;
+  constexpr int kAhead = kPasses < 8 ? kPasses : 8, es = F32 ? 4 : 2;
+  static_assert(kPasses % kAhead == 0, "whole groups of rows");
+  typedef typename std::conditional<F32, u32x4, u32x2>::type Piece;
+  LDS_AS float* rows = (LDS_AS float*)rows_p;
+  const int lane = threadIdx.x & 63, r = lane & 15, gq = lane >> 4;
+  const int left = g.M - m_wave < 16 * MT ? g.M - m_wave : 16 * MT;
+  const int row0 = lane / kLanesPerRow, n = n_wave + (lane % kLanesPerRow) * 4;
+  const bool inside = n < g.N;  // (the four columns are inside or outside together; outside: an offset no descriptor covers)
+  const auto view = [&](const uint8_t* p, int64_t stride, int64_t ld) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p) + (batch * stride + (int64_t)m_wave * ld) * es, 0,
+                                             left > 0 ? ((left - 1) * (int)ld + g.N) * es : 0, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t to = view(g.C, g.stride_c, g.ldc), from = view(HAS_D ? g.D : g.C, HAS_D ? g.stride_d : g.stride_c, HAS_D ? g.ldd : g.ldc);
+  const int to0 = inside ? (row0 * (int)g.ldc + n) * es : 0x7fffffff, to_step = inside ? kRowsPerPass * (int)g.ldc * es : 0;
+  const int from0 = inside ? (row0 * (int)g.ldd + n) * es : 0x7fffffff, from_step = inside ? kRowsPerPass * (int)g.ldd * es : 0;
+  const auto fetch = [&](Piece (&d)[HAS_D ? kAhead : 1], int pass) {
+    if constexpr (HAS_D) {
+#pragma unroll
+      for (int p = 0; p < kAhead; ++p) {
+        if constexpr (F32) d[p] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b128(from, from0 + (pass + p) * from_step, 0, 0));
+        else d[p] = __builtin_bit_cast(Piece, __builtin_amdgcn_raw_buffer_load_b64(from, from0 + (pass + p) * from_step, 0, 0));
+      }
+    }
+  };
+  Piece d[HAS_D ? kAhead : 1];
+  fetch(d, 0);
+  const bool a_rows = g.sa_mode == MI355Q_GS_PER_ROW, b_rows = g.sb_mode == MI355Q_GS_PER_ROW;
+  float sa_c[4], sb_c[4], bias_c[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int ne = inside ? n + e : g.N - 1;
+    sa_c[e] = g.sa_mode == MI355Q_GS_PER_COL ? g.sa[ne] : scalars.sa;
+    sb_c[e] = g.sb_mode == MI355Q_GS_PER_COL ? g.sb[ne] : scalars.sb;
+    bias_c[e] = g.bias_mode == MI355Q_BIAS_ROW_VECTOR ? load_out_as_f32(g.bias + batch * g.stride_bias * es, ne, !F32) : 0.0f;
+  }
+#pragma unroll
+  for (int t = 0; t < 16 * MT; t += 64) {
+    const int row = t + lane, m = m_wave + row < g.M ? m_wave + row : g.M - 1;
+    if (row < 16 * MT) {
+      rows[row * kPitch + 16 * NT] = a_rows ? g.sa[m] : 1.0f;
+      rows[row * kPitch + 16 * NT + 1] = b_rows ? g.sb[m] : 1.0f;
+    }
+  }
+  static_for<MT>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *reinterpret_cast<LDS_AS f32x4*>(rows + (16 * i + r) * kPitch + 16 * j + 4 * gq) = acc[i][j];
+  });
+#pragma unroll 1
+  for (int pass = 0; pass < kPasses && pass * kRowsPerPass < left; pass += kAhead) {
+    Piece next[HAS_D ? kAhead : 1];
+    fetch(next, pass + kAhead);  // (rows past the last one touch no memory)
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p) {
+      LDS_AS const float* row = rows + ((pass + p) * kRowsPerPass + row0) * kPitch;
+      const f32x4 a = *reinterpret_cast<LDS_AS const f32x4*>(row + (lane % kLanesPerRow) * 4);
+      const f32x2 s = *reinterpret_cast<LDS_AS const f32x2*>(row + 16 * NT);
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float t = a[e] * (a_rows ? s[0] : sa_c[e]);
+        v[e] = t * (b_rows ? s[1] : sb_c[e]) + bias_c[e];
+        if constexpr (HAS_D) v[e] += F32 ? __uint_as_float(d[p][F32 ? e : 0]) : __uint_as_float(e & 1 ? d[p][e >> 1] & 0xffff0000u : d[p][e >> 1] << 16);
+      }
+      const int at = to0 + (pass + p) * to_step;
+      if constexpr (F32) __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, to, at, 0, 2);
+      else __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}, to, at, 0, 2);  // aux 2: nontemporal
+    }
+    if constexpr (HAS_D) {
+#pragma unroll
+      for (int p = 0; p < kAhead; ++p) d[p] = next[p];
+    }
+  }
+}
+
+// Every other form (rows of C or D that are no aligned pieces of four, a full bias beside an accumulate input): the wave's sums go to
+// LDS as they are, then a rolled loop takes four columns of a row per lane.
 template <int MT, int NT>
 __device__ __forceinline__ void ring_epilogue_any(const GemmArgs& g, int64_t batch, f32x4 (&acc)[MT][NT], int m_wave, int n_wave,
                                                   float* rows, ScalarScales scalars) {
@@ -413,7 +511,7 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
 
   Consumer c;
   const int wm = (wave / Shape::kWavesN) * (16 * MT), wn = (wave % Shape::kWavesN) * (16 * NT);
-  if (g.fast_epi) ScaleStager::issue<(MT + 1) / 2, NT / 2>(g, batch, m0 + wm, n0 + wn, reinterpret_cast<float*>(lds_scales + wave * kRingScaleBytes));
+  if (g.fast_epi == kRingFast) ScaleStager::issue<(MT + 1) / 2, NT / 2>(g, batch, m0 + wm, n0 + wn, reinterpret_cast<float*>(lds_scales + wave * kRingScaleBytes));
   const ScalarScales scalars = load_scalar_scales(g);
   const uint32_t ring = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_ring;
   c.ra.init(ring, wm);
@@ -453,7 +551,7 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
     }
     __syncthreads();  // the word has been read
   }
-  if (g.fast_epi && g.D == nullptr) {
+  if (g.fast_epi == kRingFast) {
     const uint8_t* staged = lds_scales + wave * kRingScaleBytes;
     uint8_t* rows = lds_ring + wave * (16 * MT * 32 * NT);
     const bool per_col = g.sb_mode == MI355Q_GS_PER_COL, bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR;
@@ -461,8 +559,16 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
     else if (per_col) ring_epilogue_fast<MT, NT, true, false>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
     else if (bias) ring_epilogue_fast<MT, NT, false, true>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
     else ring_epilogue_fast<MT, NT, false, false>(g, batch, c.acc, m0 + wm, n0 + wn, staged, rows, scalars);
+    return;
+  }
+  float* rows = reinterpret_cast<float*>(lds_ring) + wave * 16 * MT * (16 * NT + 4);
+  if (g.fast_epi == kRingRows) {
+    if (g.out_bf16 && g.D != nullptr) ring_epilogue_rows<MT, NT, false, true>(g, batch, c.acc, m0 + wm, n0 + wn, rows, scalars);
+    else if (g.out_bf16) ring_epilogue_rows<MT, NT, false, false>(g, batch, c.acc, m0 + wm, n0 + wn, rows, scalars);
+    else if (g.D != nullptr) ring_epilogue_rows<MT, NT, true, true>(g, batch, c.acc, m0 + wm, n0 + wn, rows, scalars);
+    else ring_epilogue_rows<MT, NT, true, false>(g, batch, c.acc, m0 + wm, n0 + wn, rows, scalars);
   } else {
-    ring_epilogue_any<MT, NT>(g, batch, c.acc, m0 + wm, n0 + wn, reinterpret_cast<float*>(lds_ring) + wave * 16 * MT * (16 * NT + 4), scalars);
+    ring_epilogue_any<MT, NT>(g, batch, c.acc, m0 + wm, n0 + wn, rows, scalars);
   }
 }
 
@@ -474,6 +580,7 @@ void launch_ring(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipSt
   GemmArgs a = g;
   a.tiles_m = (g.M + BM - 1) / BM;
   a.tiles_n = (g.N + kRingBN - 1) / kRingBN;
+  a.fast_epi = g.fast_epi && g.D == nullptr ? kRingFast : (ring_rows_ok(g, batch) ? kRingRows : kRingAny);
   dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (split.parts > 1 ? split.parts : 1)), (unsigned)batch);
   if (a.tiles_m == 1 && (int64_t)g.N * g.K > kRingStreamBytes) fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, true><<<grid, kRingThreads, 0, st>>>(a, split);
   else fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, false><<<grid, kRingThreads, 0, st>>>(a, split);

@@ -2,6 +2,8 @@
 stage, of a ragged last stage and of more and fewer stages than the ring holds, each height whole and in parts, all layouts.
 Operands are small integers and scales powers of two, so that every fp32 sum is exact in any order and the result must match
 bit for bit."""
+import ctypes
+
 import pytest
 import torch
 
@@ -38,6 +40,39 @@ def test_ring_tiles_are_exact(M, K, N, ta, tb, dev):
     half, two = torch.tensor(0.5).to(dev), torch.tensor(2.0).to(dev)
     assert torch.equal(gemm(a8, bool(ta), b8, bool(tb), d.to(dev), torch.bfloat16, half, two, None, True).cpu(), (p + d.float()).bfloat16())
     assert torch.equal(gemm(a8, bool(ta), b8, bool(tb), None, torch.bfloat16, half, two, bias.bfloat16().to(dev), False).cpu(), (p + bias).bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(1, 256, 4), (16, 2048, 300), (31, 256, 132), (60, 14336, 516), (100, 512, 12004), (190, 1024, 12004), (1000, 512, 6404)])
+@pytest.mark.parametrize("f32", [True, False])
+def test_rows_in_pieces_of_four(pkg, dev, M, K, N, f32):
+    """fp32 results, accumulate inputs and scales per column of A or row of B, C and D in rows of their own pitch, two products a
+    launch; pitches that are and are not multiples of four: the same values, and nothing beside them."""
+    lib, out = pkg.capi(), torch.float32 if f32 else torch.bfloat16
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator().manual_seed(M + K + N)
+    a, b = torch.randint(-2, 3, (2, M, K), generator=g).float(), torch.randint(-2, 3, (2, N, K), generator=g).float()
+    a8, b8 = a.to(E4).to(dev), b.to(E5).to(dev)
+    p = (a.to(dev) @ b.to(dev).transpose(1, 2).contiguous()).cpu()  # (small integers: exact in fp32)
+    rows, cols = (torch.arange(M) % 3 - 1.0).exp2(), (torch.arange(N) % 2 - 1.0).exp2()
+    vec, d = (torch.arange(N) % 5 - 2).to(out).to(dev), torch.randint(-4, 5, (2, M, N), generator=g).to(out)
+    rs, cs = rows.to(dev), cols.to(dev)
+    need = lib.mi355q_fp8_gemm_workspace_bytes(0, K, 1, K, M, N, K, 2)
+    ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=dev)
+    for pitch in (N + 4, N + 3):
+        wide = torch.full((2, M, pitch), float("nan"), dtype=out)
+        wide[..., :N] = d
+        wide = wide.to(dev)
+        for a_rows, with_d, bias in ((1, 1, 0), (0, 1, 1), (0, 0, 1), (1, 0, 0)):
+            c = torch.full((2, M, pitch), 7.0, dtype=out, device=dev)
+            sa, sb = ((rs, pkg.GS_PER_ROW), (cs, pkg.GS_PER_COL)) if a_rows else ((cs, pkg.GS_PER_COL), (rs, pkg.GS_PER_ROW))
+            assert lib.mi355q_fp8_gemm_ws(a8.data_ptr(), pkg.E4M3FN, 0, K, b8.data_ptr(), pkg.E5M2, 1, K, c.data_ptr(), pkg.F32 if f32 else pkg.BF16, pitch, M, N, K,
+                                          sa[0].data_ptr(), 1.0, sa[1], sb[0].data_ptr(), 1.0, sb[1], vec.data_ptr() if bias else None,
+                                          pkg.BIAS_ROW_VECTOR if bias else pkg.BIAS_NONE, 0, wide.data_ptr() if with_d else None, pitch if with_d else 0, 2,
+                                          M * K, N * K, M * pitch, M * pitch if with_d else 0, 0, ws.data_ptr(), need, st) == 0
+            ref = p * rows[:, None] * cols + (vec.float().cpu() if bias else 0.0) + (d.float() if with_d else 0.0)
+            assert torch.equal(c[..., :N].cpu(), ref.to(out)), (pitch, a_rows, with_d, bias)
+            assert bool((c[..., N:] == 7.0).all())
 
 
 def test_every_height_is_reached(pkg):
