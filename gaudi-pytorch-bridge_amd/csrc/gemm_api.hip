@@ -113,11 +113,18 @@ constexpr double kLog2[kMostParts + 1] = {0.0, 0.0, 1.0, 1.5849625007211562, 2.0
 //    short products stay whole: below K = 1792 a cut of few strips gains a microsecond at most (1 x 1600 x 1024: 7.3 whole, 6.3
 //    in four parts) and a cut of many loses as much; an A [K, M], whose tiles of 128 rows send all their sums, from 2304 on.
 //  * 256 x 256 tiles take 1.42 us a stage in every pass over the compute units.
+//  * From one of those per compute unit on, the table holds for the 192-row tile, and for the others only below one pass and a half
+//    of them, with rows of A and B that start at whole 128-byte lines (a tile's rows of 128 bytes cross two lines otherwise, one of
+//    256 x 256 three per two) and six stages or more.  us on the 256-row tile / on 256 x 256: 7341 x 896 x 2176 21.9 / 30.8, 3840 x 3712 x
+//    6144 75.2 / 81.4, but 4096 x 4096 x 14336 204 / 173, 3636 x 2816 x 14752 171 / 147, 2409 x 3824 x 9600 119 / 112, 7836 x 512 x 3072 25.4 /
+//    22.8.  With fp32 results it holds throughout, since 256 x 256 tiles run as eight waves there: 2048 x 1536 x 11008 48.5 / 58.0,
+//    4096 x 8832 x 12672 376 / 396.
 //  * Up to 16 rows against B [K, N] of more than 96 MiB: the stream kernel, whose 256-byte pieces of B come in at 5.5 TB/s
 //    against 5.0 for the ring's 128 (16 x 8192 x 28672: 43.4 / 46.4 us; 16 x 8192 x 14336, 112 MiB, 26.4 / 26.3; 13 x 14144 x
 //    5248, 71 MiB, 23.2 / 16.8).  Its cut: a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where
 //    more of them run; no part shorter than 512, two turns of its eight waves.
-SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
+                     bool fp32_rows) {
   SplitPlan best;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
   const int64_t cus = compute_units(), stages = (K + kBK - 1) / kBK;
@@ -141,13 +148,16 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
     return best;
   }
   double best_us = 1e30;
+  bool full_chip = false;
   if (M > 128 && N > 128) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256) * batch;
     best_us = (double)((tiles + cus - 1) / cus) * (double)stages * 1.42 + 6.0;
+    full_chip = tiles >= cus && !fp32_rows && (2 * tiles >= 3 * cus || stages < 6 || lda % 128 != 0 || ldb % 128 != 0);
   }
   const double per_cu = 1.0 / (double)cus;
   for (const RingCost& c : kRingCosts) {
     if (a_kmajor ? (c.rows == 16) != (M <= 16) || (c.rows > 32 && c.rows >= 2 * M) : c.rows != 128 && c.rows != 256) continue;
+    if (full_chip && c.rows != 192) continue;
     const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + kRingBN - 1) / kRingBN), wgs = tiles * batch, rounds = (wgs + cus - 1) / cus;
     double fill = (double)std::min(wgs, cus) * per_cu;
     double us = c.fixed + (double)stages * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round);
@@ -287,7 +297,9 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const
     if (tiled_ok(gb.A, trans_a, lda, gb.B, trans_b, ldb, M, N, K, stride_a, stride_b)) {
       const bool ak = !trans_a, bk = trans_b != 0;
       // (K is walked in parts if the caller brought the room where they meet)
-      const SplitPlan plan = split_plan(ak, lda, bk, ldb, M, N, K, nb, workspace != nullptr && nb == batch);
+      // (fp32 results change the choice only where nothing is cut)
+      const bool fp32_rows = !gb.out_bf16 && ring_rows_ok(gb, nb);
+      const SplitPlan plan = split_plan(ak, lda, bk, ldb, M, N, K, nb, workspace != nullptr && nb == batch, fp32_rows);
       SplitArgs split{plan.parts, nullptr, nullptr};
       if (plan.parts > 1) {
         if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;

@@ -42,7 +42,8 @@ struct SplitPlan {
     return parts < 2 ? 0 : kTicketBytes + (size_t)parts * strips * batch * tile_rows * nb * sizeof(float);
   }
 };
-SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split);
+SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
+                     bool fp32_rows = false);  // fp32 results that ring_epilogue_rows writes
 
 // The counter, looked at ahead of time (before waits that the workgroup has anyway): parts - 1 means that every other
 // part has arrived; then this workgroup is the last whatever happens, and its own sums need not travel.

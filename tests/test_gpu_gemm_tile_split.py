@@ -73,3 +73,15 @@ def test_few_and_long_parts(pkg):
         assert sums(m, k, n) <= 64 * 1024 + 2 * tiles * 128 * 128 * 4, (m, k, n)
     for k in (14336, 16384, 32768):
         assert 64 * 1024 < sums(130, k, 128) <= 64 * 1024 + 16 * 2 * 128 * 128 * 4, k
+
+
+def test_products_that_fill_the_chip_keep_the_largest_tiles(pkg):
+    """From one and a half 256 x 256 tiles per compute unit on the 256-row tiles of the ring took up to a fifth longer, and below that
+    with rows off the 128-byte lines or few stages; the 192-row tile and the other products below it gained."""
+    name = pkg.capi().mi355q_fp8_gemm_ws_variant
+    tile = lambda m, k, n, nk=0: name(0, k, nk, k if nk else n, m, n, k, 1).decode().split("_")[0]  # noqa: E731
+    for m, k, n in [(4096, 4096, 14336), (3636, 2816, 14752), (1792, 1536, 21248), (5888, 3072, 9728), (2409, 3824, 9600), (7836, 512, 3072),
+                    (8192, 4096, 14336), (4096, 14336, 4096)]:
+        assert tile(m, k, n) == tile(m, k, n, 1) == "tile256x256x128", (m, k, n)
+    assert tile(7341, 896, 2176) == tile(3840, 3712, 6144, 1) == "tile256x128x128"
+    assert tile(8005, 3968, 2304, 1) == tile(1766, 896, 9632) == "tile192x128x128"
