@@ -121,8 +121,10 @@ constexpr double kLog2[kMostParts + 1] = {0.0, 0.0, 1.0, 1.5849625007211562, 2.0
 //    4096 x 8832 x 12672 376 / 396.
 //  * Up to 16 rows against B [K, N] of more than 96 MiB: the stream kernel, whose 256-byte pieces of B come in at 5.5 TB/s
 //    against 5.0 for the ring's 128 (16 x 8192 x 28672: 43.4 / 46.4 us; 16 x 8192 x 14336, 112 MiB, 26.4 / 26.3; 13 x 14144 x
-//    5248, 71 MiB, 23.2 / 16.8).  Its cut: a workgroup takes in its share of B at 37 GB/s, or at its share of 6.5 TB/s where
-//    more of them run; no part shorter than 512, two turns of its eight waves.
+//    5248, 71 MiB, 23.2 / 16.8).  Batches of 256 MiB and more in all, which the memory-side cache does not hold, take it too from
+//    K = 2048 on (1 x 4096 x 4096, 25 of them 74 against 97; 100 of 1 x 2048 x 2048 82 against 90, but 1600 of 1 x 512 x 512 117 against
+//    92; below, 12 of 1 x 4096 x 4096 37 against 34, but cold 38 against 50).  Its cut: a workgroup takes in its share of B at 37 GB/s,
+//    or at its share of 6.5 TB/s where more of them run; no part shorter than 512, two turns of its eight waves.
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
                      bool fp32_rows) {
   SplitPlan best;
@@ -130,7 +132,8 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   const int64_t cus = compute_units(), stages = (K + kBK - 1) / kBK;
   best.batch = batch;
   // (the stream kernel addresses an operand with 31-bit offsets)
-  if (a_kmajor && !b_kmajor && M <= 16 && N * K > (96LL << 20) && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) {
+  const bool much = N * K > (96LL << 20) || (K >= 2048 && N * K >= (256LL << 20) / batch);
+  if (a_kmajor && !b_kmajor && M <= 16 && much && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) {
     best.kind = GemmKind::kStream;
     best.nb = 256;
     best.strips = (int)((N + 255) / 256);

@@ -161,6 +161,27 @@ def test_short_products_stay_whole(pkg):
         assert 2 <= parts <= 8, (n, parts)
 
 
+def test_large_batches_are_streamed(pkg):
+    """Few rows against many matrices [K, N]: on the 16-row tiles of the ring 25 of 1 x 4096 x 4096 took a third longer."""
+    name = pkg.capi().mi355q_fp8_gemm_ws_variant
+    kernel = lambda m, k, n, batch: name(0, k, 0, n, m, n, k, batch)  # noqa: E731
+    for m, k, n, batch in [(1, 4096, 4096, 16), (16, 4096, 2048, 64), (4, 2048, 2048, 100)]:
+        assert b"registers" in kernel(m, k, n, batch), (m, k, n, batch)
+    for m, k, n, batch in [(1, 4096, 4096, 15), (1, 512, 512, 1600), (16, 1024, 1024, 400), (17, 4096, 4096, 25)]:
+        assert b"ring" in kernel(m, k, n, batch), (m, k, n, batch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16])
+def test_large_batches_are_exact(M, dev):
+    g = torch.Generator(device=dev).manual_seed(M)
+    a = torch.randint(-2, 3, (17, M, 4096), generator=g, device=dev).float()
+    b = torch.randint(-2, 3, (17, 4096, 4080), generator=g, device=dev).float()
+    want = a @ b
+    for out in (torch.float32, torch.bfloat16):
+        assert torch.equal(torch.ops.hpu.fp8_gemm_v2(a.to(E4), False, b.to(E5), False, None, out), want.to(out))
+
+
 def test_few_rows_of_an_mn_major_a_stay_whole_longer(pkg):
     """A [K, M] runs on tiles of 128 rows, whose parts send all their sums: 16 x 1792 x 128 takes 12.0 us whole and 16.4 in parts."""
     need = pkg.capi().mi355q_fp8_gemm_workspace_bytes
