@@ -9,8 +9,8 @@
 //    address register;
 //  * as many stages as the LDS holds (3 at 256 and 192 rows, 4, 6, 7, 7 below), counted waits, and load addresses without arithmetic;
 //  * low tiles where they fill the chip better, and K in parts only then (gemm_api.hip has the figures that choose);
-//  * plain loads for a B of at most 64 MiB: the nontemporal hint keeps a matrix out of the 256 MB memory-side cache, from
-//    which a second call would read it (64 x 8192 x 4096 warm: 40 us with the hint, 23 without; cold 0 to 10 % for it).
+//  * plain loads for a B of at most 64 MiB (ring_streams_b): the nontemporal hint keeps a matrix out of the 256 MB memory-side
+//    cache, from which a second call would read it.
 // Measured against the strip, 128 x 128 and 256 x 128 kernels it replaces (us, weights [K, N] but where nk, three sets of them in
 // turn): 256 x 8192 x 28672 88.8 -> 68.3 (nk 93.3 -> 66.5; the load stream alone takes 64), 1000 x 3008 x 5000 29.3 -> 24.3, 669 x 8704 x
 // 7808 nk 54.8 -> 44.7, 64 x 14336 x 4096 25.0 -> 17.5, 83 x 6640 x 864 23.9 -> 11.0, 7 x 10816 x 704 nk 16.1 -> 9.7, 1 x 4096 x 4096
@@ -437,7 +437,7 @@ struct RingConsumer {
   }
 };
 
-// NT_B: every byte of B is read by one workgroup alone (one row of tiles).
+// NT_B: B is loaded with the nontemporal hint (ring_streams_b).
 template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B, bool NT_B>
 __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g, SplitArgs split) {
   using Producer = RingProducer<BM, A_KMAJOR, B_KMAJOR>;
@@ -572,8 +572,18 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
   }
 }
 
-// B larger than this and read once is loaded past the caches (the nontemporal hint).
-constexpr int64_t kRingStreamBytes = 64LL << 20;
+// Whether B is loaded past the caches: every byte of it is read by one workgroup alone (one row of tiles, one product), and it is
+// too large to be found in the memory-side cache by a later call.  Time without the hint over that with it, 1 to 128 rows, B [K, N]:
+//   MiB          24    32    44    56    64    80    batches in all: 32    64    128   256   512
+//   B cold       1.03  1.05  1.02  1.01  1.07  1.04                  1.09  1.08  1.07  1.05  1.06
+//   B in there   0.85  0.93  0.87  0.95  0.93  0.86                  0.90  0.98  0.92  0.93  1.05
+// So what decides is whether it is still there: of a matrix of more than a quarter of the cache a decoder's other layers leave
+// nothing until its next turn, while a batch was mostly written just before.
+inline bool ring_streams_b(const GemmArgs& g, int64_t batch) {
+  if (g.tiles_m != 1 || (batch > 1 && g.stride_b == 0)) return false;
+  const int64_t bytes = (int64_t)g.N * g.K;
+  return bytes > (64LL << 20) || bytes > (256LL << 20) / batch;
+}
 
 template <int BM, bool AK, bool BK_, int FA, int FB>
 void launch_ring(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
@@ -582,7 +592,7 @@ void launch_ring(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipSt
   a.tiles_n = (g.N + kRingBN - 1) / kRingBN;
   a.fast_epi = g.fast_epi && g.D == nullptr ? kRingFast : (ring_rows_ok(g, batch) ? kRingRows : kRingAny);
   dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (split.parts > 1 ? split.parts : 1)), (unsigned)batch);
-  if (a.tiles_m == 1 && (int64_t)g.N * g.K > kRingStreamBytes) fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, true><<<grid, kRingThreads, 0, st>>>(a, split);
+  if (ring_streams_b(a, batch)) fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, true><<<grid, kRingThreads, 0, st>>>(a, split);
   else fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, false><<<grid, kRingThreads, 0, st>>>(a, split);
 }
 
