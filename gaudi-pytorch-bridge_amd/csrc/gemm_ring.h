@@ -544,6 +544,8 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
       __syncthreads();
       const bool others_in = *word == (uint32_t)split.parts - 1;
       __syncthreads();
+      // (rows past M travel too: whole lines of sums are stored and read faster than those of the rows that exist, 1 x 8192 x 1024
+      // 8.1 us against 8.7 without them, 1 x 14336 x 4096 14.2 against 14.5)
       if (!split_exchange<4 * MT * NT, kRingWaves * 64>(
               split, slot, slots, part, true, others_in, word, [&](int j) { return c.acc[j / (4 * NT)][j / 4 % NT][j % 4]; },
               [&](int j, float v) { c.acc[j / (4 * NT)][j / 4 % NT][j % 4] = v; }))
