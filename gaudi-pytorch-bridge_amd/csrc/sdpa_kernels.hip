@@ -207,15 +207,17 @@ __global__ void sdpa_clear_amax_kernel(float* a, float* b) {
   if (b != nullptr) *b = 0.0f;
 }
 
+enum { kWithoutMask, kWithMask, kEither };
+
 // One block of 64 keys for a wave's 32 query rows: S^T = K Q^T from the K tile at kb, masks, the
 // online-softmax update of (m_run, l_run, o), and O^T += V^T P^T from the V tile at vb.  qpos is the
-// lane's query position (for the causal comparison), mrow its row of the mask.  Wave-uniform: `edge` says that some score of
+// lane's query position (for the causal comparison), mrow its row of the mask (some row's where it has none).  Wave-uniform: `edge` says that some score of
 // the block may lie behind the last key, `general` that there is a mask, a first key, or a scale that is not positive; PLAIN:
-// neither, at compile time.  (The kernels walk their plain blocks in a loop of its own: with the other forms in the same
+// neither, at compile time; MASK: whether there is a mask.  (The kernels walk their plain blocks in a loop of its own: with the other forms in the same
 // loop the compiler copies all 32 scores on the way to where the paths meet, 5 % of the prefill.)
-template <int DKC, int DVT, int FMT, bool QL, bool PLAIN>
+template <int DKC, int DVT, int FMT, bool QL, bool PLAIN, int MASK>
 __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb, const uint8_t* vb, int kv0, bool edge, bool general, int qpos,
-                                           bool q_ok, const uint8_t* mrow, const i32x8 (&qf)[DKC], float sc2, float lqs, bool clamp_p,
+                                           const uint8_t* mrow, const i32x8 (&qf)[DKC], float sc2, float lqs, bool clamp_p,
                                            f32x16 (&o)[DVT], float& m_run, float& l_run, const uint8_t* qbase = nullptr,
                                            int klo = 0, int khi = 0x7fffffff) {
   constexpr int KROW = DKC * 64;
@@ -303,22 +305,45 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
       for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, s[t][r]);
     mx *= sc2;
   } else {
+    // One form per kind of mask, 16 scores' masks requested together; in the last block key by key.  A test in front of each of the 32
+    // loads had them wait for one another, each for the block just requested as well, and kept its conditions in spilled scalar
+    // registers: 2048 x 2048, 32 heads of 128, bf16 mask 280 -> 106 us, bool 287 -> 104; one query against 8192 keys, 8 x 32 heads of 128,
+    // 76 -> 40; against 19296, 2 x 64 heads of 256, 2154 -> 760.
+    int last = khi < a.S ? khi : a.S;
+    if (a.causal && qpos < last) last = qpos + 1;
+    last -= kv0 + 4 * h;
+    const int first = klo - kv0 - 4 * h;
+    constexpr bool kBounds = MASK != kWithoutMask;  // (without a mask two lane values are more than head dimension 256 has registers for)
+    const auto scores = [&](auto kindc, auto wholec) {
+      constexpr int KIND = decltype(kindc)::value, SIZE = KIND == kMaskBool ? 1 : KIND == kMaskBf16 ? 2 : 4;
+      constexpr bool WHOLE = decltype(wholec)::value;  // no key of the block lies behind the last one
+      const uint8_t* mr = mrow + (int64_t)(kv0 + 4 * h) * SIZE;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kv = kv0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-        float x = s[t][r] * sc2;
-        bool dead = kv >= a.S || kv >= khi || kv < klo || (a.causal && kv > qpos);
-        if (a.mask_kind != kMaskNone && q_ok && kv < a.S) {
-          if (a.mask_kind == kMaskBool) dead = dead || mrow[kv] == 0;
-          else if (a.mask_kind == kMaskBf16) x += bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(mrow)[kv]) * kLog2e;
-          else x += reinterpret_cast<const float*>(mrow)[kv] * kLog2e;
+        for (int r = 0; r < 16; ++r) {
+          const int key = 32 * t + 8 * (r >> 2) + (r & 3), kv = kv0 + key + 4 * h;
+          const bool dead = kBounds ? key >= last || key < first : kv >= a.S || kv >= khi || kv < klo || (a.causal && kv > qpos);
+          float x = s[t][r] * sc2;
+          if (WHOLE || kv < a.S) {
+            if constexpr (KIND == kMaskBool) x = mr[key] == 0 ? -__builtin_inff() : x;
+            if constexpr (KIND == kMaskBf16) x += bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(mr)[key]) * kLog2e;
+            if constexpr (KIND == kMaskF32) x += reinterpret_cast<const float*>(mr)[key] * kLog2e;
+          }
+          s[t][r] = dead ? -__builtin_inff() : x;
+          mx = __builtin_fmaxf(mx, s[t][r]);
+          if (r % 16 == 15 || (!WHOLE && r % 4 == 3)) __builtin_amdgcn_sched_barrier(0);
         }
-        x = dead ? -__builtin_inff() : x;
-        s[t][r] = x;
-        mx = __builtin_fmaxf(mx, x);
       }
+    };
+    const auto by_kind = [&](auto wholec) {
+      if (a.mask_kind == kMaskBool) scores(std::integral_constant<int, kMaskBool>{}, wholec);
+      else if (a.mask_kind == kMaskBf16) scores(std::integral_constant<int, kMaskBf16>{}, wholec);
+      else scores(std::integral_constant<int, kMaskF32>{}, wholec);
+    };
+    if (MASK == kWithoutMask || (MASK == kEither && a.mask_kind == kMaskNone)) scores(std::integral_constant<int, kMaskNone>{}, std::true_type{});
+    else if (kv0 + kSdpaBN <= a.S) by_kind(std::true_type{});
+    else by_kind(std::false_type{});
   }
   {  // the other half-wave's maximum for the same query row: a swap of register halves, no trip through LDS
     typedef unsigned u32x2v __attribute__((ext_vector_type(2)));
@@ -436,7 +461,7 @@ constexpr bool sdpa_q_in_lds(int dkc, int dvt, bool dma) { return dma && dkc == 
 // direct loads and a ring of two stages (255 registers, 64 KiB of LDS): 850 -> 1765 TFLOP/s at 32 / 8 heads and 8192
 // causal tokens against one workgroup with four stages.  Through registers (unaligned tensors) the same bound spills
 // 216 bytes per lane, so that form stays at one.
-constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma) { return sdpa_q_in_lds(dkc, dvt, dma) ? 3 : (dvt <= 4 || dma) ? 2 : 1; }
+constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { return sdpa_q_in_lds(dkc, dvt, dma) && !masked ? 3 : (dvt <= 4 || (dma && !masked)) ? 2 : 1; }
 
 // DKC: 64-byte steps of the q.k depth (head_dim_qk <= 64 DKC); DVT: 32-column tiles of v
 // (head_dim_v <= 32 DVT).
@@ -445,8 +470,12 @@ constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma) { return sdpa_q
 // has to assume the register route's loads outstanding wherever their registers are reused, and the wait it
 // puts there (vmcnt(0), in front of the first MFMA of every block) also waits for the blocks just requested
 // by the direct route.
-template <int DKC, int DVT, int FMT, bool DMA>
-__global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
+// MASK: with a mask no block is plain.  Two kernels from head dimension 128 on, since one with both forms spills in either (3 to 5 %
+// of the unmasked prefill at 256); with a mask two workgroups per CU at 128, whose mask needs registers, and one at 256.  At 64 one
+// kernel (apart, the one without a mask was 4 to 5 % slower where a SIMD has one wave of it).
+constexpr bool sdpa_kernel_per_mask(int dvt) { return dvt > 2; }
+template <int DKC, int DVT, int FMT, bool DMA, int MASK>
+__global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA, MASK == kWithMask)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
   constexpr bool kQLds = sdpa_q_in_lds(DKC, DVT, DMA);
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = DVT <= 4 ? 128 : 256;  // bytes of an LDS row of V
@@ -612,7 +641,8 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   float m_run = -__builtin_inff();  // running maximum of the scaled scores, in units of log2
   float l_run = 0.0f;               // this half-wave's share of the running sum (times q_scale_s)
 
-  const uint8_t* mrow = a.mask + (m_off + (int64_t)qrow * a.ldm) * (a.mask_kind == kMaskBool ? 1 : a.mask_kind == kMaskBf16 ? 2 : 4);
+  // (a row past the last one, which is not stored, reads the first one's mask)
+  const uint8_t* mrow = a.mask + (q_ok ? m_off + (int64_t)qrow * a.ldm : 0) * (a.mask_kind == kMaskBool ? 1 : a.mask_kind == kMaskBf16 ? 2 : 4);
   // The first blocks (ring positions count from the window's first one) are requested behind the query fragments, and the
   // wait for those covers them: one trip to memory at the start instead of two.
   if constexpr (DMA) {
@@ -645,7 +675,7 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   }
   __syncthreads();
 
-  const bool masked = a.mask_kind != kMaskNone || !(sc2 > 0.0f);
+  const bool masked = MASK == kWithMask || (MASK == kEither && a.mask_kind != kMaskNone) || !(sc2 > 0.0f);
   auto step = [&](auto pc, int blk) {
     constexpr bool PLAIN = decltype(pc)::value;
     const int kv0 = blk * kSdpaBN;
@@ -661,8 +691,8 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
     // a wave whose 32 rows all lie above this block's first key has nothing to add
     if (PLAIN || !(a.causal && kv0 > wq0 + 31)) {
       const bool edge = (a.causal && kv0 + kSdpaBN - 1 > wq0) || kv0 + kSdpaBN > khi;
-      sdpa_block<DKC, DVT, FMT, kQLds, PLAIN>(a, kb, vb, kv0, edge, masked || kv0 < klo, qrow, q_ok, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run,
-                                              qbase, klo, khi);
+      sdpa_block<DKC, DVT, FMT, kQLds, PLAIN, MASK>(a, kb, vb, kv0, edge, masked || kv0 < klo, qrow, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run,
+                                                    qbase, klo, khi);
     }
 
     if constexpr (DMA) {
@@ -686,7 +716,7 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA)
   if (a.causal && (q0 + 1) / kSdpaBN < plain) plain = (q0 + 1) / kSdpaBN;
   if (masked || klo > 0) plain = 0;
   int blk = blk0;
-  if constexpr (DVT <= 4 || DMA) {  // (through registers a second loop does not fit at head dimension 256)
+  if constexpr (MASK != kWithMask && (DVT <= 4 || DMA)) {  // (through registers a second loop does not fit at head dimension 256)
     for (; blk < plain; ++blk) step(std::true_type{}, blk);
   }
   for (; blk < nblk; ++blk) step(std::false_type{}, blk);
@@ -947,7 +977,7 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
   const int inner = a.pack ? lq / a.L : 0, qpos = a.pack ? lq - inner * a.L : lq;
   const bool q_ok = lq < a.rows;
   const uint8_t* qrowp = a.q + q_off + (int64_t)inner * a.q_bs[2] + (int64_t)qpos * a.ldq;
-  const uint8_t* mrow = a.mask + (m_off + (int64_t)inner * a.m_bs[2] + (int64_t)qpos * a.ldm) *
+  const uint8_t* mrow = a.mask + (q_ok ? m_off + (int64_t)inner * a.m_bs[2] + (int64_t)qpos * a.ldm : 0) *
                                      (a.mask_kind == kMaskBool ? 1 : a.mask_kind == kMaskBf16 ? 2 : 4);
 
   SdpaScales sc;
@@ -1033,7 +1063,7 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
       __builtin_amdgcn_s_waitcnt(0x0f70);
     }
     const uint8_t* kb = mine + buf * kStage;
-    sdpa_block<DKC, DVT, FMT, false, decltype(pc)::value>(a, kb, kb + KBYTES, kv0, a.causal || kv0 + kSdpaBN > a.S, masked, qpos, q_ok, mrow, qf, sc2,
+    sdpa_block<DKC, DVT, FMT, false, decltype(pc)::value, kEither>(a, kb, kb + KBYTES, kv0, a.causal || kv0 + kSdpaBN > a.S, masked, qpos, mrow, qf, sc2,
                                                           lqs, clamp_p, o, m_run, l_run);
     buf ^= 1;
   };
@@ -1112,16 +1142,22 @@ static SdpaDecodePlan sdpa_decode_plan(const mi355q_sdpa_desc* d, int cus) {
   return p;
 }
 
+template <int DKC, int DVT, int FMT, int MASK>
+static void sdpa_launch_kernel(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
+  const dim3 grid((unsigned)blocks), block(kSdpaThreads);
+  if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, false, MASK>), grid, block, 0, st, a);
+}
+template <int DKC, int DVT, int FMT>
+static void sdpa_launch_fmt(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
+  if constexpr (!sdpa_kernel_per_mask(DVT)) sdpa_launch_kernel<DKC, DVT, FMT, kEither>(a, blocks, st);
+  else if (a.mask_kind != kMaskNone) sdpa_launch_kernel<DKC, DVT, FMT, kWithMask>(a, blocks, st);
+  else sdpa_launch_kernel<DKC, DVT, FMT, kWithoutMask>(a, blocks, st);
+}
 template <int DKC, int DVT>
 static int sdpa_launch(const SdpaArgs& a, int fmt, int64_t blocks, hipStream_t st) {
-  const dim3 grid((unsigned)blocks), block(kSdpaThreads);
-  if (fmt == MI355Q_E5M2) {
-    if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, MI355Q_E5M2, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, MI355Q_E5M2, false>), grid, block, 0, st, a);
-  } else {
-    if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, MI355Q_E4M3FN, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, MI355Q_E4M3FN, false>), grid, block, 0, st, a);
-  }
+  if (fmt == MI355Q_E5M2) sdpa_launch_fmt<DKC, DVT, MI355Q_E5M2>(a, blocks, st);
+  else sdpa_launch_fmt<DKC, DVT, MI355Q_E4M3FN>(a, blocks, st);
   return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;
 }
 

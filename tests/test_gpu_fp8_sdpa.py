@@ -655,3 +655,19 @@ def test_rows_of_the_output_at_any_pitch(oracle, pkg, dev, pitch):
                                           1 / math.sqrt(D), 0, None, None, None, None, None, 0, st) == 0
     torch.cuda.synchronize()
     assert torch.equal(out[..., :D], run_op(dev, q, k, v)[0]) and bool((out[..., D:] == 7.0).all())
+
+
+@pytest.mark.parametrize("D", [64, 68, 128, 132, 256])
+@pytest.mark.parametrize("L,S", [(1, 64), (33, 65), (130, 63), (5, 128), (70, 191)])
+@pytest.mark.parametrize("kind", ["bool", "bf16", "f32"])
+def test_masks_at_the_edges_of_blocks(oracle, dev, D, L, S, kind):
+    """Whole blocks and last ones, whose masks are read together and key by key; rows of an odd number of keys; head dimensions
+    that go to LDS directly and through registers, with kernels of their own for masks and without; rows past the last one."""
+    gen = torch.Generator().manual_seed(D + L + S)
+    q, k, v = make_qkv(gen, (2, 2, L, D), (2, 2, S, D), (2, 2, S, D))
+    keep = torch.rand(2, 1, L, S, generator=gen) > 0.3
+    keep[..., S - 1] = True
+    mask = keep if kind == "bool" else torch.where(keep, torch.randn(2, 1, L, S, generator=gen), float("-inf")).to(torch.bfloat16 if kind == "bf16" else torch.float32)
+    out = run_op(dev, q, k, v, mask=mask, scales=(None, None, None, 128.0, None, 1 / 128.0))[0]
+    ref, _, _ = oracle.torch_fp8_sdpa(q, k, v, attn_mask=mask, q_scale_s=128.0, d_scale_s=1 / 128.0)
+    check_bf16(out, ref, f"{kind} {L} x {S}, D {D}")
