@@ -183,23 +183,23 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   return best;
 }
 
-// What launch_by_kind and launch_gemm_stream run; may_split: the caller brings the workspace.  A tile's extents (rows, columns,
-// bytes of K per stage) stand in falling order.
+// What launch_by_kind and launch_gemm_stream run; may_split: the caller brings the workspace.  A name gives the kernel and its
+// tile (rows x columns x bytes of K per stage), with "split_" in front where K goes in parts.
 const char* variant_name(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
   if (lda % 16 || ldb % 16 || lda > (1LL << 22) || ldb > (1LL << 22) || !k_chunks_ok(trans_a, trans_b, K)) return "simple";
   const SplitPlan p = split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, may_split);
   const bool cut = p.parts > 1;
-  if (p.kind == GemmKind::kStream) return cut ? "split_stream_Mx256_registers_mfma16x16" : "stream_Mx256_registers_mfma16x16";
-  if (p.kind == GemmKind::kRing16 && !trans_b && cut) return "split_stream_Mx128x128_ring_mfma16x16x128";
-  if (M <= 128) return cut ? "split_strip_Mx128x128_ring_mfma16x16x128" : "strip_Mx128x128_ring_mfma16x16x128";
   switch (p.kind) {
-    case GemmKind::kRing32: return cut ? "split_tile128x128x32_ring_mfma16x16x128" : "tile128x128x32_ring_mfma16x16x128";
-    case GemmKind::kRing64: return cut ? "split_tile128x128x64_ring_mfma16x16x128" : "tile128x128x64_ring_mfma16x16x128";
-    case GemmKind::kRing128: return cut ? "split_tile128x128x128_ring_mfma16x16x128" : "tile128x128x128_ring_mfma16x16x128";
-    case GemmKind::kRing192: return cut ? "split_tile192x128x128_ring_mfma16x16x128" : "tile192x128x128_ring_mfma16x16x128";
-    case GemmKind::kRing256: return cut ? "split_tile256x128x128_ring_mfma16x16x128" : "tile256x128x128_ring_mfma16x16x128";
-    default: return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
+    case GemmKind::kStream: return cut ? "split_stream_16x256_registers_mfma16x16" : "stream_16x256_registers_mfma16x16";
+    case GemmKind::kRing16: return cut ? "split_ring16x128x128_mfma16x16x128" : "ring16x128x128_mfma16x16x128";
+    case GemmKind::kRing32: return cut ? "split_ring32x128x128_mfma16x16x128" : "ring32x128x128_mfma16x16x128";
+    case GemmKind::kRing64: return cut ? "split_ring64x128x128_mfma16x16x128" : "ring64x128x128_mfma16x16x128";
+    case GemmKind::kRing128: return cut ? "split_ring128x128x128_mfma16x16x128" : "ring128x128x128_mfma16x16x128";
+    case GemmKind::kRing192: return cut ? "split_ring192x128x128_mfma16x16x128" : "ring192x128x128_mfma16x16x128";
+    case GemmKind::kRing256: return cut ? "split_ring256x128x128_mfma16x16x128" : "ring256x128x128_mfma16x16x128";
+    case GemmKind::kTile256: break;
   }
+  return "tile256x256x128_mfma16x16x128";  // 32x32x64 with eight waves for epilogues beyond the fast bf16 one
 }
 
 }  // namespace mi355q

@@ -9,15 +9,22 @@ import torch
 
 from helpers import E4, E5
 
-CASES = [  # M, K, N, trans_a, trans_b
-    (16, 144, 130, 0, 0), (1, 16, 256, 0, 1), (3, 8176, 8210, 0, 1), (16, 2064, 129, 0, 0), (1, 8192, 8208, 0, 1),     # 16 rows
-    (17, 128, 128, 0, 0), (32, 2064, 130, 0, 1), (33, 400, 1000, 0, 0), (49, 896, 384, 0, 1),                          # 32
-    (64, 4112, 4100, 0, 0), (100, 8192, 11264, 0, 0), (128, 1168, 13000, 0, 1), (65, 768, 9000, 0, 0),                 # 64
-    (257, 272, 8200, 0, 1), (129, 512, 12000, 0, 0), (257, 1040, 5000, 0, 0),                                           # 128
-    (300, 7168, 7168, 0, 0), (129, 1040, 20000, 0, 0), (513, 2576, 7168, 0, 1), (700, 8208, 4090, 0, 0), (385, 272, 9366, 0, 0), (520, 8208, 2190, 0, 1),   # 192
-    (249, 1040, 20000, 0, 0), (1000, 2576, 6400, 0, 1), (249, 7168, 13000, 0, 0),                                      # 256
-    (65, 2576, 250, 1, 0), (144, 1040, 5000, 1, 1), (600, 1303, 3000, 1, 0), (16, 4096, 256, 1, 1), (1000, 4096, 4096, 1, 0),  # A [K, M]
-]
+# M, K, N, trans_a, trans_b by the tile height that the plan gives them; whole, then in parts
+CASES_OF = {
+    "ring16": [(16, 144, 130, 0, 0), (1, 16, 256, 0, 1)],
+    "split_ring16": [(16, 2064, 129, 0, 0), (3, 8176, 8210, 0, 1), (1, 8192, 8208, 0, 1)],
+    "ring32": [(17, 128, 128, 0, 0), (33, 400, 1000, 0, 0), (65, 768, 9000, 0, 0), (49, 896, 384, 0, 1)],
+    "split_ring32": [(64, 4112, 4100, 0, 0), (32, 2064, 130, 0, 1)],
+    "ring64": [(257, 1040, 5000, 0, 0), (65, 144, 11570, 0, 0), (128, 1168, 13000, 0, 1)],
+    "split_ring64": [(35, 2720, 6598, 0, 0), (64, 14336, 4096, 0, 0), (33, 3024, 5789, 0, 1)],
+    "ring128": [(129, 512, 12000, 0, 0), (257, 272, 8200, 0, 1), (600, 1303, 3000, 1, 0), (1000, 4096, 4096, 1, 0), (144, 1040, 5000, 1, 1)],
+    "split_ring128": [(100, 8192, 11264, 0, 0), (72, 4640, 8612, 0, 1), (65, 2576, 250, 1, 0), (16, 4096, 256, 1, 1)],
+    "ring192": [(129, 1040, 20000, 0, 0), (385, 272, 9366, 0, 0), (513, 2576, 7168, 0, 1)],
+    "split_ring192": [(300, 7168, 7168, 0, 0), (700, 8208, 4090, 0, 0), (520, 8208, 2190, 0, 1)],
+    "ring256": [(249, 1040, 20000, 0, 0), (1000, 2576, 6400, 0, 1), (275, 260, 10996, 1, 0), (258, 272, 11841, 1, 1)],
+    "split_ring256": [(249, 7168, 13000, 0, 0), (200, 6672, 8488, 0, 1), (130, 6538, 8787, 1, 0), (129, 6576, 8357, 1, 1)],
+}
+CASES = [c for cases in CASES_OF.values() for c in cases]
 
 
 @pytest.mark.gpu
@@ -76,11 +83,12 @@ def test_rows_in_pieces_of_four(pkg, dev, M, K, N, f32):
 
 
 def test_every_height_is_reached(pkg):
-    """The cases above run on every tile height, whole and in parts."""
+    """The cases above run on the tile heights they stand under: all six, whole and in parts, with both layouts of B."""
     name = pkg.capi().mi355q_fp8_gemm_ws_variant
     up = lambda x: (x + 15) // 16 * 16  # noqa: E731
-    # (A [K, M] with a ragged K is the one form whose K is not rounded up before the launch)
-    got = {name(ta, up(M if ta else K), tb, up(K if tb else N), M, N, K if ta and not tb else up(K), 1).decode().split("_ring")[0] for M, K, N, ta, tb in CASES}
-    want = {"strip_Mx128x128", "split_strip_Mx128x128", "split_stream_Mx128x128", "tile128x128x128",
-            "tile192x128x128", "split_tile192x128x128", "tile256x128x128", "split_tile256x128x128"}
-    assert want <= got, want - got
+    for want, cases in CASES_OF.items():
+        for M, K, N, ta, tb in cases:
+            # (A [K, M] with a ragged K is the one form whose K is not rounded up before the launch)
+            got = name(ta, up(M if ta else K), tb, up(K if tb else N), M, N, K if ta and not tb else up(K), 1).decode()
+            assert got.startswith(want + "x"), (want, M, K, N, ta, tb, got)
+        assert {c[4] for c in cases} == {0, 1}, want

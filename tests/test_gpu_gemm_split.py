@@ -1,5 +1,5 @@
-"""Products of at most 128 rows of A: the kernel that streams B into registers (gemm_stream.h), the strip kernel, and the
-split of K over workgroups with which both run.  Operands are small integers and scales powers of two, so that every
+"""Products of few rows of A on the ring kernel (gemm_ring.h) and the split of K over workgroups; test_gpu_gemm_stream.py has
+the kernel that streams B into registers.  Operands are small integers and scales powers of two, so that every
 fp32 sum is exact in any order and the result must match bit for bit."""
 import ctypes
 
@@ -105,8 +105,9 @@ def test_one_workspace_serves_several_shapes(pkg, dev):
 
 # per kernel that splits K: rows, K off the stages' 128, N off 16
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,N,name", [(1, 4112, 1000, b"split_stream"), (16, 4112, 16378, b"split_stream"), (40, 4112, 1000, b"split_strip"),
-                                        (128, 14352, 250, b"split_strip"), (300, 8208, 1000, b"split_tile128"), (2000, 14352, 1000, b"split_tile256")])
+@pytest.mark.parametrize("M,K,N,name", [(1, 4112, 1000, b"split_ring16"), (16, 4112, 16378, b"split_ring16"), (40, 4112, 1000, b"split_ring32"),
+                                        (128, 14352, 250, b"split_ring32"), (300, 8208, 1000, b"split_ring64"), (100, 8208, 11250, b"split_ring128"),
+                                        (700, 8208, 4090, b"split_ring192"), (2000, 14352, 1000, b"split_ring256")])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_what_lies_beside_the_operands_stays_out(pkg, dev, M, K, N, name, ta, tb):
     """Operands in wider rows with NaN codes behind every row, and a row of NaN behind the last: exact results all the same.
@@ -126,7 +127,8 @@ def test_what_lies_beside_the_operands_stays_out(pkg, dev, M, K, N, name, ta, tb
         aw, bw = beside(a.t() if ta else a).to(E5).to(dev), beside(b.t() if tb else b).to(E5).to(dev)
         lda, ldb = aw.shape[1], bw.shape[1]
         variant = lib.mi355q_fp8_gemm_ws_variant(ta, lda, tb, ldb, M, N, K, 1)
-        assert variant.startswith(name) or (M <= 16 and (ta or tb) and b"strip_" in variant), variant
+        # (an A [K, M] has tiles of 128 and 256 rows alone, cut or not)
+        assert variant.startswith(name + b"x") or (ta and variant.replace(b"split_", b"").startswith((b"ring128x", b"ring256x"))), variant
         need = lib.mi355q_fp8_gemm_workspace_bytes(ta, lda, tb, ldb, M, N, K, 1)
         ws = torch.full((need,), 255, dtype=torch.uint8, device=dev)  # NaN where the sums will lie
         ws[: 64 * 1024] = 0
@@ -156,7 +158,7 @@ def test_short_products_stay_whole(pkg):
                 assert all(bytes_of(m, k, n, nk) == 0 for k in (16, 512, 1024, 1280, 1536, 1776)), (m, n, nk)
                 assert bytes_of(m, 8192, n, nk) > 0, (m, n, nk)
     counters = 64 * 1024
-    for n in (512, 1024, 4096):  # sums of 16 rows and 256 columns: parts of the stream kernel, 512 k each at least
+    for n in (512, 1024, 4096):  # sums of 16 rows and 128 columns a strip
         parts = (bytes_of(1, 4096, n, 0) - counters) // (n * 16 * 4)
         assert 2 <= parts <= 8, (n, parts)
 

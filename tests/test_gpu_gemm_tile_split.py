@@ -83,5 +83,5 @@ def test_products_that_fill_the_chip_keep_the_largest_tiles(pkg):
     for m, k, n in [(4096, 4096, 14336), (3636, 2816, 14752), (1792, 1536, 21248), (5888, 3072, 9728), (2409, 3824, 9600), (7836, 512, 3072),
                     (8192, 4096, 14336), (4096, 14336, 4096)]:
         assert tile(m, k, n) == tile(m, k, n, 1) == "tile256x256x128", (m, k, n)
-    assert tile(7341, 896, 2176) == tile(3840, 3712, 6144, 1) == "tile256x128x128"
-    assert tile(8005, 3968, 2304, 1) == tile(1766, 896, 9632) == "tile192x128x128"
+    assert tile(7341, 896, 2176) == tile(3840, 3712, 6144, 1) == "ring256x128x128"
+    assert tile(8005, 3968, 2304, 1) == tile(1766, 896, 9632) == "ring192x128x128"

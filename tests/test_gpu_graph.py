@@ -79,8 +79,9 @@ def test_graph_replays_of_a_ragged_product(dev):
         assert torch.equal(got, eager) and torch.equal(got.cpu(), a @ w8.cpu().float()), rep
 
 
-# one product per kernel that splits K: the stream kernel, the strip kernel, tiles that meet in pairs
-@pytest.mark.parametrize("M,K,N,name", [(1, 4096, 1024, b"split_stream"), (64, 14336, 256, b"split_strip"), (300, 8192, 1024, b"split_tile")])
+# the kernels that split K: 16-row tiles, 32-row tiles, tiles that meet in pairs, the kernel that streams B
+@pytest.mark.parametrize("M,K,N,name", [(1, 4096, 1024, b"split_ring16x"), (64, 14336, 256, b"split_ring32x"), (100, 8192, 11264, b"split_ring128x"),
+                                        (3, 4112, 24576, b"split_stream_")])
 def test_graph_replays_of_split_products(pkg, dev, M, K, N, name):
     """The arrival counters lie in a tensor of the graph's own, cleared by a fill kernel of the graph; here that memory is
     full of ones when the allocator hands it out, in the capture and in every replay."""

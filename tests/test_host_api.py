@@ -88,9 +88,10 @@ def test_variant_names_are_those_of_the_entry(pkg):
                                    lib.mi355q_fp8_gemm_ws_variant(0, k, nk, k if nk else n, m, n, k, 1))
     for m, k, n in [(1, 4096, 1024), (1, 14336, 4096), (1, 4096, 4096)]:
         plain, ws = names(m, k, n)
-        assert plain.startswith(b"strip_") and ws.startswith(b"split_stream_"), (m, k, n, plain, ws)
-    assert names(64, 14336, 4096)[1].startswith(b"split_strip_")
-    assert names(256, 14336, 1024)[1].startswith(b"split_tile128x128")
+        assert plain.startswith(b"ring16x") and ws.startswith(b"split_ring16x"), (m, k, n, plain, ws)
+    assert names(64, 14336, 4096)[1].startswith(b"split_ring64x")
+    assert names(256, 14336, 1024)[1].startswith(b"split_ring64x") and names(100, 8192, 11264)[1].startswith(b"split_ring128x")
+    assert names(16, 8192, 28672) == (b"stream_16x256_registers_mfma16x16", b"split_stream_16x256_registers_mfma16x16")
     assert names(8192, 4096, 14336) == (b"tile256x256x128_mfma16x16x128",) * 2
     for m in (1, 8, 16, 17, 64, 128, 129, 256, 300, 1000, 4096):
         for k in (512, 2048, 4096, 14336):
