@@ -49,39 +49,42 @@ def test_exact_small_integers_tiled(dev, fa, fb, ta, tb, M, N, K):
     assert torch.equal(out16.cpu(), expect.bfloat16())
 
 
-# One shape per kernel the dispatcher can pick (256 CUs): 256 x 256 tiles need at least 256 of them
-# (a last pass that fills at most a quarter of the CUs is split off as columns of 256 x 128 tiles:
-# 272 and 528 tiles do that, 464 do not);
-# below that the eight-wave kernel runs with 256 x 128 tiles while those fill more than half the CUs
-# (more, or fewer, tiles than CUs), else with 128 x 128 tiles, two workgroups per CU; the strip kernel
-# has three row-tile heights, and 128 x 128 tiles also serve N <= 128 < M (fewer, or more, tiles than
-# the 512 workgroup slots).  Edges are ragged in M, N and K.
+# Per kernel that the plan can pick (256 CUs): M, N, K and what runs it with A [M, K] and with A [K, M].  256 x 256 tiles as one
+# launch and with a last pass of few tiles split off as columns of the ring's (528 tiles), K in two stages, an odd and an even number
+# of them and a ragged last one; K % 256 == 0 is the form without per-lane K tests.  Products with other epilogues than the
+# fast bf16 one run the eight-wave kernel (an accumulate input) or, with fp32 results, what the plan prefers for those.  Then the
+# ring's heights, more and fewer tiles than CUs.  Edges are ragged in M, N and K.
 KERNEL_SHAPES = {
-    "tile256_one_pass_and_tail_columns": (4000, 4112, 208),
-    "tile256_two_passes_and_tail_columns": (4000, 8208, 208),
-    "tile256_two_passes_no_split": (4000, 7184, 144),
-    "tile256_ten_k_stages": (4000, 4112, 1168),
-    "tile256_whole_stage_pairs_and_tail_columns": (4000, 4112, 512),   # K % 256 == 0: the kernel without per-lane K tests
-    "tile256_whole_stage_pairs_two_passes": (4000, 8208, 256),
-    "tile256x128_more_tiles_than_cus": (1008, 12304, 208),
-    "tile256x128_fewer_tiles_than_cus": (272, 10256, 272),
-    "tile128_underfilled": (272, 4112, 400),
-    "strip_32_rows": (16, 1040, 400),
-    "strip_64_rows": (48, 1040, 400),
-    "strip_128_rows": (112, 1040, 400),
-    "tile128": (400, 112, 272),
-    "tile128_more_tiles_than_slots": (66576, 112, 144),
+    "tile256_two_passes_and_tail_columns": (4000, 8208, 208, "tile256x256", "tile256x256"),
+    "tile256_two_passes_no_split": (4000, 7184, 144, "tile256x256", "tile256x256"),
+    "tile256_ten_k_stages": (4000, 7184, 1168, "tile256x256", "tile256x256"),
+    "tile256_nine_k_stages_and_tail_columns": (4000, 8208, 1104, "tile256x256", "tile256x256"),
+    "tile256_odd_whole_stages": (4000, 7184, 640, "tile256x256", "tile256x256"),
+    "tile256_whole_stage_pairs_and_tail_columns": (4000, 8208, 1024, "tile256x256", "tile256x256"),
+    "tile256_whole_stage_pairs_two_passes": (4000, 8208, 256, "tile256x256", "tile256x256"),
+    "tile256_few_rows": (1008, 12304, 208, "tile256x256", "tile256x256"),
+    "ring192_or_tile256_one_pass": (4000, 4112, 208, "ring192", "tile256x256"),
+    "ring192_or_tile256_ten_k_stages": (4000, 4112, 1168, "ring192", "tile256x256"),
+    "ring192_or_tile256_whole_stages": (4000, 4112, 512, "ring192", "tile256x256"),
+    "ring128_few_rows": (272, 10256, 272, "ring128", "ring128"),
+    "ring64_underfilled": (272, 4112, 400, "ring64", "ring128"),
+    "ring16": (16, 1040, 400, "ring16", "ring128"),
+    "ring32": (48, 1040, 400, "ring32", "ring128"),
+    "ring32_four_tiles": (112, 1040, 400, "ring32", "ring128"),
+    "ring32_narrow": (400, 112, 272, "ring32", "ring128"),
+    "ring192_narrow_more_tiles_than_cus": (66576, 112, 144, "ring192", "ring128"),
 }
 
 
 @pytest.mark.parametrize("ta", [False, True])
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("kernel", sorted(KERNEL_SHAPES))
-def test_every_kernel_path(oracle, dev, kernel, ta, tb):
+def test_every_kernel_path(oracle, pkg, dev, kernel, ta, tb):
     """Exact small-integer products through each kernel (fp32 output: general epilogue), then the
     same operands with per-row x per-column scales, a bias vector and bf16 output (fast epilogue)
     against the fp32-accumulated CPU reference, with and without an accumulate input."""
-    M, N, K = KERNEL_SHAPES[kernel]
+    M, N, K, *kernels = KERNEL_SHAPES[kernel]
+    assert pkg.capi().mi355q_fp8_gemm_ws_variant(ta, M if ta else K, tb, K if tb else N, M, N, K, 1).decode().startswith(kernels[ta])
     g = torch.Generator().manual_seed(M + N + K)
     A = small_int_fp8((K, M) if ta else (M, K), E4, g)
     B = small_int_fp8((N, K) if tb else (K, N), E5, g)
@@ -105,6 +108,21 @@ def test_every_kernel_path(oracle, dev, kernel, ta, tb):
     assert torch.equal(out_d.cpu(), (expect * 0.125 + bias.float() + D.float()).bfloat16())
     out_d = ops.fp8_gemm_v2(A.to(dev), ta, B.to(dev), tb, D.to(dev), torch.bfloat16, sa.to(dev), sb.to(dev), None, True, [1, N])
     check(out_d, oracle.torch_fp8_gemm(A, ta, B, tb, torch.float32, sa, sb.reshape(1, N), D=D), kernel + " accumulate")
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_eight_wave_tiles_and_rows_at_any_alignment(pkg, dev, ta, tb):
+    """256 x 256 tiles whose results start at odd elements, with and without an accumulate input and a full bias: the general epilogue."""
+    M, N, K = 4000, 7173, 1104
+    assert pkg.capi().mi355q_fp8_gemm_ws_variant(ta, M if ta else K, tb, K if tb else N + 11, M, N, K, 1).startswith(b"tile256x256")
+    g = torch.Generator(device=dev).manual_seed(5)
+    a, b, d = (torch.randint(-2, 3, shape, generator=g, device=dev).float() for shape in ((M, K), (K, N), (M, N)))
+    p = a @ b
+    a8, b8 = (a.t().contiguous() if ta else a).to(E4), (b.t().contiguous() if tb else b).to(E5)
+    for out in (torch.float32, torch.bfloat16):
+        assert torch.equal(ops.fp8_gemm_v2(a8, ta, b8, tb, None, out), p.to(out))
+        assert torch.equal(ops.fp8_gemm_v2(a8, ta, b8, tb, d.to(out), out, 0.5, 2.0, d.to(out), True), (p + 2 * d).to(out))
 
 
 @pytest.mark.parametrize("shape", [(24, 12, 36), (22, 10, 34), (26, 16, 38), (1, 7, 3), (17, 1, 5), (33, 65, 129)])
