@@ -213,3 +213,38 @@ def test_ops_follow_the_current_stream(oracle, dev):
     assert torch.equal(y.cpu().view(torch.uint8), ref.view(torch.uint8))
     assert amax.cpu() == ref_amax
     assert torch.equal(back.cpu().float(), ref.float())
+
+
+@pytest.mark.parametrize("M", [40, 100])
+def test_graph_replays_of_4bit_products_in_two_and_three_launches(pkg, dev, M):
+    """Above 32 rows the parts of K are added up by a launch of their own, which belongs to the graph like the ones before it; the
+    memory of its workspace is full of ones when the allocator hands it out."""
+    g = torch.Generator().manual_seed(M)
+    K, N = 4096, 512
+    counters = 1024
+    assert pkg.capi().mi355q_w4a8_gemm_workspace_bytes(M, N, K, 128, pkg.BF16) >= counters + 3 * M * N * 4  # three parts at least
+    pk = torch.randint(-2 ** 31, 2 ** 31 - 1, (K, N // 8), generator=g, dtype=torch.int64).to(torch.int32).to(dev)
+    s = (torch.rand(K // 128, N, generator=g) * 0.019 + 0.001).bfloat16().to(dev)
+    z = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 128, N // 8), generator=g, dtype=torch.int64).to(torch.int32).to(dev)
+    static_x = torch.zeros(M, K, dtype=torch.bfloat16, device=dev)
+
+    def run(x):
+        own = torch.ops.mi355q
+        return own.w4a8_gemm(x.to(E4), pk, s, z, False, torch.bfloat16, None, None), own.w4a16_gemm(x, pk, s, z, False, torch.bfloat16, None)
+
+    run(static_x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ones = [torch.empty(n, dtype=torch.uint8, device=dev).fill_(255) for n in (48 << 20, 1 << 20, 1 << 20)]
+        del ones
+        outs = run(static_x)
+    for rep in range(4):
+        x = torch.randn(M, K, generator=g).bfloat16().to(dev)
+        static_x.copy_(x)
+        want = run(x)  # eager work between the replays
+        for out in outs:
+            out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(out, ref) for out, ref in zip(outs, want)), rep
