@@ -39,6 +39,7 @@ GemmArgs columns_from(const GemmArgs& g, int64_t n_off, int64_t batch) {
   t.N = g.N - (int)n_off;
   t.B = g.B + (B_KMAJOR ? n_off * g.ldb : n_off);
   t.C = g.C + n_off * es;
+  if (g.sa_mode == MI355Q_GS_PER_COL) t.sa = g.sa + n_off;
   if (g.sb_mode == MI355Q_GS_PER_COL) t.sb = g.sb + n_off;
   if (g.bias_mode != MI355Q_BIAS_NONE) t.bias = g.bias + n_off * es;
   if (g.D) t.D = g.D + n_off * es;

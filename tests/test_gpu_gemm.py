@@ -110,6 +110,21 @@ def test_every_kernel_path(oracle, pkg, dev, kernel, ta, tb):
     check(out_d, oracle.torch_fp8_gemm(A, ta, B, tb, torch.float32, sa, sb.reshape(1, N), D=D), kernel + " accumulate")
 
 
+@pytest.mark.parametrize("kind_a", ["row", "col"])
+@pytest.mark.parametrize("kind_b", ["row", "col"])
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+def test_scales_of_split_off_columns(pkg, dev, kind_a, kind_b, out):
+    """A last pass of few 256 x 256 tiles runs as a second launch over the last columns: with their scales, A's as well as B's."""
+    M, N, K = 4000, 8208, 256
+    assert pkg.capi().mi355q_fp8_gemm_ws_variant(0, K, 0, N, M, N, K, 1).startswith(b"tile256x256")
+    g = torch.Generator(device=dev).manual_seed(6)
+    a, b = (torch.randint(-2, 3, shape, generator=g, device=dev).float() for shape in ((M, K), (K, N)))
+    rows, cols = (torch.arange(M, device=dev) % 3 - 1.0).exp2()[:, None], (torch.arange(N, device=dev) // 4000 - 1.0).exp2()[None]
+    sa, sb = rows if kind_a == "row" else cols, rows if kind_b == "row" else cols
+    c = ops.fp8_gemm_v2(a.to(E4), False, b.to(E4), False, None, out, sa, sb, None, False, list(sb.shape))
+    assert torch.equal(c, (a @ b * sa * sb).to(out))
+
+
 @pytest.mark.parametrize("ta", [False, True])
 @pytest.mark.parametrize("tb", [False, True])
 def test_eight_wave_tiles_and_rows_at_any_alignment(pkg, dev, ta, tb):
