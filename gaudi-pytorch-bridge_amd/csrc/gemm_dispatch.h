@@ -11,13 +11,11 @@
 
 namespace mi355q {
 
-// Tile columns to split off a 256 x 256 tiling whose last pass over the tiles would
-// leave at least three quarters of the compute units idle (320 tiles on 256
-// CUs: one full pass and one of 64 tiles).  Those last columns then run as a second
-// launch with 256 x 128 tiles, twice as many for about 0.6 of the time each
-// (2048 x 10240 x 8192: 0.156 -> 0.145 ms).  With a last pass that is half
-// full the second launch costs what it saves (4096 x 14336 x 4096: 0.177 ms
-// either way), so those are left alone.  0: no split.
+// Tile columns to split off a 256 x 256 tiling whose last pass over the tiles would leave at least three quarters of the compute
+// units idle (544 tiles on 256 CUs: two full passes and one of 32 tiles).  Those last columns then run as a second launch with the
+// ring's 256 x 128 tiles, twice as many for about 0.6 of the time each (without -> with: 4096 x 4096 x 8704 126 -> 116 us, with an
+// accumulate input 150 -> 139; 4096 x 2048 x 8448 73.7 -> 70.2; 8704 x 2048 x 8192, 1088 tiles, 125 -> 123).  A last pass that is more
+// than a quarter full is left alone: the second launch then needs a pass of its own as long as what it saves.  0: no split.
 inline int64_t tail_tile_columns(int64_t M, int64_t N, int64_t batch) {
   const int64_t cus = compute_units();
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256;
@@ -51,7 +49,7 @@ template <bool AK, bool BK_, int FA, int FB>
 void launch_256x256(const GemmArgs& g, int64_t batch, hipStream_t st) {
   // the fast bf16 epilogue without an accumulate input: four waves on the 16x16x128 MFMA (gemm_tile16.h)
   if (g.fast_epi && g.D == nullptr) launch_tile16<AK, BK_, FA, FB>(g, batch, st);
-  else launch_tile<256, 256, 4, false, AK, BK_, FA, FB>(g, batch, st);
+  else launch_tile<AK, BK_, FA, FB>(g, batch, st);
 }
 
 template <bool AK, bool BK_, int FA, int FB>

@@ -1,6 +1,6 @@
 // fp8 x fp8 -> fp32-accumulate -> bf16/fp32 GEMM for gfx950 (fp8_gemm_v2).
 //
-// Tiled kernel: a workgroup of 2 x WN waves owns a BM x BN tile of C and walks K
+// Tiled kernel: a workgroup of 2 x 4 waves owns a 256 x 256 tile of C and walks K
 // in steps of 128 bytes.  Operand tiles travel from global memory straight into
 // LDS (buffer_load_dwordx4 ... lds: no staging registers, and the buffer
 // descriptor's bounds check zero-fills rows past the matrix edge) into one of
@@ -9,19 +9,17 @@
 // which keeps the 128-bit and transposing fragment reads free of bank
 // conflicts; since a DMA load places lane l's chunk at LDS offset 16 l, the
 // swizzle is applied by choosing which global chunk each lane fetches.  Each
-// wave computes its (BM/2) x (BN/WN) sub-tile with v_mfma_f32_32x32x64_f8f6f4
+// wave computes its 128 x 64 sub-tile with v_mfma_f32_32x32x64_f8f6f4
 // (fp8/bf8 operands, 64 k per instruction), reading the fragments of the next
 // half-step while the MFMAs of the current one run.  The buffer descriptors
 // walk along K by scalar arithmetic, so the per-lane offsets are small
 // constants and operands of any size are addressable.
 //
-// Two wave grids are built.  2 x 4 (eight waves, two per SIMD, 128 x 64 wave
-// tiles at BM = BN = 256): while one wave of a SIMD sits in its epilogue or
-// waits for a fragment, the other keeps the matrix pipe busy; this grid carries
-// both epilogues.  2 x 2 (four waves, one per SIMD, 128 x 128 wave tiles, all
-// 256 accumulation registers): a third fewer LDS fragment bytes per MFMA, which
-// is what matters once the chip runs at its power limit; its epilogue is not
-// hidden by a second wave, so it exists with the fast bf16 epilogue only.
+// The wave grid is 2 x 4 (eight waves, two per SIMD): while one wave of a SIMD
+// sits in its epilogue or waits for a fragment, the other keeps the matrix pipe
+// busy.  Products whose results the fast bf16 epilogue writes without an
+// accumulate input run on four waves of 128 x 128 instead (gemm_tile16.h); this
+// kernel has the fast epilogue with an accumulate input, and the general one.
 //
 // Operand layouts.  An operand whose K index is contiguous in memory (A with
 // trans_a == 0, B with trans_b != 0) is "K-major": a lane's 32-byte MFMA
@@ -56,7 +54,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define LDS_AS __attribute__((address_space(3)))
 
-constexpr int kWavesM = 2;  // the waves of a workgroup form a 2 x WN grid over its tile
+constexpr int kTile = 256, kTileWavesM = 2, kTileWavesN = 4;  // a workgroup's tile of C, and the grid of its waves over it
 constexpr int kBK = 128;  // bytes (= fp8 elements) of K per LDS stage
 
 // Number of compute units of the current device (workgroups of the persistent kernel).
@@ -676,7 +674,7 @@ constexpr int fast_epilogue_stores() { return MT * 2 * NT; }
 // rows (fp32).  Values of a kind the problem does not have are zeros.
 constexpr int kStagedColScale = 0, kStagedBias = 512, kStagedRowScale = 768, kStagedBytes = 1280;
 
-template <int MT, int NT, bool PER_COL, bool HAS_BIAS, bool HAS_D = false>
+template <int MT, int NT, bool PER_COL, bool HAS_BIAS>
 __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t batch, f32x16 (&acc)[MT][NT],
                                                    int m_wave, int n_wave, float* stage_f, ScalarScales scalars) {
   static_assert(MT <= 4 && NT <= 4, "staged layout");
@@ -741,27 +739,21 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
 
   // The accumulate input, read in the accumulator layout (4 bf16 per lane and
   // column group): rows past M fall outside the descriptor and read as zero.
-  __amdgpu_buffer_rsrc_t rsrc_d = rsrc;
-  int d_off0 = 0, d_pitch = 0;
-  if constexpr (HAS_D) {
-    const uint16_t* dbase = reinterpret_cast<const uint16_t*>(g.D) + batch * g.stride_d + (int64_t)m_wave * g.ldd;
-    rsrc_d = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(dbase), 0, rows > 0 ? rows * (int)g.ldd * 2 : 0, 0x00020000);
-    d_pitch = (int)g.ldd * 2;
-    d_off0 = r * d_pitch + (n_wave + 4 * h) * 2;
-  }
+  const uint16_t* dbase = reinterpret_cast<const uint16_t*>(g.D) + batch * g.stride_d + (int64_t)m_wave * g.ldd;
+  const __amdgpu_buffer_rsrc_t rsrc_d =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(dbase), 0, rows > 0 ? rows * (int)g.ldd * 2 : 0, 0x00020000);
+  const int d_pitch = (int)g.ldd * 2, d_off0 = r * d_pitch + (n_wave + 4 * h) * 2;
 
   // scaled, rounded values of the 32 rows of accumulator row i -> staging area
   auto write_rows = [&](auto ic) {
     constexpr int i = decltype(ic)::value;
-    u32x2 dv[HAS_D ? NT : 1][4];
-    if constexpr (HAS_D) {
+    u32x2 dv[NT][4];
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          dv[j][q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
-              rsrc_d, d_off0 + 32 * i * d_pitch + (32 * j + 8 * q) * 2, 0, 0));
-    }
+      for (int q = 0; q < 4; ++q)
+        dv[j][q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+            rsrc_d, d_off0 + 32 * i * d_pitch + (32 * j + 8 * q) * 2, 0, 0));
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -773,12 +765,10 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
           if constexpr (PER_COL) v[e] = __builtin_fmaf(acc[i][j][4 * q + e] * ra[i], cs[j][q][e], b);
           else v[e] = __builtin_fmaf(acc[i][j][4 * q + e], ra[i], b);
         }
-        if constexpr (HAS_D) {
-          v[0] += __uint_as_float(dv[j][q][0] << 16);
-          v[1] += __uint_as_float(dv[j][q][0] & 0xffff0000u);
-          v[2] += __uint_as_float(dv[j][q][1] << 16);
-          v[3] += __uint_as_float(dv[j][q][1] & 0xffff0000u);
-        }
+        v[0] += __uint_as_float(dv[j][q][0] << 16);
+        v[1] += __uint_as_float(dv[j][q][0] & 0xffff0000u);
+        v[2] += __uint_as_float(dv[j][q][1] << 16);
+        v[3] += __uint_as_float(dv[j][q][1] & 0xffff0000u);
         const u32x2 o = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
         const int slot = (8 * j + 2 * q + h) ^ f_w;
         *reinterpret_cast<LDS_AS u32x2*>(stage + r * kRowBytes + slot * 8) = o;
@@ -819,20 +809,10 @@ __device__ __forceinline__ void epilogue_bf16_fast(const GemmArgs& g, int64_t ba
   });
 }
 
-// ALLOW_D false: the caller guarantees there is no accumulate input (the
-// kernel with 256 accumulator registers per lane keeps its epilogue to four
-// variants; with more, the compiler copies accumulators to scratch memory).
-template <int MT, int NT, bool ALLOW_D = true>
+template <int MT, int NT>
 __device__ __forceinline__ void epilogue_bf16_fast_any(const GemmArgs& g, int64_t batch, f32x16 (&acc)[MT][NT],
                                                        int m_wave, int n_wave, float* stage, ScalarScales scalars) {
   const bool per_col = g.sb_mode == MI355Q_GS_PER_COL, bias = g.bias_mode == MI355Q_BIAS_ROW_VECTOR;
-  if (ALLOW_D && g.D != nullptr) {
-    if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else if (per_col) epilogue_bf16_fast<MT, NT, true, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else if (bias) epilogue_bf16_fast<MT, NT, false, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    else epilogue_bf16_fast<MT, NT, false, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
-    return;
-  }
   if (per_col && bias) epilogue_bf16_fast<MT, NT, true, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
   else if (per_col) epilogue_bf16_fast<MT, NT, true, false>(g, batch, acc, m_wave, n_wave, stage, scalars);
   else if (bias) epilogue_bf16_fast<MT, NT, false, true>(g, batch, acc, m_wave, n_wave, stage, scalars);
@@ -884,24 +864,22 @@ struct ScaleStager {
 
 // Per-wave state of the K loop: accumulators, fragments, loaders.
 //
-// Register budget.  Two waves per SIMD (WN = 4) leave 256 registers per lane:
-// 128 hold the accumulators of the 128 x 64 wave tile, so the fragments get 64.
-// One wave per SIMD (WN = 2) has 512: 256 accumulators of the 128 x 128 wave
-// tile, 96 for fragments.  In both the B fragments are double-buffered (the
-// next half-step's set is read while the current one is in use), the A
-// fragments are single-buffered and rolled: MFMAs run row by row, A_i is dead
-// after the last MFMA of row i, and the next half-step's A_i is read into the
-// same registers right then.
-template <int BM, int BN, int WN, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
+// Register budget.  Two waves per SIMD leave 256 registers per lane: 128 hold the
+// accumulators of the 128 x 64 wave tile, so the fragments get 64.  The B
+// fragments are double-buffered (the next half-step's set is read while the
+// current one is in use), the A fragments single-buffered and rolled: MFMAs run
+// row by row, A_i is dead after the last MFMA of row i, and the next half-step's
+// A_i is read into the same registers right then.
+template <bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
 struct TileCore {
-  static constexpr int TM = BM / kWavesM, TN = BN / WN;
-  using LoaderA = DmaLoader<A_KMAJOR, BM, kBK, kWavesM * WN>;
-  using LoaderB = DmaLoader<B_KMAJOR, BN, kBK, kWavesM * WN>;
+  static constexpr int TM = kTile / kTileWavesM, TN = kTile / kTileWavesN;
+  using LoaderA = DmaLoader<A_KMAJOR, kTile, kBK, kTileWavesM * kTileWavesN>;
+  using LoaderB = DmaLoader<B_KMAJOR, kTile, kBK, kTileWavesM * kTileWavesN>;
   static constexpr int MT = TM / 32, NT = TN / 32;
-  using ReaderA = FragReader<A_KMAJOR, BM, MT>;
-  using ReaderB = FragReader<B_KMAJOR, BN, NT>;
+  using ReaderA = FragReader<A_KMAJOR, kTile, MT>;
+  using ReaderB = FragReader<B_KMAJOR, kTile, NT>;
   // LDS ring: the two stages of A, then the two stages of B
-  static constexpr int kStageA = BM * kBK, kStageB = BN * kBK;
+  static constexpr int kStageA = kTile * kBK, kStageB = kTile * kBK;
   static constexpr int kRingBytes = 2 * (kStageA + kStageB);
   f32x16 acc[MT][NT];
   i32x8 fa[MT], fb0[NT], fb1[NT];
@@ -1062,12 +1040,10 @@ __device__ __forceinline__ void tile_coords(int logical, int tiles_m, int tiles_
 // a contiguous range of the tile order, and in pass r its workgroups take the
 // next gridDim.x / 8 tiles of that range, so that the tiles in flight on one
 // XCD form a compact patch that shares A and B panels in its L2.
-template <int BM, int BN, int WN, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B, bool FAST_ONLY>
-__global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmArgs g) {
-  constexpr int kWaves = kWavesM * WN;
-  constexpr int TM = BM / kWavesM, TN = BN / WN;   // per-wave tile
-  constexpr int MT = TM / 32, NT = TN / 32;             // MFMA tiles per wave
-  using Core = TileCore<BM, BN, WN, A_KMAJOR, B_KMAJOR, FMT_A, FMT_B>;
+template <bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
+__global__ __launch_bounds__(kTileWavesM * kTileWavesN * 64) void fp8_gemm_tile_kernel(GemmArgs g) {
+  using Core = TileCore<A_KMAJOR, B_KMAJOR, FMT_A, FMT_B>;
+  constexpr int kWaves = kTileWavesM * kTileWavesN, MT = Core::MT, NT = Core::NT;
   // two stages of each operand; the epilogue has its own staging area
   __shared__ __attribute__((aligned(1024))) uint8_t lds_ring[Core::kRingBytes];
   __shared__ __attribute__((aligned(16))) float lds_epi[kWaves * epilogue_stage_floats<MT, NT>()];
@@ -1082,7 +1058,7 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
 
   const int64_t batch = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = (wave / WN) * TM, wn = (wave % WN) * TN;
+  const int wm = (wave / kTileWavesN) * Core::TM, wn = (wave % kTileWavesN) * Core::TN;
   float* stage = lds_epi + wave * epilogue_stage_floats<MT, NT>();
 
   Core core;
@@ -1101,13 +1077,13 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
   int tile_m, tile_n;
   tile_coords(first + idx, g.tiles_m, g.tiles_n, &tile_m, &tile_n);
   core.set_lane_addresses(g);
-  core.retarget(g, batch, tile_m * BM, tile_n * BN, true);
+  core.retarget(g, batch, tile_m * kTile, tile_n * kTile, true);
   core.template issue_stage<0>(0);
   core.template issue_stage<1>(1);
   const ScalarScales scalars = load_scalar_scales(g);
   bool stores_pending = false;  // the fast epilogue's stores of the previous tile
   for (;;) {
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * kTile, n0 = tile_n * kTile;
     core.first_fragments(stores_pending);
     // Two stages per step; the step that issues the last loads of this tile's
     // stages (the last one) first points the loaders at the next tile.
@@ -1116,20 +1092,20 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
         idx += slots;
         const bool more = idx < count;
         if (more) tile_coords(first + idx, g.tiles_m, g.tiles_n, &tile_m, &tile_n);
-        core.retarget(g, batch, tile_m * BM, tile_n * BN, more);
+        core.retarget(g, batch, tile_m * kTile, tile_n * kTile, more);
       }
       // stage numbers restart at 0 for the next tile
       core.template k_pair<decltype(first_c)::value>(kt + 2 == KT2 ? -2 : kt, stores_pending, [&] {
-        if (FAST_ONLY || g.fast_epi) ScaleStager::issue<MT, NT>(g, batch, m0 + wm, n0 + wn, stage);
+        if (g.fast_epi) ScaleStager::issue<MT, NT>(g, batch, m0 + wm, n0 + wn, stage);
       });
     };
     k_step(std::true_type{}, 0);
     for (int kt = 2; kt < KT2; kt += 2) k_step(std::false_type{}, kt);
-    if (FAST_ONLY || g.fast_epi) {
-      epilogue_bf16_fast_any<MT, NT, !FAST_ONLY>(g, batch, core.acc, m0 + wm, n0 + wn, stage, scalars);
+    if (g.fast_epi) {
+      epilogue_bf16_fast_any<MT, NT>(g, batch, core.acc, m0 + wm, n0 + wn, stage, scalars);
       // A store whose lanes are all past M or N completes at once and must not be counted as
       // outstanding: after a tile on the matrix edge the next tile waits for everything.
-      stores_pending = m0 + BM <= g.M && n0 + BN <= g.N;
+      stores_pending = m0 + kTile <= g.M && n0 + kTile <= g.N;
     } else {
       epilogue<MT, NT>(g, batch, core.acc, m0 + wm, n0 + wn, stage);
     }
@@ -1140,18 +1116,17 @@ __global__ __launch_bounds__(kWavesM * WN * 64) void fp8_gemm_tile_kernel(GemmAr
   __builtin_amdgcn_s_waitcnt(0);
 }
 
-// WN: waves along n (the workgroup has 2 x WN); FAST_ONLY: the kernel carries
-// the fast bf16 epilogue alone, without an accumulate input: the launch must
-// satisfy epilogue_fast_ok() and have no D.
-template <int BM, int BN, int WN, bool FAST_ONLY, bool AK, bool BK_, int FA, int FB>
+// The launch has fp32 results, an accumulate input, or another form that the four-wave kernel does not write.
+template <bool AK, bool BK_, int FA, int FB>
 void launch_tile(const GemmArgs& g, int64_t batch, hipStream_t st) {
   GemmArgs a = g;
-  a.tiles_m = (g.M + BM - 1) / BM;
-  a.tiles_n = (g.N + BN - 1) / BN;
+  a.fast_epi = g.fast_epi && g.D != nullptr;  // (the fast epilogue of this kernel has an accumulate input)
+  a.tiles_m = (g.M + kTile - 1) / kTile;
+  a.tiles_n = (g.N + kTile - 1) / kTile;
   const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
   const int cus = compute_units();
   dim3 grid((unsigned)(tiles < cus ? tiles : cus), (unsigned)batch);
-  fp8_gemm_tile_kernel<BM, BN, WN, AK, BK_, FA, FB, FAST_ONLY><<<grid, kWavesM * WN * 64, 0, st>>>(a);
+  fp8_gemm_tile_kernel<AK, BK_, FA, FB><<<grid, kTileWavesM * kTileWavesN * 64, 0, st>>>(a);
 }
 
 }  // namespace mi355q
