@@ -16,7 +16,7 @@ ops = torch.ops.hpu
     (520, 1024, 1001),    # only N ragged
     (515, 1024, 1008),    # only M ragged
     (512, 1030, 512),     # only K ragged
-    (70, 4100, 1999),     # few rows: the strip kernel
+    (70, 4100, 1999),     # few rows: K in parts
 ])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 def test_ragged_large_products_are_exact(dev, M, K, N, ta, tb):

@@ -199,8 +199,8 @@ def test_parts_of_k_meet_by_device_scope_accesses_in_order():
     """Sums stored (sc1), acknowledged, barrier, ticket, barrier, counter reset, sums read (sc1); nothing cache-wide."""
     import re
     from concurrent.futures import ThreadPoolExecutor
-    # the strip kernel has three heights with an A [M, K] and one with an A [K, M], the tiles two sizes, four pairs of formats
-    sources = (("gemm_stream.hip", 4), ("gemm_inst_kk.hip", 20), ("gemm_inst_km.hip", 20), ("gemm_inst_mk.hip", 12), ("gemm_inst_mm.hip", 12))
+    # the ring kernel has six heights with an A [M, K] and two with an A [K, M], each for four pairs of formats and B with the nontemporal hint or not
+    sources = (("gemm_stream.hip", 4), ("gemm_inst_kk.hip", 48), ("gemm_inst_km.hip", 48), ("gemm_inst_mk.hip", 16), ("gemm_inst_mm.hip", 16))
     with ThreadPoolExecutor(max_workers=4) as ex:
         texts = list(ex.map(isa_check.compile_to_isa, [src for src, _ in sources]))
     for (src, least), text in zip(sources, texts):
