@@ -51,21 +51,21 @@ MEASURED_TRAFFIC = {
     "convert_from_int4": 43.10e6,
     "fp8_gemm_v2": 939.89e6,
     "fp8_gemm_v2_B_NK": 939.33e6,
-    "fp8_gemm_v2_decode_M16": 236.92e6,
+    "fp8_gemm_v2_decode_M16": 244.33e6,
     "fp8_gemm_v2_decode_M64": 242.92e6,
-    "fp8_gemm_v2_decode_M256": 266.37e6,
-    "w4a8_gemm_M16": 130.86e6,      # the partial sums of the two K parts on top of the 124 MB of operands
-    "w4a8_gemm_M32": 139.63e6,
-    "w4a8_gemm_M64": 157.22e6,
-    "w4a8_gemm_M256": 153.68e6,     # two row blocks of 128 on one XCD share a strip's weights in its L2
-    "w4a16_gemm_M16": 131.96e6,     # split_rows_vec_kernel + w4a8_wide_kernel<two planes>
-    "w4a16_gemm_M64": 161.49e6,
-    "w4a16_gemm_M256": 178.91e6,
-    "fp8_sdpa_B1_L8192": 124.63e6,
-    "fp8_sdpa_B4_L4096": 235.55e6,
-    "fp8_sdpa_B1_L8192_D256": 347.00e6,   # k and v are re-read by the query blocks of a head group beyond L2
-    "fp8_sdpa_decode_B64_S4096": 537.37e6,
-    "fp8_sdpa_decode_B8_S8192": 143.15e6,   # fp8_sdpa_decode_kernel 138.81 + 4.34 written and read back by the merge
+    "fp8_gemm_v2_decode_M256": 266.36e6,
+    "w4a8_gemm_M16": 129.02e6,      # the partial sums of the two K parts on top of the 124 MB of operands
+    "w4a8_gemm_M32": 135.97e6,
+    "w4a8_gemm_M64": 149.87e6,
+    "w4a8_gemm_M256": 153.59e6,     # two row blocks of 128 on one XCD share a strip's weights in its L2
+    "w4a16_gemm_M16": 130.15e6,     # split_rows_vec_kernel + w4a8_wide_kernel<two planes>
+    "w4a16_gemm_M64": 154.13e6,
+    "w4a16_gemm_M256": 178.81e6,
+    "fp8_sdpa_B1_L8192": 124.80e6,
+    "fp8_sdpa_B4_L4096": 235.33e6,
+    "fp8_sdpa_B1_L8192_D256": 354.91e6,   # k and v are re-read by the query blocks of a head group beyond L2
+    "fp8_sdpa_decode_B64_S4096": 537.24e6,
+    "fp8_sdpa_decode_B8_S8192": 136.71e6,   # fp8_sdpa_decode_kernel 135.57 + 1.14 written and read back by the merge
     "softmax_fp8": 1609.32e6,
     "sum_fp8_rows": 67.32e6,
     "sum_fp8_columns": 73.44e6,   # sum_columns_kernel 69.20 + sum_finish_kernel 4.24

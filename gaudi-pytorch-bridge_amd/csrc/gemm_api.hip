@@ -86,10 +86,11 @@ struct RingCost {
 };
 // Least-squares fits to 480 products (1 to 4096 rows, K from 512 to 16384, N from 256 to 28672, both layouts of B, whole and
 // in 2 to 24 parts), each timed with the weights hot in the caches and cold and counted half and half.  The choice they make is
-// 1.8 % slower in the mean than the best one measured.  The line of the 256-row tile is lowered by a tenth, which costs nothing
-// over the sample and halves the reads of B where it decides.
-// The line of the 192-row tile lies between its neighbours' and a little above where they would meet: of 70 products timed on
-// the tiles of 128, 192 and 256 rows and of 256 x 256 it is chosen for 8, which are 7.6 % faster in the mean and none slower.
+// 1.8 % slower in the mean than the best one measured, and 2.5 % over 240 other products of the
+// same ranges.  The line of the 256-row tile is lowered by a tenth, which changed none of the 240
+// choices.  The line of the 192-row tile lies between its neighbours' and a little above where they would meet: without it the 240
+// take 3.0 %; of the 19 it is chosen for 16 are 1 to 20 % faster than on what would be chosen else, 3 slower (129 x 8992 x 7888 40 us
+// against 31 on two parts of 128 rows).
 constexpr RingCost kRingCosts[] = {
     {GemmKind::kRing16, 16, 2.84, 0.28, 0.44, 0.75, 0.83, 0.41, 1.10},
     {GemmKind::kRing32, 32, 3.18, 0.29, 0.26, 0.61, 1.29, 1.25, 1.34},

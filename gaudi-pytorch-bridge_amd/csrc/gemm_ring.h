@@ -3,7 +3,10 @@
 //
 // What bounds it.  A compute unit keeps about 32 KB of lines on their way, whatever asks for them (a loop that only loads, into
 // LDS or registers, 4 to 16 waves: 48 to 55 KB/us from HBM at 0.63 us a load, 150 to 200 KB/us from the XCD's L2): its intake is
-// what a stage costs, (rows + 128) x 128 bytes, and a wave that issues loads beyond that limit stalls.  Hence
+// what a stage costs, (rows + 128) x 128 bytes, and a wave that issues loads beyond that limit stalls.  Where both kinds mix, all of it
+// comes at HBM's rate: 256 x 8192 x 28672 takes 64 us for a workgroup's 3 MiB (49 KB/us) though the 2 MiB of A are found in the L2
+// (252 MB read from HBM in all), so A's lines, which a wave requests in turn with B's and gets back in that order, gain nothing
+// from it.  Loading waves of their own for either operand have not been tried with this ring.  Hence
 //  * four waves that only load and four that only multiply, one of each per SIMD, meeting at one barrier per stage: the
 //    loading waves' stalls hold up no MFMA, and the multiplying waves' loop is MFMAs, fragment reads and one addition per
 //    address register;

@@ -507,8 +507,9 @@ int mi355q_pad_rows(const mi355q_pad_desc* desc, int count, void* stream);
 
 /* Name of the kernel variant that mi355q_fp8_gemm picks for a problem of one
  * batch with 16-byte aligned operands, and of the one that mi355q_fp8_gemm_ws
- * picks with a workspace ("split_...": K in parts over workgroups).  For logs
- * and profiles; static strings. */
+ * picks with a workspace ("split_...": K in parts over workgroups): the kernel
+ * (ring, stream, tile or simple) and its tile, rows x columns x bytes of K per
+ * stage.  For logs and profiles; static strings. */
 const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb,
                                     int64_t M, int64_t N, int64_t K);
 const char* mi355q_fp8_gemm_ws_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb,
