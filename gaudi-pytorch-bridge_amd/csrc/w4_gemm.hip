@@ -1150,11 +1150,15 @@ struct W4WidePlan {
   }
 };
 // What a part of K costs, in microseconds: a stage of a tile, the parts' meeting, what each part adds to it and what a full chip
-// does.  From products of 7 to 490 rows, K from 1408 to 12288 and N from 1312 to 28672, timed in one to 24 parts: 7 x 1408 x 1664 with
+// does, and what it does on top to parts of fewer than ten stages where two compute units in five have a workgroup and more (short_full).
+// From products of 7 to 490 rows, K from 1408 to 12288 and N from 1312 to 28672, timed in one to 24 parts: 7 x 1408 x 1664 with
 // two planes takes 14.9 us whole, 12.2 in four parts and 13.6 in eleven, 48 rows 20.4, 14.0 and 13.9.  fp8 activations: parts of
-// eight stages at least (a part more of short products gained a microsecond at most up to 32 rows).
+// eight stages at least (a part more of short products gained a microsecond at most up to 32 rows).  The last term, for two planes up to
+// 64 rows: 470 products of 1 to 64 rows, K from 1024 to 16384 and N from 1024 to 28672, in every number of parts; without it one in ten
+// up to 32 rows was slower than in parts of eight stages and more (3 x 1024 x 14208 in four parts 12.8 us, in two 11.8; 2 x 3840 x 10368 in six
+// 16.8, in five 16.0; 40 x 2560 x 20480 in three 23.6, in two 21.5).
 struct W4Cost {
-  double stage, meet, part, crowd;
+  double stage, meet, part, crowd, short_full;
 };
 inline W4WidePlan w4_wide_plan(int64_t M, int64_t N, int64_t K, int64_t group, int scale_f32, bool a16) {
   W4WidePlan p{0, 0, 0, 0};
@@ -1165,14 +1169,16 @@ inline W4WidePlan w4_wide_plan(int64_t M, int64_t N, int64_t K, int64_t group, i
   const int64_t kt = (K + kBK - 1) / kBK, groups = (int64_t)p.strips * p.row_blocks;
   // at most one workgroup per compute unit
   const int64_t most = std::min<int64_t>(256 / groups, kt / (a16 ? 2 : 8));
-  const W4Cost c = p.rows == 16   ? W4Cost{0.57, 1.0, 0.40, 0.5}
-                   : p.rows == 32 ? W4Cost{0.63, 1.0, 0.50, 2.0}
-                   : p.rows == 64 ? W4Cost{a16 ? 0.98 : 0.70, 1.0, 0.25, 6.0}
-                                  : W4Cost{a16 ? 1.65 : 1.15, 1.0, 0.25, 9.0};
+  const W4Cost c = p.rows == 16   ? W4Cost{0.57, 1.0, 0.40, 0.5, a16 ? 1.5 : 0.0}
+                   : p.rows == 32 ? W4Cost{0.63, 1.0, 0.50, 2.0, a16 ? 6.0 : 0.0}
+                   : p.rows == 64 ? W4Cost{a16 ? 0.98 : 0.70, 1.0, 0.25, 6.0, a16 ? 3.0 : 0.0}
+                                  : W4Cost{a16 ? 1.65 : 1.15, 1.0, 0.25, 9.0, 0.0};
   double best = (double)kt * c.stage;
   p.parts = 1;
   for (int64_t n = 2; n <= most; ++n) {
-    const double us = (double)((kt + n - 1) / n) * c.stage + c.meet + c.part * (double)n + c.crowd * (double)(groups * n) / 256.0;
+    const double share = (double)(groups * n) / 256.0, over = std::max(0.0, share - 0.4) / 0.6;
+    double us = (double)((kt + n - 1) / n) * c.stage + c.meet + c.part * (double)n + c.crowd * share;
+    if (n * 10 > kt) us += c.short_full * over * over;
     if (us >= best) continue;
     best = us;
     p.parts = (int)n;

@@ -180,3 +180,16 @@ def test_one_workspace_serves_shapes_with_and_without_a_split(oracle, pkg, dev):
         torch.cuda.synchronize()
         assert torch.equal(C.cpu().double(), expect), (M, K, N)
         assert torch.count_nonzero(ws[:1024]) == 0
+
+
+def test_parts_that_fill_the_chip_are_not_taken_for_their_own_sake(pkg):
+    """bf16 activations of few rows went in as many parts of two stages as the chip holds, slower than in fewer (and than whole, at K = 1024)."""
+    def parts(M, K, N):
+        up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+        sums = pkg.capi().mi355q_w4a16_gemm_workspace_bytes(M, N, K, 128, pkg.BF16) - 2 * up(M * K) - up(4 * M) - 1024
+        return sums / ((N + 255) // 256 * (64 if M > 32 else 32) * 256 * 4)
+
+    for m, k, n, most in [(3, 1024, 14208, 2), (5, 1024, 14848, 2), (2, 3840, 10368, 5), (40, 2560, 20480, 2)]:
+        assert parts(m, k, n) <= most, (m, k, n, parts(m, k, n))
+    # parts of ten stages and more, and those that leave most of the chip idle
+    assert parts(16, 8192, 28672) == 2 and parts(7, 1408, 1664) >= 4 and parts(20, 14592, 7616) == 8 and parts(53, 2816, 2496) == 8
