@@ -43,7 +43,7 @@
 #include <algorithm>
 #include <mutex>
 
-#include "gemm_tile.h"
+#include "w4_stream.h"
 
 namespace mi355q {
 
@@ -57,23 +57,6 @@ constexpr int kW4PackedStage = kBK * kW4BN / 2;  // bytes of packed weights per 
 constexpr int kW4ScaleRow = 1024;
 constexpr int kW4ZpRow = 1024;
 
-struct W4Args {
-  GemmArgs g;              // A, C, M, N, K, lda, ldc, sa*, bias*, out_bf16 (B, sb*, D unused)
-  const uint8_t* packed;   // int32 [K, N / 8]
-  int64_t ld_packed;       // bytes between k-rows
-  const uint8_t* scale;    // [K / group, N] bf16 or fp32
-  const uint8_t* zp;       // packed int32 [K / group, N / 8] or nullptr
-  int scale_f32, is_signed;
-  int stages_per_group;    // group / 128
-  // wide kernel: K is walked in `ksplit` parts by as many workgroups per strip
-  int ksplit;
-  uint32_t* tickets;       // one per strip, zero between launches
-  float* partials;         // [ksplit][strips] partial sums of 32 x 256, in the consumers' register order
-  // 16-bit activations as two fp8 planes (wide kernel, A16): g.A holds the leading part of every value and a_lo,
-  // with the same pitch, 16 times what is left of it (split_rows_kernel); a = (A + a_lo / 16) / row scale
-  const uint8_t* a_lo;
-};
-
 template <int BM>
 constexpr int w4_stage_bytes() { return BM * kBK + kW4PackedStage + kW4ScaleRow + kW4ZpRow; }
 
@@ -81,25 +64,6 @@ template <int BM>
 constexpr int w4_stages() {
   constexpr int s = (160 * 1024) / w4_stage_bytes<BM>();
   return s > 10 ? 10 : s;
-}
-
-// One 16-byte piece per lane, straight copy into LDS (lane l lands at dst + 16 l).  The
-// s_nop covers a descriptor word that reached its scalar register through a vector
-// instruction (five wait states before a memory instruction may read it).
-// STREAM adds the nontemporal hint, for weights that the launch reads once.
-template <bool STREAM = false>
-__device__ __forceinline__ void w4_dma16(const i32x4& rsrc, int voff, uint32_t lds_dst) {
-  if constexpr (STREAM) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
-                 :
-                 : "s"(lds_dst), "v"(voff), "s"(rsrc)
-                 : "memory", "m0");
-  } else {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :
-                 : "s"(lds_dst), "v"(voff), "s"(rsrc)
-                 : "memory", "m0");
-  }
 }
 
 // A buffer descriptor that walks through memory in fixed steps: base and the bytes left behind it.
@@ -537,7 +501,6 @@ constexpr int kW4SumRing = 4;  // stages of row sums kept
 // that lane i of its group of 16 addresses, so the lanes address the rows in the order that leaves k ascending
 // over the two registers (w4_nibble_row).
 constexpr int kW4ByteScale = 127 + 9;
-__device__ __forceinline__ int w4_nibble_row(int i) { return (i & 8) | ((i & 1) << 2) | ((i >> 1) & 3); }
 __device__ __forceinline__ i32x8 w4_bytes(const i32x2& w0, const i32x2& w1, uint32_t flip) {
   i32x8 r;
 #pragma unroll
@@ -557,50 +520,6 @@ template <int FMT_A>
 __device__ __forceinline__ f32x4 w4_mfma16(const u32x4& plane, const i32x8& fa, const f32x4& c, int e) {
   const i32x8 b = {(int)plane[0], (int)plane[1], (int)plane[2], (int)plane[3], 0, 0, 0, 0};
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b, fa, c, 4, mfma_code<FMT_A>(), 0, e, 0, 127);
-}
-
-// What the epilogue multiplies a row by and adds to its columns.  Loaded for all of a lane's results before the first is stored: a
-// load behind a store waits for a trip to the L2 of its own, and a lane of a 128-row tile has
-// sixteen (uint4, us, before and after: 512 x 4096 x 16384 54.5 -> 51.8, two planes 74.5 -> 70.9; 60 x 4096 x 40960 36.3 -> 34.7,
-// 41.7 -> 40.5; 133 x 10112 x 21696 two planes 140.5 -> 135.5; parts added up by a second launch +- 0).  (Rows and columns past the
-// edge read the last ones; they are not stored.)
-__device__ __forceinline__ float w4_row_scale(const GemmArgs& g, const ScalarScales& scalars, int m) {
-  return g.sa_mode == MI355Q_GS_PER_ROW ? g.sa[m < g.M ? m : g.M - 1] : scalars.sa;
-}
-__device__ __forceinline__ f32x4 w4_bias4(const GemmArgs& g, int n) {
-  f32x4 b = {0.f, 0.f, 0.f, 0.f};
-  if (g.bias_mode == MI355Q_BIAS_ROW_VECTOR) {
-    const int from = n < g.N ? n : g.N - 4;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) b[e] = load_out_as_f32(g.bias, from + e, g.out_bf16);
-  }
-  return b;
-}
-
-// The epilogue of four columns of a row: N is a multiple of 32, so they are inside or outside together.
-__device__ __forceinline__ void w4_store4(const GemmArgs& g, int m, int n, const f32x4& sums, float sa, const f32x4& bias) {
-  if (m >= g.M || n >= g.N) return;
-  const int es = g.out_bf16 ? 2 : 4;
-  float v[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = __fmul_rn(sums[e], sa) + bias[e];  // rounded as the other epilogues round
-  uint8_t* cp = g.C + ((int64_t)m * g.ldc + n) * es;
-  const bool vec_ok = (reinterpret_cast<uintptr_t>(cp) % (4 * es)) == 0;
-  if (g.out_bf16) {
-    if (vec_ok) {
-      *reinterpret_cast<u32x2*>(cp) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) reinterpret_cast<uint16_t*>(cp)[e] = (uint16_t)(pack_bf16x2(v[e], v[e]) & 0xffffu);
-    }
-  } else {
-    if (vec_ok) {
-      *reinterpret_cast<f32x4*>(cp) = f32x4{v[0], v[1], v[2], v[3]};
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) reinterpret_cast<float*>(cp)[e] = v[e];
-    }
-  }
 }
 
 // Whether the parts are added up by w4_finish_kernel.  Two parts of 64 rows are not: there the launch costs more than the one
@@ -1144,7 +1063,7 @@ struct W4WidePlan {
   // The counters sit in front of the partial sums, in an area of a fixed size: a workspace that is used for
   // problems of different shapes then finds them zero whatever the last shape left in the partial sums.
   // K is only split for at most 128 strips (256 / groups >= 2 below).
-  static constexpr size_t ticket_bytes() { return 1024; }
+  static constexpr size_t ticket_bytes() { return kW4TicketBytes; }
   size_t workspace_bytes() const {
     return parts < 2 ? 0 : ticket_bytes() + (size_t)parts * strips * row_blocks * w4_wide_partial_bytes(tile_rows());
   }
@@ -1188,6 +1107,17 @@ inline W4WidePlan w4_wide_plan(int64_t M, int64_t N, int64_t K, int64_t group, i
   if (p.parts < 2 && groups < 100) p.parts = 0;
   if (p.row_blocks > 65535) p.parts = 0;
   if (p.parts >= 2 && (size_t)groups * 4 > W4WidePlan::ticket_bytes()) p.parts = 1;  // (cannot happen: 256 / groups >= 2)
+  return p;
+}
+
+// The stream kernel's plan for a call (see w4_stream.hip), in as many parts as the caller's workspace has room for; parts 0 where the
+// kernel does not take the call or would want parts and has no room.
+inline W4StreamPlan w4_stream_plan_for(int64_t M, int64_t N, int64_t K, int64_t group, int scale_f32, bool a16, int64_t lda, int64_t ld_packed, size_t workspace_bytes) {
+  W4StreamPlan p = w4_stream_plan(M, N, K, group, scale_f32, a16);
+  if (lda > kW4StMostPitch || ld_packed > kW4StMostPitch) p.parts = 0;
+  const int wanted = p.parts;
+  while (p.parts > 1 && p.workspace_bytes() > workspace_bytes) --p.parts;
+  if (wanted > 1 && p.parts < 2) p.parts = 0;
   return p;
 }
 
@@ -1261,7 +1191,8 @@ using namespace mi355q;
 
 extern "C" size_t mi355q_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int scale_dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || group <= 0) return 0;
-  return w4a16_layout(M, N, K, group, scale_dtype == MI355Q_F32).total;
+  const int scale_f32 = scale_dtype == MI355Q_F32;
+  return std::max(w4a16_layout(M, N, K, group, scale_f32).total, w4_stream_plan(M, N, K, group, scale_f32, true).workspace_bytes());
 }
 
 extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const int32_t* packed, int64_t ld_packed,
@@ -1288,20 +1219,13 @@ extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const 
   float* sx_inv = reinterpret_cast<float*>(ws + l.scale_off);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const std::lock_guard<std::mutex> in_order(w4_launch_order(workspace));
-  const int sp = mi355q_split_rows_fp8x2(A, a_dtype, lda, M, K, ws + l.plane_off, ws + l.lo_off, l.ld, sx_inv, stream);
-  if (sp != MI355Q_OK) return sp;
   W4Args a{};
-  a.g.A = ws + l.plane_off;
-  a.a_lo = ws + l.lo_off;
   a.g.C = static_cast<uint8_t*>(C);
-  a.g.lda = l.ld;
   a.g.ldc = ldc;
   a.g.M = (int)M;
   a.g.N = (int)N;
   a.g.K = (int)K;
-  a.g.sa = sx_inv;
   a.g.sa_host = 1.0f;
-  a.g.sa_mode = MI355Q_GS_PER_ROW;
   a.g.sb_mode = MI355Q_GS_NONE;
   a.g.sb_host = 1.0f;
   a.g.bias = static_cast<const uint8_t*>(bias);
@@ -1314,6 +1238,21 @@ extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const 
   a.scale_f32 = 0;
   a.is_signed = is_signed != 0;
   a.stages_per_group = 1;
+  const W4StreamPlan stream_plan = w4_stream_plan_for(M, N, K, group, 0, true, lda, ld_packed, split_k ? workspace_bytes : 0);
+  if (stream_plan.parts > 0) {
+    a.g.A = static_cast<const uint8_t*>(A);
+    a.g.lda = lda;
+    a.g.sa_mode = MI355Q_GS_NONE;
+    launch_w4_stream(a, kW4Bf16, stream_plan, workspace, split_k < 0, st);
+    return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;
+  }
+  const int sp = mi355q_split_rows_fp8x2(A, a_dtype, lda, M, K, ws + l.plane_off, ws + l.lo_off, l.ld, sx_inv, stream);
+  if (sp != MI355Q_OK) return sp;
+  a.g.A = ws + l.plane_off;
+  a.a_lo = ws + l.lo_off;
+  a.g.lda = l.ld;
+  a.g.sa = sx_inv;
+  a.g.sa_mode = MI355Q_GS_PER_ROW;
   const W4WidePlan plan = w4_wide_plan(M, N, K, group, 0, true);
   a.ksplit = 1;
   if (plan.parts >= 2 && split_k) {
@@ -1327,7 +1266,9 @@ extern "C" int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const 
 }
 
 extern "C" size_t mi355q_w4a8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int scale_dtype) {
-  return w4_wide_plan(M, N, K, group, scale_dtype == MI355Q_F32, false).workspace_bytes();
+  const int scale_f32 = scale_dtype == MI355Q_F32;
+  const size_t wide = w4_wide_plan(M, N, K, group, scale_f32, false).workspace_bytes();
+  return std::max(wide, w4_stream_plan(M, N, K, group, scale_f32, false).workspace_bytes());
 }
 
 extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int32_t* packed, int64_t ld_packed,
@@ -1389,9 +1330,12 @@ extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int
     // an empty sum: bias (or zero) through the same epilogue, with no stage to walk
     a.stages_per_group = 1;
   }
+  // up to 16 rows the stream kernel
+  const W4StreamPlan stream_plan = w4_stream_plan_for(M, N, K, group, a.scale_f32, false, lda, ld_packed, workspace != nullptr && al16(workspace) ? workspace_bytes : 0);
   std::unique_lock<std::mutex> in_order;
   if (a.partials != nullptr) in_order = std::unique_lock<std::mutex>(w4_launch_order(workspace));
-  if (fmt_a == MI355Q_E4M3FN) w4a8_launch_by_m<MI355Q_E4M3FN>(a, st);
+  if (stream_plan.parts > 0) launch_w4_stream(a, fmt_a, stream_plan, workspace, false, st);
+  else if (fmt_a == MI355Q_E4M3FN) w4a8_launch_by_m<MI355Q_E4M3FN>(a, st);
   else w4a8_launch_by_m<MI355Q_E5M2>(a, st);
   return hipGetLastError() == hipSuccess ? MI355Q_OK : MI355Q_ERR_LAUNCH;
 }

@@ -313,7 +313,7 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
  * with mi355q_dequant_4bit.
  *
  * workspace: with groups of 128 and bf16 scales, K is walked in parts by several workgroups per
- * 256 columns where that fills the chip better, which meet through `workspace`:
+ * 256 columns (512 up to 16 rows) where that fills the chip better, which meet through `workspace`:
  * mi355q_w4a8_gemm_workspace_bytes() of device memory, 16-byte aligned (0: the shape is not split
  * and no workspace is read).  Its first KiB holds arrival counters (whatever the shape): they have
  * to be zero when a call starts and every call leaves them zero, so a workspace is zero-filled
@@ -389,7 +389,8 @@ int mi355q_softmax_fp8(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * with a bf16.  This is what the reference composes from convert_from_int4 / convert_from_uint4 to
  * bf16 (Int4BaseOp::AddNode, hpu_ops/backend/int4_ops.cpp:40-56: nibble order, (q - z) * s, the
  * group layout of its test, tests/pytest_working/any_mode/test_hpu_convert_from_int4.py:398-476)
- * and a bf16 matmul; here the bf16 [K, N] matrix never exists.  The activations are first cut into
+ * and a bf16 matmul; here the bf16 [K, N] matrix never exists.  Up to 16 rows the product runs in bf16, to
+ * which the nibbles are expanded, exactly, in registers.  Above that the activations are first cut into
  * two e4m3fn planes per row (mi355q_split_rows_fp8x2: a * s = hi + lo / 16 with a power-of-two row
  * scale s, exact for every element within a factor 2^15 of the row's largest and to 3e-8 of that
  * largest otherwise), and both planes meet the packed nibbles in the matrix unit as in
@@ -399,7 +400,8 @@ int mi355q_softmax_fp8(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * aligned, for the planes, the row scales and, in front, the arrival counters and partial sums of
  * the split over K: its first 1 KiB has to be zero before the first use and is left zero, so the
  * buffer can be passed again (calls that may overlap need buffers of their own).  split_k = 0 keeps
- * K in one piece (no counters are touched).  Nothing is allocated.
+ * K in one piece (no counters are touched); with split_k < 0 the parts of up to 16 rows are added up by the
+ * one that comes last alone, where they share that work otherwise (the same bits).  Nothing is allocated.
  */
 size_t mi355q_w4a16_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t group, int scale_dtype);
 int mi355q_w4a16_gemm(const void* A, int a_dtype, int64_t lda, const int32_t* packed, int64_t ld_packed,
