@@ -21,7 +21,7 @@ LIB_KERNELS = os.path.join(HERE, "libmi355q.so")
 LIB_TORCH = os.path.join(HERE, "mi355q_torch.so")
 LIB_PROBE = os.path.join(HERE, "libmi355q_probe.so")
 
-HIP_SOURCES = ["cast_kernels.hip", "int4_kernels.hip", "reduce_kernels.hip", "gemm_api.hip", "gemm_inst_kk.hip", "gemm_inst_km.hip", "gemm_inst_mk.hip", "gemm_inst_mm.hip", "gemm_stream.hip", "w4_gemm.hip", "w4_stream.hip", "sdpa_kernels.hip", "api.cpp"]
+HIP_SOURCES = ["cast_kernels.hip", "int4_kernels.hip", "reduce_kernels.hip", "gemm_api.hip", "gemm_inst_kk.hip", "gemm_inst_km.hip", "gemm_inst_mk.hip", "gemm_inst_mm.hip", "gemm_stream.hip", "gemm_ragged_kk.hip", "gemm_ragged_km.hip", "w4_gemm.hip", "w4_stream.hip", "sdpa_kernels.hip", "api.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

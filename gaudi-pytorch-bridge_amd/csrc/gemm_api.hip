@@ -127,14 +127,14 @@ constexpr double kLog2[kMostParts + 1] = {0.0, 0.0, 1.0, 1.5849625007211562, 2.0
 //    92; below, 12 of 1 x 4096 x 4096 37 against 34, but cold 38 against 50).  Its cut: a workgroup takes in its share of B at 37 GB/s,
 //    or at its share of 6.5 TB/s where more of them run; no part shorter than 512, two turns of its eight waves.
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
-                     bool fp32_rows) {
+                     bool fp32_rows, bool ring_only) {
   SplitPlan best;
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
   const int64_t cus = compute_units(), stages = (K + kBK - 1) / kBK;
   best.batch = batch;
   // (the stream kernel addresses an operand with 31-bit offsets)
   const bool much = N * K > (96LL << 20) || (K >= 2048 && N * K >= (256LL << 20) / batch);
-  if (a_kmajor && !b_kmajor && M <= 16 && much && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) {
+  if (!ring_only && a_kmajor && !b_kmajor && M <= 16 && much && K * ldb < 0x7fff0000LL && M * lda < 0x7fff0000LL) {
     best.kind = GemmKind::kStream;
     best.nb = 256;
     best.strips = (int)((N + 255) / 256);
@@ -153,7 +153,7 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   }
   double best_us = 1e30;
   bool full_chip = false;
-  if (M > 128 && N > 128) {
+  if (!ring_only && M > 128 && N > 128) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256) * batch;
     best_us = (double)((tiles + cus - 1) / cus) * (double)stages * 1.42 + 6.0;
     full_chip = tiles >= cus && !fp32_rows && (2 * tiles >= 3 * cus || stages < 6 || lda % 128 != 0 || ldb % 128 != 0);
@@ -164,13 +164,14 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
     if (full_chip && c.rows != 192) continue;
     const int64_t tiles = ((M + c.rows - 1) / c.rows) * ((N + kRingBN - 1) / kRingBN), wgs = tiles * batch, rounds = (wgs + cus - 1) / cus;
     double fill = (double)std::min(wgs, cus) * per_cu;
-    double us = c.fixed + (double)stages * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round);
+    double in_stages = (double)stages * (c.stage + c.busy * fill) * (1.0 + (double)(rounds - 1) * c.round), us = c.fixed + in_stages;
     const bool in_parts = may_split && (M > 128 || K >= (a_kmajor ? 1792 : 2304));
     const int most = in_parts && stages >= 4 && rounds == 1 ? (int)std::min<int64_t>({cus / wgs, stages / 2, kMostParts}) : 1;
     for (int parts = 1; parts <= most; ++parts) {
       if (parts > 1) {
         fill = (double)(parts * (int)wgs) * per_cu;
-        us = c.fixed + (double)(((unsigned)stages + (unsigned)parts - 1) / (unsigned)parts) * (c.stage + c.busy * fill) + c.meet + c.level * kLog2[parts] + c.crowd * fill;
+        in_stages = (double)(((unsigned)stages + (unsigned)parts - 1) / (unsigned)parts) * (c.stage + c.busy * fill);
+        us = c.fixed + in_stages + c.meet + c.level * kLog2[parts] + c.crowd * fill;
       }
       if (us >= best_us) continue;
       best_us = us;
@@ -179,9 +180,26 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
       best.strips = (int)tiles;
       best.parts = parts;
       best.tile_rows = c.rows;
+      best.stages_us = in_stages;
     }
   }
   return best;
+}
+
+// The plan of a product whose operands lie anywhere (launch_gemm_ragged_*), A [M, K].  parts 0: not served, its operands are better copied
+// first.  That is so where the copies end in 256 x 256 tiles, and where the loads' detour costs more than the copies would: it lengthens
+// the stages by 0.3 for rows at whole dwords (DwordProducer) and by 0.8 for others, and a copy is 4.5 us and twice the bytes at 5 TB/s.
+// us with the copies / without: 1000 x 3000 x 5000 31.4 / 25.1, 16 x 8191 x 28671 122 / 65, 64 x 4100 x 9999 38.1 / 23.9, 1 x 8191 x 20000 B [N, K]
+// 87.7 / 51.6, 300 x 2049 x 1003 16.7 / 13.1, 256 x 8190 x 8190 53.0 / 44.6, but 1000 x 3001 x 5001 35.3 / 36.6, 3779 x 13824 x 1411 82.7 / 96.0.
+SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+  SplitPlan none;
+  none.parts = 0;
+  if (trans_a || M < 1 || N < 16 || K < 256 || batch < 1 || lda > (1LL << 22) || ldb > (1LL << 22)) return none;
+  const auto up = [](int64_t v) { return (v + 15) & ~(int64_t)15; };
+  if (split_plan(true, up(lda), trans_b != 0, up(ldb), M, N, K, batch, may_split).kind == GemmKind::kTile256) return none;
+  const SplitPlan p = split_plan(true, up(lda), trans_b != 0, up(ldb), M, N, K, batch, may_split, false, true);
+  const double copied = (double)batch * ((K % 16 != 0 || lda % 16 != 0 ? (double)M * (double)K : 0.0) + ((trans_b ? K : N) % 16 != 0 || ldb % 16 != 0 ? (double)N * (double)K : 0.0));
+  return p.stages_us * ((lda | ldb) % 4 == 0 ? 0.3 : 0.8) < 4.5 + 0.4e-6 * copied ? p : none;
 }
 
 // What launch_by_kind and launch_gemm_stream run; may_split: the caller brings the workspace.  A name gives the kernel and its
@@ -207,43 +225,14 @@ const char* variant_name(int trans_a, int64_t lda, int trans_b, int64_t ldb, int
 
 using namespace mi355q;
 
-extern "C" {
-
-const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
-                                    int64_t N, int64_t K) {
-  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, 1, false);
-}
-
-const char* mi355q_fp8_gemm_ws_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
-                                       int64_t N, int64_t K, int64_t batch) {
-  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
-}
-
-size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                                       int64_t batch) {
-  if (lda % 16 || ldb % 16 || !k_chunks_ok(trans_a, trans_b, K)) return 0;
-  return batch > 65535 ? 0 : split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, true).workspace_bytes();
-}
-
-int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
-                    int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
-                    int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
-                    const float* sb_dev, float sb_host, int sb_mode, const void* bias,
-                    int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
-                    int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
-                    int64_t stride_bias, void* stream) {
-  return mi355q_fp8_gemm_ws(A, fmt_a, trans_a, lda, B, fmt_b, trans_b, ldb, C, out_dtype, ldc, M, N, K, sa_dev, sa_host,
-                            sa_mode, sb_dev, sb_host, sb_mode, bias, bias_mode, ldbias, D, ldd, batch, stride_a, stride_b,
-                            stride_c, stride_d, stride_bias, nullptr, 0, stream);
-}
-
-int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
-                       int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
-                       int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
-                       const float* sb_dev, float sb_host, int sb_mode, const void* bias,
-                       int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
-                       int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
-                       int64_t stride_bias, void* workspace, size_t workspace_bytes, void* stream) {
+// mi355q_fp8_gemm_ws and mi355q_fp8_gemm_unaligned_ws (`unaligned`: ragged_plan decides, not tiled_ok).
+static int gemm_call(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
+                     int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
+                     int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
+                     const float* sb_dev, float sb_host, int sb_mode, const void* bias,
+                     int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
+                     int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
+                     int64_t stride_bias, void* workspace, size_t workspace_bytes, void* stream, bool unaligned) {
   auto fmt_ok = [](int f) { return f == MI355Q_E4M3FN || f == MI355Q_E5M2; };
   auto mode_ok = [](int m, const float* p) {
     if (m < MI355Q_GS_NONE || m > MI355Q_GS_PER_COL) return false;
@@ -298,7 +287,18 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const
       gb.bias_mode = MI355Q_BIAS_NONE;
     }
     gb.fast_epi = epilogue_fast_ok(gb, nb);
-    if (tiled_ok(gb.A, trans_a, lda, gb.B, trans_b, ldb, M, N, K, stride_a, stride_b)) {
+    if (unaligned) {
+      const SplitPlan plan = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, nb, workspace != nullptr && nb == batch);
+      if (plan.parts == 0) return MI355Q_ERR_UNSUPPORTED;
+      SplitArgs split{plan.parts, nullptr, nullptr, plan.kind};
+      if (plan.parts > 1) {
+        if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;
+        split.tickets = static_cast<uint32_t*>(workspace);
+        split.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
+      }
+      if (trans_b) launch_gemm_ragged_kk(gb, split, fmt_a, fmt_b, nb, st);
+      else launch_gemm_ragged_km(gb, split, fmt_a, fmt_b, nb, st);
+    } else if (tiled_ok(gb.A, trans_a, lda, gb.B, trans_b, ldb, M, N, K, stride_a, stride_b)) {
       const bool ak = !trans_a, bk = trans_b != 0;
       // (K is walked in parts if the caller brought the room where they meet)
       // (fp32 results change the choice only where nothing is cut)
@@ -329,6 +329,66 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const
     if (hipGetLastError() != hipSuccess) return MI355Q_ERR_LAUNCH;
   }
   return MI355Q_OK;
+}
+
+extern "C" {
+
+const char* mi355q_fp8_gemm_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
+                                    int64_t N, int64_t K) {
+  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, 1, false);
+}
+
+const char* mi355q_fp8_gemm_ws_variant(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M,
+                                       int64_t N, int64_t K, int64_t batch) {
+  return variant_name(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
+}
+
+size_t mi355q_fp8_gemm_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                       int64_t batch) {
+  if (lda % 16 || ldb % 16 || !k_chunks_ok(trans_a, trans_b, K)) return 0;
+  return batch > 65535 ? 0 : split_plan(!trans_a, lda, trans_b != 0, ldb, M, N, K, batch, true).workspace_bytes();
+}
+
+int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
+                    int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
+                    int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
+                    const float* sb_dev, float sb_host, int sb_mode, const void* bias,
+                    int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
+                    int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
+                    int64_t stride_bias, void* stream) {
+  return mi355q_fp8_gemm_ws(A, fmt_a, trans_a, lda, B, fmt_b, trans_b, ldb, C, out_dtype, ldc, M, N, K, sa_dev, sa_host,
+                            sa_mode, sb_dev, sb_host, sb_mode, bias, bias_mode, ldbias, D, ldd, batch, stride_a, stride_b,
+                            stride_c, stride_d, stride_bias, nullptr, 0, stream);
+}
+
+int64_t mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                                  int64_t batch) {
+  const SplitPlan p = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
+  return p.parts == 0 ? -1 : (int64_t)p.workspace_bytes();
+}
+
+int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
+                       int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
+                       int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
+                       const float* sb_dev, float sb_host, int sb_mode, const void* bias,
+                       int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
+                       int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
+                       int64_t stride_bias, void* workspace, size_t workspace_bytes, void* stream) {
+  return gemm_call(A, fmt_a, trans_a, lda, B, fmt_b, trans_b, ldb, C, out_dtype, ldc, M, N, K, sa_dev, sa_host, sa_mode, sb_dev, sb_host,
+                   sb_mode, bias, bias_mode, ldbias, D, ldd, batch, stride_a, stride_b, stride_c, stride_d, stride_bias, workspace,
+                   workspace_bytes, stream, false);
+}
+
+int mi355q_fp8_gemm_unaligned_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,
+                                 int trans_b, int64_t ldb, void* C, int out_dtype, int64_t ldc, int64_t M,
+                                 int64_t N, int64_t K, const float* sa_dev, float sa_host, int sa_mode,
+                                 const float* sb_dev, float sb_host, int sb_mode, const void* bias,
+                                 int bias_mode, int64_t ldbias, const void* D, int64_t ldd, int64_t batch,
+                                 int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t stride_d,
+                                 int64_t stride_bias, void* workspace, size_t workspace_bytes, void* stream) {
+  return gemm_call(A, fmt_a, trans_a, lda, B, fmt_b, trans_b, ldb, C, out_dtype, ldc, M, N, K, sa_dev, sa_host, sa_mode, sb_dev, sb_host,
+                   sb_mode, bias, bias_mode, ldbias, D, ldd, batch, stride_a, stride_b, stride_c, stride_d, stride_bias, workspace,
+                   workspace_bytes, stream, true);
 }
 
 }  // extern "C"

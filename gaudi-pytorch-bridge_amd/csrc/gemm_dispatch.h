@@ -81,6 +81,26 @@ void launch_by_format(const GemmArgs& g, const SplitArgs& split, int fmt_a, int 
   else launch_by_kind<AK, BK_, MI355Q_E5M2, MI355Q_E5M2>(g, split, batch, st);
 }
 
+// Operands at any alignment (gemm_ragged_*.hip): A [M, K] on the ring kernel alone.
+template <bool BK_, int FA, int FB>
+void launch_ragged_by_kind(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
+  if (split.kind == GemmKind::kRing16) launch_ring_ragged<16, BK_, FA, FB>(g, split, batch, st);
+  else if (split.kind == GemmKind::kRing32) launch_ring_ragged<32, BK_, FA, FB>(g, split, batch, st);
+  else if (split.kind == GemmKind::kRing64) launch_ring_ragged<64, BK_, FA, FB>(g, split, batch, st);
+  else if (split.kind == GemmKind::kRing128) launch_ring_ragged<128, BK_, FA, FB>(g, split, batch, st);
+  else if (split.kind == GemmKind::kRing192) launch_ring_ragged<192, BK_, FA, FB>(g, split, batch, st);
+  else launch_ring_ragged<256, BK_, FA, FB>(g, split, batch, st);
+}
+template <bool BK_>
+void launch_ragged_by_format(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st) {
+  if (fmt_a == MI355Q_E4M3FN && fmt_b == MI355Q_E4M3FN) launch_ragged_by_kind<BK_, MI355Q_E4M3FN, MI355Q_E4M3FN>(g, split, batch, st);
+  else if (fmt_a == MI355Q_E4M3FN) launch_ragged_by_kind<BK_, MI355Q_E4M3FN, MI355Q_E5M2>(g, split, batch, st);
+  else if (fmt_b == MI355Q_E4M3FN) launch_ragged_by_kind<BK_, MI355Q_E5M2, MI355Q_E4M3FN>(g, split, batch, st);
+  else launch_ragged_by_kind<BK_, MI355Q_E5M2, MI355Q_E5M2>(g, split, batch, st);
+}
+void launch_gemm_ragged_kk(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+void launch_gemm_ragged_km(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
+
 // A K-major / B K-major etc.; defined in gemm_inst_*.hip
 void launch_gemm_kk(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);
 void launch_gemm_km(const GemmArgs& g, const SplitArgs& split, int fmt_a, int fmt_b, int64_t batch, hipStream_t st);

@@ -393,6 +393,215 @@ struct RingProducer {
   }
 };
 
+// RingLoader for an operand whose rows begin anywhere: its chunks go through registers, 16 bytes per lane from any address, and are
+// stored in the places of LDS that the other loader's DMA would give them.  Only the last stage of K has chunks that are partly, or not at
+// all, inside the operand: fetch_edge() takes those from its last 16 bytes, and trim_edge() shifts them and clears what lies past K.
+template <bool KMAJOR, int EXT>
+struct RaggedLoader {
+  using G = typename RingLoader<KMAJOR, EXT>::G;
+  static constexpr int kCPR = G::kChunksPerRow, kRowsPerRegion = 64 / kCPR, kPerWave = RingLoader<KMAJOR, EXT>::kPerWave;
+  typedef uint32_t Any __attribute__((ext_vector_type(4), aligned(1)));
+  typedef const __attribute__((address_space(1))) uint8_t* Global;
+  Global base;              // the next stage to fetch
+  Global last16;            // the operand's last 16 bytes
+  int64_t step;
+  uint32_t at[kPerWave];    // a lane's offsets in a stage
+  int limit[kPerWave];      // and their k in it
+  u32x4 v[2][kPerWave];     // of two stages
+  uint32_t out;             // where the lane's first chunk goes, from the start of the operand's tile in LDS
+
+  // p, ld, valid, wave: as in RingLoader; last: the operand's last 16 bytes
+  __device__ __forceinline__ void init(const uint8_t* p, int64_t ld, int valid, int wave, const uint8_t* last) {
+    const uint64_t b = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+    base = reinterpret_cast<Global>(((uint64_t)hi << 32) | lo);
+    last16 = reinterpret_cast<Global>(reinterpret_cast<uint64_t>(last));
+    step = KMAJOR ? kBK : (int64_t)kBK * ld;
+    const int lane = threadIdx.x & 63;
+    out = (uint32_t)(wave * kPerWave * 1024 + lane * 16);
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int row = (wave * kPerWave + i) * kRowsPerRegion + lane / kCPR;
+      const int c16 = ((lane % kCPR) ^ G::swizzle(row)) * 16;
+      // (rows and columns past the edge take others: their products are never stored)
+      if constexpr (KMAJOR) at[i] = (uint32_t)((row < valid ? row : valid - 1) * (int)ld + c16);
+      else at[i] = (uint32_t)(row * (int)ld + (c16 < valid ? c16 : 0));
+      limit[i] = KMAJOR ? c16 : row;
+    }
+  }
+  __device__ __forceinline__ static u32x4 load(Global p) { return *reinterpret_cast<const __attribute__((address_space(1))) Any*>(p); }
+  template <int P, int I>
+  __device__ __forceinline__ void fetch() { v[P][I] = load(base + at[I]); }
+  // A chunk of the last stage, of valid_k k: how many of its bytes count, where it begins, and how far that is past the last 16 bytes.
+  struct Edge {
+    int inside, over;
+    Global p;
+  };
+  template <int I>
+  __device__ __forceinline__ Edge edge(Global from, int valid_k) const {
+    Edge e;
+    e.inside = KMAJOR ? valid_k - limit[I] : (limit[I] < valid_k ? 16 : 0);
+    const Global p = e.inside > 0 ? from + at[I] : last16;
+    e.p = p < last16 ? p : last16;
+    e.over = (int)(p - e.p);
+    return e;
+  }
+  template <int P, int I>
+  __device__ __forceinline__ void fetch_edge(int valid_k) { v[P][I] = load(edge<I>(base, valid_k).p); }
+  // and the same chunk once it has come (the loader points past its stage by then)
+  template <int P, int I>
+  __device__ __forceinline__ void trim_edge(int valid_k) {
+    const Edge e = edge<I>(base - step, valid_k);
+    u32x4 w = v[P][I];
+    if (__builtin_amdgcn_ballot_w64(e.over > 0) != 0) {  // rare: the operand's last rows
+      uint64_t w0 = ((uint64_t)w[1] << 32) | w[0], w1 = ((uint64_t)w[3] << 32) | w[2];
+      const int s = 8 * e.over;
+      w0 = s >= 64 ? w1 >> (s - 64) : (s > 0 ? (w0 >> s) | (w1 << (64 - s)) : w0);
+      w1 = s >= 64 ? 0 : w1 >> s;
+      w = u32x4{(uint32_t)w0, (uint32_t)(w0 >> 32), (uint32_t)w1, (uint32_t)(w1 >> 32)};
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int n = e.inside - 4 * d;
+      const uint32_t part = (1u << ((8 * n) & 31)) - 1u;
+      v[P][I][d] = w[d] & (n >= 4 ? 0xffffffffu : (n > 0 ? part : 0u));
+    }
+  }
+  // straight into LDS (whole stages of rows that begin at whole dwords)
+  template <int I>
+  __device__ __forceinline__ void to_lds(uint32_t tile, int wave) const {
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
+    const i32x4 rsrc = {(int)(uint32_t)b, (int)((uint32_t)(b >> 32) & 0xffffu), 0x7ffffff0, 0x00020000};
+    const uint32_t dst = tile + (uint32_t)((wave * kPerWave + I) * 1024);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(dst), "v"(at[I]), "s"(rsrc) : "memory", "m0");
+  }
+  template <int P, int I>
+  __device__ __forceinline__ void store(uint32_t tile) const { *reinterpret_cast<LDS_AS u32x4*>(tile + out + I * 1024) = v[P][I]; }
+};
+
+// The load side for such operands.  Two stages are on their way in registers; each chunk's register is stored to LDS and at once asked for
+// the stage after next.  (One stage on its way: 1000 x 3000 x 5000 31 us, two: 27.2.)
+template <int BM, bool A_KMAJOR, bool B_KMAJOR>
+struct RaggedProducer {
+  using Shape = RingShape<BM>;
+  static constexpr int R = Shape::kStages, kStage = Shape::kStage, kOffB = Shape::kOffB;
+  using LoaderA = RaggedLoader<A_KMAJOR, Shape::kRows>;
+  using LoaderB = RaggedLoader<B_KMAJOR, kRingBN>;
+  LoaderA la;
+  LoaderB lb;
+  uint32_t slot, ring;
+  int next, stages, last_k;  // next: the stage the loaders point at
+
+  template <int P, int STORE, int FETCH>  // 0 nothing, 1 a whole stage, 2 the last stage
+  __device__ __forceinline__ void move() {
+    const int last = last_k;
+    static_for<LoaderA::kPerWave>([&](auto ic) { chunk<P, decltype(ic)::value, STORE, FETCH>(la, slot, last); });
+    static_for<LoaderB::kPerWave>([&](auto ic) { chunk<P, decltype(ic)::value, STORE, FETCH>(lb, slot + kOffB, last); });
+    if constexpr (STORE != 0) slot = slot + kStage == ring + R * kStage ? ring : slot + kStage;
+    if constexpr (FETCH != 0) {
+      la.base += la.step;
+      lb.base += lb.step;
+      ++next;
+    }
+  }
+  template <int P, int I, int STORE, int FETCH, typename Loader>
+  __device__ __forceinline__ static void chunk(Loader& l, uint32_t tile, int last) {
+    if constexpr (STORE == 2) l.template trim_edge<P, I>(last);
+    if constexpr (STORE != 0) l.template store<P, I>(tile);
+    if constexpr (FETCH == 1) l.template fetch<P, I>();
+    if constexpr (FETCH == 2) l.template fetch_edge<P, I>(last);
+  }
+  template <int P>
+  __device__ __forceinline__ void fetch_only() {
+    if (next < stages - 1) move<P, 0, 1>();
+    else if (next == stages - 1) move<P, 0, 2>();
+  }
+  // Stage s, in register set P = s % 2, to LDS; the stage after next into its place.
+  template <int P>
+  __device__ __forceinline__ void advance(int s) {
+    if (next < stages - 1) move<P, 1, 1>();
+    else if (next == stages - 1) move<P, 1, 2>();
+    else if (s < stages - 1) move<P, 1, 0>();
+    else if (s == stages - 1) move<P, 2, 0>();
+  }
+  // (the loads on their way stay there: only what was stored to LDS is waited for)
+  __device__ __forceinline__ static void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
+  __device__ __forceinline__ void run() {
+    next = 0;
+    fetch_only<0>();
+    fetch_only<1>();
+    advance<0>(0);
+    barrier();  // the first stage is in LDS
+    // stage s + 1 to LDS, into the slot of a stage that the consumers have had in their registers since the last barrier
+    int s = 0;
+    for (; s + 1 < stages; s += 2) {
+      advance<1>(s + 1);
+      barrier();
+      advance<0>(s + 2);
+      barrier();
+    }
+    if (s < stages) barrier();
+  }
+};
+
+// The load side where rows begin at whole dwords, which is all that a load into LDS needs: every stage but the last comes that way,
+// as in RingProducer.  The last one's chunks are asked for first of all and wait in registers for their turn.  (us, through registers
+// / straight into LDS: 1000 x 3000 x 5000 27.2 / 25.3, 256 x 8188 x 8188 42.2 / 38.1, 64 x 4100 x 9996 22.2 / 21.9.)
+template <int BM, bool A_KMAJOR, bool B_KMAJOR>
+struct DwordProducer {
+  using Shape = RingShape<BM>;
+  static constexpr int R = Shape::kStages, kStage = Shape::kStage, kOffB = Shape::kOffB;
+  using LoaderA = RaggedLoader<A_KMAJOR, Shape::kRows>;
+  using LoaderB = RaggedLoader<B_KMAJOR, kRingBN>;
+  static constexpr int kOps = LoaderA::kPerWave + LoaderB::kPerWave;
+  LoaderA la;
+  LoaderB lb;
+  uint32_t slot, ring;
+  int wave, stages, last_k;
+
+  __device__ __forceinline__ void issue_stage() {
+    static_for<LoaderA::kPerWave>([&](auto ic) { la.template to_lds<decltype(ic)::value>(slot, wave); });
+    static_for<LoaderB::kPerWave>([&](auto ic) { lb.template to_lds<decltype(ic)::value>(slot + kOffB, wave); });
+    slot = slot + kStage == ring + R * kStage ? ring : slot + kStage;
+    la.base += la.step;
+    lb.base += lb.step;
+  }
+  __device__ __forceinline__ void run() {
+    const int whole = stages - 1;
+    la.base += la.step * whole;
+    lb.base += lb.step * whole;
+    static_for<LoaderA::kPerWave>([&](auto ic) { la.template fetch_edge<0, decltype(ic)::value>(last_k); });
+    static_for<LoaderB::kPerWave>([&](auto ic) { lb.template fetch_edge<0, decltype(ic)::value>(last_k); });
+    la.base -= la.step * whole;
+    lb.base -= lb.step * whole;
+    for (int s = 0; s < R && s < whole; ++s) issue_stage();
+    // (a stage's landing is what its barrier waits for; the last stage's chunks are older than any of them)
+    RingProducer<BM, A_KMAJOR, B_KMAJOR>::wait_upto((whole < R ? whole : R) - 1);
+    if (whole == 0) store_last();
+    RaggedProducer<BM, A_KMAJOR, B_KMAJOR>::barrier();
+    for (int s = 0; s < stages; ++s) {
+      const bool more = s + R < whole;
+      if (s + 1 == whole) store_last();
+      else RingProducer<BM, A_KMAJOR, B_KMAJOR>::wait_upto(more ? R - 2 : whole - 2 - s);
+      RaggedProducer<BM, A_KMAJOR, B_KMAJOR>::barrier();
+      if (more) issue_stage();
+    }
+  }
+  // the last stage into its slot (of a stage that the consumers are long done with); the loaders point past the stages before it
+  __device__ __forceinline__ void store_last() {
+    la.base += la.step;
+    lb.base += lb.step;
+    static_for<LoaderA::kPerWave>([&](auto ic) {
+      la.template trim_edge<0, decltype(ic)::value>(last_k);
+      la.template store<0, decltype(ic)::value>(slot);
+    });
+    static_for<LoaderB::kPerWave>([&](auto ic) {
+      lb.template trim_edge<0, decltype(ic)::value>(last_k);
+      lb.template store<0, decltype(ic)::value>(slot + kOffB);
+    });
+  }
+};
+
 // The multiply side.  Fragments are single-buffered as in gemm_tile16.h: those of the next stage replace this stage's as
 // they die, so the barrier early in a stage finds every wave done with the stage's ring slot, and the next stage landed.
 template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B>
@@ -440,8 +649,8 @@ struct RingConsumer {
   }
 };
 
-// NT_B: B is loaded with the nontemporal hint (ring_streams_b).
-template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B, bool NT_B>
+// NT_B: B is loaded with the nontemporal hint (ring_streams_b).  RAGGED: rows of A and B at any address, K of any length.
+template <int BM, bool A_KMAJOR, bool B_KMAJOR, int FMT_A, int FMT_B, bool NT_B, bool RAGGED = false>
 __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g, SplitArgs split) {
   using Producer = RingProducer<BM, A_KMAJOR, B_KMAJOR>;
   using Consumer = RingConsumer<BM, A_KMAJOR, B_KMAJOR, FMT_A, FMT_B>;
@@ -483,6 +692,27 @@ __global__ __launch_bounds__(kRingThreads) void fp8_gemm_ring_kernel(GemmArgs g,
   const int stages = (g.K + kBK - 1) / kBK;
 
   if (wave >= kRingWaves) {
+    if constexpr (RAGGED) {
+      const auto run = [&](auto& p) {
+        p.slot = p.ring = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_ring;
+        p.stages = stages;
+        p.last_k = g.K - (stages - 1) * kBK;
+        const uint8_t *a = g.A + batch * g.stride_a, *b = g.B + batch * g.stride_b;
+        p.la.init(a + (int64_t)m0 * (A_KMAJOR ? g.lda : 1), g.lda, g.M - m0, wave - kRingWaves, a + (A_KMAJOR ? (g.M - 1) * g.lda + g.K : (g.K - 1) * g.lda + g.M) - 16);
+        p.lb.init(b + (int64_t)n0 * (B_KMAJOR ? g.ldb : 1), g.ldb, g.N - n0, wave - kRingWaves, b + (B_KMAJOR ? (g.N - 1) * g.ldb + g.K : (g.K - 1) * g.ldb + g.N) - 16);
+        p.run();
+      };
+      const uint64_t places = reinterpret_cast<uint64_t>(g.A) | reinterpret_cast<uint64_t>(g.B) | (uint64_t)(g.lda | g.ldb | g.stride_a | g.stride_b);
+      if ((places & 3u) == 0) {
+        DwordProducer<BM, A_KMAJOR, B_KMAJOR> p;
+        p.wave = wave - kRingWaves;
+        run(p);
+      } else {
+        RaggedProducer<BM, A_KMAJOR, B_KMAJOR> p;
+        run(p);
+      }
+      return;
+    }
     Producer p;
     p.slot = p.ring = (uint32_t)(uintptr_t)(LDS_AS uint8_t*)lds_ring;
     p.stages = stages;
@@ -599,6 +829,18 @@ void launch_ring(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipSt
   dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (split.parts > 1 ? split.parts : 1)), (unsigned)batch);
   if (ring_streams_b(a, batch)) fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, true><<<grid, kRingThreads, 0, st>>>(a, split);
   else fp8_gemm_ring_kernel<BM, AK, BK_, FA, FB, false><<<grid, kRingThreads, 0, st>>>(a, split);
+}
+
+// Operands at any alignment: A [M, K], either layout of B.  Without it they were copied into padded buffers first, a launch of its own
+// that reads and writes both (ragged_plan in gemm_api.hip has figures and the rule).
+template <int BM, bool BK_, int FA, int FB>
+void launch_ring_ragged(const GemmArgs& g, const SplitArgs& split, int64_t batch, hipStream_t st) {
+  GemmArgs a = g;
+  a.tiles_m = (g.M + BM - 1) / BM;
+  a.tiles_n = (g.N + kRingBN - 1) / kRingBN;
+  a.fast_epi = g.fast_epi && g.D == nullptr ? kRingFast : (ring_rows_ok(g, batch) ? kRingRows : kRingAny);
+  dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (split.parts > 1 ? split.parts : 1)), (unsigned)batch);
+  fp8_gemm_ring_kernel<BM, true, BK_, FA, FB, false, true><<<grid, kRingThreads, 0, st>>>(a, split);
 }
 
 }  // namespace mi355q

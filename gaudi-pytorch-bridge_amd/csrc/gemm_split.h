@@ -38,12 +38,14 @@ struct SplitPlan {
   int strips = 0, parts = 1;   // strips, or tiles
   int64_t tile_rows = 0;     // rows of sums a workgroup leaves in the workspace
   int64_t batch = 1;
+  double stages_us = 0.0;    // ring kernel: what the stages of K are expected to take
   size_t workspace_bytes() const {
     return parts < 2 ? 0 : kTicketBytes + (size_t)parts * strips * batch * tile_rows * nb * sizeof(float);
   }
 };
 SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
-                     bool fp32_rows = false);  // fp32 results that ring_epilogue_rows writes
+                     bool fp32_rows = false,   // fp32 results that ring_epilogue_rows writes
+                     bool ring_only = false);  // the ring kernel's forms alone
 
 // The counter, looked at ahead of time (before waits that the workgroup has anyway): parts - 1 means that every other
 // part has arrived; then this workgroup is the last whatever happens, and its own sums need not travel.

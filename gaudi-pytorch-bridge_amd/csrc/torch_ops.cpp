@@ -594,8 +594,8 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   Tensor out = at::empty(out_shape, A.options().dtype(out_dtype));
   if (out.numel() == 0) return out;
 
-  // The MFMA kernels move 16-byte chunks: they need 16-byte aligned operands and pitches and, where K is an operand's
-  // contiguous dimension, K % 16 == 0; anything else runs on a kernel that takes about 80 ns per k (1 x 3001 x 8000:
+  // Most MFMA kernels move 16-byte chunks: they need 16-byte aligned operands and pitches and, where K is an operand's
+  // contiguous dimension, K % 16 == 0; anything that mi355q_fp8_gemm_unaligned_ws does not take either runs on a kernel that takes about 80 ns per k (1 x 3001 x 8000:
   // 0.7 ms).  Where that is more than a second launch costs, such operands go into zero-filled buffers with every extent
   // rounded up to 16, both in one launch (zeros along K add nothing to any sum; padding along m or n is never read into
   // a stored output).  Without -> with the copies, us a call:
@@ -606,7 +606,12 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   auto misaligned = [](const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) != 0; };
   const bool k_ragged = K % 16 != 0 && !(ta && !tb);
   const double outputs = (double)M * (double)N;
-  if ((ac % 16 || bc % 16 || k_ragged || misaligned(ac_t) || misaligned(bc_t)) &&
+  const bool ragged = ac % 16 || bc % 16 || k_ragged || misaligned(ac_t) || misaligned(bc_t);
+  // A [M, K] times one matrix B is one product over all rows of A (see below)
+  const bool flat = batch > 1 && stride_b == 0 && stride_a != 0 && !ta;
+  // From K = 256 on the ring kernel takes such operands as they lie (A [M, K]), where copies would not end in 256 x 256 tiles.
+  const int64_t unaligned_ws = ragged ? mi355q_fp8_gemm_unaligned_workspace_bytes(ta ? 1 : 0, ac, tb ? 1 : 0, bc, flat ? batch * M : M, N, K, flat ? 1 : batch) : -1;
+  if (ragged && unaligned_ws < 0 &&
       (K >= 128 || outputs * (double)K >= (double)(1 << 26) || (tb && K >= 64 && outputs >= (double)(1 << 17)))) {
     const int64_t kp = (ta && !tb) ? K : (K + 15) / 16 * 16;  // K is contiguous in neither operand: any K
     mi355q_pad_desc jobs[2];
@@ -687,11 +692,13 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
     stride_d = M * N;
   }
 
-  const size_t ws_bytes = mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
+  const size_t ws_bytes = unaligned_ws >= 0 ? (size_t)unaligned_ws
+                                            : mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
   const bool kept = ws_bytes == 0 || !stream_is_capturing();
   Tensor ws = kept ? ticket_workspace(A, ws_bytes, kWsGemm) : captured_ticket_workspace(A, ws_bytes, MI355Q_FP8_GEMM_COUNTER_BYTES);
   const int st =
-      mi355q_fp8_gemm_ws(ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
+      (unaligned_ws >= 0 ? mi355q_fp8_gemm_unaligned_ws : mi355q_fp8_gemm_ws)(
+                      ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
                       bc_t.data_ptr(), to_mi355q_dtype(B.scalar_type()), tb ? 1 : 0, ldb,
                       out.data_ptr(), to_mi355q_dtype(out_dtype), N, m_call, N, k_call, sa.dev, sa.host, sa.mode,
                       sb.dev, sb.host, sb.mode, bias_mode != MI355Q_BIAS_NONE ? bias_t.data_ptr() : nullptr,

@@ -292,6 +292,25 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
                     int64_t batch, int64_t stride_a, int64_t stride_b,
                     int64_t stride_c, int64_t stride_d, int64_t stride_bias,
                     void* workspace, size_t workspace_bytes, void* stream);
+/*
+ * The same product for operands that lie anywhere: base addresses, pitches and batch strides of A and B need no alignment and K may
+ * be any length.  Served are A [M, K], K >= 256, N >= 16, pitches up to 4 Mi elements, and sizes that do not fill the chip with
+ * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows); mi355q_fp8_gemm_unaligned_workspace_bytes() is -1
+ * and the call MI355Q_ERR_UNSUPPORTED otherwise.  The workspace is that of mi355q_fp8_gemm_ws.
+ */
+int64_t mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                                  int64_t batch);
+int mi355q_fp8_gemm_unaligned_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
+                    const void* B, int fmt_b, int trans_b, int64_t ldb,
+                    void* C, int out_dtype, int64_t ldc,
+                    int64_t M, int64_t N, int64_t K,
+                    const float* sa_dev, float sa_host, int sa_mode,
+                    const float* sb_dev, float sb_host, int sb_mode,
+                    const void* bias, int bias_mode, int64_t ldbias,
+                    const void* D, int64_t ldd,
+                    int64_t batch, int64_t stride_a, int64_t stride_b,
+                    int64_t stride_c, int64_t stride_d, int64_t stride_bias,
+                    void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Fused int4-dequant GEMM, fp8 activations times 4-bit weights (W4A8):
