@@ -361,10 +361,12 @@ int mi355q_fp8_gemm(const void* A, int fmt_a, int trans_a, int64_t lda, const vo
                             stride_c, stride_d, stride_bias, nullptr, 0, stream);
 }
 
-int64_t mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                                                  int64_t batch) {
+int mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                              int64_t batch, size_t* bytes) {
+  if (bytes == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
   const SplitPlan p = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
-  return p.parts == 0 ? -1 : (int64_t)p.workspace_bytes();
+  *bytes = p.parts == 0 ? 0 : p.workspace_bytes();
+  return p.parts == 0 ? MI355Q_ERR_UNSUPPORTED : MI355Q_OK;
 }
 
 int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda, const void* B, int fmt_b,

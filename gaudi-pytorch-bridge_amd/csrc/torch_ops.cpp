@@ -610,8 +610,10 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   // A [M, K] times one matrix B is one product over all rows of A (see below)
   const bool flat = batch > 1 && stride_b == 0 && stride_a != 0 && !ta;
   // From K = 256 on the ring kernel takes such operands as they lie (A [M, K]), where copies would not end in 256 x 256 tiles.
-  const int64_t unaligned_ws = ragged ? mi355q_fp8_gemm_unaligned_workspace_bytes(ta ? 1 : 0, ac, tb ? 1 : 0, bc, flat ? batch * M : M, N, K, flat ? 1 : batch) : -1;
-  if (ragged && unaligned_ws < 0 &&
+  size_t unaligned_ws = 0;
+  const bool unaligned = ragged && mi355q_fp8_gemm_unaligned_workspace_bytes(ta ? 1 : 0, ac, tb ? 1 : 0, bc, flat ? batch * M : M, N, K,
+                                                                             flat ? 1 : batch, &unaligned_ws) == MI355Q_OK;
+  if (ragged && !unaligned &&
       (K >= 128 || outputs * (double)K >= (double)(1 << 26) || (tb && K >= 64 && outputs >= (double)(1 << 17)))) {
     const int64_t kp = (ta && !tb) ? K : (K + 15) / 16 * 16;  // K is contiguous in neither operand: any K
     mi355q_pad_desc jobs[2];
@@ -692,12 +694,12 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
     stride_d = M * N;
   }
 
-  const size_t ws_bytes = unaligned_ws >= 0 ? (size_t)unaligned_ws
-                                            : mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
+  const size_t ws_bytes = unaligned ? unaligned_ws
+                                    : mi355q_fp8_gemm_workspace_bytes(ta ? 1 : 0, lda, tb ? 1 : 0, ldb, m_call, N, k_call, batch_call);
   const bool kept = ws_bytes == 0 || !stream_is_capturing();
   Tensor ws = kept ? ticket_workspace(A, ws_bytes, kWsGemm) : captured_ticket_workspace(A, ws_bytes, MI355Q_FP8_GEMM_COUNTER_BYTES);
   const int st =
-      (unaligned_ws >= 0 ? mi355q_fp8_gemm_unaligned_ws : mi355q_fp8_gemm_ws)(
+      (unaligned ? mi355q_fp8_gemm_unaligned_ws : mi355q_fp8_gemm_ws)(
                       ac_t.data_ptr(), to_mi355q_dtype(A.scalar_type()), ta ? 1 : 0, lda,
                       bc_t.data_ptr(), to_mi355q_dtype(B.scalar_type()), tb ? 1 : 0, ldb,
                       out.data_ptr(), to_mi355q_dtype(out_dtype), N, m_call, N, k_call, sa.dev, sa.host, sa.mode,

@@ -295,11 +295,11 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
 /*
  * The same product for operands that lie anywhere: base addresses, pitches and batch strides of A and B need no alignment and K may
  * be any length.  Served are A [M, K], K >= 256, N >= 16, pitches up to 4 Mi elements, and sizes that do not fill the chip with
- * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows); mi355q_fp8_gemm_unaligned_workspace_bytes() is -1
- * and the call MI355Q_ERR_UNSUPPORTED otherwise.  The workspace is that of mi355q_fp8_gemm_ws.
+ * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows), nor others where such copies cost less; both calls
+ * return MI355Q_ERR_UNSUPPORTED otherwise.  The workspace is that of mi355q_fp8_gemm_ws; its size goes to *bytes.
  */
-int64_t mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
-                                                  int64_t batch);
+int mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                                              int64_t batch, size_t* bytes);
 int mi355q_fp8_gemm_unaligned_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
                     const void* B, int fmt_b, int trans_b, int64_t ldb,
                     void* C, int out_dtype, int64_t ldc,

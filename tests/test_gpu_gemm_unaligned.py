@@ -29,20 +29,17 @@ def operands(gen, batch, M, K, N, trans_b, lda, ldb, offset, dev):
 
 def call(pkg, dev, batch, M, K, N, trans_b, lda, ldb, offset, out_dtype=torch.float32):
     lib = pkg.capi()
-    lib.mi355q_fp8_gemm_unaligned_workspace_bytes.restype = ctypes.c_int64
     gen = torch.Generator().manual_seed(M + K + N + offset)
     a, b, ((araw, sa), (braw, sb)) = operands(gen, batch, M, K, N, trans_b, lda, ldb, offset, dev)
-    need = lib.mi355q_fp8_gemm_unaligned_workspace_bytes(0, ctypes.c_int64(lda), int(trans_b), ctypes.c_int64(ldb), ctypes.c_int64(M), ctypes.c_int64(N),
-                                                         ctypes.c_int64(K), ctypes.c_int64(batch))
-    assert need >= 0
+    size = ctypes.c_size_t()
+    assert lib.mi355q_fp8_gemm_unaligned_workspace_bytes(0, lda, int(trans_b), ldb, M, N, K, batch, ctypes.byref(size)) == 0
+    need = size.value
     ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=dev)
     c = torch.full((batch, M, N), -7.0, dtype=out_dtype, device=dev)
-    i64 = ctypes.c_int64
     st = lib.mi355q_fp8_gemm_unaligned_ws(
-        ctypes.c_void_p(araw.data_ptr() + offset), pkg.E4M3FN, 0, i64(lda), ctypes.c_void_p(braw.data_ptr() + offset), pkg.E5M2, int(trans_b), i64(ldb),
-        ctypes.c_void_p(c.data_ptr()), pkg.F32 if out_dtype == torch.float32 else pkg.BF16, i64(N), i64(M), i64(N), i64(K), None, ctypes.c_float(1.0), pkg.GS_NONE, None,
-        ctypes.c_float(1.0), pkg.GS_NONE, None, 0, i64(0), None, i64(0), i64(batch), i64(sa), i64(sb), i64(M * N), i64(0), i64(0),
-        ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(need), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        araw.data_ptr() + offset, pkg.E4M3FN, 0, lda, braw.data_ptr() + offset, pkg.E5M2, int(trans_b), ldb, c.data_ptr(),
+        pkg.F32 if out_dtype == torch.float32 else pkg.BF16, N, M, N, K, None, 1.0, pkg.GS_NONE, None, 1.0, pkg.GS_NONE, None, 0, 0, None, 0, batch,
+        sa, sb, M * N, 0, 0, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
     assert st == 0
     ref = a @ b
     assert ref.abs().max() < 2 ** 24
