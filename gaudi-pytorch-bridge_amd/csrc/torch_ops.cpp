@@ -1366,7 +1366,13 @@ SdpaOut fp8_sdpa_recomp_fwd_common(const Tensor& q, const Tensor& k, const Tenso
   // for: they are not filled here (a fill is a launch of its own in front of every call); the amax words that
   // are asked for are cleared by the C entry point.
   Tensor pool = at::empty({40}, opts.dtype(at::kByte));
-  auto one = [&](int slot, at::ScalarType t) { return pool.slice(0, 8 * slot, 8 * slot + (int64_t)c10::elementSize(t)).view(t); };
+  // (tensors over its storage, made here: slice and view are a trip through the dispatcher each, ten of them 3 of a call's 11.4 us)
+  auto one = [&](int slot, at::ScalarType t) {
+    Tensor word = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(pool.storage()), c10::DispatchKeySet(c10::DispatchKey::CUDA), c10::scalarTypeToTypeMeta(t));
+    word.unsafeGetTensorImpl()->set_storage_offset(8 * slot / (int64_t)c10::elementSize(t));
+    word.unsafeGetTensorImpl()->set_sizes_contiguous({1});
+    return word;
+  };
   Tensor m = one(0, stat_dt), linv = one(1, linv_dt), seed = one(2, at::kInt), amax_s = one(3, at::kFloat), amax_o = one(4, at::kFloat);
   DeviceGuard guard(q.device());
   TORCH_CHECK(k.device() == q.device() && v.device() == q.device(), "fp8_sdpa_recomp_fwd: q, k and v must be on one device");
