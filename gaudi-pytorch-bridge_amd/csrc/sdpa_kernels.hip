@@ -39,6 +39,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kSdpaThreads = 256;
 constexpr int kSdpaBM = 128;  // query rows per workgroup
 constexpr int kSdpaBN = 64;   // keys per block
+constexpr int kSdpaResident = 1024;  // workgroups that are resident at once, four on each of 256 CUs
 constexpr float kLog2e = 1.44269504088896341f;
 
 enum { kMaskNone = MI355Q_SDPA_MASK_NONE, kMaskBool = MI355Q_SDPA_MASK_BOOL, kMaskBf16 = MI355Q_SDPA_MASK_BF16, kMaskF32 = MI355Q_SDPA_MASK_F32 };
@@ -54,6 +55,8 @@ struct SdpaArgs {
   int64_t ldq, ldk, ldv, ldm, ldo;
   int L, S, Dk, Dv;
   int mask_kind, causal, out_fp8;
+  // the order of the workgroups (sdpa_place): heads of a group, 0 = contiguous ranges; heads per XCD (all of them where xcd_shift is 0)
+  int head_group, heads, xcd_shift;
   int vec_q, vec_k, vec_v, vec_o;  // 16-byte (q, k, v) / 4-element (out; 2: 8-element) accesses are possible
   int dma;                         // k and v go global -> LDS directly
   int nqb;                         // query blocks per (batch, head)
@@ -111,6 +114,31 @@ __device__ __forceinline__ int64_t sdpa_batch_index(const SdpaArgs& a, int d, ui
   const uint32_t q = rest / n, b = rest - q * n;
   rest = q;
   return b;
+}
+
+// Which (batch, head) `bi` and query block `qb` workgroup `id` of `total` takes.  Workgroups go to the 8 XCDs round robin, in the order
+// of their numbers, and an XCD's are to share K and V in its L2.
+// Without a causal mask all take as long: each XCD gets a contiguous range of (batch, head, query block).
+// Under one the last query block takes nqb times as long as the first, and what counts is that the long ones start first, over all
+// heads of the XCD and not head by head: with the last head's longest workgroups started last the CUs stood idle for a fifth of the
+// prefill (32 / 8 heads of 128, 8192 tokens, 360 -> 320 us; 8 x 1024 tokens 78 -> 60).  So the heads go in groups, block by block
+// down from the last: a group is what the caches hold of K and V (sdpa_order).  If every workgroup is resident from the start, the
+// order decides which ones share a CU, and every second round over the 32 CUs of an XCD runs backwards, so that each CU gets long and short
+// ones (16 / 4 heads, 8192 tokens, 180 -> 169 us; where workgroups wait for their turn it costs 1.5 %).
+__device__ __forceinline__ void sdpa_place(const SdpaArgs& a, int id, int total, uint32_t& bi, int& qb) {
+  if (a.head_group > 0) {
+    const int k = id >> 3;
+    if (total <= kSdpaResident && (k & 32) != 0 && (k | 31) < (total >> 3)) id ^= 31 << 3;
+    const uint32_t xcd = (uint32_t)id & ((1u << a.xcd_shift) - 1), i = (uint32_t)id >> a.xcd_shift;
+    const uint32_t per = (uint32_t)a.head_group * (uint32_t)a.nqb, g = i / per, j = i - g * per, first = g * (uint32_t)a.head_group;
+    const uint32_t left = (uint32_t)a.heads - first, n = left < (uint32_t)a.head_group ? left : (uint32_t)a.head_group, r = j / n;
+    qb = a.nqb - 1 - (int)r;
+    bi = xcd * (uint32_t)a.heads + first + (j - r * n);
+  } else {
+    if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+    bi = (uint32_t)id / (uint32_t)a.nqb;
+    qb = a.nqb - 1 - (id - (int)bi * a.nqb);
+  }
 }
 
 // LDS offset of 16-byte chunk `chunk` of K row `row` (ROW_BYTES per row).  The 16 lanes of one
@@ -500,13 +528,9 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // the same in every lane, and known to be
   const int lq = lane & 31, h = lane >> 5;
 
-  // Workgroups go to the 8 XCDs round robin: give each XCD a contiguous range of (batch, head,
-  // query block), so that the query blocks that share a K and V meet in one L2.
-  int id = blockIdx.x;
-  const int total = gridDim.x;
-  if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
-  uint32_t bi = (uint32_t)id / (uint32_t)a.nqb;
-  const int qb = a.nqb - 1 - (id - (int)bi * a.nqb);  // under a causal mask the long rows start first
+  uint32_t bi;
+  int qb;
+  sdpa_place(a, blockIdx.x, gridDim.x, bi, qb);
   int64_t q_off = 0, k_off = 0, v_off = 0, m_off = 0, o_off = 0;
   int64_t b_valid = 0;
 #pragma unroll
@@ -1141,6 +1165,24 @@ static SdpaDecodePlan sdpa_decode_plan(const mi355q_sdpa_desc* d, int cus) {
   return p;
 }
 
+// The order of a launch's workgroups (see sdpa_place).  With one workgroup per CU or fewer it is of no account.
+// A number of heads that 8 divides leaves each head on one XCD, GQA's heads of a K and V together, in groups of equal size whose K
+// and V are at most 8 MiB, twice an XCD's L2 (4096 tokens of 32 heads per XCD, each with its own K and V: 8 heads 679 us, 4 689, 16 697,
+// all 745; 2048 tokens, 16 heads per XCD: 16 heads 96, 8 110).  Any other number goes through all heads at once, over all XCDs:
+// 9 heads, 8192 tokens, 190 -> 136 us; 30 heads, 357 -> 308, whose K and V are 60 MiB.
+static void sdpa_order(SdpaArgs& a, const mi355q_sdpa_desc* d, int64_t batches, bool causal) {
+  if (!causal || a.nqb * batches <= 256) return;
+  a.xcd_shift = batches % 8 == 0 ? 3 : 0;
+  a.heads = (int)(batches >> a.xcd_shift);
+  a.head_group = a.heads;
+  if (a.xcd_shift == 0) return;
+  int64_t sharing = 1;  // heads with the same K and V
+  for (int i = 2; i >= 0 && (d->batch[i] == 1 || (d->k_bstride[i] == 0 && d->v_bstride[i] == 0)); --i) sharing *= d->batch[i];
+  const int64_t most = (int64_t)(8 << 20) / (d->kv_len > 0 ? d->kv_len * (d->head_dim_qk + d->head_dim_v) : 1) * sharing;
+  const int64_t groups = most > 0 ? (a.heads + most - 1) / most : a.heads;
+  a.head_group = (int)((a.heads + groups - 1) / groups);
+}
+
 template <int DKC, int DVT, int FMT, int MASK>
 static void sdpa_launch_kernel(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
   const dim3 grid((unsigned)blocks), block(kSdpaThreads);
@@ -1258,6 +1300,7 @@ int mi355q_fp8_sdpa_fwd(const void* q, const void* k, const void* v, int fp8_fmt
   // direct loads address a block's rows with 32-bit offsets from a base that moves with the block
   a.dma = vk && vv && d->ldk < (1 << 24) && d->ldv < (1 << 24);
   a.nqb = (int)nqb;
+  sdpa_order(a, d, batches, is_causal != 0);
   a.scale = softmax_scale;
   for (int i = 0; i < 6; ++i) {
     a.sc_dev[i] = scale_dev != nullptr ? scale_dev[i] : nullptr;
