@@ -17,8 +17,8 @@
 // and the V^T fragment is gathered from LDS in the same key order by the transposing reads
 // (ds_read_b64_tr_b8 takes each of its 8 k-rows from its own address).
 //
-// K and V blocks are double buffered in LDS, one barrier per block.  Aligned tensors (16-byte
-// rows and head dimensions) go global -> LDS directly (buffer_load ... lds: the loads of block
+// K and V blocks are double buffered in LDS, one barrier per block (the form for many workgroups of head
+// dimension 128: one V, two barriers).  Aligned tensors (16-byte rows and head dimensions) go global -> LDS directly (buffer_load ... lds: the loads of block
 // i + 1 are issued before the arithmetic of block i and waited for after it, and cost the waves
 // neither registers nor vector instructions); anything else goes through registers, byte by
 // byte where it must.  Rows are XOR-swizzled so that the fragment reads are bank-conflict free;
@@ -230,6 +230,12 @@ __device__ __forceinline__ f32x16 sdpa_mfma(const i32x8& first, const i32x8& sec
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(first, second, acc, code, code, 0, 0, 0, 0);
 }
 
+__device__ __forceinline__ uint32_t sdpa_lds(const uint8_t* p) { return (uint32_t)(uintptr_t)(SDPA_LDS_AS const uint8_t*)p; }
+__device__ __forceinline__ u32x4 sdpa_lds_read(uint32_t at, int off) { return *(SDPA_LDS_AS const u32x4*)(uintptr_t)(at + off); }
+__device__ __forceinline__ i32x8 sdpa_join(const u32x4& lo, const u32x4& hi) {
+  return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 __global__ void sdpa_clear_amax_kernel(float* a, float* b) {
@@ -245,10 +251,10 @@ enum { kWithoutMask, kWithMask, kEither };
 // the block may lie behind the last key, `general` that there is a mask, a first key, or a scale that is not positive; PLAIN:
 // neither, at compile time; MASK: whether there is a mask.  (The kernels walk their plain blocks in a loop of its own: with the other forms in the same
 // loop the compiler copies all 32 scores on the way to where the paths meet, 5 % of the prefill.)
-template <int DKC, int DVT, int FMT, bool QL, bool PLAIN, int MASK>
+template <int DKC, int DVT, int FMT, bool QL, bool PLAIN, int MASK, typename BeforeV>
 __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb, const uint8_t* vb, int kv0, bool edge, bool general, int qpos,
                                            const uint8_t* mrow, const i32x8 (&qf)[DKC], float sc2, float lqs, bool clamp_p,
-                                           f32x16 (&o)[DVT], float& m_run, float& l_run, const uint8_t* qbase = nullptr,
+                                           f32x16 (&o)[DVT], float& m_run, float& l_run, const BeforeV& before_v, const uint8_t* qbase = nullptr,
                                            int klo = 0, int khi = 0x7fffffff) {
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = DVT <= 4 ? 128 : 256;
@@ -256,22 +262,20 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   const int lane = threadIdx.x & 63, lq = lane & 31, h = lane >> 5;
   f32x16 s[2];
   if constexpr (QL) {
-    // the query fragments come from LDS, one depth step at a time (registers for a third wave per SIMD)
+    // the query fragments come from LDS, one depth step at a time (registers for more waves per SIMD)
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+    // One address, the other chunks of the row by XOR: four kept over the block would be four registers.
+    const uint32_t k0 = sdpa_lds(kb) + k_lds_offset<KROW>(lq, h * 2);
 #pragma unroll
     for (int c = 0; c < DKC; ++c) {
-      const u32x4 qlo = *reinterpret_cast<const u32x4*>(qbase + (c * 2) * 1024);
-      const u32x4 qhi = *reinterpret_cast<const u32x4*>(qbase + (c * 2 + 1) * 1024);
-      const i32x8 q = {(int)qlo[0], (int)qlo[1], (int)qlo[2], (int)qlo[3], (int)qhi[0], (int)qhi[1], (int)qhi[2], (int)qhi[3]};
+      if (c > 0) __builtin_amdgcn_sched_barrier(0);
+      const i32x8 q = sdpa_join(sdpa_lds_read(sdpa_lds(qbase), c * 2048), sdpa_lds_read(sdpa_lds(qbase), c * 2048 + 1024));
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const int row = 32 * t + lq;
-        const u32x4 lo = *reinterpret_cast<const u32x4*>(kb + k_lds_offset<KROW>(row, c * 4 + h * 2));
-        const u32x4 hi = *reinterpret_cast<const u32x4*>(kb + k_lds_offset<KROW>(row, c * 4 + h * 2 + 1));
-        const i32x8 kf = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+        const i32x8 kf = sdpa_join(sdpa_lds_read(k0 ^ (c * 64), 32 * KROW * t), sdpa_lds_read(k0 ^ (c * 64 + 16), 32 * KROW * t));
         s[t] = sdpa_mfma<FMT>(kf, q, s[t]);
       }
     }
@@ -319,8 +323,29 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   // Scores in units of log2, masks applied.  Where only a last key is set (the causal rule, the end of the keys), a lane
   // knows how many of the block's keys it may see and the scores stay as the MFMA left them.
   float mx = -__builtin_inff();
-  if (PLAIN || !general) {
-    if (!PLAIN && edge) {
+  // Fold: the scores of a block with a first key or a scale that is not positive are scaled and masked in place and then go the
+  // way of the others with a scale of 1.  (With a way of their own behind this point the kernel of four waves per SIMD keeps a
+  // tile of O in scratch memory, in its plain blocks too.)
+  constexpr bool kFold = QL && MASK == kWithoutMask;
+  float sc = sc2;
+  if constexpr (kFold && !PLAIN) {
+    if (general) {
+      int last = khi < a.S ? khi : a.S;
+      if (a.causal && qpos < last) last = qpos + 1;
+      last -= kv0 + 4 * h;
+      const int first = klo - kv0 - 4 * h;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = 32 * t + 8 * (r >> 2) + (r & 3);
+          s[t][r] = key >= last || key < first ? -__builtin_inff() : s[t][r] * sc2;
+        }
+      sc = 1.0f;
+    }
+  }
+  if (PLAIN || kFold || !general) {
+    if (!PLAIN && edge && (!kFold || !general)) {
       int last = khi < a.S ? khi : a.S;
       if (a.causal && qpos < last) last = qpos + 1;
       const int left = last - kv0 - 4 * h;
@@ -333,7 +358,7 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, s[t][r]);
-    mx *= sc2;
+    mx *= sc;
   } else {
     // One form per kind of mask, 16 scores' masks requested together; in the last block key by key.  A test in front of each of the 32
     // loads had them wait for one another, each for the block just requested as well, and kept its conditions in spilled scalar
@@ -402,7 +427,7 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float x = s[t][4 * j + i];
-          p[i] = fast_exp2(RAW ? __builtin_fmaf(x, sc2, shift) : x + shift);
+          p[i] = fast_exp2(RAW ? __builtin_fmaf(x, sc, shift) : x + shift);
           psum += p[i];
           if (CLAMP) p[i] = __builtin_elementwise_minimum(p[i], kMax8);
         }
@@ -422,24 +447,27 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
         pf[4 * t + j] = w;
       }
   };
-  if ((PLAIN || !general) && !clamp_p) exponentials(std::true_type{}, std::false_type{});
-  else if (PLAIN || !general) exponentials(std::true_type{}, std::true_type{});
+  if ((PLAIN || kFold || !general) && !clamp_p) exponentials(std::true_type{}, std::false_type{});
+  else if (PLAIN || kFold || !general) exponentials(std::true_type{}, std::true_type{});
   else exponentials(std::false_type{}, std::true_type{});
   l_run = l_run * alpha + psum;
 
-  // With the queries in LDS (three workgroups per CU, no registers for V fragments during the softmax) the V fragments
+  // With the queries in LDS (three or four workgroups per CU, no registers for V fragments during the softmax) the V fragments
   // are read here: the 32 score registers are dead, and the reads' latency passes under the rescaling of O instead of
   // standing in front of each P V product.
+  before_v();
   constexpr bool kMidV = DVT <= 4 && QL;
   i32x8 vfm[kMidV ? DVT : 1];
   if constexpr (kMidV) {
+    uint32_t v0 = sdpa_lds(vb) + v_lds_offset<kVRow>(8 * (r8 >> 2) + 4 * h + (r8 & 3), g & 1) + hh * 8;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(v0));  // the other tiles' addresses are made here, not kept over the loop
+#endif
 #pragma unroll
     for (int t = 0; t < DVT; ++t) {
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-        const int krow = 32 * (p >> 1) + 8 * (2 * (p & 1) + (r8 >> 2)) + 4 * h + (r8 & 3);
-        const int off = v_lds_offset<kVRow>(krow, 2 * t + (g & 1)) + hh * 8;
-        const i32x2 w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((SDPA_LDS_AS i32x2*)((SDPA_LDS_AS uint8_t*)vb + off));
+        const i32x2 w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((SDPA_LDS_AS i32x2*)(uintptr_t)((v0 ^ (t * 32)) + 16 * p * kVRow));
         vfm[t][2 * p] = w[0];
         vfm[t][2 * p + 1] = w[1];
       }
@@ -484,19 +512,26 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
 // Head dimension 128 with direct loads: the query fragments live in LDS instead of 16 registers and the ring has
 // two stages instead of four, which brings a workgroup to 161 registers and 48 KB of LDS, so that three
 // workgroups fit a CU (three waves per SIMD).  A wave alone needs about 3500 cycles for a block of 64 keys (a
-// chain of LDS reads, MFMAs, the softmax and MFMAs again) of which 1200 are vector work and 512 MFMA time, so a
+// chain of LDS reads, MFMAs, the softmax and MFMAs again) of which 1000 are vector work and 512 MFMA time, so a
 // SIMD is as busy as it has waves to switch between.
 constexpr bool sdpa_q_in_lds(int dkc, int dvt, bool dma) { return dma && dkc == 2 && dvt == 4; }
 // Workgroups per CU the kernel is compiled for.  Head dimension 256 (eight tiles of O: 128 registers) fits two with the
 // direct loads and a ring of two stages (255 registers, 64 KiB of LDS): 850 -> 1765 TFLOP/s at 32 / 8 heads and 8192
 // causal tokens against one workgroup with four stages.  Through registers (unaligned tensors) the same bound spills
 // 216 bytes per lane, so that form stays at one.
+// More workgroups than three per CU run four at a time (MANY): two stages of K but one of V, 40 KB with the queries, and 128
+// registers.  The values of a block are requested at its start and waited for, with the next block's keys, behind the softmax: a
+// second barrier.  32 / 8 heads, 8192 causal tokens, 324 -> 315 us; 16 heads 183 -> 169; 4096 tokens without causality 173 -> 168;
+// 64 heads x 4 x 4096 688 -> 668; 28 heads, 8192 tokens, 285 -> 277.  With fewer the fourth place stays empty and the barrier
+// costs: 4 heads, 8192 tokens, 122 -> 129; 32 heads, 2048 tokens, 39 -> 41; 20 heads, 4096 tokens, 72 -> 74.
+constexpr int kSdpaMany = 3 * 256;
+constexpr bool sdpa_four_per_cu(int dkc, int dvt, bool dma, int mask) { return sdpa_q_in_lds(dkc, dvt, dma) && mask == kWithoutMask; }
 constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { return sdpa_q_in_lds(dkc, dvt, dma) && !masked ? 3 : (dvt <= 4 || (dma && !masked)) ? 2 : 1; }
 
 // DKC: 64-byte steps of the q.k depth (head_dim_qk <= 64 DKC); DVT: 32-column tiles of v
 // (head_dim_v <= 32 DVT).
 // DMA: K and V blocks go from global memory straight into LDS (aligned tensors), a ring of kStages blocks;
-// otherwise through registers, two buffers.  A compile-time choice: with both routes in one loop the compiler
+// otherwise through registers, two buffers.  MANY: four workgroups per CU, see above.  A compile-time choice: with both routes in one loop the compiler
 // has to assume the register route's loads outstanding wherever their registers are reused, and the wait it
 // puts there (vmcnt(0), in front of the first MFMA of every block) also waits for the blocks just requested
 // by the direct route.
@@ -504,8 +539,8 @@ constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { 
 // of the unmasked prefill at 256); with a mask two workgroups per CU at 128, whose mask needs registers, and one at 256.  At 64 one
 // kernel (apart, the one without a mask was 4 to 5 % slower where a SIMD has one wave of it).
 constexpr bool sdpa_kernel_per_mask(int dvt) { return dvt > 2; }
-template <int DKC, int DVT, int FMT, bool DMA, int MASK>
-__global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA, MASK == kWithMask)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
+template <int DKC, int DVT, int FMT, bool DMA, int MASK, bool MANY>
+__global__ __launch_bounds__(kSdpaThreads, MANY ? 4 : sdpa_workgroups_per_cu(DKC, DVT, DMA, MASK == kWithMask)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
   constexpr bool kQLds = sdpa_q_in_lds(DKC, DVT, DMA);
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = DVT <= 4 ? 128 : 256;  // bytes of an LDS row of V
@@ -518,15 +553,19 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
   static_assert(KLOADS >= 1 && VLOADS >= 1, "block too small for the workgroup");
   // Direct loads run kStages - 1 blocks ahead of the arithmetic (a block's arithmetic takes about a
   // microsecond, less than a load from HBM under load; with the queries in LDS one block ahead, which the
-  // third workgroup on the CU covers, and at head dimension 256, where two stages are what leaves room for a second
+  // other workgroups on the CU cover, and at head dimension 256, where two stages are what leaves room for a second
   // workgroup); the route through registers uses two buffers.
   constexpr int kStages = (kQLds || DVT > 4) ? 2 : 4;
-  __shared__ __align__(1024) uint8_t lds[kStages * (KBYTES + VBYTES)];
+  constexpr bool kOneV = MANY;
+  static_assert(!MANY || sdpa_four_per_cu(DKC, DVT, DMA, MASK));
+  constexpr int kPitch = kOneV ? KBYTES : KBYTES + VBYTES;  // from one stage's K to the next one's
+  __shared__ __align__(1024) uint8_t lds[kStages * KBYTES + (kOneV ? 1 : kStages) * VBYTES];
   __shared__ __align__(16) uint8_t qlds[kQLds ? 4 * 4096 : 16];  // per wave: [depth chunk of 16 bytes][half-wave][row]
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
+  int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // the same in every lane, and known to be
-  const int lq = lane & 31, h = lane >> 5;
+  int lq = lane & 31, h = lane >> 5;
 
   uint32_t bi;
   int qb;
@@ -559,8 +598,8 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
 
   const int q0 = qb * kSdpaBM;
   const int wq0 = q0 + wave * 32;  // first query row of this wave
-  const int qrow = wq0 + lq;
-  const bool q_ok = qrow < a.L;
+  int qrow = wq0 + lq;
+  bool q_ok = qrow < a.L;
 
   SdpaScales sc;
   sc.load(a);
@@ -632,28 +671,50 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
     wv.base += (uint64_t)blk0 * kSdpaBN * a.ldv;
 #pragma unroll
     for (int n = 0; n < KREG; ++n) {
-      const int pos = (wave * KREG + n) * 64 + lane;  // 16-byte slot of the tile this lane fills
+      const int pos = (kOneV ? wave + 4 * n : wave * KREG + n) * 64 + lane;  // 16-byte slot of the tile this lane fills
       const int row = pos / KCPR, chunk = (pos % KCPR) ^ k_swizzle<KROW>(pos / KCPR);
       kvoff[n] = chunk * 16 < a.Dk ? row * (int)a.ldk + chunk * 16 : 0x7fffffff;
     }
 #pragma unroll
     for (int n = 0; n < VREG; ++n) {
-      const int pos = (wave * VREG + n) * 64 + lane;
+      const int pos = (kOneV ? wave + 4 * n : wave * VREG + n) * 64 + lane;
       const int row = pos / (kVRow / 16), chunk = (pos % (kVRow / 16)) ^ v_swizzle<kVRow>(pos / (kVRow / 16));
       vvoff[n] = chunk * 16 < a.Dv ? row * (int)a.ldv + chunk * 16 : 0x7fffffff;
     }
   }
   // the loads of the next block into buffer `buf`; the descriptors then move on by one block
-  auto issue_block = [&](int buf) {
-    const uint32_t kdst = (uint32_t)(uintptr_t)(SDPA_LDS_AS uint8_t*)(lds + buf * (KBYTES + VBYTES));
+  // (an offset that the compiler cannot make before the loop and keep: with one V, registers are what the fourth wave needs)
+  const auto later = [](int off, int n, int ld) {
+    if (n == 0) return off;
+    int add = n * 32 * ld;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(add));
+#endif
+    return (int)((uint32_t)off + (uint32_t)add);  // (a lane with nothing to load stays beyond any descriptor)
+  };
+  auto issue_k = [&](int buf) {
+    const uint32_t dst = (uint32_t)(uintptr_t)(SDPA_LDS_AS uint8_t*)(lds + buf * kPitch);
     const i32x4 rk = wk.rsrc(rows_left, (int)a.ldk, a.Dk);
 #pragma unroll
-    for (int n = 0; n < KREG; ++n) sdpa_dma16(rk, kvoff[n], kdst + (wave * KREG + n) * 1024);
-    const i32x4 rv = wv.rsrc(rows_left, (int)a.ldv, a.Dv);
-#pragma unroll
-    for (int n = 0; n < VREG; ++n) sdpa_dma16(rv, vvoff[n], kdst + KBYTES + (wave * VREG + n) * 1024);
+    for (int n = 0; n < KREG; ++n) {
+      if constexpr (kOneV) sdpa_dma16(rk, later(kvoff[0], n, (int)a.ldk), dst + (wave + 4 * n) * 1024);
+      else sdpa_dma16(rk, kvoff[n], dst + (wave * KREG + n) * 1024);
+    }
     wk.base += (uint64_t)kSdpaBN * a.ldk;
+  };
+  auto issue_v = [&](int buf, int rows) {
+    const uint32_t dst = (uint32_t)(uintptr_t)(SDPA_LDS_AS uint8_t*)(kOneV ? lds + kStages * KBYTES : lds + buf * kPitch + KBYTES);
+    const i32x4 rv = wv.rsrc(rows, (int)a.ldv, a.Dv);
+#pragma unroll
+    for (int n = 0; n < VREG; ++n) {
+      if constexpr (kOneV) sdpa_dma16(rv, later(vvoff[0], n, (int)a.ldv), dst + (wave + 4 * n) * 1024);
+      else sdpa_dma16(rv, vvoff[n], dst + (wave * VREG + n) * 1024);
+    }
     wv.base += (uint64_t)kSdpaBN * a.ldv;
+  };
+  auto issue_block = [&](int buf) {
+    issue_k(buf);
+    if constexpr (!kOneV) issue_v(buf, rows_left);
     rows_left -= kSdpaBN;
   };
 
@@ -706,20 +767,31 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
     const int pos = blk - blk0;
     if constexpr (DMA) {
       if (blk + kStages - 1 < nblk) issue_block((unsigned)(pos + kStages - 1) % kStages);
+      if constexpr (kOneV) issue_v(0, a.S - kv0);
     } else {
       if (blk + 1 < nblk) fetch(blk + 1);
     }
-    const uint8_t* kb = lds + (DMA ? (unsigned)pos % kStages : pos & 1) * (KBYTES + VBYTES);
-    const uint8_t* vb = kb + KBYTES;
+    const uint8_t* kb = lds + (DMA ? (unsigned)pos % kStages : pos & 1) * kPitch;
+    const uint8_t* vb = kOneV ? lds + kStages * KBYTES : kb + KBYTES;
+    const auto v_landed = [&] {
+      if constexpr (kOneV) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+      }
+    };
 
     // a wave whose 32 rows all lie above this block's first key has nothing to add
     if (PLAIN || !(a.causal && kv0 > wq0 + 31)) {
       const bool edge = (a.causal && kv0 + kSdpaBN - 1 > wq0) || kv0 + kSdpaBN > khi;
       sdpa_block<DKC, DVT, FMT, kQLds, PLAIN, MASK>(a, kb, vb, kv0, edge, masked || kv0 < klo, qrow, mrow, qf, sc2, lqs, clamp_p, o, m_run, l_run,
-                                                    qbase, klo, khi);
+                                                    v_landed, qbase, klo, khi);
+    } else {
+      v_landed();
     }
 
-    if constexpr (DMA) {
+    if constexpr (kOneV) {
+      // (the next block's keys were waited for with this one's values)
+    } else if constexpr (DMA) {
       // The next block has landed once only the loads of the blocks after it are outstanding.  Loads
       // retire in issue order as long as every one of them goes to memory; one whose lanes all lie
       // beyond kv_len completes at once, so the count is only trusted while every block in flight is
@@ -742,6 +814,13 @@ __global__ __launch_bounds__(kSdpaThreads, sdpa_workgroups_per_cu(DKC, DVT, DMA,
   int blk = blk0;
   if constexpr (MASK != kWithMask && (DVT <= 4 || DMA)) {  // (through registers a second loop does not fit at head dimension 256)
     for (; blk < plain; ++blk) step(std::true_type{}, blk);
+  }
+  if constexpr (kOneV) {  // made again from the lane's number: none of these need a register over the plain blocks
+    lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    lq = lane & 31;
+    h = lane >> 5;
+    qrow = wq0 + lq;
+    q_ok = qrow < a.L;
   }
   for (; blk < nblk; ++blk) step(std::false_type{}, blk);
 
@@ -1087,7 +1166,7 @@ __global__ __launch_bounds__(kSdpaThreads) void fp8_sdpa_decode_kernel(const Sdp
     }
     const uint8_t* kb = mine + buf * kStage;
     sdpa_block<DKC, DVT, FMT, false, decltype(pc)::value, kEither>(a, kb, kb + KBYTES, kv0, a.causal || kv0 + kSdpaBN > a.S, masked, qpos, mrow, qf, sc2,
-                                                          lqs, clamp_p, o, m_run, l_run);
+                                                          lqs, clamp_p, o, m_run, l_run, [] {});
     buf ^= 1;
   };
   int plain = a.S / kSdpaBN < b1 ? a.S / kSdpaBN : b1;
@@ -1186,8 +1265,14 @@ static void sdpa_order(SdpaArgs& a, const mi355q_sdpa_desc* d, int64_t batches, 
 template <int DKC, int DVT, int FMT, int MASK>
 static void sdpa_launch_kernel(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
   const dim3 grid((unsigned)blocks), block(kSdpaThreads);
-  if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, false, MASK>), grid, block, 0, st, a);
+  if constexpr (sdpa_four_per_cu(DKC, DVT, true, MASK)) {
+    if (a.dma && blocks > kSdpaMany) {
+      hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK, true>), grid, block, 0, st, a);
+      return;
+    }
+  }
+  if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK, false>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, false, MASK, false>), grid, block, 0, st, a);
 }
 template <int DKC, int DVT, int FMT>
 static void sdpa_launch_fmt(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
