@@ -1,7 +1,8 @@
-"""The order in which a causal prefill's workgroups take heads and query blocks (sdpa_place): every block is served, once.
+"""The order in which a causal prefill's workgroups take heads and query blocks (sdpa_place): every block is served, once; and the
+form of the kernel for many workgroups (MANY).
 
 A block of query rows does not depend on which workgroup served it, so the whole call equals its heads called one by one, which
-are too few workgroups for the order to be changed, bit for bit.
+are too few workgroups for the order to be changed or for that form, bit for bit.
 """
 import math
 
@@ -36,3 +37,28 @@ def test_every_block_once(dev, heads, kv_heads, length, keys, dim):
     for a in range(kv_heads):
         for b in range(heads // kv_heads):
             assert torch.equal(out[a, b], run(q[a:a + 1, b:b + 1], k[a:a + 1], v[a:a + 1])[0, 0]), (a, b)
+
+
+@pytest.mark.parametrize("keys", [1, 63, 65, 128, 500])
+@pytest.mark.parametrize("causal,scale,p_scale,pad", [
+    (False, 0.1, 128.0, None),
+    (True, 0.1, 128.0, None),
+    (True, -0.1, 128.0, None),      # scores scaled in place: a scale that is not positive
+    (False, 0.0, 1.0, None),
+    (True, 0.1, 1000.0, None),      # probabilities that have to be limited
+    (True, 0.1, 128.0, "left"),     # a first key
+    (True, 0.1, 128.0, "right"),
+])
+def test_many_workgroups(dev, keys, causal, scale, p_scale, pad):
+    batch, heads, length, dim = 4, 50, 500, 128  # 800 workgroups: more than three per CU
+    gen = torch.Generator(device=dev).manual_seed(keys)
+    q, k, v = (torch.randn((batch, heads, n, dim), generator=gen, device=dev).to(E4) for n in (length, keys, keys))
+    valid = None if pad is None else torch.tensor([keys, (keys + 1) // 2, max(keys - 64, 0), 1], dtype=torch.int32, device=dev)
+
+    def run(q, k, v, valid):
+        return torch.ops.hpu.fp8_sdpa_recomp_fwd.scalar(q, k, v, None, 0.0, scale, causal, False, "None", 1.0, 1.0, 1.0,
+                                                        p_scale, 0.0, 1.0 / p_scale, False, False, valid, pad or "left")[0]
+    out = run(q, k, v, valid)
+    for b in range(batch):
+        one = slice(b, b + 1)
+        assert torch.equal(out[one], run(q[one], k[one], v[one], None if valid is None else valid[one])), b
