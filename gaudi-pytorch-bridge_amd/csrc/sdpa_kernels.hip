@@ -238,6 +238,14 @@ __device__ __forceinline__ i32x8 sdpa_join(const u32x4& lo, const u32x4& hi) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// A wave's largest value into the launch's.  The word only grows, so a value that does not exceed what is read changes nothing,
+// and nearly none do: with an atomic operation of every wave on one address, 4096 of them, 2 x 32 heads x 2048 causal tokens took
+// 87 us, now 59 as without the amax.
+__device__ __forceinline__ void sdpa_raise_amax(float* amax, uint32_t bits) {
+  unsigned int* word = reinterpret_cast<unsigned int*>(amax);
+  if (bits > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, bits);
+}
+
 __global__ void sdpa_clear_amax_kernel(float* a, float* b) {
   if (a != nullptr) *a = 0.0f;
   if (b != nullptr) *b = 0.0f;
@@ -890,14 +898,14 @@ __global__ __launch_bounds__(kSdpaThreads, MANY ? 4 : sdpa_workgroups_per_cu(DKC
       }
     if (a.amax_o != nullptr) {
       const uint32_t m = wave_max_u32(__float_as_uint(amax_o));
-      if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), m);
+      if (lane == 0) sdpa_raise_amax(a.amax_o, m);
     }
   }
 
   if (a.amax_s != nullptr) {
     // the largest probability of a row is the one at the row maximum: 1 / l
     const uint32_t m = wave_max_u32(__float_as_uint(q_ok ? inv_l : 0.0f));
-    if (lane == 0 && m != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_s), m);
+    if (lane == 0) sdpa_raise_amax(a.amax_s, m);
   }
 }
 
@@ -1029,11 +1037,11 @@ __device__ __forceinline__ void sdpa_decode_finish(const SdpaArgs& a, uint8_t* l
   const int lane = tid & 63;
   if (a.amax_s != nullptr) {
     const uint32_t mx = wave_max_u32(__float_as_uint(row_ok && dv0 == 0 ? inv_l : 0.0f));
-    if (lane == 0 && mx != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_s), mx);
+    if (lane == 0) sdpa_raise_amax(a.amax_s, mx);
   }
   if (a.amax_o != nullptr) {
     const uint32_t mx = wave_max_u32(__float_as_uint(amax_o));
-    if (lane == 0 && mx != 0u) atomicMax(reinterpret_cast<unsigned int*>(a.amax_o), mx);
+    if (lane == 0) sdpa_raise_amax(a.amax_o, mx);
   }
 }
 
