@@ -54,16 +54,16 @@ MEASURED_TRAFFIC = {
     "fp8_gemm_v2_decode_M16": 244.33e6,
     "fp8_gemm_v2_decode_M64": 242.92e6,
     "fp8_gemm_v2_decode_M256": 266.36e6,
-    "w4a8_gemm_M16": 129.02e6,      # the partial sums of the two K parts on top of the 124 MB of operands
+    "w4a8_gemm_M16": 138.79e6,      # the partial sums of the four K parts, written and read, on top of the 123 MB of operands
     "w4a8_gemm_M32": 135.97e6,
     "w4a8_gemm_M64": 149.87e6,
     "w4a8_gemm_M256": 153.59e6,     # two row blocks of 128 on one XCD share a strip's weights in its L2
-    "w4a16_gemm_M16": 130.15e6,     # split_rows_vec_kernel + w4a8_wide_kernel<two planes>
-    "w4a16_gemm_M64": 154.13e6,
+    "w4a16_gemm_M16": 139.84e6,
+    "w4a16_gemm_M64": 154.13e6,     # split_rows_vec_kernel + w4a8_wide_kernel<two planes>
     "w4a16_gemm_M256": 178.81e6,
-    "fp8_sdpa_B1_L8192": 124.80e6,
-    "fp8_sdpa_B4_L4096": 235.33e6,
-    "fp8_sdpa_B1_L8192_D256": 354.91e6,   # k and v are re-read by the query blocks of a head group beyond L2
+    "fp8_sdpa_B1_L8192": 133.81e6,
+    "fp8_sdpa_B4_L4096": 346.11e6,   # an XCD walks the heads of four k and v together, 4 MiB
+    "fp8_sdpa_B1_L8192_D256": 306.55e6,   # k and v are re-read by the query blocks of a head group beyond L2
     "fp8_sdpa_decode_B64_S4096": 537.24e6,
     "fp8_sdpa_decode_B8_S8192": 136.71e6,   # fp8_sdpa_decode_kernel 135.57 + 1.14 written and read back by the merge
     "softmax_fp8": 1609.32e6,
@@ -587,7 +587,7 @@ def bench_w4a8(oracle, dev, steps, warmup, cpu):
                  "sample": f"M=16, {rows_n} of the 28672 output columns: unpack, (q - z) * s in float64, matmul, per-row scale"}
         out.append(hbm_entry(f"w4a8_gemm_M{M}", f"w4a8_gemm M={M} K=8192 N=28672: uint4 weights (group 128, bf16 scales, packed "
                                                 "zero points) x per-token e4m3fn activations -> bf16",
-                             nbytes, ms, steps, "w4a8_wide_kernel", c,
+                             nbytes, ms, steps, "w4_stream_kernel" if M <= 16 else "w4a8_wide_kernel", c,
                              extra={"tflops": round(2.0 * M * N * K / (ms * 1e-3) / 1e12, 2)}))
     return out
 
@@ -619,7 +619,8 @@ def bench_w4a16(oracle, dev, steps, warmup, cpu):
             c = {"value": round((K * cols_n // 2) / t / 1e9, 3), "unit": "GB/s", "cores": torch.get_num_threads(), "kind": "port",
                  "sample": f"M=16, {cols_n} of the 28672 output columns: unpack, (q - z) * s in float64, matmul"}
         out.append(hbm_entry(f"w4a16_gemm_M{M}", f"w4a16_gemm M={M} K=8192 N=28672: uint4 weights (group 128, bf16 scales, packed zero points) "
-                                                 "x bf16 activations -> bf16", nbytes, ms, steps, "split_rows_vec_kernel + w4a8_wide_kernel<two planes>", c,
+                                                 "x bf16 activations -> bf16", nbytes, ms, steps,
+                             "w4_stream_kernel" if M <= 16 else "split_rows_vec_kernel + w4a8_wide_kernel<two planes>", c,
                              extra={"tflops": round(2.0 * M * N * K / (ms * 1e-3) / 1e12, 2)}))
     return out
 
