@@ -17,8 +17,8 @@
 // and the V^T fragment is gathered from LDS in the same key order by the transposing reads
 // (ds_read_b64_tr_b8 takes each of its 8 k-rows from its own address).
 //
-// K and V blocks are double buffered in LDS, one barrier per block (the form for many workgroups of head
-// dimension 128: one V, two barriers).  Aligned tensors (16-byte rows and head dimensions) go global -> LDS directly (buffer_load ... lds: the loads of block
+// K and V blocks are double buffered in LDS, one barrier per block (the form for many workgroups: one V,
+// two barriers).  Aligned tensors (16-byte rows and head dimensions) go global -> LDS directly (buffer_load ... lds: the loads of block
 // i + 1 are issued before the arithmetic of block i and waited for after it, and cost the waves
 // neither registers nor vector instructions); anything else goes through registers, byte by
 // byte where it must.  Rows are XOR-swizzled so that the fragment reads are bank-conflict free;
@@ -332,7 +332,7 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   // knows how many of the block's keys it may see and the scores stay as the MFMA left them.
   float mx = -__builtin_inff();
   // Fold: the scores of a block with a first key or a scale that is not positive are scaled and masked in place and then go the
-  // way of the others with a scale of 1.  (With a way of their own behind this point the kernel of four waves per SIMD keeps a
+  // way of the others with a scale of 1.  (With a way of their own behind this point the form of four waves per SIMD keeps a
   // tile of O in scratch memory, in its plain blocks too.)
   constexpr bool kFold = QL && MASK == kWithoutMask;
   float sc = sc2;
@@ -527,19 +527,21 @@ constexpr bool sdpa_q_in_lds(int dkc, int dvt, bool dma) { return dma && dkc == 
 // direct loads and a ring of two stages (255 registers, 64 KiB of LDS): 850 -> 1765 TFLOP/s at 32 / 8 heads and 8192
 // causal tokens against one workgroup with four stages.  Through registers (unaligned tensors) the same bound spills
 // 216 bytes per lane, so that form stays at one.
-// More workgroups than three per CU run four at a time (MANY): two stages of K but one of V, 40 KB with the queries, and 128
-// registers.  The values of a block are requested at its start and waited for, with the next block's keys, behind the softmax: a
-// second barrier.  32 / 8 heads, 8192 causal tokens, 324 -> 315 us; 16 heads 183 -> 169; 4096 tokens without causality 173 -> 168;
-// 64 heads x 4 x 4096 688 -> 668; 28 heads, 8192 tokens, 285 -> 277.  With fewer the fourth place stays empty and the barrier
-// costs: 4 heads, 8192 tokens, 122 -> 129; 32 heads, 2048 tokens, 39 -> 41; 20 heads, 4096 tokens, 72 -> 74.
+// More workgroups than three per CU, the most of the other form, run four at a time at head dimension 128 and five at 64 (MANY): two
+// stages of K but one of V, 40 and 24 KB with the queries, 128 and 96 registers.  The values of a block are requested at its
+// start and waited for, with the next block's keys, behind the softmax: a second barrier.  128, us: 32 / 8 heads, 8192 causal tokens,
+// 324 -> 315; 16 heads 183 -> 169; 4096 tokens without causality 173 -> 168; 64 heads x 4 x 4096 688 -> 668; 28 heads, 8192 tokens,
+// 285 -> 277.  64, us: 32 / 8 heads, 8192 tokens, 243 -> 228 (four at a time 232), 8 x 1024 44 -> 41, 64 heads x 16 x 512 60 -> 53, 32 x 32 / 8 x 333
+// 39 -> 33, the same without causality 42 -> 37.  With fewer workgroups the further places stay empty and the barrier costs, at 128: 4 heads, 8192
+// tokens, 122 -> 129; 32 heads, 2048 tokens, 39 -> 41; 20 heads, 4096 tokens, 72 -> 74.
 constexpr int kSdpaMany = 3 * 256;
-constexpr bool sdpa_four_per_cu(int dkc, int dvt, bool dma, int mask) { return sdpa_q_in_lds(dkc, dvt, dma) && mask == kWithoutMask; }
+constexpr int sdpa_many_per_cu(int dkc, int dvt) { return dkc == 2 && dvt == 4 ? 4 : dkc == 1 && dvt == 2 ? 5 : 0; }  // 0: there is no such form
 constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { return sdpa_q_in_lds(dkc, dvt, dma) && !masked ? 3 : (dvt <= 4 || (dma && !masked)) ? 2 : 1; }
 
 // DKC: 64-byte steps of the q.k depth (head_dim_qk <= 64 DKC); DVT: 32-column tiles of v
 // (head_dim_v <= 32 DVT).
 // DMA: K and V blocks go from global memory straight into LDS (aligned tensors), a ring of kStages blocks;
-// otherwise through registers, two buffers.  MANY: four workgroups per CU, see above.  A compile-time choice: with both routes in one loop the compiler
+// otherwise through registers, two buffers.  MANY: see above.  A compile-time choice: with both routes in one loop the compiler
 // has to assume the register route's loads outstanding wherever their registers are reused, and the wait it
 // puts there (vmcnt(0), in front of the first MFMA of every block) also waits for the blocks just requested
 // by the direct route.
@@ -548,8 +550,8 @@ constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { 
 // kernel (apart, the one without a mask was 4 to 5 % slower where a SIMD has one wave of it).
 constexpr bool sdpa_kernel_per_mask(int dvt) { return dvt > 2; }
 template <int DKC, int DVT, int FMT, bool DMA, int MASK, bool MANY>
-__global__ __launch_bounds__(kSdpaThreads, MANY ? 4 : sdpa_workgroups_per_cu(DKC, DVT, DMA, MASK == kWithMask)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
-  constexpr bool kQLds = sdpa_q_in_lds(DKC, DVT, DMA);
+__global__ __launch_bounds__(kSdpaThreads, MANY ? sdpa_many_per_cu(DKC, DVT) : sdpa_workgroups_per_cu(DKC, DVT, DMA, MASK == kWithMask)) void fp8_sdpa_fwd_kernel(const SdpaArgs a) {
+  constexpr bool kQLds = MANY || sdpa_q_in_lds(DKC, DVT, DMA);
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = DVT <= 4 ? 128 : 256;  // bytes of an LDS row of V
   constexpr int KCPR = KROW / 16;           // chunks per K row
@@ -565,10 +567,10 @@ __global__ __launch_bounds__(kSdpaThreads, MANY ? 4 : sdpa_workgroups_per_cu(DKC
   // workgroup); the route through registers uses two buffers.
   constexpr int kStages = (kQLds || DVT > 4) ? 2 : 4;
   constexpr bool kOneV = MANY;
-  static_assert(!MANY || sdpa_four_per_cu(DKC, DVT, DMA, MASK));
+  static_assert(!MANY || (DMA && MASK == kWithoutMask && sdpa_many_per_cu(DKC, DVT) > 0));
   constexpr int kPitch = kOneV ? KBYTES : KBYTES + VBYTES;  // from one stage's K to the next one's
   __shared__ __align__(1024) uint8_t lds[kStages * KBYTES + (kOneV ? 1 : kStages) * VBYTES];
-  __shared__ __align__(16) uint8_t qlds[kQLds ? 4 * 4096 : 16];  // per wave: [depth chunk of 16 bytes][half-wave][row]
+  __shared__ __align__(16) uint8_t qlds[kQLds ? 4 * DKC * 2048 : 16];  // per wave: [depth chunk of 16 bytes][half-wave][row]
 
   const int tid = threadIdx.x;
   int lane = tid & 63;
@@ -748,13 +750,13 @@ __global__ __launch_bounds__(kSdpaThreads, MANY ? 4 : sdpa_workgroups_per_cu(DKC
 #pragma unroll
   for (int c = 0; c < DKC; ++c) asm volatile("" : : "v"(qf[c]));
 #endif
-  const uint8_t* qbase = qlds + (kQLds ? wave * 4096 + h * 512 + lq * 16 : 0);
+  const uint8_t* qbase = qlds + (kQLds ? wave * DKC * 2048 + h * 512 + lq * 16 : 0);
   if constexpr (kQLds) {
 #pragma unroll
     for (int c = 0; c < DKC; ++c) {
-      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2) * 1024 + h * 512 + lq * 16) =
+      *reinterpret_cast<u32x4*>(qlds + wave * DKC * 2048 + (c * 2) * 1024 + h * 512 + lq * 16) =
           u32x4{(uint32_t)qf[c][0], (uint32_t)qf[c][1], (uint32_t)qf[c][2], (uint32_t)qf[c][3]};
-      *reinterpret_cast<u32x4*>(qlds + wave * 4096 + (c * 2 + 1) * 1024 + h * 512 + lq * 16) =
+      *reinterpret_cast<u32x4*>(qlds + wave * DKC * 2048 + (c * 2 + 1) * 1024 + h * 512 + lq * 16) =
           u32x4{(uint32_t)qf[c][4], (uint32_t)qf[c][5], (uint32_t)qf[c][6], (uint32_t)qf[c][7]};
     }
   }
@@ -1273,9 +1275,9 @@ static void sdpa_order(SdpaArgs& a, const mi355q_sdpa_desc* d, int64_t batches, 
 template <int DKC, int DVT, int FMT, int MASK>
 static void sdpa_launch_kernel(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
   const dim3 grid((unsigned)blocks), block(kSdpaThreads);
-  if constexpr (sdpa_four_per_cu(DKC, DVT, true, MASK)) {
-    if (a.dma && blocks > kSdpaMany) {
-      hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK, true>), grid, block, 0, st, a);
+  if constexpr (MASK != kWithMask && sdpa_many_per_cu(DKC, DVT) > 0) {
+    if (a.dma && a.mask_kind == kMaskNone && blocks > kSdpaMany) {
+      hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, kWithoutMask, true>), grid, block, 0, st, a);
       return;
     }
   }

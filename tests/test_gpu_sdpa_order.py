@@ -39,6 +39,7 @@ def test_every_block_once(dev, heads, kv_heads, length, keys, dim):
             assert torch.equal(out[a, b], run(q[a:a + 1, b:b + 1], k[a:a + 1], v[a:a + 1])[0, 0]), (a, b)
 
 
+@pytest.mark.parametrize("dim", [128, 112, 64, 48])
 @pytest.mark.parametrize("keys", [1, 63, 65, 128, 500])
 @pytest.mark.parametrize("causal,scale,p_scale,pad", [
     (False, 0.1, 128.0, None),
@@ -49,8 +50,8 @@ def test_every_block_once(dev, heads, kv_heads, length, keys, dim):
     (True, 0.1, 128.0, "left"),     # a first key
     (True, 0.1, 128.0, "right"),
 ])
-def test_many_workgroups(dev, keys, causal, scale, p_scale, pad):
-    batch, heads, length, dim = 4, 50, 500, 128  # 800 workgroups: more than three per CU
+def test_many_workgroups(dev, dim, keys, causal, scale, p_scale, pad):
+    batch, heads, length = 4, 50, 500  # 800 workgroups: more than three per CU
     gen = torch.Generator(device=dev).manual_seed(keys)
     q, k, v = (torch.randn((batch, heads, n, dim), generator=gen, device=dev).to(E4) for n in (length, keys, keys))
     valid = None if pad is None else torch.tensor([keys, (keys + 1) // 2, max(keys - 64, 0), 1], dtype=torch.int32, device=dev)
