@@ -53,10 +53,9 @@ __device__ __forceinline__ void block_amax_commit(uint32_t m, uint32_t* amax) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) wave_part[wave] = m;
   __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const uint32_t r = max_of_waves(wave_part);
   if (threadIdx.x == 0) {
-    uint32_t r = wave_part[0];
-    const int nwaves = (int)(blockDim.x >> 6);
-    for (int w = 1; w < nwaves; ++w) r = r > wave_part[w] ? r : wave_part[w];
     // Atomics on one address serialise in L2.  The running maximum only grows,
     // so a block whose maximum does not beat the value already there has
     // nothing to add: read it first (device-scope load, not from L1) and skip
@@ -664,10 +663,7 @@ __device__ __forceinline__ float row_scale_of_block(uint32_t am, float target, i
   am = wave_max_u32(am);
   if ((threadIdx.x & 63) == 0) wave_part[threadIdx.x >> 6] = am;
   __syncthreads();
-  uint32_t r = wave_part[0];
-  const int waves = (int)(blockDim.x >> 6);
-  for (int w = 1; w < waves; ++w) r = r > wave_part[w] ? r : wave_part[w];
-  const float scale = row_scale(target, __uint_as_float(r));
+  const float scale = row_scale(target, __uint_as_float(max_of_waves(wave_part)));
   if (threadIdx.x == 0) {
     if (scale_out) scale_out[row] = scale;
     if (scale_inv_out) scale_inv_out[row] = 1.0f / scale;
