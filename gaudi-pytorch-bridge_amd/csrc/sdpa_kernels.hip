@@ -267,7 +267,11 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   constexpr int KROW = DKC * 64;
   constexpr int kVRow = DVT <= 4 ? 128 : 256;
   constexpr float kMax8 = FMT == MI355Q_E5M2 ? 57344.0f : 448.0f;
-  const int lane = threadIdx.x & 63, lq = lane & 31, h = lane >> 5;
+  constexpr bool kFold = QL && MASK == kWithoutMask;  // (see below)
+  // (head dimension 64: made again in the loop of the blocks that are not plain: the parts of addresses that both loops share would stay in registers over
+  // the plain one)
+  const int lane = kFold && !PLAIN && DVT <= 2 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : (int)(threadIdx.x & 63);
+  const int lq = lane & 31, h = lane >> 5;
   f32x16 s[2];
   if constexpr (QL) {
     // the query fragments come from LDS, one depth step at a time (registers for more waves per SIMD)
@@ -334,7 +338,6 @@ __device__ __forceinline__ void sdpa_block(const SdpaArgs& a, const uint8_t* kb,
   // Fold: the scores of a block with a first key or a scale that is not positive are scaled and masked in place and then go the
   // way of the others with a scale of 1.  (With a way of their own behind this point the form of four waves per SIMD keeps a
   // tile of O in scratch memory, in its plain blocks too.)
-  constexpr bool kFold = QL && MASK == kWithoutMask;
   float sc = sc2;
   if constexpr (kFold && !PLAIN) {
     if (general) {
