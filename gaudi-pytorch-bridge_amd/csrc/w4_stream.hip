@@ -38,7 +38,9 @@ constexpr int kW4StStages = 3;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Eight k of one operand of v_mfma_f32_16x16x32_bf16.  Weights are q x 2^-kW4StShift, with which the sums of a group stay inside fp32
-// whatever the activations; sums of activations alone are taken with ones of the same size.
+// whatever the activations, and with denormal ones too every product is still a multiple of fp32's smallest value; sums of activations
+// alone are taken with ones of the same size.  The sums over the groups are in the results' own units: at 2^-kW4StShift of them
+// results below 2^-113 lost bits (rows of 2^-120 under scales of 2^-27 all of them).
 constexpr int kW4StShift = 12;
 __device__ __forceinline__ u32x4 w4_st_weights(uint32_t w) {  // eight nibbles, the even ones for k 0 .. 3
   const int even = (int)(w & 0x0f0f0f0fu), odd = (int)((w >> 4) & 0x0f0f0f0fu);
@@ -78,8 +80,8 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
   static_assert(kStage % 256 == 0, "rows of weights stay aligned");
   static_assert(S == 3, "the loaders' waits are for one stage behind the one they wait for");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[S * kStage];
-  __shared__ __attribute__((aligned(16))) float scales[2][kW4StBN], zeros[2][HAS_Z ? kW4StBN : 4];  // zeros: minus zero-point x scale
-  __shared__ uint32_t word;
+  __shared__ __attribute__((aligned(16))) float scales[2][kW4StBN], zeros[2][HAS_Z ? kW4StBN : 4];  // zeros: minus the zero-points
+  __shared__ uint32_t word, again;
 
   const GemmArgs& g = a.g;
   const int strips = (g.N + kW4StBN - 1) / kW4StBN;
@@ -92,6 +94,15 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
   f32x4 total[kW4StTiles];
 #pragma unroll
   for (int t = 0; t < kW4StTiles; ++t) total[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // bf16 activations near the end of fp32's range: where a sum may not be finite the workgroup walks its part once more, at
+  // 2^-kW4StShift of the size, for the sums that are not.  The question costs 0.2 us of 12 to 28; both sums side by side 0.3 to 1.2.
+  bool second = false;
+  const auto once_more = [&] {
+    if (!A16 || second) return false;
+    second = __builtin_amdgcn_readfirstlane((int)again) != 0;
+    return second;
+  };
+  if (A16 && threadIdx.x == 0) again = 0;  // (in front of the barrier of the first stage)
 
   if (wave >= kW4StConsumers) {
     const int wq = wave - kW4StConsumers;
@@ -136,34 +147,36 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
       if (bring_zp) w4_dma4(view(row_from + group * row_step), vo_row, base + off + row_at);
       else w4_dma16(view(row_from + group * row_step), vo_row, base + off + row_at);
     };
-    // the scales of a stage as fp32 and minus zero-point times scale, two columns per lane, for the fold one stage later
+    // the scales of a stage and minus its zero-points as fp32, two columns per lane, for the fold one stage later
     const uint32_t flip = a.is_signed ? 0x88u : 0u;
     auto rows = [&](int off, int slot) {
       const int n = (wq * 64 + lane) * 2;
       const uint32_t s2 = *reinterpret_cast<const uint32_t*>(lds + off + kOffScale + 2 * n);
-      const f32x2 s = {__uint_as_float(s2 << 16), __uint_as_float(s2 & 0xffff0000u)};
-      *reinterpret_cast<f32x2*>(&scales[slot][n]) = s;
+      const float up = second ? 1.0f : (float)(1 << kW4StShift);
+      *reinterpret_cast<f32x2*>(&scales[slot][n]) = f32x2{__uint_as_float(s2 << 16) * up, __uint_as_float(s2 & 0xffff0000u) * up};
       if constexpr (HAS_Z) {
         const uint32_t z2 = (a.zp != nullptr ? lds[off + kOffZp + n / 2] : 0u) ^ flip;
-        *reinterpret_cast<f32x2*>(&zeros[slot][n]) = f32x2{-(float)(z2 & 15u) * s[0], -(float)(z2 >> 4) * s[1]};
+        *reinterpret_cast<f32x2*>(&zeros[slot][n]) = f32x2{-(float)(z2 & 15u), -(float)(z2 >> 4)};
       }
     };
+    do {
 #pragma unroll
-    for (int s = 0; s < S - 1; ++s)
-      if (s < KT) issue(s * kStage, s);
-    int wr_off = (S - 1) * kStage, rd_off = 0;
-    for (int kt = 0; kt < KT; ++kt) {
-      // stage kt has landed when only the loads of those after it are on their way
-      constexpr int c = (S - 2) * kOps;
-      if (kt + S - 2 < KT) __builtin_amdgcn_s_waitcnt((c & 15) | ((c >> 4) << 14) | 0x0f70);
-      else __builtin_amdgcn_s_waitcnt(0x0f70);
-      __syncthreads();  // stage kt is in LDS for the consumers, who are done with stage kt - 1
-      if (kt + S - 1 < KT) issue(wr_off, kt + S - 1);
-      rows(rd_off, kt & 1);
-      wr_off = wr_off + kStage == S * kStage ? 0 : wr_off + kStage;
-      rd_off = rd_off + kStage == S * kStage ? 0 : rd_off + kStage;
-    }
-    __syncthreads();  // the consumers' fold of the last stage
+      for (int s = 0; s < S - 1; ++s)
+        if (s < KT) issue(s * kStage, s);
+      int wr_off = (S - 1) * kStage, rd_off = 0;
+      for (int kt = 0; kt < KT; ++kt) {
+        // stage kt has landed when only the loads of those after it are on their way
+        constexpr int c = (S - 2) * kOps;
+        if (kt + S - 2 < KT) __builtin_amdgcn_s_waitcnt((c & 15) | ((c >> 4) << 14) | 0x0f70);
+        else __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();  // stage kt is in LDS for the consumers, who are done with stage kt - 1
+        if (kt + S - 1 < KT) issue(wr_off, kt + S - 1);
+        rows(rd_off, kt & 1);
+        wr_off = wr_off + kStage == S * kStage ? 0 : wr_off + kStage;
+        rd_off = rd_off + kStage == S * kStage ? 0 : rd_off + kStage;
+      }
+      __syncthreads();  // the consumers' fold of the last stage
+    } while (once_more());
   } else {
     const uint32_t flip = a.is_signed ? 0x88888888u : 0u;  // signed nibble s = (q ^ 8) - 8
     // lane: row m = lane % 16 of A; columns n0 + 64 wave + 16 t + 4 gk + e.  The transposing read of step pair p points at k-row
@@ -188,13 +201,14 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
 #pragma unroll
       for (int t = 0; t < kW4StTiles; ++t) {
         const f32x4 s = *reinterpret_cast<const f32x4*>(&scales[B][col + 16 * t]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) total[t][e] = __builtin_fmaf(acc[B][t][e], s[e], total[t][e]);
+        f32x4 d = acc[B][t];  // the zero-points first, so that what cancels does so here
         if constexpr (HAS_Z) {
           const f32x4 z = *reinterpret_cast<const f32x4*>(&zeros[B][col + 16 * t]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) total[t][e] = __builtin_fmaf(z[e], sums[B], total[t][e]);
+          for (int e = 0; e < 4; ++e) d[e] = __builtin_fmaf(z[e], sums[B], d[e]);
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[t][e] = __builtin_fmaf(d[e], s[e], total[t][e]);
       }
     };
     auto stage = [&](auto bc, auto hpc) {
@@ -241,20 +255,53 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
     };
     using T = std::true_type;
     using F = std::false_type;
-    stage(std::integral_constant<int, 0>{}, F{});
-    int kt = 1;
-    for (; kt + 1 < KT; kt += 2) {
-      stage(std::integral_constant<int, 1>{}, T{});
-      stage(std::integral_constant<int, 0>{}, T{});
+    // Before the barrier of the last stage's rows: whether the sums are finite so far, and that stage's far from the end of the range.
+    const auto in_range = [&](auto bc) {
+      constexpr int B = decltype(bc)::value;
+      float so_far = 0.0f, most = 0.0f;  // so_far: or NaN
+#pragma unroll
+      for (int t = 0; t < kW4StTiles; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          so_far = __builtin_fmaf(total[t][e], 0.0f, so_far);
+          most = __builtin_fmaxf(most, __builtin_fabsf(acc[B][t][e]));
+        }
+      if (!(so_far == 0.0f && most < 0x1p80f)) again = 1;
+    };
+    f32x4 first[A16 ? kW4StTiles : 1];
+    do {
+      if (second) {
+        rd_off = 0;
+#pragma unroll
+        for (int t = 0; t < kW4StTiles; ++t) {
+          first[A16 ? t : 0] = total[t];
+          total[t] = zero;
+        }
+      }
+      stage(std::integral_constant<int, 0>{}, F{});
+      int kt = 1;
+      for (; kt + 1 < KT; kt += 2) {
+        stage(std::integral_constant<int, 1>{}, T{});
+        stage(std::integral_constant<int, 0>{}, T{});
+      }
+      if (kt < KT) stage(std::integral_constant<int, 1>{}, T{});
+      if constexpr (A16) {
+        if (KT & 1) in_range(std::integral_constant<int, 0>{});
+        else in_range(std::integral_constant<int, 1>{});
+      }
+      __syncthreads();  // the fp32 rows of the last stage
+      if (KT & 1) fold(std::integral_constant<int, 0>{});
+      else fold(std::integral_constant<int, 1>{});
+    } while (once_more());
+    if (second) {
+#pragma unroll
+      for (int t = 0; t < kW4StTiles; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = first[A16 ? t : 0][e];
+          total[t][e] = __builtin_isfinite(v) ? v : total[t][e] * (float)(1 << kW4StShift);
+        }
     }
-    if (kt < KT) stage(std::integral_constant<int, 1>{}, T{});
-    __syncthreads();  // the fp32 rows of the last stage
-    if (KT & 1) fold(std::integral_constant<int, 0>{});
-    else fold(std::integral_constant<int, 1>{});
-#pragma unroll
-    for (int t = 0; t < kW4StTiles; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) total[t][e] *= (float)(1 << kW4StShift);
   }
 
   const ScalarScales scalars = load_scalar_scales(g);

@@ -71,6 +71,46 @@ def test_extreme_activations_in_bf16(oracle, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", [512, 4096])      # in one part, in several
+@pytest.mark.parametrize("scale", [-27, 0])
+def test_rows_of_small_activations(oracle, dev, K, scale):
+    """Results down to fp32's smallest values keep the bits that fp32 has for them, beside rows near the largest bf16 values."""
+    gen = torch.Generator().manual_seed(K + scale)
+    M, N = 16, 1056
+    q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True)
+    s = (s.float() * 2.0 ** scale).bfloat16()
+    x = (torch.randn(M, K, generator=gen).double() * torch.exp2(torch.tensor([*range(-90, -132, -3), 118, 120]).double())[:, None]).bfloat16()
+    out = torch.ops.mi355q.w4a16_gemm(x.to(dev), pk.to(dev), s.to(dev), pz.to(dev), False, torch.float32, None).cpu()
+    ref = x.double() @ ((q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0))
+    # 2^-24 of the sum of magnitudes for each of K products, of q a and z a apart, and half of fp32's smallest value wherever a group or a
+    # part is added (sixteen parts at most)
+    bound = (x.double().abs() @ (15 * s.double().repeat_interleave(128, 0))) * (2 * K * 2.0 ** -24) + (K // 128 + 16) * 2.0 ** -150
+    assert ((out.double() - ref).abs() <= bound).all(), ((out.double() - ref).abs() / bound).amax(1)
+
+
+@pytest.mark.gpu
+def test_sums_past_the_range(oracle, dev):
+    """Groups whose sums are past fp32's largest value: an infinity of the result's sign, and a finite result stays finite."""
+    gen = torch.Generator().manual_seed(6)
+    M, K, N = 8, 512, 544
+    q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True)
+    x = torch.randn(M, K, generator=gen)
+    x[:, 256:] = -x[:, :256]             # with the weights below: the last two groups take the first two back, but for one activation
+    q[256:], z[2:], s[2:] = q[:256], z[:2], s[:2]
+    pk, pz = oracle.pack_nibbles(q), oracle.pack_nibbles(z)
+    x[1::2, 300] += 4.0
+    s = (s.float() * 2.0 ** 20).bfloat16()
+    x = (x * 2.0 ** 110).bfloat16()
+    out = torch.ops.mi355q.w4a16_gemm(x.to(dev), pk.to(dev), s.to(dev), pz.to(dev), False, torch.float32, None).cpu()
+    ref = x.double() @ ((q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0))
+    top = torch.finfo(torch.float32).max
+    assert (ref[1::2].abs() > 2 * top).any() and (ref.abs() < top / 2).any()
+    assert torch.isfinite(out[ref.abs() < top / 2]).all()
+    past = ref.abs() > 2 * top
+    assert torch.equal(out[past].double(), ref[past].sign() * float("inf"))
+
+
+@pytest.mark.gpu
 def test_same_bits_whoever_adds_the_parts_up(oracle, pkg, dev):
     """The parts share the sum, or the last one adds all of them up (split_k < 0); the counters are zero afterwards; fewer parts where
     the workspace has less room than the plan wants."""
