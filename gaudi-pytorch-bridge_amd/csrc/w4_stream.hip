@@ -41,16 +41,23 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // whatever the activations, and with denormal ones too every product is still a multiple of fp32's smallest value; sums of activations
 // alone are taken with ones of the same size.  The sums over the groups are in the results' own units: at 2^-kW4StShift of them
 // results below 2^-113 lost bits (rows of 2^-120 under scales of 2^-27 all of them).
+// fp8 activations need none of that: their sums of a group are below 2^27.
 constexpr int kW4StShift = 12;
+constexpr int w4_st_shift(int act) { return act == kW4Bf16 ? kW4StShift : 0; }
+template <int ACT>
 __device__ __forceinline__ u32x4 w4_st_weights(uint32_t w) {  // eight nibbles, the even ones for k 0 .. 3
   const int even = (int)(w & 0x0f0f0f0fu), odd = (int)((w >> 4) & 0x0f0f0f0fu);
-  constexpr float s = 0x1p-3f;  // 2^9 for the code, 2^-12
+  constexpr float s = 512.0f / (float)(1 << w4_st_shift(ACT));  // 2^9 for the code
   return u32x4{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, s, false)),
                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, s, true)),
                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, s, false)),
                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, s, true))};
 }
-__device__ __forceinline__ u32x4 w4_st_ones() { return u32x4{0x39803980u, 0x39803980u, 0x39803980u, 0x39803980u}; }
+template <int ACT>
+__device__ __forceinline__ u32x4 w4_st_ones() {
+  constexpr uint32_t one = (uint32_t)(127 - w4_st_shift(ACT)) << 7, two = one << 16 | one;
+  return u32x4{two, two, two, two};
+}
 template <int ACT>
 __device__ __forceinline__ u32x4 w4_st_widen(uint32_t lo, uint32_t hi) {  // eight fp8 activations
   const auto two = [](uint32_t v, auto hc) {
@@ -152,8 +159,14 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
     auto rows = [&](int off, int slot) {
       const int n = (wq * 64 + lane) * 2;
       const uint32_t s2 = *reinterpret_cast<const uint32_t*>(lds + off + kOffScale + 2 * n);
-      const float up = second ? 1.0f : (float)(1 << kW4StShift);
-      *reinterpret_cast<f32x2*>(&scales[slot][n]) = f32x2{__uint_as_float(s2 << 16) * up, __uint_as_float(s2 & 0xffff0000u) * up};
+      f32x2 s = {__uint_as_float(s2 << 16), __uint_as_float(s2 & 0xffff0000u)};
+      if constexpr (A16) {
+        if (!second) {
+          s *= (float)(1 << kW4StShift);
+          if (!(__builtin_fabsf(s[0]) < __builtin_inff() && __builtin_fabsf(s[1]) < __builtin_inff())) again = 1;  // scales from 2^116 on
+        }
+      }
+      *reinterpret_cast<f32x2*>(&scales[slot][n]) = s;
       if constexpr (HAS_Z) {
         const uint32_t z2 = (a.zp != nullptr ? lds[off + kOffZp + n / 2] : 0u) ^ flip;
         *reinterpret_cast<f32x2*>(&zeros[slot][n]) = f32x2{-(float)(z2 & 15u), -(float)(z2 >> 4)};
@@ -244,9 +257,9 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
       for (int p = 0; p < 2; ++p)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          if constexpr (HAS_Z) rs = w4_st_mfma(w4_st_ones(), act[p][h], rs);
+          if constexpr (HAS_Z) rs = w4_st_mfma(w4_st_ones<ACT>(), act[p][h], rs);
 #pragma unroll
-          for (int t = 0; t < kW4StTiles; ++t) acc[B][t] = w4_st_mfma(w4_st_weights((uint32_t)w[p][t][h] ^ flip), act[p][h], p == 0 && h == 0 ? zero : acc[B][t]);
+          for (int t = 0; t < kW4StTiles; ++t) acc[B][t] = w4_st_mfma(w4_st_weights<ACT>((uint32_t)w[p][t][h] ^ flip), act[p][h], p == 0 && h == 0 ? zero : acc[B][t]);
         }
       // the stage before this one, whose MFMAs finished long ago, behind those just issued
       if constexpr (decltype(hpc)::value) fold(std::integral_constant<int, 1 - B>{});

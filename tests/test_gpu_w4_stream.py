@@ -111,6 +111,32 @@ def test_sums_past_the_range(oracle, dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", ["bf16", "e5m2"])
+@pytest.mark.parametrize("K", [256, 2048])      # in one part, in several
+def test_scales_near_the_end_of_the_range(oracle, dev, K, act):
+    """Scales of 2^120 beside ordinary ones, in the last group and in others: rows of zeros stay zeros, small activations give what they should."""
+    gen = torch.Generator().manual_seed(K)
+    M, N = 16, 544
+    q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
+    s[0, 1::2] = s[-1, 2::4] = 2.0 ** 120
+    x = torch.randint(-3, 4, (M, K), generator=gen).double()
+    x[3] = x[8, -128:] = 0.0
+    tiny = 2.0 ** (-100 if act == "bf16" else -16)
+    x *= torch.where(torch.arange(M) < 12, tiny, 1.0)[:, None]
+    ref = x @ ((q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0))
+    if act == "bf16":
+        out = torch.ops.mi355q.w4a16_gemm(x.bfloat16().to(dev), pk.to(dev), s.to(dev), pz.to(dev), False, torch.float32, None).cpu()
+    else:
+        out = torch.ops.mi355q.w4a8_gemm(x.to(E5).to(dev), pk.to(dev), s.to(dev), pz.to(dev), False, torch.float32, None, None).cpu()
+    assert (out[3] == 0).all()
+    # fp32 sums: a rounding of 2^-24 of the sum of magnitudes per group and part
+    bound = (x.abs() @ (15 * s.double().repeat_interleave(128, 0))) * ((K // 128 + 16) * 2.0 ** -23)
+    inside = (x.abs() @ (15 * s.double().repeat_interleave(128, 0))) < torch.finfo(torch.float32).max / 2   # every partial sum too
+    assert inside[:12].all()
+    assert torch.isfinite(out[inside]).all() and ((out.double() - ref).abs() <= bound)[inside].all()
+
+
+@pytest.mark.gpu
 def test_same_bits_whoever_adds_the_parts_up(oracle, pkg, dev):
     """The parts share the sum, or the last one adds all of them up (split_k < 0); the counters are zero afterwards; fewer parts where
     the workspace has less room than the plan wants."""
