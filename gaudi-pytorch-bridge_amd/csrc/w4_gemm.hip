@@ -1333,7 +1333,7 @@ extern "C" int mi355q_w4a8_gemm(const void* A, int fmt_a, int64_t lda, const int
   // up to 16 rows the stream kernel
   const W4StreamPlan stream_plan = w4_stream_plan_for(M, N, K, group, a.scale_f32, false, lda, ld_packed, workspace != nullptr && al16(workspace) ? workspace_bytes : 0);
   std::unique_lock<std::mutex> in_order;
-  if (a.partials != nullptr) in_order = std::unique_lock<std::mutex>(w4_launch_order(workspace));
+  if (a.partials != nullptr || stream_plan.parts > 1) in_order = std::unique_lock<std::mutex>(w4_launch_order(workspace));
   if (stream_plan.parts > 0) launch_w4_stream(a, fmt_a, stream_plan, workspace, false, st);
   else if (fmt_a == MI355Q_E4M3FN) w4a8_launch_by_m<MI355Q_E4M3FN>(a, st);
   else w4a8_launch_by_m<MI355Q_E5M2>(a, st);

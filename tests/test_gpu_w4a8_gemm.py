@@ -356,3 +356,36 @@ def test_two_threads_share_a_workspace_of_the_c_entries(oracle, pkg, dev, M):
     torch.cuda.synchronize()
     assert not failed and all(torch.equal(y.cpu(), j[-1]) for j in jobs for y in j[-2])
     assert int(ws[:1024].count_nonzero()) == 0
+
+
+def test_one_launch_call_stays_out_of_another_calls_launches(oracle, pkg, dev):
+    """A product of 16 rows that only the stream kernel walks in parts, beside one of two launches, on one stream with one workspace."""
+    import ctypes
+    import threading
+    lib, calls = pkg.capi(), 1000
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    shapes = [(100, 4096, 512), (16, 1024, 4096)]
+    needs = [lib.mi355q_w4a8_gemm_workspace_bytes(M, N, K, 128, pkg.BF16) for M, K, N in shapes]
+    assert min(needs) > 1024
+    ws = torch.zeros(max(needs), dtype=torch.uint8, device=dev)
+    jobs, failed = [], []
+    for M, K, N in shapes:
+        gen = torch.Generator().manual_seed(M)
+        q, z, s, pk, pz = weights(oracle, gen, K, N, 128, False, True, pow2=True)
+        a = torch.randint(-4, 5, (M, K), generator=gen).float()
+        w = (q - z.repeat_interleave(128, 0)).double() * s.double().repeat_interleave(128, 0)
+        jobs.append((M, K, N, a.to(E4).to(dev), pk.to(dev), s.to(dev), pz.to(dev), [torch.empty(M, N, device=dev) for _ in range(calls)], (a.double() @ w).float().to(dev)))
+
+    def work(M, K, N, a8, pk, s, pz, ys, ref):
+        for y in ys:
+            r = lib.mi355q_w4a8_gemm(a8.data_ptr(), pkg.E4M3FN, K, pk.data_ptr(), N // 8, s.data_ptr(), pkg.BF16, pz.data_ptr(), 0, 128, y.data_ptr(), pkg.F32, N, M, N, K,
+                                     None, 1.0, pkg.GS_NONE, None, ws.data_ptr(), ws.numel(), st)
+            failed.extend([r] if r else [])
+
+    jobs.append((*jobs[1][:7], [torch.empty_like(y) for y in jobs[1][7]], jobs[1][8]))
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    torch.cuda.synchronize()
+    assert not failed and all(torch.equal(y, j[-1]) for j in jobs for y in j[-2])
