@@ -186,6 +186,12 @@ SplitPlan split_plan(bool a_kmajor, int64_t lda, bool b_kmajor, int64_t ldb, int
   return best;
 }
 
+inline int64_t round_up16(int64_t v) { return (v + 15) & ~(int64_t)15; }
+// The ring kernel's form and cut for operands that lie anywhere: those of aligned ones.
+SplitPlan ragged_ring_plan(int trans_b, int64_t lda, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+  return split_plan(true, round_up16(lda), trans_b != 0, round_up16(ldb), M, N, K, batch, may_split, false, true);
+}
+
 // The plan of a product whose operands lie anywhere (launch_gemm_ragged_*), A [M, K].  parts 0: not served, its operands are better copied
 // first.  That is so where the copies end in 256 x 256 tiles, and where the loads' detour costs more than the copies would: it lengthens
 // the stages by 0.3 for rows at whole dwords (DwordProducer) and by 0.8 for others, and a copy is 4.5 us and twice the bytes at 5 TB/s.
@@ -195,9 +201,8 @@ SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_
   SplitPlan none;
   none.parts = 0;
   if (trans_a || M < 1 || N < 16 || K < 256 || batch < 1 || lda > (1LL << 22) || ldb > (1LL << 22)) return none;
-  const auto up = [](int64_t v) { return (v + 15) & ~(int64_t)15; };
-  if (split_plan(true, up(lda), trans_b != 0, up(ldb), M, N, K, batch, may_split).kind == GemmKind::kTile256) return none;
-  const SplitPlan p = split_plan(true, up(lda), trans_b != 0, up(ldb), M, N, K, batch, may_split, false, true);
+  if (split_plan(true, round_up16(lda), trans_b != 0, round_up16(ldb), M, N, K, batch, may_split).kind == GemmKind::kTile256) return none;
+  const SplitPlan p = ragged_ring_plan(trans_b, lda, ldb, M, N, K, batch, may_split);
   const double copied = (double)batch * ((K % 16 != 0 || lda % 16 != 0 ? (double)M * (double)K : 0.0) + ((trans_b ? K : N) % 16 != 0 || ldb % 16 != 0 ? (double)N * (double)K : 0.0));
   return p.stages_us * ((lda | ldb) % 4 == 0 ? 0.3 : 0.8) < 4.5 + 0.4e-6 * copied ? p : none;
 }
@@ -268,6 +273,12 @@ static int gemm_call(const void* A, int fmt_a, int trans_a, int64_t lda, const v
   g.tiles_m = g.tiles_n = 0;
 
   const int64_t kMaxBatch = 65535;
+  // Whether the call is served is settled here, on what the query was asked, and not by a piece of the batch or by the workspace.
+  SplitPlan ragged;
+  if (unaligned) {
+    ragged = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= kMaxBatch);
+    if (ragged.parts == 0) return MI355Q_ERR_UNSUPPORTED;
+  }
   for (int64_t b0 = 0; b0 < batch; b0 += kMaxBatch) {
     const int64_t nb = (batch - b0) < kMaxBatch ? (batch - b0) : kMaxBatch;
     GemmArgs gb = g;
@@ -288,8 +299,8 @@ static int gemm_call(const void* A, int fmt_a, int trans_a, int64_t lda, const v
     }
     gb.fast_epi = epilogue_fast_ok(gb, nb);
     if (unaligned) {
-      const SplitPlan plan = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, nb, workspace != nullptr && nb == batch);
-      if (plan.parts == 0) return MI355Q_ERR_UNSUPPORTED;
+      const bool as_asked = nb == batch && (workspace != nullptr || ragged.parts == 1);
+      const SplitPlan plan = as_asked ? ragged : ragged_ring_plan(trans_b, lda, ldb, M, N, K, nb, false);
       SplitArgs split{plan.parts, nullptr, nullptr, plan.kind};
       if (plan.parts > 1) {
         if (!al16(workspace) || workspace_bytes < plan.workspace_bytes()) return MI355Q_ERR_WORKSPACE;

@@ -67,6 +67,25 @@ def test_batches_and_bf16(pkg, dev, trans_b):
     call(pkg, dev, 2, 200, 516, 260, trans_b, 520, (516 if trans_b else 260) + 4, 8)
 
 
+@pytest.mark.parametrize("batch,room", [(65536, True), (65600, True), (65600, False), (1, False)])
+def test_a_product_that_the_query_accepts_is_served(pkg, dev, batch, room):
+    """More matrices than a launch takes, whose last piece alone would not be worth it, and calls without a workspace."""
+    lib = pkg.capi()
+    gen = torch.Generator().manual_seed(batch)
+    M, N, K = 1, 64, 2801
+    a, b, ((araw, _), (braw, _)) = operands(gen, 1, M, K, N, True, K, K, 0, dev)
+    size = ctypes.c_size_t()
+    assert lib.mi355q_fp8_gemm_unaligned_workspace_bytes(0, K, 1, K, M, N, K, batch, ctypes.byref(size)) == 0
+    ws = torch.zeros(max(size.value, 16), dtype=torch.uint8, device=dev)
+    c = torch.full((batch, M, N), -7.0, device=dev)
+    st = lib.mi355q_fp8_gemm_unaligned_ws(
+        araw.data_ptr(), pkg.E4M3FN, 0, K, braw.data_ptr(), pkg.E5M2, 1, K, c.data_ptr(), pkg.F32, N, M, N, K, None, 1.0, pkg.GS_NONE, None, 1.0, pkg.GS_NONE,
+        None, 0, 0, None, 0, batch, 0, 0, M * N, 0, 0, ws.data_ptr() if room else None, size.value if room else 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert st == 0
+    assert torch.equal(c, (a @ b).to(dev).expand(batch, M, N))
+
+
 def test_what_is_copied_and_what_is_not(pkg, dev):
     """Both sides of the rule, by the buffers that a call allocates: the result alone, or two copies as well."""
     for M, K, N, copied in [(1, 3001, 8000, 0), (300, 2049, 1003, 0), (64, 4100, 9999, 0), (1000, 3000, 5000, 0), (1000, 3001, 5001, 2), (2600, 2999, 6001, 2), (300, 255, 1003, 2)]:
