@@ -201,6 +201,8 @@ SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_
   SplitPlan none;
   none.parts = 0;
   if (trans_a || M < 1 || N < 16 || K < 256 || batch < 1 || lda > (1LL << 22) || ldb > (1LL << 22)) return none;
+  // A chunk at the end of a row of B [K, N] is read into the next row, up to 15 bytes, so that one has to lie as far on.
+  if (lda < 0 || ldb < (trans_b ? 0 : 16)) return none;
   if (split_plan(true, round_up16(lda), trans_b != 0, round_up16(ldb), M, N, K, batch, may_split).kind == GemmKind::kTile256) return none;
   const SplitPlan p = ragged_ring_plan(trans_b, lda, ldb, M, N, K, batch, may_split);
   const double copied = (double)batch * ((K % 16 != 0 || lda % 16 != 0 ? (double)M * (double)K : 0.0) + ((trans_b ? K : N) % 16 != 0 || ldb % 16 != 0 ? (double)N * (double)K : 0.0));

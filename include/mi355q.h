@@ -294,7 +294,7 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
                     void* workspace, size_t workspace_bytes, void* stream);
 /*
  * The same product for operands that lie anywhere: base addresses, pitches and batch strides of A and B need no alignment and K may
- * be any length.  Served are A [M, K], K >= 256, N >= 16, pitches up to 4 Mi elements, and sizes that do not fill the chip with
+ * be any length.  Served are A [M, K], K >= 256, N >= 16, pitches up to 4 Mi elements and of B [K, N] from 16 on, and sizes that do not fill the chip with
  * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows), nor others where such copies cost less; both calls
  * return MI355Q_ERR_UNSUPPORTED otherwise.  The workspace is that of mi355q_fp8_gemm_ws; its size goes to *bytes.
  */

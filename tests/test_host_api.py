@@ -415,3 +415,17 @@ def test_w4a8_gemm_rejects_a_zero_point_or_bias_on_another_device(pkg):
         torch.ops.mi355q.w4a8_gemm(A, packed, scale, torch.zeros(2, 32, dtype=torch.int32), False, torch.bfloat16, None, None)
     with pytest.raises(RuntimeError, match="bias must be on the same device as A"):
         torch.ops.mi355q.w4a8_gemm(A, packed, scale, None, False, torch.bfloat16, None, torch.zeros(256, dtype=torch.bfloat16))
+
+
+def test_unaligned_products_whose_loads_would_leave_the_operand_are_refused(pkg):
+    """Chunks at the end of a row of B [K, N] reach into the next row, which has to be there; rows run forwards."""
+    import ctypes
+    size = ctypes.c_size_t()
+
+    def ask(trans_b, lda, ldb):
+        return pkg.capi().mi355q_fp8_gemm_unaligned_workspace_bytes(0, lda, trans_b, ldb, 1, 500, 3001, 1, ctypes.byref(size))
+
+    for trans_b, lda, ldb in ((0, 3001, 0), (0, 3001, 15), (0, -3001, 500), (1, -3001, 3001), (1, 3001, -3001)):
+        assert ask(trans_b, lda, ldb) == 2, (trans_b, lda, ldb)
+    for trans_b, lda, ldb in ((0, 3001, 16), (0, 3001, 500), (0, 0, 500), (1, 3001, 3001), (1, 1, 7)):
+        assert ask(trans_b, lda, ldb) == 0, (trans_b, lda, ldb)
