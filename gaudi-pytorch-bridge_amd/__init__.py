@@ -71,6 +71,7 @@ def capi():
     L.mi355q_fp8_gemm_ws.argtypes = L.mi355q_fp8_gemm.argtypes[:-1] + [vp, c.c_size_t, vp]
     L.mi355q_fp8_gemm_unaligned_ws.argtypes = L.mi355q_fp8_gemm_ws.argtypes
     L.mi355q_fp8_gemm_unaligned_workspace_bytes.argtypes = [i32, i64, i32, i64, i64, i64, i64, i64, c.POINTER(c.c_size_t)]
+    L.mi355q_fp8_gemm_unaligned_query.argtypes = [vp, i32, i64, i64, vp, i32, i64, i64, i64, i64, i64, i64, c.POINTER(c.c_size_t)]
     L.mi355q_fp8_gemm_workspace_bytes.argtypes = [i32, i64, i32, i64, i64, i64, i64, i64]
     L.mi355q_fp8_gemm_workspace_bytes.restype = c.c_size_t
     L.mi355q_pad_rows.argtypes = [vp, i32, vp]
@@ -97,7 +98,7 @@ def capi():
     L.mi355q_fp8_gemm_ws_variant.argtypes = [i32, i64, i32, i64, i64, i64, i64, i64]
     L.mi355q_fp8_gemm_ws_variant.restype = c.c_char_p
     for name in ("mi355q_amax", "mi355q_rowwise_amax", "mi355q_quantize_rows", "mi355q_silu_mul_quantize_rows", "mi355q_cast_to_fp8", "mi355q_cast_to_fp8_running_amax", "mi355q_cast_to_fp8_amax_chain", "mi355q_cast_to_fp8_sr", "mi355q_cast_to_fp8_hybrid", "mi355q_cast_from_fp8",
-                 "mi355q_dequant_4bit", "mi355q_fp8_gemm", "mi355q_fp8_gemm_ws", "mi355q_fp8_gemm_unaligned_ws", "mi355q_fp8_gemm_unaligned_workspace_bytes", "mi355q_pad_rows", "mi355q_w4a8_gemm", "mi355q_w4a16_gemm", "mi355q_split_rows_fp8x2", "mi355q_sum_fp8", "mi355q_sum_fp8_static", "mi355q_softmax_fp8", "mi355q_fp8_sdpa_fwd"):
+                 "mi355q_dequant_4bit", "mi355q_fp8_gemm", "mi355q_fp8_gemm_ws", "mi355q_fp8_gemm_unaligned_ws", "mi355q_fp8_gemm_unaligned_workspace_bytes", "mi355q_fp8_gemm_unaligned_query", "mi355q_pad_rows", "mi355q_w4a8_gemm", "mi355q_w4a16_gemm", "mi355q_split_rows_fp8x2", "mi355q_sum_fp8", "mi355q_sum_fp8_static", "mi355q_softmax_fp8", "mi355q_fp8_sdpa_fwd"):
         getattr(L, name).restype = i32
     L._typed = True
     return L
@@ -134,7 +135,7 @@ SDPA_MASK_NONE, SDPA_MASK_BOOL, SDPA_MASK_BF16, SDPA_MASK_F32 = 0, 1, 2, 3
 
 EXPORTED_SYMBOLS = (
     "mi355q_abi_version", "mi355q_status_string", "mi355q_amax", "mi355q_rowwise_amax",
-    "mi355q_quantize_rows", "mi355q_silu_mul_quantize_rows", "mi355q_cast_to_fp8", "mi355q_cast_to_fp8_running_amax", "mi355q_cast_to_fp8_amax_chain", "mi355q_cast_to_fp8_sr", "mi355q_cast_to_fp8_hybrid", "mi355q_cast_from_fp8", "mi355q_dequant_4bit", "mi355q_fp8_gemm", "mi355q_fp8_gemm_ws", "mi355q_fp8_gemm_unaligned_ws", "mi355q_fp8_gemm_unaligned_workspace_bytes", "mi355q_fp8_gemm_workspace_bytes", "mi355q_pad_rows",
+    "mi355q_quantize_rows", "mi355q_silu_mul_quantize_rows", "mi355q_cast_to_fp8", "mi355q_cast_to_fp8_running_amax", "mi355q_cast_to_fp8_amax_chain", "mi355q_cast_to_fp8_sr", "mi355q_cast_to_fp8_hybrid", "mi355q_cast_from_fp8", "mi355q_dequant_4bit", "mi355q_fp8_gemm", "mi355q_fp8_gemm_ws", "mi355q_fp8_gemm_unaligned_ws", "mi355q_fp8_gemm_unaligned_workspace_bytes", "mi355q_fp8_gemm_unaligned_query", "mi355q_fp8_gemm_workspace_bytes", "mi355q_pad_rows",
     "mi355q_w4a8_gemm", "mi355q_w4a8_gemm_workspace_bytes", "mi355q_w4a16_gemm", "mi355q_w4a16_gemm_workspace_bytes", "mi355q_split_rows_fp8x2", "mi355q_fp8_gemm_variant", "mi355q_fp8_gemm_ws_variant", "mi355q_sum_fp8_workspace_bytes", "mi355q_sum_fp8", "mi355q_sum_fp8_static", "mi355q_softmax_fp8", "mi355q_fp8_sdpa_fwd", "mi355q_fp8_sdpa_workspace_bytes", "mi355q_fp8_sdpa_key_splits",
 )
 

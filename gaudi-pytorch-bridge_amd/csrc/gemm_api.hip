@@ -192,12 +192,23 @@ SplitPlan ragged_ring_plan(int trans_b, int64_t lda, int64_t ldb, int64_t M, int
   return split_plan(true, round_up16(lda), trans_b != 0, round_up16(ldb), M, N, K, batch, may_split, false, true);
 }
 
+// Where the operands of a product of several matrices lie, for what depends on more than the pitches.
+struct RaggedPlaces {
+  const void *a, *b;
+  int64_t stride_a, stride_b;
+};
+
 // The plan of a product whose operands lie anywhere (launch_gemm_ragged_*), A [M, K].  parts 0: not served, its operands are better copied
 // first.  That is so where the copies end in 256 x 256 tiles, and where the loads' detour costs more than the copies would: it lengthens
-// the stages by 0.3 for rows at whole dwords (DwordProducer) and by 0.8 for others, and a copy is 4.5 us and twice the bytes at 5 TB/s.
-// us with the copies / without: 1000 x 3000 x 5000 31.4 / 25.1, 16 x 8191 x 28671 122 / 65, 64 x 4100 x 9999 38.1 / 23.9, 1 x 8191 x 20000 B [N, K]
-// 87.7 / 51.6, 300 x 2049 x 1003 16.7 / 13.1, 256 x 8190 x 8190 53.0 / 44.6, but 1000 x 3001 x 5001 35.3 / 36.6, 3779 x 13824 x 1411 82.7 / 96.0.
-SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split) {
+// the stages by 0.3 for rows at whole dwords (DwordProducer), by 0.5 where only those of B are not and by 0.8 for others, and a copy is
+// 4.6 us and twice the bytes at 5 TB/s.  Copied is what fp8_gemm_v2 would copy: an operand off the grid of 16 bytes, and both where K is
+// off it, for they are filled up along K.  us a call with the copies / without: 1000 x 3000 x 5000 31.4 / 25.1, 16 x 8191 x 28671 122 / 65, 16 x
+// 8191 x 28672 121 / 48, 64 x 4100 x 9999 38.1 / 23.9, 1 x 8191 x 20000 B [N, K] 87.7 / 51.6, 300 x 2049 x 1008 16.1 / 11.2, 1000 x 3008 x 5001 39.9 / 34.3,
+// 256 x 8190 x 8192 51.8 / 41.5, but 1000 x 3001 x 5001 35.3 / 36.6, 3779 x 13824 x 1411 82.7 / 96.0; with A an odd byte from the grid 1000 x 3008 x 5008
+// 29.5 / 34.0, 256 x 8192 x 8192 36.7 / 42.1, 300 x 2048 x 1024 11.5 / 10.2.  Of 150 such products the rule's way was never more than 5 % the slower.
+// `at` nullptr: addresses and batch strides as aligned as the pitches, one matrix after the other; either: one of both will do.
+SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split,
+                      const RaggedPlaces* at = nullptr, bool either = false) {
   SplitPlan none;
   none.parts = 0;
   if (trans_a || M < 1 || N < 16 || K < 256 || batch < 1 || lda > (1LL << 22) || ldb > (1LL << 22)) return none;
@@ -205,8 +216,15 @@ SplitPlan ragged_plan(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_
   if (lda < 0 || ldb < (trans_b ? 0 : 16)) return none;
   if (split_plan(true, round_up16(lda), trans_b != 0, round_up16(ldb), M, N, K, batch, may_split).kind == GemmKind::kTile256) return none;
   const SplitPlan p = ragged_ring_plan(trans_b, lda, ldb, M, N, K, batch, may_split);
-  const double copied = (double)batch * ((K % 16 != 0 || lda % 16 != 0 ? (double)M * (double)K : 0.0) + ((trans_b ? K : N) % 16 != 0 || ldb % 16 != 0 ? (double)N * (double)K : 0.0));
-  return p.stages_us * ((lda | ldb) % 4 == 0 ? 0.3 : 0.8) < 4.5 + 0.4e-6 * copied ? p : none;
+  const auto pays = [&](const RaggedPlaces& w) {
+    const uint64_t a = reinterpret_cast<uint64_t>(w.a) | (uint64_t)(lda | (batch > 1 ? w.stride_a : 0));
+    const uint64_t b = reinterpret_cast<uint64_t>(w.b) | (uint64_t)(ldb | (batch > 1 ? w.stride_b : 0));
+    const double copied = (K % 16 != 0 || a % 16 != 0 ? (double)M * (double)K * (double)(w.stride_a == 0 ? 1 : batch) : 0.0) +
+                          (K % 16 != 0 || b % 16 != 0 ? (double)N * (double)K * (double)(w.stride_b == 0 ? 1 : batch) : 0.0);
+    return p.stages_us * (a % 4 != 0 ? 0.8 : (b % 4 != 0 ? 0.5 : 0.3)) < 4.6 + 0.4e-6 * copied;
+  };
+  const RaggedPlaces one_after_the_other{nullptr, nullptr, M * lda, (trans_b ? N : K) * ldb};
+  return (at != nullptr && pays(*at)) || ((at == nullptr || either) && pays(one_after_the_other)) ? p : none;
 }
 
 // What launch_by_kind and launch_gemm_stream run; may_split: the caller brings the workspace.  A name gives the kernel and its
@@ -275,11 +293,13 @@ static int gemm_call(const void* A, int fmt_a, int trans_a, int64_t lda, const v
   g.tiles_m = g.tiles_n = 0;
 
   const int64_t kMaxBatch = 65535;
-  // Whether the call is served is settled here, on what the query was asked, and not by a piece of the batch or by the workspace.
+  // Whether the call is served is settled here, on what either query was asked, and not by a piece of the batch or by the workspace.
   SplitPlan ragged;
   if (unaligned) {
-    ragged = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= kMaxBatch);
+    const RaggedPlaces at{A, B, stride_a, stride_b};
+    ragged = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= kMaxBatch, &at, true);
     if (ragged.parts == 0) return MI355Q_ERR_UNSUPPORTED;
+    if (batch == 1) g.stride_a = g.stride_b = 0;  // (the kernel asks whether they are whole dwords)
   }
   for (int64_t b0 = 0; b0 < batch; b0 += kMaxBatch) {
     const int64_t nb = (batch - b0) < kMaxBatch ? (batch - b0) : kMaxBatch;
@@ -378,6 +398,15 @@ int mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int tran
                                               int64_t batch, size_t* bytes) {
   if (bytes == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
   const SplitPlan p = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535);
+  *bytes = p.parts == 0 ? 0 : p.workspace_bytes();
+  return p.parts == 0 ? MI355Q_ERR_UNSUPPORTED : MI355Q_OK;
+}
+
+int mi355q_fp8_gemm_unaligned_query(const void* A, int trans_a, int64_t lda, int64_t stride_a, const void* B, int trans_b, int64_t ldb,
+                                    int64_t stride_b, int64_t M, int64_t N, int64_t K, int64_t batch, size_t* bytes) {
+  if (bytes == nullptr) return MI355Q_ERR_INVALID_ARGUMENT;
+  const RaggedPlaces at{A, B, stride_a, stride_b};
+  const SplitPlan p = ragged_plan(trans_a, lda, trans_b, ldb, M, N, K, batch, batch <= 65535, &at);
   *bytes = p.parts == 0 ? 0 : p.workspace_bytes();
   return p.parts == 0 ? MI355Q_ERR_UNSUPPORTED : MI355Q_OK;
 }

@@ -607,12 +607,14 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
   const bool k_ragged = K % 16 != 0 && !(ta && !tb);
   const double outputs = (double)M * (double)N;
   const bool ragged = ac % 16 || bc % 16 || k_ragged || misaligned(ac_t) || misaligned(bc_t);
-  // A [M, K] times one matrix B is one product over all rows of A (see below)
-  const bool flat = batch > 1 && stride_b == 0 && stride_a != 0 && !ta;
+  // A [..., M, K] times one matrix B is one product over all batch * M rows: B is streamed once
+  // and the rows fill the kernels' tiles, where batch separate problems would each re-read B with
+  // M rows only (a [64, 1, K] decode activation against [K, N] weights would be 64 one-row products).
+  const bool can_flatten = batch > 1 && stride_b == 0 && stride_a != 0 && !ta;
   // From K = 256 on the ring kernel takes such operands as they lie (A [M, K]), where copies would not end in 256 x 256 tiles.
   size_t unaligned_ws = 0;
-  const bool unaligned = ragged && mi355q_fp8_gemm_unaligned_workspace_bytes(ta ? 1 : 0, ac, tb ? 1 : 0, bc, flat ? batch * M : M, N, K,
-                                                                             flat ? 1 : batch, &unaligned_ws) == MI355Q_OK;
+  const bool unaligned = ragged && mi355q_fp8_gemm_unaligned_query(ac_t.data_ptr(), ta ? 1 : 0, ac, stride_a, bc_t.data_ptr(), tb ? 1 : 0, bc, stride_b,
+                                                                   can_flatten ? batch * M : M, N, K, can_flatten ? 1 : batch, &unaligned_ws) == MI355Q_OK;
   if (ragged && !unaligned &&
       (K >= 128 || outputs * (double)K >= (double)(1 << 26) || (tb && K >= 64 && outputs >= (double)(1 << 17)))) {
     const int64_t kp = (ta && !tb) ? K : (K + 15) / 16 * 16;  // K is contiguous in neither operand: any K
@@ -638,10 +640,6 @@ Tensor fp8_gemm_v2_impl(const Tensor& A, bool trans_A, const Tensor& B, bool tra
     k_call = kp;
   }
 
-  // A [..., M, K] times one matrix B is one product over all batch * M rows: B is streamed once
-  // and the rows fill the kernels' tiles, where batch separate problems would each re-read B with
-  // M rows only (a [64, 1, K] decode activation against [K, N] weights would be 64 one-row products).
-  const bool can_flatten = batch > 1 && stride_b == 0 && stride_a != 0 && !ta;
   // Per-row scales that cover the batch as well ([..., M, 1], what quantize_rows returns for a
   // batched activation) are per-row scales of the flattened product.
   auto batched_rows = [&](const IValue& sc) {

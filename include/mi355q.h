@@ -295,9 +295,14 @@ int mi355q_fp8_gemm_ws(const void* A, int fmt_a, int trans_a, int64_t lda,
 /*
  * The same product for operands that lie anywhere: base addresses, pitches and batch strides of A and B need no alignment and K may
  * be any length.  Served are A [M, K], K >= 256, N >= 16, pitches up to 4 Mi elements and of B [K, N] from 16 on, and sizes that do not fill the chip with
- * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows), nor others where such copies cost less; both calls
+ * 256 x 256 tiles (those gain more from operands copied with mi355q_pad_rows), nor others where such copies cost less; all three
  * return MI355Q_ERR_UNSUPPORTED otherwise.  The workspace is that of mi355q_fp8_gemm_ws; its size goes to *bytes.
+ * mi355q_fp8_gemm_unaligned_query looks at the addresses and batch strides, which count for both sides: rows off whole dwords are the
+ * slower ones to load, and what lies on whole 16 bytes need not be copied.  mi355q_fp8_gemm_unaligned_workspace_bytes takes them
+ * to be as aligned as the pitches, each matrix after the one before.  A product that either of them accepts is served.
  */
+int mi355q_fp8_gemm_unaligned_query(const void* A, int trans_a, int64_t lda, int64_t stride_a, const void* B, int trans_b, int64_t ldb,
+                                    int64_t stride_b, int64_t M, int64_t N, int64_t K, int64_t batch, size_t* bytes);
 int mi355q_fp8_gemm_unaligned_workspace_bytes(int trans_a, int64_t lda, int trans_b, int64_t ldb, int64_t M, int64_t N, int64_t K,
                                               int64_t batch, size_t* bytes);
 int mi355q_fp8_gemm_unaligned_ws(const void* A, int fmt_a, int trans_a, int64_t lda,

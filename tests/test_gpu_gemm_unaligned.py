@@ -86,6 +86,31 @@ def test_a_product_that_the_query_accepts_is_served(pkg, dev, batch, room):
     assert torch.equal(c, (a @ b).to(dev).expand(batch, M, N))
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("offset", [1, 8, 15])
+@pytest.mark.parametrize("M,K,N", [(1, 1024, 64), (33, 512, 160), (200, 400, 272), (256, 2304, 512)])
+def test_whole_pitches_off_the_grid(pkg, dev, M, K, N, trans_b, offset):
+    """Extents of whole chunks, and only the addresses are not."""
+    call(pkg, dev, 1, M, K, N, trans_b, K, K if trans_b else N, offset)
+    call(pkg, dev, 3, M, K, N, trans_b, K + 16, (K if trans_b else N) + 32, offset)
+
+
+@pytest.mark.parametrize("M,K,N,off_a,off_b,copied", [
+    (16, 8191, 4096, 0, 0, 0), (300, 2049, 1008, 0, 0, 0),                              # only K is ragged: B is filled up along it too
+    (1000, 3001, 5008, 0, 0, 2), (1000, 3008, 5008, 4, 4, 0), (1000, 3008, 5001, 0, 0, 0),
+    (1000, 3008, 5008, 1, 0, 1), (300, 2048, 1024, 1, 0, 0), (1000, 3008, 5008, 0, 1, 0), (1000, 3000, 5000, 1, 0, 2),
+])
+def test_what_is_copied_looks_at_addresses_and_at_what_a_copy_holds(dev, M, K, N, off_a, off_b, copied):
+    a8 = torch.zeros(M * K + 64, dtype=torch.uint8, device=dev)[off_a:off_a + M * K].view(M, K).view(E4)
+    b8 = torch.zeros(K * N + 64, dtype=torch.uint8, device=dev)[off_b:off_b + K * N].view(K, N).view(E4)
+    run = lambda: torch.ops.hpu.fp8_gemm_v2(a8, False, b8, False, None, torch.bfloat16, None, None, None, False)  # noqa: E731
+    run()
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    c = run()
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 1 + copied
+    assert not c.any()
+
+
 def test_what_is_copied_and_what_is_not(pkg, dev):
     """Both sides of the rule, by the buffers that a call allocates: the result alone, or two copies as well."""
     for M, K, N, copied in [(1, 3001, 8000, 0), (300, 2049, 1003, 0), (64, 4100, 9999, 0), (1000, 3000, 5000, 0), (1000, 3001, 5001, 2), (2600, 2999, 6001, 2), (300, 255, 1003, 2)]:

@@ -429,3 +429,26 @@ def test_unaligned_products_whose_loads_would_leave_the_operand_are_refused(pkg)
         assert ask(trans_b, lda, ldb) == 2, (trans_b, lda, ldb)
     for trans_b, lda, ldb in ((0, 3001, 16), (0, 3001, 500), (0, 0, 500), (1, 3001, 3001), (1, 1, 7)):
         assert ask(trans_b, lda, ldb) == 0, (trans_b, lda, ldb)
+
+
+def test_the_query_with_addresses_and_the_one_without(pkg):
+    """Where addresses and strides are as aligned as the pitches both answer alike; odd addresses make loads slower and copies necessary."""
+    import ctypes
+    lib, size, size_at = pkg.capi(), ctypes.c_size_t(), ctypes.c_size_t()
+
+    def ask(M, K, N, trans_b, off_a, off_b, batch=1, stride_a=None, stride_b=None):
+        ldb = K if trans_b else N
+        return lib.mi355q_fp8_gemm_unaligned_query(4096 + off_a, 0, K, M * K if stride_a is None else stride_a, 4096 + off_b, trans_b, ldb,
+                                                   N * K if stride_b is None else stride_b, M, N, K, batch, ctypes.byref(size_at))
+
+    for M, K, N, batch in ((16, 8191, 28672, 1), (1000, 3000, 5000, 1), (1000, 3001, 5001, 1), (3, 515, 77, 40), (300, 2048, 1024, 1), (129, 1001, 516, 65600)):
+        for trans_b in (0, 1):
+            st = lib.mi355q_fp8_gemm_unaligned_workspace_bytes(0, K, trans_b, K if trans_b else N, M, N, K, batch, ctypes.byref(size))
+            assert (ask(M, K, N, trans_b, 0, 0, batch), size_at.value) == (st, size.value)
+    assert [ask(1000, 3008, 5008, 0, *off) for off in ((4, 4), (1, 0), (0, 1))] == [0, 2, 0]
+    assert [ask(1000, 3000, 5000, 0, *off) for off in ((0, 0), (1, 0), (0, 2))] == [0, 2, 0]
+    # a matrix that a batch shares is copied once: with a stride of its own there is more to save
+    assert ask(600, 4001, 512, 0, 0, 0, 8) == 0 and ask(600, 4001, 512, 0, 0, 0, 8, 0, 0) == 2
+    # strides off the dwords count as addresses do, but not those of a single matrix
+    assert ask(600, 2000, 1000, 0, 0, 0, 1, 1, 1) == ask(600, 2000, 1000, 0, 0, 0)
+    assert lib.mi355q_fp8_gemm_unaligned_query(0, 0, 3001, 0, 0, 0, 500, 0, 1, 500, 3001, 1, None) == 1
