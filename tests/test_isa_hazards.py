@@ -80,8 +80,9 @@ def test_scanner_flags_m0_used_at_once():
 
 @pytest.mark.timeout(900)
 def test_gemm_kernels_have_no_uncovered_hazard():
-    sources = ["gemm_inst_kk.hip", "gemm_inst_km.hip", "gemm_inst_mk.hip", "gemm_inst_mm.hip", "w4_gemm.hip", "sdpa_kernels.hip"]
-    with ThreadPoolExecutor(max_workers=6) as ex:
+    sources = ["gemm_inst_kk.hip", "gemm_inst_km.hip", "gemm_inst_mk.hip", "gemm_inst_mm.hip", "gemm_ragged_kk.hip", "gemm_ragged_km.hip", "w4_gemm.hip",
+               "sdpa_kernels.hip"]
+    with ThreadPoolExecutor(max_workers=8) as ex:
         texts = list(ex.map(isa_check.compile_to_isa, sources))
     sharing = 0
     for src, text in zip(sources, texts):
