@@ -39,7 +39,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kSdpaThreads = 256;
 constexpr int kSdpaBM = 128;  // query rows per workgroup
 constexpr int kSdpaBN = 64;   // keys per block
-constexpr int kSdpaResident = 1024;  // workgroups that are resident at once, four on each of 256 CUs
 constexpr float kLog2e = 1.44269504088896341f;
 
 enum { kMaskNone = MI355Q_SDPA_MASK_NONE, kMaskBool = MI355Q_SDPA_MASK_BOOL, kMaskBf16 = MI355Q_SDPA_MASK_BF16, kMaskF32 = MI355Q_SDPA_MASK_F32 };
@@ -57,6 +56,7 @@ struct SdpaArgs {
   int mask_kind, causal, out_fp8;
   // the order of the workgroups (sdpa_place): heads of a group, 0 = contiguous ranges; heads per XCD (all of them where xcd_shift is 0)
   int head_group, heads, xcd_shift;
+  int mixed;  // launches of at most so many workgroups give each CU long and short ones
   int vec_q, vec_k, vec_v, vec_o;  // 16-byte (q, k, v) / 4-element (out; 2: 8-element) accesses are possible
   int dma;                         // k and v go global -> LDS directly
   int nqb;                         // query blocks per (batch, head)
@@ -122,13 +122,15 @@ __device__ __forceinline__ int64_t sdpa_batch_index(const SdpaArgs& a, int d, ui
 // Under one the last query block takes nqb times as long as the first, and what counts is that the long ones start first, over all
 // heads of the XCD and not head by head: with the last head's longest workgroups started last the CUs stood idle for a fifth of the
 // prefill (32 / 8 heads of 128, 8192 tokens, 360 -> 320 us; 8 x 1024 tokens 78 -> 60).  So the heads go in groups, block by block
-// down from the last: a group is what the caches hold of K and V (sdpa_order).  If every workgroup is resident from the start, the
-// order decides which ones share a CU, and every second round over the 32 CUs of an XCD runs backwards, so that each CU gets long and short
-// ones (16 / 4 heads, 8192 tokens, 180 -> 169 us; where workgroups wait for their turn it costs 1.5 %).
+// down from the last: a group is what the caches hold of K and V (sdpa_order).  In a launch of few workgroups the order decides
+// which ones share a CU, and every second round over the 32 CUs of an XCD runs backwards, so that each CU gets long and short
+// ones: up to four per CU (16 / 4 heads of 128, 8192 tokens, 180 -> 169 us; of 256, two at a time, 304 -> 295, 9 heads 207 -> 203, 30 heads x
+// 4096 160 -> 153; of 72, through registers, no difference), and up to the five that are resident at head dimension 64 (20 / 5 heads, 8192
+// tokens, 157 -> 144, 32 / 8 x 4608 86 -> 79).  In longer launches it costs 1.5 %.
 __device__ __forceinline__ void sdpa_place(const SdpaArgs& a, int id, int total, uint32_t& bi, int& qb) {
   if (a.head_group > 0) {
     const int k = id >> 3;
-    if (total <= kSdpaResident && (k & 32) != 0 && (k | 31) < (total >> 3)) id ^= 31 << 3;
+    if (total <= a.mixed && (k & 32) != 0 && (k | 31) < (total >> 3)) id ^= 31 << 3;
     const uint32_t xcd = (uint32_t)id & ((1u << a.xcd_shift) - 1), i = (uint32_t)id >> a.xcd_shift;
     const uint32_t per = (uint32_t)a.head_group * (uint32_t)a.nqb, g = i / per, j = i - g * per, first = g * (uint32_t)a.head_group;
     const uint32_t left = (uint32_t)a.heads - first, n = left < (uint32_t)a.head_group ? left : (uint32_t)a.head_group, r = j / n;
@@ -537,7 +539,6 @@ constexpr bool sdpa_q_in_lds(int dkc, int dvt, bool dma) { return dma && dkc == 
 // 285 -> 277.  64, us: 32 / 8 heads, 8192 tokens, 243 -> 228 (four at a time 232), 8 x 1024 44 -> 41, 64 heads x 16 x 512 60 -> 53, 32 x 32 / 8 x 333
 // 39 -> 33, the same without causality 42 -> 37.  With fewer workgroups the further places stay empty and the barrier costs, at 128: 4 heads, 8192
 // tokens, 122 -> 129; 32 heads, 2048 tokens, 39 -> 41; 20 heads, 4096 tokens, 72 -> 74.
-constexpr int kSdpaMany = 3 * 256;
 constexpr int sdpa_many_per_cu(int dkc, int dvt) { return dkc == 2 && dvt == 4 ? 4 : dkc == 1 && dvt == 2 ? 5 : 0; }  // 0: there is no such form
 constexpr int sdpa_workgroups_per_cu(int dkc, int dvt, bool dma, bool masked) { return sdpa_q_in_lds(dkc, dvt, dma) && !masked ? 3 : (dvt <= 4 || (dma && !masked)) ? 2 : 1; }
 
@@ -1257,13 +1258,23 @@ static SdpaDecodePlan sdpa_decode_plan(const mi355q_sdpa_desc* d, int cus) {
   return p;
 }
 
+static int compute_units_sdpa() {
+  static const int n = [] {
+    int dev = 0, cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
+      cu = 256;
+    return cu;
+  }();
+  return n;
+}
+
 // The order of a launch's workgroups (see sdpa_place).  With one workgroup per CU or fewer it is of no account.
 // A number of heads that 8 divides leaves each head on one XCD, GQA's heads of a K and V together, in groups of equal size whose K
 // and V are at most 8 MiB, twice an XCD's L2 (4096 tokens of 32 heads per XCD, each with its own K and V: 8 heads 679 us, 4 689, 16 697,
 // all 745; 2048 tokens, 16 heads per XCD: 16 heads 96, 8 110).  Any other number goes through all heads at once, over all XCDs:
 // 9 heads, 8192 tokens, 190 -> 136 us; 30 heads, 357 -> 308, whose K and V are 60 MiB.
 static void sdpa_order(SdpaArgs& a, const mi355q_sdpa_desc* d, int64_t batches, bool causal) {
-  if (!causal || a.nqb * batches <= 256) return;
+  if (!causal || a.nqb * batches <= compute_units_sdpa()) return;
   a.xcd_shift = batches % 8 == 0 ? 3 : 0;
   a.heads = (int)(batches >> a.xcd_shift);
   a.head_group = a.heads;
@@ -1275,17 +1286,22 @@ static void sdpa_order(SdpaArgs& a, const mi355q_sdpa_desc* d, int64_t batches, 
   a.head_group = (int)((a.heads + groups - 1) / groups);
 }
 
+template <int DKC, int DVT, int FMT, bool DMA, int MASK, bool MANY>
+static void sdpa_launch_form(SdpaArgs a, int64_t blocks, hipStream_t st) {
+  // (sdpa_place deals with 32 CUs per XCD)
+  a.mixed = compute_units_sdpa() != 256 ? 0 : 256 * (MANY && sdpa_many_per_cu(DKC, DVT) > 4 ? sdpa_many_per_cu(DKC, DVT) : 4);
+  hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, DMA, MASK, MANY>), dim3((unsigned)blocks), dim3(kSdpaThreads), 0, st, a);
+}
 template <int DKC, int DVT, int FMT, int MASK>
 static void sdpa_launch_kernel(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
-  const dim3 grid((unsigned)blocks), block(kSdpaThreads);
   if constexpr (MASK != kWithMask && sdpa_many_per_cu(DKC, DVT) > 0) {
-    if (a.dma && a.mask_kind == kMaskNone && blocks > kSdpaMany) {
-      hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, kWithoutMask, true>), grid, block, 0, st, a);
+    if (a.dma && a.mask_kind == kMaskNone && blocks > 3 * compute_units_sdpa()) {
+      sdpa_launch_form<DKC, DVT, FMT, true, kWithoutMask, true>(a, blocks, st);
       return;
     }
   }
-  if (a.dma) hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, true, MASK, false>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((fp8_sdpa_fwd_kernel<DKC, DVT, FMT, false, MASK, false>), grid, block, 0, st, a);
+  if (a.dma) sdpa_launch_form<DKC, DVT, FMT, true, MASK, false>(a, blocks, st);
+  else sdpa_launch_form<DKC, DVT, FMT, false, MASK, false>(a, blocks, st);
 }
 template <int DKC, int DVT, int FMT>
 static void sdpa_launch_fmt(const SdpaArgs& a, int64_t blocks, hipStream_t st) {
@@ -1301,16 +1317,6 @@ static int sdpa_launch(const SdpaArgs& a, int fmt, int64_t blocks, hipStream_t s
 }
 
 static bool aligned_to(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) % n) == 0; }
-
-static int compute_units_sdpa() {
-  static const int n = [] {
-    int dev = 0, cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
-      cu = 256;
-    return cu;
-  }();
-  return n;
-}
 
 }  // namespace mi355q
 

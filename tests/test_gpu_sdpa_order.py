@@ -20,6 +20,8 @@ pytestmark = pytest.mark.gpu
     (88, 22, 385, 385, 128),       # all resident, every second round backwards, shared K and V
     (16, 4, 2100, 2100, 256),      # 17 query blocks of 16 heads: one round more than the first
     (544, 136, 300, 300, 64),      # more workgroups than are resident
+    (144, 36, 1000, 1000, 64),     # five per CU, resident: every second round backwards
+    (160, 160, 1000, 1000, 64),    # as many as are
     (136, 136, 130, 8192, 128),    # 17 heads per XCD in groups of 4, the last one of 1
     (24, 24, 1500, 1500, 72),      # rows through registers
 ])
