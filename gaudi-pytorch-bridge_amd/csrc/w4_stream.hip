@@ -17,8 +17,8 @@
 // arrives last also takes the shares of those that gave up.  Nobody waits longer than those looks.  (16 x 8192 x 28672 28.0 -> 26.7 us,
 // 16 x 14336 x 4096 in eight parts 18.6 -> 18.0.)
 //
-// Against w4a8_wide_kernel, us, weights cold: bf16 activations 16 x 8192 x 28672 33.3 -> 27.2, 16 x 14336 x 4096 22.7 -> 15.7, 8 x 4096 x
-// 4096 15.6 -> 10.0; fp8 29.7 -> 26.5, 19.5 -> 14.8, 13.2 -> 10.0.  What is left of the 27: 20 of loads, 3 for the parts' meeting, and the
+// Against w4a8_wide_kernel, us, weights cold: bf16 activations 16 x 8192 x 28672 33.3 -> 27.4, 16 x 14336 x 4096 22.7 -> 15.9, 8 x 4096 x
+// 4096 15.6 -> 10.2; fp8 29.7 -> 26.5, 19.5 -> 14.8, 13.2 -> 10.0.  What is left of the 27: 20 of loads, 3 for the parts' meeting, and the
 // first stage's way in and the last one's through the multiplying waves.
 #include <algorithm>
 
@@ -268,18 +268,15 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
     };
     using T = std::true_type;
     using F = std::false_type;
-    // Before the barrier of the last stage's rows: whether the sums are finite so far, and that stage's far from the end of the range.
-    const auto in_range = [&](auto bc) {
-      constexpr int B = decltype(bc)::value;
-      float so_far = 0.0f, most = 0.0f;  // so_far: or NaN
+    // Before the barrier of the last stage's rows: whether the sums of the stages before it are finite.  (The last fold rounds once: it
+    // leaves an infinity only where the part's sum is one.)
+    const auto in_range = [&] {
+      f32x4 v = zero;  // or NaN
 #pragma unroll
       for (int t = 0; t < kW4StTiles; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          so_far = __builtin_fmaf(total[t][e], 0.0f, so_far);
-          most = __builtin_fmaxf(most, __builtin_fabsf(acc[B][t][e]));
-        }
-      if (!(so_far == 0.0f && most < 0x1p80f)) again = 1;
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(total[t][e], 0.0f, v[e]);
+      if (!((v[0] + v[1]) + (v[2] + v[3]) == 0.0f)) again = 1;
     };
     f32x4 first[A16 ? kW4StTiles : 1];
     do {
@@ -298,10 +295,7 @@ __global__ __launch_bounds__(kW4StThreads, 1) void w4_stream_kernel(W4Args a, in
         stage(std::integral_constant<int, 0>{}, T{});
       }
       if (kt < KT) stage(std::integral_constant<int, 1>{}, T{});
-      if constexpr (A16) {
-        if (KT & 1) in_range(std::integral_constant<int, 0>{});
-        else in_range(std::integral_constant<int, 1>{});
-      }
+      if constexpr (A16) in_range();
       __syncthreads();  // the fp32 rows of the last stage
       if (KT & 1) fold(std::integral_constant<int, 0>{});
       else fold(std::integral_constant<int, 1>{});
