@@ -976,7 +976,8 @@ Tensor w4a8_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, con
 
 // mi355q::w4a16_gemm: the same weights against bf16 activations (what the reference gets from
 // convert_from_[u]int4 to bf16 followed by a bf16 matmul, hpu_ops/backend/int4_ops.cpp:40-56), without the
-// bf16 [K, N] matrix: the activations go through the matrix unit as two fp8 planes (mi355q_w4a16_gemm).
+// bf16 [K, N] matrix: up to 16 rows the nibbles are widened to bf16, above that the activations go through the matrix unit as
+// two fp8 planes (mi355q_w4a16_gemm).
 Tensor w4a16_gemm(const Tensor& A, const Tensor& packed, const Tensor& scale, const c10::optional<Tensor>& zero_point,
                   bool is_signed, at::ScalarType out_dtype, const c10::optional<Tensor>& bias) {
   TORCH_CHECK(A.scalar_type() == at::kBFloat16, "mi355q::w4a16_gemm A must be bfloat16, got ", A.scalar_type());

@@ -18,7 +18,7 @@ struct W4Args {
   // wide and stream kernels: K is walked in `ksplit` parts by as many workgroups per strip
   int ksplit;
   uint32_t* tickets;       // one per strip, zero between launches
-  float* partials;         // [ksplit][strips] partial sums of 32 x 256, in the consumers' register order
+  float* partials;         // partial sums [ksplit][strips], in the consumers' register order: the wide kernel's tiles of its rows x 256, the stream kernel's 16 x 512
   int ticket_stride;       // stream kernel: 32-bit words between the counters
   // 16-bit activations as two fp8 planes (wide kernel, A16): g.A holds the leading part of every value and a_lo,
   // with the same pitch, 16 times what is left of it (split_rows_kernel); a = (A + a_lo / 16) / row scale

@@ -414,11 +414,12 @@ int mi355q_softmax_fp8(const void* x, int x_dtype, int64_t rows, int64_t cols,
  * bf16 (Int4BaseOp::AddNode, hpu_ops/backend/int4_ops.cpp:40-56: nibble order, (q - z) * s, the
  * group layout of its test, tests/pytest_working/any_mode/test_hpu_convert_from_int4.py:398-476)
  * and a bf16 matmul; here the bf16 [K, N] matrix never exists.  Up to 16 rows the product runs in bf16, to
- * which the nibbles are expanded, exactly, in registers.  Above that the activations are first cut into
+ * which the nibbles are expanded, exactly, in registers (fp32 results 1e-7 from the exact ones, 2-norm).  Above that, with a
+ * pitch of A or of the weights above 4 Mi elements, and with split_k = 0 where K would go in parts, the activations are first cut into
  * two e4m3fn planes per row (mi355q_split_rows_fp8x2: a * s = hi + lo / 16 with a power-of-two row
  * scale s, exact for every element within a factor 2^15 of the row's largest and to 3e-8 of that
  * largest otherwise), and both planes meet the packed nibbles in the matrix unit as in
- * mi355q_w4a8_gemm, so the integers (q - z) and the products enter the fp32 sums exactly.
+ * mi355q_w4a8_gemm (1e-5 to 5e-5 from the exact results: the matrix unit rounds inside a product).
  * Serves groups of 128 with bf16 scales, N a multiple of 32 and K of 16 (MI355Q_ERR_UNSUPPORTED
  * otherwise).  `workspace`: mi355q_w4a16_gemm_workspace_bytes(...) bytes of device memory, 16-byte
  * aligned, for the planes, the row scales and, in front, the arrival counters and partial sums of
