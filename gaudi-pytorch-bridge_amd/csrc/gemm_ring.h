@@ -396,6 +396,8 @@ struct RingProducer {
 // RingLoader for an operand whose rows begin anywhere: its chunks go through registers, 16 bytes per lane from any address, and are
 // stored in the places of LDS that the other loader's DMA would give them.  Only the last stage of K has chunks that are partly, or not at
 // all, inside the operand: fetch_edge() takes those from its last 16 bytes, and trim_edge() shifts them and clears what lies past K.
+// (Before it rows and columns past the edge read others, and the last chunk of a row of an operand that is not K-major reads up to 15 bytes into
+// the next row: there is one, of 16 bytes at least and 16 bytes on at least.)
 template <bool KMAJOR, int EXT>
 struct RaggedLoader {
   using G = typename RingLoader<KMAJOR, EXT>::G;
